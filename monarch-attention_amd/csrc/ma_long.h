@@ -8,8 +8,9 @@
 //  * longer ones loop over their strips, with the next strip's rows loaded ahead, in as many waves as registers and LDS allow
 //    (Cfg below).  Their logits are packed to 16 bits as they leave the first product (they are rounded to the operand type
 //    there anyway) and the probabilities take their place: half the accumulator registers; probabilities enter the second
-//    product unnormalised (at most 1) and its result is divided by their sum - the same relative rounding, one
-//    multiplication per entry less -, the exponent is one FMA from the packed logit;
+//    product unnormalised, relative to the largest of their row (at most 1, at least as large as the normalised ones), and
+//    its result is divided by their sum - the same relative rounding, one multiplication per entry less -, the exponent is
+//    one FMA from the packed logit;
 //  * head dims of 81 .. 96 have a column class of their own.
 // Measured before (the kernels of ma_mfma.h) -> after, one launch: 32 heads of 16384, D = 96, 160-row blocks: R step 158 ->
 // 94 us (with V 221 -> 156); 16 heads of 32768, D = 128, 181 rows: L step 259 -> 164, R with V 236 -> 192; 48 heads of
@@ -506,7 +507,15 @@ __global__ __launch_bounds__(64 * W, EU) void r_step_long(Problem P, int first) 
             // (rounding is monotonic: the largest rounded logit is the largest logit, rounded)
             mx = fmaxf(mx, fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3])));
         });
-        mx = fmaxf(round_to<T>(mfma::quad_rows_max(mx)) * cj, P.eps * kLog2e);   // clamped row maximum (ma_torch.py:15)
+        // The row maximum is clamped from below (ma_torch.py:15), so a row whose logits are all negative has probabilities far
+        // below 1, which 16 bits would not hold (fp16: two bits at a maximum of -15, zero below -17).  So p is formed from
+        // the row's own maximum and `shift` octaves are put back per row, in fp32.  60 octaves are enough (eps, at -40, rules
+        // the sum long before) and keep the rows of fully masked blocks at 0.  (A few
+        // instructions a row: 48 heads of 65536 tokens, D = 64, 256 rows, one step: 996.2 us without, 996.3 with.)
+        mx = round_to<T>(mfma::quad_rows_max(mx)) * cj;
+        const float clamped = fmaxf(mx, P.eps * kLog2e);
+        mx = fmaxf(mx, clamped - 60.f);
+        const float shift = mx - clamped, scale = __builtin_amdgcn_exp2f(shift);
         float sum = 0.f, ent = 0.f;
         auto softmax = [&](auto has_mask) {
             constexpr bool kMasked = decltype(has_mask)::value;
@@ -529,10 +538,10 @@ __global__ __launch_bounds__(64 * W, EU) void r_step_long(Problem P, int first) 
         else softmax(std::false_type{});
         sum = mfma::quad_rows_sum(sum);
         ent = mfma::quad_rows_sum(ent);
-        const float den = sum + P.eps, inv = mfma::rcp(den);
+        const float den = fmaf(scale, sum, P.eps), inv = scale * mfma::rcp(den);
         const unsigned lrow = static_cast<unsigned>(j * M + k);   // row of aL / cL / Y: (j, k)
-        if (q == 0)   // cL = sum_i r log r with r = p / den (ma_torch.py:20)
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, kLn2 * (ent * inv - mfma::log2_normal(den) * (sum * inv))),
+        if (q == 0)   // cL = sum_i r log r with r = p scale / den (ma_torch.py:20)
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, kLn2 * (ent * inv + (shift - mfma::log2_normal(den)) * (sum * inv))),
                                                   state_slice(P.cL, eh, np, 4), j < B ? lrow * 4u : kOob, 0, 0);
         f32x4 O[DT];
         gemm2<T, DT, NWT>(O, Kt, C, r, q);

@@ -12,7 +12,7 @@ import torch
 
 from helpers import (DT, assert_parity, block_safe_mask, err_metrics, golden_names, load_golden, seeded_qkv)
 from ma import _hip_lib as L
-from ma.ma_hip import make_params, monarch_attention_hip, monarch_matrix_hip, sync_status
+from ma.ma_hip import make_params, monarch_attention_hip, monarch_attention_hip_backward, monarch_matrix_hip, sync_status
 from ma.monarch_attention import MonarchAttention, PadType
 from oracle.ma_oracle import OracleTrace, monarch_attention_oracle, monarch_matrix_oracle
 
@@ -938,3 +938,36 @@ def test_long_stages_at_strip_edges(i, B, M, heads, dt):
         ref = monarch_attention_oracle(q, k, v, mask, T, B, pre, upcast=True)
         out = monarch_attention_hip(*(t.to(DEV) for t in (q, k, v)), None if mask is None else mask.to(DEV), T, B, pre, variant="staged")
         assert_parity(out.cpu(), ref, dt)
+
+
+@pytest.mark.parametrize("kind", ["plain", "mask", "dead_block", "one_key"])
+@pytest.mark.parametrize("B", [129, 181, 192, 256])
+def test_rows_of_negative_logits_in_long_blocks(B, kind):
+    """fp16 logits around -10, -15 and -20: the row maximum is clamped at eps before it is subtracted (ma/ma_torch.py:15), so
+    the exponentials are far below what 16 bits resolve while the normalised probabilities are ordinary numbers.  A mask, a
+    block without a live key and a block with one (at -20 the empty block outweighs the others in the reference as well).
+
+    Against the oracle in fp32.  Bound: logits of up to 32 before their softmax are rounded to 16 bits, by 2^-7 at most, and
+    three such roundings (S, aR, U) lie one behind the other: sqrt(3) 2^-7 / sqrt(3) = 7.8e-3 root mean square."""
+    E, H, M, D = 1, 2, 3, 64
+    N = B * M - 5
+    mask = None if kind == "plain" else block_safe_mask(E, N, B, seed=B)
+    if mask is not None:
+        mask[:, :B] = True   # (every position keeps a query)
+        if kind != "mask":
+            mask[:, B:2 * B] = False
+        if kind == "one_key":
+            mask[:, B + 77] = True
+    for i, offset in enumerate((10.0, 15.0, 20.0) if kind in ("plain", "mask") else (10.0, 15.0)):
+        q, k, v = seeded_qkv(E, H, N, D, torch.float32, seed=B + i)
+        common = (offset / D ** 0.5) ** 0.5 * (1 - 2 * (torch.arange(D) % 2))   # q.k / sqrt(D): -offset on top
+        q, k, v = (t.half() for t in (q + common, k - common, v))
+        w = torch.randn(v.shape, generator=torch.Generator().manual_seed(B)).half()
+        for T in (1, 2):
+            leaves = [t.float().requires_grad_() for t in (q, k, v)]
+            ref = monarch_attention_oracle(*leaves, mask, T, B, False)
+            ref.backward(w.float())
+            dev = to_dev(q, k, v, mask, w)
+            got = [monarch_attention_hip(*dev[:4], T, B, False, variant="staged"), *monarch_attention_hip_backward(*dev, T, B, False)]
+            for name, x, r in zip(("out", "dq", "dk", "dv"), got, [ref] + [t.grad for t in leaves]):
+                assert err_metrics(x, r)["rel_fro"] <= 1e-2, (name, offset, T)
