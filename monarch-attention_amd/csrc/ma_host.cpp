@@ -13,6 +13,7 @@
 
 #include <dlfcn.h>
 
+#include <initializer_list>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -21,6 +22,7 @@
 
 #include <ATen/ATen.h>
 #include <ATen/DeviceGuard.h>
+#include <c10/core/AutogradState.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
@@ -154,6 +156,14 @@ bool valid(const Call& c) {
             mask_code(c.mask.scalar_type()) < 0)
             return false;
     return true;
+}
+
+// Forward-mode AD: the operator has no jvp, and a result without a tangent would pass for a zero derivative.
+void refuse_tangents(std::initializer_list<const Tensor*> tensors) {
+    if (!c10::AutogradState::get_tls_state().get_fw_grad_mode()) return;
+    for (const Tensor* t : tensors)
+        TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(/*level=*/0).defined(),
+                                    "monarch_attention_hip has no forward-mode derivative (jvp): q, k, v and the output gradient must not be dual tensors");
 }
 
 // The library wants unit stride along the last dimension and token rows that do not overlap; batch and head dimensions
@@ -310,6 +320,7 @@ struct MonarchAttentionHipBackward : public torch::autograd::Node {
         std::lock_guard<std::mutex> lock(mutex_);
         torch::autograd::variable_list out(3);
         if (!grads[0].defined()) return out;
+        refuse_tangents({&grads[0]});
         Call c = call;
         c.q = q.unpack();
         c.k = k.unpack();
@@ -388,9 +399,9 @@ bool tensor_or_none(PyObject* o, Tensor* t) { return o == Py_None || tensor(o, t
 PyObject* py_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Call c;
-    if (n != 9 || !tensor(args[0], &c.q) || !tensor(args[1], &c.k) || !tensor(args[2], &c.v) || !tensor_or_none(args[3], &c.mask) ||
-        !scalars(args + 4, &c) || !valid(c))
-        Py_RETURN_NONE;
+    if (n != 9 || !tensor(args[0], &c.q) || !tensor(args[1], &c.k) || !tensor(args[2], &c.v)) Py_RETURN_NONE;
+    refuse_tangents({&c.q, &c.k, &c.v});
+    if (!tensor_or_none(args[3], &c.mask) || !scalars(args + 4, &c) || !valid(c)) Py_RETURN_NONE;
     const bool record = c10::GradMode::is_enabled() && (c.q.requires_grad() || c.k.requires_grad() || c.v.requires_grad());
     return THPVariable_Wrap(record ? run_recorded(c) : run_forward(c, nullptr));
     END_HANDLE_TH_ERRORS

@@ -175,7 +175,8 @@ def monarch_attention_hip(q: Tensor, k: Tensor, v: Tensor, attn_mask: Tensor | N
     contiguous v; backed by ``(E, N, H, Dv)`` when v is such a permuted view).
     Differentiable with respect to q, k and v: when one of them requires grad
     (and grad mode is on) the call is recorded as one autograd node that keeps
-    the states of the steps and whose backward is ``ma_bwd_kept``.
+    the states of the steps and whose backward is ``ma_bwd_kept``.  There is no
+    forward-mode derivative: dual tensors raise ``NotImplementedError``.
 
     The one-launch kernels wait for each other's workgroups with bounded waits:
     a call whose wait ran out is reported by a RuntimeError from the first later

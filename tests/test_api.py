@@ -92,3 +92,22 @@ def test_argument_validation(mutate, exc):
     mutate(a)
     with pytest.raises(exc):
         monarch_attention_hip(a["q"], a["k"], a["v"], a["mask"], a["T"], a["B"], False)
+
+
+@pytest.mark.parametrize("requires_grad", [False, True])
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_forward_mode_derivatives_are_refused_not_dropped(which, requires_grad):
+    """There is no jvp: a result without a tangent would pass for a zero derivative."""
+    import torch.autograd.forward_ad as fwd
+
+    args = [t.requires_grad_(requires_grad) for t in _qkv(torch.float32)]
+    with fwd.dual_level():
+        args[which] = fwd.make_dual(args[which], torch.ones_like(args[which]))
+        with pytest.raises(NotImplementedError, match="forward-mode"):
+            monarch_attention_hip(*args, None, 1, 4, False)
+        with fwd._set_fwd_grad_enabled(False), pytest.raises(ValueError, match="GPU"):   # tangents are not wanted
+            monarch_attention_hip(*args, None, 1, 4, False)
+    args = list(_qkv(torch.float32))
+    with pytest.raises(NotImplementedError, match="forward-mode"):
+        torch.func.jvp(lambda x: monarch_attention_hip(*args[:which], x, *args[which + 1:], None, 1, 4, False),
+                       (args[which],), (torch.ones_like(args[which]),))
