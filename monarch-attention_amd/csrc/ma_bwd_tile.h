@@ -85,9 +85,13 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
     auto v_off = [&](int i) { return i < B ? mfma::tok_off(t0 + i, P.N, vst) : kOob; };
     auto x_off = [&](int j) { return j >= B ? kOob : first ? mfma::tok_off(t0 + j, P.N, qst) : static_cast<unsigned>(k * B + j) * row_b; };
     auto g_off = [&](int j) { return j < B ? static_cast<unsigned>(j * M + k) * row_b : kOob; };
-    auto cj_of = [&](int j) {   // 1 / (cR + eps)
-        const float c = first ? 1.f : mfma::bloadf<0>(scR, j < B ? static_cast<unsigned>(k * B + j) * 4u : kOob);
-        return 1.0f / ((j < B ? c : 1.f) + P.eps);
+    auto cr_of = [&](int j) { return first ? 1.f : mfma::bloadf<0>(scR, j < B ? static_cast<unsigned>(k * B + j) * 4u : kOob); };
+    // 1 / (cR + eps).  A row with cR = 0 (its position's queries are all masked) has aR = 0 too, so its logits are 0 whatever
+    // the factor is, and neither its dDot, which multiplies aR, nor its gaR, which L = 0 multiplies, reaches a gradient: the
+    // factor 0 stands for 1 / eps there, whose products would leave the range of fp16 and come back as 0 * inf.
+    auto over_cr = [&](float c) {
+        const float f = mfma::fp32_value(1.0f / (c + P.eps));   // (a value of its own: no branch around the division)
+        return c == 0.f ? 0.f : f;
     };
     auto gcl_of = [&](int j) { return mfma::bloadf<0>(sgcL, j < B ? static_cast<unsigned>(j * M + k) * 4u : kOob); };
     auto key_ok = [&](int i) { return i < B && token_ok(P, e, t0 + i); };
@@ -107,7 +111,7 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
         T* Vt = tiles + 16 * CT1 * MT::LD;
         typename MT::Row xb, ga, gy;
         f32x4 S[NWT], Gg[NWT], O[DT];
-        float cj, gcl;
+        float cr, cj, gcl;
         for (int c = 0; c < PL::NC1; ++c) {   // (one chunk but for the largest fp32 problems)
             TileIn<MT, T, 16 * CT1, NTH> kc, vc;
             kc.issue(sk, D, wide, [&](int i) { return k_off(16 * CT1 * c + i); });
@@ -116,7 +120,7 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
                 MT::load(xb, sx, x_off(own), D, wide, q);
                 MT::load(ga, sga, g_off(own), D, wide, q);
                 if (with_v) MT::load(gy, sgy, g_off(own), D, wide, q);
-                cj = cj_of(own);
+                cr = cr_of(own);
                 gcl = gcl_of(own);
                 for (int i = threadIdx.x; i < ROWS; i += NTH) kok[i] = key_ok(i) ? 1.f : 0.f;
                 MT::scale(ga, sm);
@@ -126,6 +130,7 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
             kc.commit(Kt);
             if (with_v) vc.commit(Vt);
             __syncthreads();
+            if (c == 0) cj = over_cr(cr);   // (not where it is loaded: the tiles would wait for it)
 #pragma unroll
             for (int w = 0; w < CT1; ++w) {
                 f32x4 a = {0.f, 0.f, 0.f, 0.f}, g = {0.f, 0.f, 0.f, 0.f};
@@ -224,15 +229,6 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
         }
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) O[dt] += dq0[dt];
-        if constexpr (std::is_same<T, f16>::value) {
-            // the row of a position whose queries are all masked has cR = 0, a factor 1 / eps here and the factor 0 in the
-            // L stage: it stays finite
-            if (!first)
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) O[dt][v] = __builtin_amdgcn_fmed3f(O[dt][v], -65504.f, 65504.f);
-        }
         if (first) MT::store(token_slice<T>(G.out[0], G.outs[0], e, h, P.N, D),
                              own_in ? mfma::tok_off(own_t, P.N, static_cast<unsigned>(G.outs[0][2]) * sizeof(T)) : kOob, D, O, q, wide);
         else MT::store(state_slice(G.gaR, eh, np, row_b), own_in ? static_cast<unsigned>(k * B + own) * row_b : kOob, D, O, q, D % 8 == 0);
@@ -271,7 +267,7 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
                 if (with_v) yc.issue(sgy, D, wide, [&](int j) { return g_off(16 * CT2 * c + j); });
                 if (c == 0) {
                     for (int j = threadIdx.x; j < ROWS; j += NTH) {
-                        cjs[j] = cj_of(j);
+                        cjs[j] = over_cr(cr_of(j));
                         gcls[j] = gcl_of(j);
                         f32x4 s = {0.f, 0.f, 0.f, 0.f};
                         if (j < B) s = *reinterpret_cast<const f32x4*>(G.stat + 4 * (eh * np + k * B + j));
