@@ -7,13 +7,13 @@
 // its products contract over three different indices and a lane can feed a B operand only from accumulators whose ROWS
 // are the contraction index:
 //
-//   R, pass 1, strip of query rows j (accumulator rows = keys i): S = X K^T, Gg = Ga K^T + Gy V^T -> r, g, dDot;
+//   R, pass 1, strip of query rows j (accumulator rows = keys i): S = X K^T, Gg = Ga K^T + Gy V^T -> r, g, dDot  (Ga = sm gaL);
 //      gaR[j] = sum_i dDot[j,i] K[i], gcR[j]; the row statistics (max, 1 / sum, sum_i g r).
 //   R, pass 2, strip of keys i (accumulator rows = query rows j): r and dDot again from the statistics;
 //      dK[i] (+)= sum_j r[j,i] Ga[j] + dDot[j,i] X[j],  dV[i] = sum_j r[j,i] Gy[j].
 //   L / Z, pass 1, strip of query blocks l (accumulator rows = key blocks k): U, g -> p, dU;
 //      dq[(l,j)] (+)= sum_k dU[l,k] aL[j,k]  (L: + round(mask_q p)[l,k] gaR[k,j]); the row statistics.
-//   L / Z, pass 2, strip of key blocks k: gaL[j,k] = sum_l dU[l,k] Q[l], gcL[j,k] = -sum_l dU[l,k],
+//   L / Z, pass 2, strip of key blocks k: Ga[j,k] = sm sum_l dU[l,k] Q[l], gcL[j,k] = -sum_l dU[l,k],
 //      Z: gY[j,k] = sum_l round(p)[l,k] dout[l].
 //
 // The second evaluation of the logits costs matrix instructions that are otherwise idle; it saves the n x n matrices.
@@ -123,7 +123,6 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
                 cr = cr_of(own);
                 gcl = gcl_of(own);
                 for (int i = threadIdx.x; i < ROWS; i += NTH) kok[i] = key_ok(i) ? 1.f : 0.f;
-                MT::scale(ga, sm);
             } else {
                 __syncthreads();
             }
@@ -280,7 +279,7 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
                     __syncthreads();
                 }
                 xc.commit(Xt);
-                ac.commit(Gat, sm);
+                ac.commit(Gat);
                 if (with_v) yc.commit(Gyt);
             }
             __syncthreads();
@@ -591,6 +590,10 @@ __global__ __launch_bounds__(64 * W) void lz_bwd_tile(Problem P, BwdBuffers G) {
         }
         gcl = quad_rows_sum(gcl);
         if (q == 0 && own_in) G.gcL[eh * np + jm + own] = gcl;   // gcL[j,k] = -sum_l dU
+        // sm gaL is what the R stage multiplies with.  gaL, gY and gaR are matrix operands wherever they are read, so they are
+        // rounded to the operand type once: here, where the sum is complete in fp32.
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) Oa[dt] *= P.sm_scale;
         MT::store(state_slice(G.gaL, eh, np, row_b), a_off(own), D, Oa, q, wide_s);
         if (kZ) MT::store(state_slice(G.gY, eh, np, row_b), a_off(own), D, Oy, q, wide_s);
     }

@@ -143,7 +143,7 @@ struct BwdBuffers {
     int state16;   // gaL, gY, gaR hold the operand dtype instead of fp32 (see bwd_state16_ok)
     // tiled != 0: every stage runs a kernel of ma_bwd_tile.h (see bwd_tiled).  The stage that completes a gradient then
     // rounds it into the caller's tensor itself - dv in the R stage that forms it, dq and dk in the R stage of the first
-    // step -, gaL, gY, gaR hold the operand dtype, nothing has to be zeroed and no conversion kernel runs.  out = {dq, dk,
+    // step -, gaL (times sm_scale), gY, gaR hold the operand dtype, nothing has to be zeroed and no conversion kernel runs.  out = {dq, dk,
     // dv} of the caller, outs their element strides (e, h, token); rows16: every row of the caller's tensors starts on a
     // 16-byte boundary (else 8-byte ones, 16-bit operands only); stat: (E,H,Np) rows of four floats for the stages that
     // run as two launches.

@@ -39,19 +39,9 @@ struct Mat {   // 16-bit
         const u32x2 b = __builtin_amdgcn_raw_buffer_load_b64(s, c + 4 < D ? ro + 2 * c + 8 : kOob, 0, 0);
         return u32x4{a[0], a[1], b[0], b[1]};
     }
-    static __device__ __forceinline__ u32x4 scaled(u32x4 v, float f) {
-        V8 a = __builtin_bit_cast(V8, v);
-#pragma unroll
-        for (int u = 0; u < 8; ++u) a[u] = from_f<T>(f * to_f(a[u]));
-        return __builtin_bit_cast(u32x4, a);
-    }
     static __device__ __forceinline__ void load(Row& w, rsrc_t s, unsigned ro, int D, bool wide, int q) {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) w.x[ks] = __builtin_bit_cast(V8, piece(s, ro, 32 * ks + 8 * q, D, wide));
-    }
-    static __device__ __forceinline__ void scale(Row& w, float f) {
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) w.x[ks] = __builtin_bit_cast(V8, scaled(__builtin_bit_cast(u32x4, w.x[ks]), f));
     }
     static __device__ __forceinline__ void from_tile(Row& w, const T* tile, int row, int q) {
 #pragma unroll
@@ -133,21 +123,9 @@ struct Mat<float, DT> {   // fp32: k slot q of step (t, u) is column 16 t + 4 q 
     static __device__ __forceinline__ u32x4 piece(rsrc_t s, unsigned ro, int c, int D, bool) {
         return __builtin_amdgcn_raw_buffer_load_b128(s, c < D ? ro + 4 * c : kOob, 0, 0);
     }
-    static __device__ __forceinline__ u32x4 scaled(u32x4 v, float f) {
-        f32x4 a = __builtin_bit_cast(f32x4, v);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) a[u] *= f;
-        return __builtin_bit_cast(u32x4, a);
-    }
     static __device__ __forceinline__ void load(Row& w, rsrc_t s, unsigned ro, int D, bool, int q) {
 #pragma unroll
         for (int t = 0; t < DT; ++t) w.x[t] = __builtin_bit_cast(f32x4, piece(s, ro, 16 * t + 4 * q, D, true));
-    }
-    static __device__ __forceinline__ void scale(Row& w, float f) {
-#pragma unroll
-        for (int t = 0; t < DT; ++t)
-#pragma unroll
-            for (int u = 0; u < 4; ++u) w.x[t][u] *= f;
     }
     static __device__ __forceinline__ void from_tile(Row& w, const float* tile, int row, int q) {
 #pragma unroll
@@ -225,12 +203,12 @@ struct TileIn {
             v[i] = MT::piece(s, (ROWS * CH % NTH == 0 || c < ROWS * CH) ? off(row) : kOob, (c % CH) * MT::PIECE, D, wide);
         }
     }
-    __device__ __forceinline__ void commit(T* tile, float scale = 1.f) const {
+    __device__ __forceinline__ void commit(T* tile) const {
 #pragma unroll
         for (int i = 0; i < CNT; ++i) {
             const int c = static_cast<int>(threadIdx.x) + i * NTH;
             if (ROWS * CH % NTH != 0 && c >= ROWS * CH) continue;
-            *reinterpret_cast<u32x4*>(tile + MT::at(c / CH, c % CH)) = scale == 1.f ? v[i] : MT::scaled(v[i], scale);
+            *reinterpret_cast<u32x4*>(tile + MT::at(c / CH, c % CH)) = v[i];
         }
     }
 };
