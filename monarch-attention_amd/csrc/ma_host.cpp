@@ -300,9 +300,10 @@ Grads run_backward(const Call& c, const Tensor& dout_, const Tensor& state) {
 // One autograd node per operator call: forward ma_fwd_keep, backward ma_bwd_kept.  A forward variant that keeps no state
 // in memory (an explicit 'fused' or 'resident') runs as ma_fwd, and ma_bwd runs the steps again.
 struct MonarchAttentionHipBackward : public torch::autograd::Node {
-    torch::autograd::SavedVariable q, k, v, mask;
-    bool has_mask = false;
-    Tensor state;
+    // the state goes through saved-tensor hooks as the inputs do: checkpointing drops it, save_on_cpu moves it
+    torch::autograd::SavedVariable q, k, v, mask, state;
+    bool has_mask = false, has_state = false;
+    int64_t state_bytes = 0;
     Call call;   // without tensors
 
     std::string name() const override { return "MonarchAttentionHipBackward"; }
@@ -313,7 +314,7 @@ struct MonarchAttentionHipBackward : public torch::autograd::Node {
         k.reset_data();
         v.reset_data();
         mask.reset_data();
-        state.reset();
+        state.reset_data();
     }
 
     torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
@@ -326,10 +327,18 @@ struct MonarchAttentionHipBackward : public torch::autograd::Node {
         c.k = k.unpack();
         c.v = v.unpack();
         if (has_mask) c.mask = mask.unpack();
+        Tensor st;
+        if (has_state) st = state.unpack();
         Grads g;
         {
             const c10::AutoGradMode no_grad(false);
-            g = run_backward(c, grads[0], state);
+            if (has_state) {   // a hook may have put it anywhere
+                TORCH_CHECK(st.defined() && st.scalar_type() == at::kByte && st.numel() == state_bytes && st.device() == c.q.device(),
+                            "the kept state of monarch_attention_hip came back from its saved-tensor hooks as another tensor: expected ", state_bytes,
+                            " bytes (uint8) on ", c.q.device());
+                if (!st.is_contiguous() || reinterpret_cast<uintptr_t>(st.data_ptr()) % 256 != 0) st = st.clone(at::MemoryFormat::Contiguous);
+            }
+            g = run_backward(c, grads[0], st);
         }
         if (task_should_compute_output(0)) out[0] = std::move(g.dq);
         if (task_should_compute_output(1)) out[1] = std::move(g.dk);
@@ -348,16 +357,21 @@ Tensor run_recorded(const Call& c) {
     auto node = std::shared_ptr<MonarchAttentionHipBackward>(new MonarchAttentionHipBackward(), torch::autograd::deleteNode);
     node->set_next_edges(torch::autograd::collect_next_edges(c.q, c.k, c.v));
     const bool keeps = c.variant != MA_VARIANT_FUSED && c.variant != MA_VARIANT_RESIDENT;
-    Tensor out;
+    Tensor out, state;
     {
         const c10::AutoGradMode no_grad(false);
-        out = run_forward(c, keeps ? &node->state : nullptr);
+        out = run_forward(c, keeps ? &state : nullptr);
     }
     node->q = torch::autograd::SavedVariable(c.q, false);
     node->k = torch::autograd::SavedVariable(c.k, false);
     node->v = torch::autograd::SavedVariable(c.v, false);
     node->has_mask = c.mask.defined();
     if (node->has_mask) node->mask = torch::autograd::SavedVariable(c.mask, false);
+    node->has_state = keeps;
+    if (keeps) {
+        node->state_bytes = state.numel();
+        node->state = torch::autograd::SavedVariable(state, false);
+    }
     node->call.T = c.T;
     node->call.B = c.B;
     node->call.pre_pad = c.pre_pad;

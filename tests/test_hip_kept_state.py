@@ -40,3 +40,51 @@ def test_kept_states_give_the_gradients_of_a_recomputation(case):
     torch.autograd.grad(out, leaves, w)
     with pytest.raises(RuntimeError, match="second time"):
         torch.autograd.grad(out, leaves, w)
+
+
+def test_kept_state_goes_through_saved_tensor_hooks():
+    """Activation checkpointing keeps nothing of the operator's own, save_on_cpu moves the state with the inputs, and a hook
+    that returns it at another address or as a strided view is served; the gradients are the same bits."""
+    from torch.autograd.graph import save_on_cpu, saved_tensors_hooks
+    from torch.utils.checkpoint import checkpoint
+
+    E, H, N, D, B, T = 2, 4, 500, 64, 32, 2
+    leaves = [t.to(DEV).requires_grad_() for t in seeded_qkv(E, H, N, D, torch.float16)]
+    mask = block_safe_mask(E, N, B).to(DEV)
+    w = torch.randn(E, H, N, D, generator=torch.Generator().manual_seed(1)).to(DEV).half()
+
+    def op(*x):
+        return monarch_attention_hip(*x, mask, T, B, False)
+
+    want = torch.autograd.grad(op(*leaves), leaves, w)
+    seen = []
+
+    def spread(t):   # every second byte of a larger buffer, one byte off
+        seen.append(t.numel() * t.element_size())
+        if t.dtype != torch.uint8:
+            return t
+        buf = torch.zeros(2 * t.numel() + 1, dtype=t.dtype, device=t.device)[1::2]
+        return buf.copy_(t)
+
+    with saved_tensors_hooks(spread, lambda t: t):
+        out = op(*leaves)
+    assert len(seen) == 5 and max(seen) > 4 * w.numel() * 2   # q, k, v, mask; 2 aL, aR, Y and the column sums
+    for a, b in zip(torch.autograd.grad(out, leaves, w), want):
+        assert torch.equal(a, b)
+    with save_on_cpu():
+        out = op(*leaves)
+    for a, b in zip(torch.autograd.grad(out, leaves, w), want):
+        assert torch.equal(a, b)
+
+    op(*leaves)   # (the workspace is there)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    out = checkpoint(op, *leaves, use_reentrant=False)
+    assert torch.cuda.memory_allocated() - before <= 2 * w.numel() * 2   # the output
+    for a, b in zip(torch.autograd.grad(out, leaves, w), want):
+        assert torch.equal(a, b)
+
+    with saved_tensors_hooks(lambda t: t[:-1] if t.dtype == torch.uint8 else t, lambda t: t):
+        out = op(*leaves)
+    with pytest.raises(RuntimeError, match="saved-tensor hooks"):
+        torch.autograd.grad(out, leaves, w)
