@@ -353,10 +353,12 @@ struct MonarchAttentionHipBackward : public torch::autograd::Node {
     }
 };
 
-Tensor run_recorded(const Call& c) {
+// keep: keep the state of the steps (the forward runs as a variant that has it in memory); else ma_fwd, and the backward
+// runs the steps again.
+Tensor run_recorded(const Call& c, bool keep) {
     auto node = std::shared_ptr<MonarchAttentionHipBackward>(new MonarchAttentionHipBackward(), torch::autograd::deleteNode);
     node->set_next_edges(torch::autograd::collect_next_edges(c.q, c.k, c.v));
-    const bool keeps = c.variant != MA_VARIANT_FUSED && c.variant != MA_VARIANT_RESIDENT;
+    const bool keeps = keep && c.variant != MA_VARIANT_FUSED && c.variant != MA_VARIANT_RESIDENT;
     Tensor out, state;
     {
         const c10::AutoGradMode no_grad(false);
@@ -409,15 +411,17 @@ bool tensor(PyObject* o, Tensor* t) {
 
 bool tensor_or_none(PyObject* o, Tensor* t) { return o == Py_None || tensor(o, t); }
 
-// forward(q, k, v, mask, T, B, pre_pad, variant, flags) -> Tensor, or None for arguments the operator does not take
+// forward(q, k, v, mask, T, B, pre_pad, variant, flags, keep_state) -> Tensor, or None for arguments the operator does not take
 PyObject* py_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Call c;
-    if (n != 9 || !tensor(args[0], &c.q) || !tensor(args[1], &c.k) || !tensor(args[2], &c.v)) Py_RETURN_NONE;
+    if (n != 10 || !tensor(args[0], &c.q) || !tensor(args[1], &c.k) || !tensor(args[2], &c.v)) Py_RETURN_NONE;
     refuse_tangents({&c.q, &c.k, &c.v});
     if (!tensor_or_none(args[3], &c.mask) || !scalars(args + 4, &c) || !valid(c)) Py_RETURN_NONE;
     const bool record = c10::GradMode::is_enabled() && (c.q.requires_grad() || c.k.requires_grad() || c.v.requires_grad());
-    return THPVariable_Wrap(record ? run_recorded(c) : run_forward(c, nullptr));
+    const int keep = PyObject_IsTrue(args[9]);
+    if (keep < 0) throw python_error();
+    return THPVariable_Wrap(record ? run_recorded(c, keep != 0) : run_forward(c, nullptr));
     END_HANDLE_TH_ERRORS
 }
 

@@ -169,19 +169,25 @@ def _refused(q, k, v, attn_mask, T, B):
 
 
 def monarch_attention_hip(q: Tensor, k: Tensor, v: Tensor, attn_mask: Tensor | None, T: int, B: int,
-                          pre_pad: bool, *, variant: str | None = None) -> Tensor:
+                          pre_pad: bool, *, variant: str | None = None, keep_state: bool = True) -> Tensor:
     """MonarchAttention forward on the current HIP stream; returns a new
     ``(E, H, N, Dv)`` tensor of ``v.dtype`` in v's memory layout (contiguous for
     contiguous v; backed by ``(E, N, H, Dv)`` when v is such a permuted view).
     Differentiable with respect to q, k and v: when one of them requires grad
     (and grad mode is on) the call is recorded as one autograd node that keeps
-    the states of the steps and whose backward is ``ma_bwd_kept``.  There is no
-    forward-mode derivative: dual tensors raise ``NotImplementedError``.
+    the states of the steps and whose backward is ``ma_bwd_kept``.  The states
+    are saved tensors like q, k and v (2T - 1 of q's size and one of v's).
+    ``keep_state=False`` keeps none of them: the forward then runs as an
+    unrecorded call does, the LDS-resident kernels included, and the backward
+    runs the steps again - for callers who need the memory, or who leave grad
+    mode on where no backward follows.  (A module takes it as an implementation:
+    ``register_impl("hip_lean", functools.partial(monarch_attention_hip,
+    keep_state=False))``.)  There is no forward-mode derivative: dual tensors raise ``NotImplementedError``.
 
     The one-launch kernels wait for each other's workgroups with bounded waits:
     a call whose wait ran out is reported by a RuntimeError from the first later
     call on the same stream that finds its error word set."""
-    out = _HOST.forward(q, k, v, attn_mask, T, B, pre_pad, _variant_code(variant), _flags())
+    out = _HOST.forward(q, k, v, attn_mask, T, B, pre_pad, _variant_code(variant), _flags(), keep_state)
     if out is None:
         _refused(q, k, v, attn_mask, T, B)
     return out

@@ -88,3 +88,20 @@ def test_kept_state_goes_through_saved_tensor_hooks():
         out = op(*leaves)
     with pytest.raises(RuntimeError, match="saved-tensor hooks"):
         torch.autograd.grad(out, leaves, w)
+
+
+@pytest.mark.parametrize("E,H,N,D,B,dt", [(16, 12, 512, 64, 32, "bf16"), (64, 12, 197, 64, 14, "f16"), (8, 8, 197, 64, 16, "f32")])
+def test_a_recorded_call_that_keeps_no_state_runs_as_an_unrecorded_one(E, H, N, D, B, dt):
+    """AUTO resolves these to the resident kernels, which keep no state in memory."""
+    leaves = [t.to(DEV).requires_grad_() for t in seeded_qkv(E, H, N, D, DT[dt])]
+    w = torch.ones_like(leaves[2])
+    with torch.no_grad():
+        plain = monarch_attention_hip(*leaves, None, 2, B, False)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    out = monarch_attention_hip(*leaves, None, 2, B, False, keep_state=False)
+    assert torch.cuda.memory_allocated() - before <= w.numel() * w.element_size() + 512
+    assert torch.equal(out.detach(), plain)
+    want = monarch_attention_hip_backward(*leaves, None, w, 2, B, False)
+    for a, b in zip(torch.autograd.grad(out, leaves, w), want):
+        assert torch.equal(a, b)
