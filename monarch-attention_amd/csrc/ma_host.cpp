@@ -19,6 +19,7 @@
 #include <mutex>
 #include <string>
 #include <utility>
+#include <vector>
 
 #include <ATen/ATen.h>
 #include <ATen/DeviceGuard.h>
@@ -70,36 +71,31 @@ void check(int status, const char* what) {
 // so they can share it).  Allocated zero-filled; every forward call leaves the sync area ready for the next one
 // (MA_FLAG_SYNC_READY).  A one-launch kernel whose bounded wait runs out stores the code of the error into a word of
 // pinned host memory, and EVERY call on the workspace looks at that word first (a plain host read).
+// Calls run without the GIL.  `lock` is held over a call's launches: those of two threads on one stream must not
+// interleave, they share the state arrays.
 struct Workspace {
+    std::mutex lock;
     Tensor buf, err_host;
     volatile int32_t* err = nullptr;
     bool dirty = false;   // a failed call: the sync area must be cleared before the next one
+
     void resize(c10::Device device, uint64_t nbytes) {
         // calls on this stream that still use the old buffer are ahead of everything queued from here on, and the
         // caching allocator hands a freed block to other streams only after that work is done
         buf = at::zeros({static_cast<int64_t>(std::max<uint64_t>(nbytes, 1u << 20))}, at::TensorOptions().dtype(at::kByte).device(device));
     }
-};
-std::mutex g_mutex;
-std::map<std::pair<int, void*>, std::shared_ptr<Workspace>> g_workspaces;
-
-std::shared_ptr<Workspace> workspace_for(c10::Device device, void* stream, uint64_t nbytes) {
-    std::lock_guard<std::mutex> lock(g_mutex);
-    auto& w = g_workspaces[{device.index(), stream}];
-    if (!w) {
-        auto fresh = std::make_shared<Workspace>();
-        fresh->resize(device, nbytes);
-        fresh->err_host = at::zeros({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-        fresh->err = fresh->err_host.data_ptr<int32_t>();
-        w = std::move(fresh);
-    } else if (static_cast<uint64_t>(w->buf.numel()) < nbytes) {
-        w->resize(device, nbytes);
-    }
-    if (*w->err != 0) {   // an earlier call on this workspace failed
-        const int code = *w->err;
-        *w->err = 0;
-        w->dirty = true;
-        w->buf.slice(0, 4, 8).zero_();   // the word in the workspace is sticky: clear it for the calls to come
+    // lock held: the buffer has nbytes, and no earlier call on it failed
+    void ready(c10::Device device, uint64_t nbytes) {
+        if (err == nullptr) {
+            err_host = at::zeros({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+            err = err_host.data_ptr<int32_t>();
+        }
+        if (!buf.defined() || static_cast<uint64_t>(buf.numel()) < nbytes) resize(device, nbytes);
+        if (*err == 0) return;
+        const int code = *err;
+        *err = 0;
+        dirty = true;
+        buf.slice(0, 4, 8).zero_();   // the word in the workspace is sticky: clear it for the calls to come
         const std::string why = code == 1 ? "a bounded wait between workgroups ran out"
                                 : code == 2 ? "workgroups of one head ran on different XCDs (the one-launch kernels rely on ids x, x + 8, ... "
                                               "sharing an XCD)"
@@ -107,8 +103,23 @@ std::shared_ptr<Workspace> workspace_for(c10::Device device, void* stream, uint6
         TORCH_CHECK(false, "monarch_attention_hip: an earlier forward call on this stream failed: ", why,
                     "; its output holds NaN rows.  The workspace has been reset; pass variant='staged' to avoid the one-launch kernels");
     }
+};
+std::mutex g_mutex;   // the map
+std::map<std::pair<int, void*>, std::shared_ptr<Workspace>> g_workspaces;
+
+std::shared_ptr<Workspace> workspace_of(c10::Device device, void* stream) {
+    const std::lock_guard<std::mutex> lock(g_mutex);
+    auto& w = g_workspaces[{device.index(), stream}];
+    if (!w) w = std::make_shared<Workspace>();
     return w;
 }
+
+// The GIL is released while a call allocates and launches: a full queue blocks the launch.  Nothing that holds one of the
+// locks above waits for them with the GIL.
+struct NoGil {
+    PyThreadState* const state = PyEval_SaveThread();
+    ~NoGil() { PyEval_RestoreThread(state); }
+};
 
 // ---- arguments
 int dtype_code(at::ScalarType t) {
@@ -242,7 +253,9 @@ Tensor run_forward(const Call& c, Tensor* state) {
         check(api.layout(&p, &unused), "monarch_attention_hip");
     }
     void* stream = current_stream(q.device());
-    const std::shared_ptr<Workspace> w = workspace_for(q.device(), stream, nbytes);
+    const std::shared_ptr<Workspace> w = workspace_of(q.device(), stream);
+    const std::lock_guard<std::mutex> lock(w->lock);
+    w->ready(q.device(), nbytes);
     p.workspace = w->buf.data_ptr();
     p.workspace_bytes = static_cast<uint64_t>(w->buf.numel());
     p.error_word = reinterpret_cast<uint32_t*>(const_cast<int32_t*>(w->err));
@@ -258,6 +271,34 @@ Tensor run_forward(const Call& c, Tensor* state) {
         check(api.fwd(&p, stream), "ma_fwd");
     }
     return out;
+}
+
+// The dense matrix (c.v unused)
+Tensor run_matrix(const Call& c) {
+    const c10::AutoGradMode no_grad(false);
+    const at::DeviceGuard guard(c.q.device());
+    const Tensor q = rows_contiguous(c.q), k = rows_contiguous(c.k);
+    ma_fwd_params p = params_of(c, q, k, q);
+    const int64_t N = q.size(2);
+    const Tensor A = at::empty({q.size(0), q.size(1), N, N}, q.options().dtype(at::kFloat));
+    p.out = A.data_ptr();
+    set_strides(p.out_stride, q);
+    if (p.E > 1 && p.out_stride[0] == 0) p.out_stride[0] = 1;   // stand-ins: the call reads neither out nor its strides
+    if (p.H > 1 && p.out_stride[1] == 0) p.out_stride[1] = 1;
+    const uint64_t nbytes = api.matrix_workspace_bytes(&p);
+    if (nbytes == 0) {
+        ma_ws_layout unused;
+        check(api.layout(&p, &unused), "monarch_matrix_hip");
+    }
+    void* stream = current_stream(q.device());
+    const std::shared_ptr<Workspace> w = workspace_of(q.device(), stream);
+    const std::lock_guard<std::mutex> lock(w->lock);
+    w->ready(q.device(), nbytes);
+    p.workspace = w->buf.data_ptr();
+    p.workspace_bytes = static_cast<uint64_t>(w->buf.numel());
+    p.flags |= MA_FLAG_SYNC_READY;
+    check(api.matrix(&p, A.data_ptr<float>(), stream), "ma_matrix");
+    return A;
 }
 
 struct Grads {
@@ -421,7 +462,12 @@ PyObject* py_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const bool record = c10::GradMode::is_enabled() && (c.q.requires_grad() || c.k.requires_grad() || c.v.requires_grad());
     const int keep = PyObject_IsTrue(args[9]);
     if (keep < 0) throw python_error();
-    return THPVariable_Wrap(record ? run_recorded(c, keep != 0) : run_forward(c, nullptr));
+    Tensor out;
+    {
+        const NoGil no_gil;
+        out = record ? run_recorded(c, keep != 0) : run_forward(c, nullptr);
+    }
+    return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }
 
@@ -433,8 +479,12 @@ PyObject* py_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (n != 10 || !tensor(args[0], &c.q) || !tensor(args[1], &c.k) || !tensor(args[2], &c.v) || !tensor_or_none(args[3], &c.mask) ||
         !tensor(args[4], &dout) || !scalars(args + 5, &c) || !valid(c) || dout.sizes() != c.v.sizes() || dout.device() != c.v.device())
         Py_RETURN_NONE;
-    const c10::AutoGradMode no_grad(false);
-    Grads g = run_backward(c, dout, Tensor());
+    Grads g;
+    {
+        const NoGil no_gil;
+        const c10::AutoGradMode no_grad(false);
+        g = run_backward(c, dout, Tensor());
+    }
     PyObject* r = PyTuple_New(3);
     if (!r) throw python_error();
     PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(std::move(g.dq)));
@@ -452,39 +502,35 @@ PyObject* py_matrix(PyObject*, PyObject* const* args, Py_ssize_t n) {
         Py_RETURN_NONE;
     c.v = c.q;
     if (!valid(c)) Py_RETURN_NONE;
-    const c10::AutoGradMode no_grad(false);
-    const at::DeviceGuard guard(c.q.device());
-    const Tensor q = rows_contiguous(c.q), k = rows_contiguous(c.k);
-    ma_fwd_params p = params_of(c, q, k, q);
-    const int64_t N = q.size(2);
-    const Tensor A = at::empty({q.size(0), q.size(1), N, N}, q.options().dtype(at::kFloat));
-    p.out = A.data_ptr();
-    set_strides(p.out_stride, q);
-    if (p.E > 1 && p.out_stride[0] == 0) p.out_stride[0] = 1;   // stand-ins: the call reads neither out nor its strides
-    if (p.H > 1 && p.out_stride[1] == 0) p.out_stride[1] = 1;
-    const uint64_t nbytes = api.matrix_workspace_bytes(&p);
-    if (nbytes == 0) {
-        ma_ws_layout unused;
-        check(api.layout(&p, &unused), "monarch_matrix_hip");
+    Tensor A;
+    {
+        const NoGil no_gil;
+        A = run_matrix(c);
     }
-    void* stream = current_stream(q.device());
-    const std::shared_ptr<Workspace> w = workspace_for(q.device(), stream, nbytes);
-    p.workspace = w->buf.data_ptr();
-    p.workspace_bytes = static_cast<uint64_t>(w->buf.numel());
-    p.flags |= MA_FLAG_SYNC_READY;
-    check(api.matrix(&p, A.data_ptr<float>(), stream), "ma_matrix");
-    return THPVariable_Wrap(A);
+    return THPVariable_Wrap(std::move(A));
     END_HANDLE_TH_ERRORS
 }
 
 // workspaces() -> list of the cached workspace buffers
 PyObject* py_workspaces(PyObject*, PyObject*) {
     HANDLE_TH_ERRORS
-    std::lock_guard<std::mutex> lock(g_mutex);
+    std::vector<Tensor> buffers;
+    {
+        const NoGil no_gil;
+        std::vector<std::shared_ptr<Workspace>> all;
+        {
+            const std::lock_guard<std::mutex> lock(g_mutex);
+            for (const auto& kv : g_workspaces) all.push_back(kv.second);
+        }
+        for (const auto& w : all) {
+            const std::lock_guard<std::mutex> lock(w->lock);
+            if (w->buf.defined()) buffers.push_back(w->buf);
+        }
+    }
     PyObject* r = PyList_New(0);
     if (!r) throw python_error();
-    for (const auto& kv : g_workspaces) {
-        PyObject* t = THPVariable_Wrap(kv.second->buf);
+    for (const Tensor& buf : buffers) {
+        PyObject* t = THPVariable_Wrap(buf);
         PyList_Append(r, t);
         Py_DECREF(t);
     }
@@ -494,12 +540,12 @@ PyObject* py_workspaces(PyObject*, PyObject*) {
 
 PyObject* py_clear(PyObject*, PyObject*) {
     HANDLE_TH_ERRORS
-    std::map<std::pair<int, void*>, std::shared_ptr<Workspace>> gone;
     {
-        std::lock_guard<std::mutex> lock(g_mutex);
+        const NoGil no_gil;
+        std::map<std::pair<int, void*>, std::shared_ptr<Workspace>> gone;
+        const std::lock_guard<std::mutex> lock(g_mutex);
         gone.swap(g_workspaces);
     }
-    gone.clear();
     Py_RETURN_NONE;
     END_HANDLE_TH_ERRORS
 }

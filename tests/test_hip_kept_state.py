@@ -105,3 +105,59 @@ def test_a_recorded_call_that_keeps_no_state_runs_as_an_unrecorded_one(E, H, N, 
     want = monarch_attention_hip_backward(*leaves, None, w, 2, B, False)
     for a, b in zip(torch.autograd.grad(out, leaves, w), want):
         assert torch.equal(a, b)
+
+
+def test_calls_release_the_gil():
+    """A call that blocks on a full queue must not hold up other Python threads.  With a switch interval longer than the test
+    a waiting thread runs only if the call lets it."""
+    import sys
+    import threading
+
+    q, k, v = (t.to(DEV) for t in seeded_qkv(1, 2, 64, 32, torch.float16))
+    monarch_attention_hip(q, k, v, None, 2, 8, False)
+    ran, gate = [], threading.Lock()
+    gate.acquire()
+
+    def other():
+        gate.acquire()
+        ran.append(True)
+
+    thread = threading.Thread(target=other)
+    interval = sys.getswitchinterval()
+    try:
+        thread.start()
+        sys.setswitchinterval(1000.0)
+        gate.release()
+        for _ in range(2000):
+            monarch_attention_hip(q, k, v, None, 2, 8, False)
+            if ran:
+                break
+        done = bool(ran)
+    finally:
+        sys.setswitchinterval(interval)
+        thread.join()
+    assert done
+
+
+def test_threads_on_one_stream_share_the_workspace():
+    """Calls of several launches that read each other's state arrays, from several threads, all on the default stream."""
+    import threading
+
+    shapes = [(2, 4, 300, 64, 20, 3), (1, 8, 1000, 64, 130, 2), (1, 3, 500, 32, 16, 2), (2, 2, 700, 96, 72, 3)]
+    problems = []
+    for i, (E, H, N, D, B, T) in enumerate(shapes):
+        x = [t.to(DEV) for t in seeded_qkv(E, H, N, D, torch.bfloat16, seed=i)]
+        problems.append((x, T, B, monarch_attention_hip(*x, None, T, B, False, variant="staged")))
+    wrong = []
+
+    def work(i):
+        x, T, B, want = problems[i % len(problems)]
+        outs = [monarch_attention_hip(*x, None, T, B, False, variant="staged") for _ in range(100)]
+        wrong.extend(i for o in outs if not torch.equal(o, want))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
