@@ -26,6 +26,7 @@
 #include <c10/core/AutogradState.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/forward_grad.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
@@ -171,7 +172,8 @@ bool valid(const Call& c) {
 
 // Forward-mode AD: the operator has no jvp, and a result without a tangent would pass for a zero derivative.
 void refuse_tangents(std::initializer_list<const Tensor*> tensors) {
-    if (!c10::AutogradState::get_tls_state().get_fw_grad_mode()) return;
+    // (outside of every dual level - one lookup - there are none, and the tensors' metadata is not touched)
+    if (!c10::AutogradState::get_tls_state().get_fw_grad_mode() || !torch::autograd::ForwardADLevel::try_get_by_idx(0)) return;
     for (const Tensor* t : tensors)
         TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(/*level=*/0).defined(),
                                     "monarch_attention_hip has no forward-mode derivative (jvp): q, k, v and the output gradient must not be dual tensors");
