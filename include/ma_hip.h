@@ -189,9 +189,7 @@ uint64_t ma_fwd_workspace_bytes(const ma_fwd_params* p);
 int ma_workspace_init(const ma_fwd_params* p, void* stream);
 
 /* The variant MA_VARIANT_AUTO resolves to for this problem (a ma_variant), or
- * a negative ma_status.  (fp32 problems with blocks or block counts of more than
- * 128 rows, or of more rows and columns than fit the LDS at once, are reported as
- * GENERIC; unless GENERIC is asked for they run on the kernels of STAGED.) */
+ * a negative ma_status. */
 int ma_fwd_select_variant(const ma_fwd_params* p);
 
 /* Name of the kernel that does the bulk of the work for this problem under the variant it resolves to

@@ -171,16 +171,6 @@ bool mfma32_supported(const ma_fwd_params* p) {
     return true;
 }
 
-// ... of them those whose operand tiles and L matrix would fit the LDS together.  The others count as GENERIC where AUTO
-// reports what it resolves to (ma_fwd_select_variant), but run on the stage kernels as well unless GENERIC is asked for.
-bool mfma32_small(const ma_fwd_params* p) {
-    const long long M = (static_cast<long long>(p->N) + p->B - 1) / p->B;
-    auto strips = [](long long n) { return n <= 16 ? 1 : n <= 32 ? 2 : n <= 64 ? 4 : 8; };
-    const long long rows = 16 * strips(p->B > M ? p->B : M), pitch = 16 * ((p->D + 15) / 16) + 4, rowsL = 16 * strips(M);
-    const long long lds = 4 * (2 * rows * pitch + rows), ldsL = 4 * (2 * rowsL * pitch + rowsL * (rowsL + 4) + 5 * rowsL);
-    return p->B <= 128 && M <= 128 && (lds > ldsL ? lds : ldsL) <= 160 * 1024;
-}
-
 int run_resident(const Problem& P, int dtype_qk, bool dry_run, hipStream_t s) {
     if (dtype_qk == MA_F32) return launch_head32(P, dry_run, s);
     const bool h = dtype_qk == MA_F16;
@@ -890,7 +880,6 @@ int ma_workspace_init(const ma_fwd_params* p, void* stream) {
 }
 
 int ma_fwd_select_variant(const ma_fwd_params* p) {
-    if (p != nullptr && p->variant == MA_VARIANT_AUTO && check_shape(p) == MA_OK && mfma32_supported(p) && !mfma32_small(p)) return MA_VARIANT_GENERIC;
     const int st = check_shape(p);
     if (st != MA_OK) return st;
     return select_variant(p);
@@ -901,7 +890,7 @@ const char* ma_fwd_kernel_name(const ma_fwd_params* p) {
     const bool f32 = p->dtype_qk == MA_F32;
     switch (select_variant(p)) {
         case MA_VARIANT_GENERIC: return "r_step_kernel";
-        case MA_VARIANT_STAGED: return f32 ? "r_step_f32" : "r_step_mfma";
+        case MA_VARIANT_STAGED: return f32 ? "r_step_f32" : p->B > 128 ? "r_step_long" : p->B > 64 ? "r_step_pair" : "r_step_mfma";   // (see runs_long)
         case MA_VARIANT_FUSED: return "fused_fwd_mfma";
         case MA_VARIANT_CHAINED: return "chain_fwd_mfma";
         case MA_VARIANT_RESIDENT: {

@@ -205,7 +205,9 @@ def test_kernel_name_follows_the_resolved_variant():
     assert name(16, 12, 512, 64, 32, T=1) == "resident_head2_mfma"
     assert name(8, 12, 512, 64, 32) == "chain_fwd_mfma"           # ... 96 heads do not fill the device
     assert name(16, 12, 1000, 32, 32, variant="resident") == "resident_fwd_mfma"   # state only
-    assert name(1, 16, 4096, 64, 256) == "r_step_mfma"
+    assert name(1, 16, 4096, 64, 256) == "r_step_long"            # stage kernels by the rows of a block
+    assert name(1, 16, 4096, 64, 128, variant="staged") == "r_step_pair"
+    assert name(1, 16, 4096, 64, 64, variant="staged") == "r_step_mfma"
     assert name(1, 1, 256, 64, 16, dt=L.MA_F32, T=1) == "head_t1_f32"
     assert name(1, 1, 256, 64, 16, dt=L.MA_F32, T=2) == "r_step_f32"
     assert name(8, 8, 197, 64, 16, dt=L.MA_F32) == "head_fwd_f32"
@@ -312,7 +314,9 @@ def test_auto_variant_policy():
     assert auto(1, 2, 128, 32, 16, dt=L.MA_F32) == "resident"       # ... and for very small heads always
     assert auto(8, 8, 272, 64, 16, dt=L.MA_F32) == "staged"         # 17 blocks
     assert auto(8, 8, 256, 80, 16, dt=L.MA_F32) == "staged"         # head dim above 64
-    assert auto(1, 16, 16384, 128, 128, dt=L.MA_F32) == "generic"   # 128 x 128 fp32 tiles do not fit the LDS
+    assert auto(1, 16, 16384, 128, 128, dt=L.MA_F32) == "staged"    # fp32 stage kernels up to 256 rows and 128 columns (tiles in chunks)
+    assert auto(1, 16, 65536, 128, 256, dt=L.MA_F32) == "staged"
+    assert auto(1, 16, 4096, 128, 257, dt=L.MA_F32) == "generic"
     assert auto(1, 16, 4096, 62, 64, dt=L.MA_F32) == "generic"      # D % 4 != 0
     assert auto(1, 16, 4096, 64, 64, Dv=128) == "generic"
     assert auto(1, 16, 4096, 60, 64) == "generic"       # D % 8 != 0
