@@ -245,7 +245,7 @@ int ma_z_step(const ma_fwd_params* p, void* stream);
  * identity, no (E,H,Np,N) Y state.  `A` is a contiguous (E,H,N,N) fp32 device
  * array.  Of *p the fields v, out, Dv, dtype_v, v_stride and out_stride are not
  * read; workspace: ma_matrix_workspace_bytes(), which has room for the
- * probabilities of the last R step.  With ma_fwd_workspace_bytes() of a problem
+ * probabilities of the last R step where the matrix-core kernels apply.  With ma_fwd_workspace_bytes() of a problem
  * of Dv = D and dtype_v = dtype_qk the call works as well, on a slower kernel.
  * Variants AUTO, GENERIC and STAGED (they select the kernels of the T steps);
  * MA_ERR_UNSUPPORTED for the one-launch variants and, where the matrix-core
@@ -287,8 +287,9 @@ int ma_bwd(const ma_bwd_params* p, void* stream);
  * memory, 256-byte aligned, the caller's until the backward pass has run; p->workspace: ma_fwd_keep_workspace_bytes(p)
  * bytes, used and kept ready (MA_FLAG_SYNC_READY) like ma_fwd's.  Variants AUTO, GENERIC, STAGED and CHAINED (the ones
  * that hold the state in memory); MA_ERR_UNSUPPORTED for the others.
- * ma_bwd_kept is ma_bwd on that state, which it only reads; it needs ma_bwd_kept_workspace_bytes() of workspace.  The
- * fwd arguments must be those of the ma_fwd_keep call. */
+ * ma_bwd_kept is ma_bwd on that state, which it only reads; it needs ma_bwd_kept_workspace_bytes() of workspace: what the
+ * kernels need that the shape, strides and pointers of *p select (without pointers: the most any of them needs).  The fwd
+ * arguments must be those of the ma_fwd_keep call. */
 uint64_t ma_fwd_state_bytes(const ma_fwd_params* p);
 uint64_t ma_fwd_keep_workspace_bytes(const ma_fwd_params* p);
 int ma_fwd_keep(const ma_fwd_params* p, void* state, uint64_t state_bytes, void* stream);

@@ -670,20 +670,29 @@ int bwd_prepare(const ma_bwd_params* b, bool kept, ma_fwd_params* pp, BwdLayout*
     if ((pp->E > 1 && (b->dq_stride[0] == 0 || b->dk_stride[0] == 0 || b->dv_stride[0] == 0)) ||
         (pp->H > 1 && (b->dq_stride[1] == 0 || b->dk_stride[1] == 0 || b->dv_stride[1] == 0)))
         return MA_ERR_STRIDE;
-    const uint64_t rows = padded_rows(pp);
+    L->tiled = bwd_tiled(b, pp, &L->rows16);
+    // What a stage of the path does not use has no room of its own.  (ma_bwd's size is one for every path, so that it does
+    // not depend on pointers a caller may not have yet; the T steps it runs again are the larger part of it anyway.)
+    const bool tight = kept && L->tiled, steps = pp->T > 1;
+    const uint64_t rows = padded_rows(pp), es = tight ? elt_size(pp->dtype_qk) : 4;
     uint64_t off = kept ? 0 : state_layout(pp).total;
-    L->stats = off; off = kept ? off : align_up(off + rows * 8);
-    L->gaR = off; off = align_up(off + rows * pp->D * 4);
-    L->gcR = off; off = align_up(off + rows * 4);
-    L->gaL = off; off = align_up(off + rows * pp->D * 4);
-    L->gcL = off; off = align_up(off + rows * 4);
-    L->gY = off; off = align_up(off + rows * pp->Dv * 4);
-    L->stat = off; off = align_up(off + rows * 16);
+    auto take = [&](uint64_t* at, bool used, uint64_t bytes) {
+        *at = off;
+        if (used) off = align_up(off + bytes);
+    };
+    const bool two_launches = pp->B > 64 || (pp->N + pp->B - 1) / pp->B > 64;   // (each_launch: longer problems may split)
+    take(&L->stats, !kept, rows * 8);
+    take(&L->gaR, !tight || steps, rows * pp->D * es);
+    take(&L->gcR, !tight || steps, rows * 4);
+    take(&L->gaL, true, rows * pp->D * es);
+    take(&L->gcL, true, rows * 4);
+    take(&L->gY, true, rows * pp->Dv * es);
+    take(&L->stat, tight && two_launches, rows * 16);
     // dq, dk, dv are contiguous: one fill kernel zeroes the three
     L->dq = off; off += rows * pp->D * 4;
-    L->dk = off; off += rows * pp->D * 4;
-    L->dv = off; off = align_up(off + rows * pp->Dv * 4);
-    L->tiled = bwd_tiled(b, pp, &L->rows16);
+    L->dk = off; off += !tight || steps ? rows * pp->D * 4 : 0;   // (a single step completes dk in registers)
+    L->dv = off; off = align_up(off + (tight ? 0 : rows * pp->Dv * 4));
+    if (L->tiled && !tight) L->stat = L->dv;   // no accumulator of dv on the tiled path (D % 4 == 0: 16 bytes a row and more)
     {
         ma_ws_layout none;
         std::memset(&none, 0, sizeof(none));
@@ -1000,12 +1009,16 @@ int ma_fwd_static(const ma_fwd_params* p, void* stream) {
 uint64_t ma_matrix_workspace_bytes(const ma_fwd_params* p) {
     if (p == nullptr) return 0;
     ma_fwd_params pp = *p;   // v and out are not read
+    pp.v = pp.q;
+    pp.out = nullptr;        // (aligned, as far as anybody knows)
     pp.Dv = pp.D;
     pp.dtype_v = pp.dtype_qk;
     for (int i = 0; i < 3; ++i) pp.v_stride[i] = pp.out_stride[i] = pp.q_stride[i];
     if (pp.E > 1 && pp.out_stride[0] == 0) pp.out_stride[0] = 1;
     if (pp.H > 1 && pp.out_stride[1] == 0) pp.out_stride[1] = 1;
-    return matrix_workspace(&pp);
+    if (pp.variant != MA_VARIANT_GENERIC && check_shape(&pp) == MA_OK && (mfma_supported(&pp) || mfma32_supported(&pp))) return matrix_workspace(&pp);
+    ma_ws_layout L;          // the FMA writer keeps no probabilities
+    return layout_of(&pp, &L) == MA_OK ? L.total : 0;
 }
 
 int ma_matrix(const ma_fwd_params* p, float* A, void* stream) {

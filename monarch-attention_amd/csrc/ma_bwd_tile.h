@@ -606,6 +606,7 @@ int launch_r(const Problem& P, const BwdBuffers& G, bool first, bool with_v, hip
     return each_launch<sizeof(T) == 4>(P.B, problems, [&](auto nwt, auto w, auto pass) {
         constexpr int NWT = decltype(nwt)::value, W = decltype(w)::value, PASS = decltype(pass)::value;
         if constexpr (PASS == 0 && !RPlan<T, DT, NWT, 0>::kFits) {   // three fp32 tiles of 128 rows: the passes one after the other
+            static_assert(NWT > 4, "the statistics of problems of up to 64 rows have no room in the workspace");
             const int st = run(r_bwd_tile<T, DT, NWT, NWT / 2, 1>, RPlan<T, DT, NWT, 1>::kLds, problems, 2, NWT / 2, s, P, G, first ? 1 : 0, with_v ? 1 : 0);
             return st ? st : run(r_bwd_tile<T, DT, NWT, NWT / 2, 2>, RPlan<T, DT, NWT, 2>::kLds, problems, 2, NWT / 2, s, P, G, first ? 1 : 0, with_v ? 1 : 0);
         } else {

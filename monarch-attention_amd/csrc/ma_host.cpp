@@ -92,7 +92,10 @@ struct Workspace {
             err = err_host.data_ptr<int32_t>();
         }
         if (!buf.defined() || static_cast<uint64_t>(buf.numel()) < nbytes) resize(device, nbytes);
-        if (*err == 0) return;
+        report();
+    }
+    void report() {
+        if (err == nullptr || *err == 0) return;
         const int code = *err;
         *err = 0;
         dirty = true;
@@ -293,12 +296,14 @@ Tensor run_matrix(const Call& c) {
         check(api.layout(&p, &unused), "monarch_matrix_hip");
     }
     void* stream = current_stream(q.device());
-    const std::shared_ptr<Workspace> w = workspace_of(q.device(), stream);
-    const std::lock_guard<std::mutex> lock(w->lock);
-    w->ready(q.device(), nbytes);
-    p.workspace = w->buf.data_ptr();
-    p.workspace_bytes = static_cast<uint64_t>(w->buf.numel());
-    p.flags |= MA_FLAG_SYNC_READY;
+    {
+        const std::shared_ptr<Workspace> w = workspace_of(q.device(), stream);
+        const std::lock_guard<std::mutex> lock(w->lock);
+        w->report();
+    }
+    const Tensor ws = device_bytes(nbytes, q);   // (with the probabilities: allocated per call and freed after it)
+    p.workspace = ws.data_ptr();
+    p.workspace_bytes = nbytes;
     check(api.matrix(&p, A.data_ptr<float>(), stream), "ma_matrix");
     return A;
 }

@@ -385,3 +385,41 @@ def test_backward_workspace_and_argument_checks_precede_any_launch():
     need = lib.ma_bwd_workspace_bytes(bad)
     bad.fwd.workspace, bad.fwd.workspace_bytes = 0x100000, need
     assert need > 0 and lib.ma_bwd(bad, None) == L.MA_ERR_UNSUPPORTED
+
+
+def test_workspaces_hold_what_the_path_uses():
+    """Bytes a row: what the tiled backward kernels keep (state gradients in the operand type, fp32 dq and, with more than one
+    step, dk) and nothing for the other kernels; the matrix call's probabilities only where they are kept."""
+    lib = L.load()
+    E, H, N, D, B, es = 1, 16, 8192, 64, 64, 2
+    rows = H * N
+
+    def params(T, align, variant="auto"):
+        b = L.BwdParams()
+        p = b.fwd
+        p.E, p.H, p.N, p.D, p.Dv, p.B, p.T = E, H, N, D, D, B, T
+        p.dtype_qk = p.dtype_v = L.MA_BF16
+        p.eps, p.variant = 1e-12, L.VARIANTS[variant]
+        for name in ("q_stride", "k_stride", "v_stride", "out_stride"):
+            setattr(p, name, (C.c_int64 * 3)(H * N * D, N * D, D))
+        for name in ("dout_stride", "dq_stride", "dk_stride", "dv_stride"):
+            setattr(b, name, (C.c_int64 * 3)(H * N * D, N * D, D))
+        if align:
+            p.q = p.k = p.v = b.dout = b.dq = b.dk = b.dv = align
+        return b
+
+    slack = 16 * 256
+    for T, per_row in ((1, 2 * D * es + 4 + 16 + 4 * D), (2, 3 * D * es + 8 + 16 + 2 * 4 * D), (3, 3 * D * es + 8 + 16 + 2 * 4 * D)):
+        need = lib.ma_bwd_kept_workspace_bytes(params(T, 0x10000))
+        assert rows * per_row <= need <= rows * per_row + slack
+        assert lib.ma_bwd_kept_workspace_bytes(params(T, 0x10002)) > need         # other kernels: fp32 throughout
+        assert lib.ma_bwd_kept_workspace_bytes(params(T, 0)) >= lib.ma_bwd_kept_workspace_bytes(params(T, 0x10002))
+        b = params(T, 0x10000)
+        b.fwd.workspace, b.fwd.workspace_bytes = 0x100000, need - 1
+        assert lib.ma_bwd_kept(b, 0x200000, lib.ma_fwd_state_bytes(b.fwd), None) == L.MA_ERR_WORKSPACE
+    p = params(2, 0).fwd
+    assert lib.ma_matrix_workspace_bytes(p) == lib.ma_fwd_workspace_bytes(p) + rows * B * 4
+    p.D = 60   # D % 8 != 0: the FMA writer
+    p.Dv = 60
+    assert lib.ma_matrix_workspace_bytes(p) == lib.ma_fwd_workspace_bytes(p)
+    assert lib.ma_matrix_workspace_bytes(params(2, 0, "generic").fwd) == lib.ma_fwd_workspace_bytes(params(2, 0).fwd)

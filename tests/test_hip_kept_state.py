@@ -161,3 +161,14 @@ def test_threads_on_one_stream_share_the_workspace():
     for t in threads:
         t.join()
     assert not wrong
+
+
+def test_matrix_call_leaves_the_cached_workspace_as_it_is():
+    from ma import ma_hip
+
+    ma_hip.clear_workspace_cache()
+    q, k, v = (t.to(DEV) for t in seeded_qkv(1, 12, 1024, 64, torch.float16))
+    monarch_attention_hip(q, k, v, None, 2, 256, False)
+    sizes = [b.numel() for b in ma_hip._HOST.workspaces()]
+    ma_hip.monarch_matrix_hip(q, k, None, 2, 256, False)
+    assert [b.numel() for b in ma_hip._HOST.workspaces()] == sizes
