@@ -752,7 +752,7 @@ int launch(const Problem& P, int stage, bool first, bool with_v, hipStream_t s) 
             if (with_v) return run(r_step_pair<T, DT, NWT, W, SP, true>, RPlan<T, DT, NWT>::kLds, problems, GR, W, s, P, first ? 1 : 0);
             return run(r_step_pair<T, DT, NWT, W, SP, false>, KPlan<T, DT, NWT>::kLds, problems, GR, W, s, P, first ? 1 : 0);
         };
-        if (problems <= 512) return go(std::integral_constant<int, 1>{}, std::integral_constant<int, 2>{});
+        if (problems <= 2 * mfma::compute_units()) return go(std::integral_constant<int, 1>{}, std::integral_constant<int, 2>{});
         return go(std::integral_constant<int, 2>{}, std::integral_constant<int, 1>{});
     };
     auto whole = [&](auto nwt) {

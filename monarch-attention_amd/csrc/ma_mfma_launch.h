@@ -3,9 +3,10 @@
 // instantiations compile in parallel.
 #pragma once
 
+#include <atomic>
 #include <map>
-#include <utility>
 #include <mutex>
+#include <utility>
 
 #include "ma_mfma.h"
 
@@ -72,6 +73,18 @@ DeviceCaps device_caps(K kernel, int threads, size_t lds) {
     if (!c.err && threads > 0) c.err = static_cast<int>(hipOccupancyMaxActiveBlocksPerMultiprocessor(&c.per_cu, key, threads, lds));
     if (!c.err) known[{key, dev}] = c;
     return c;
+}
+
+// Compute units of the current device, looked up once per device.
+inline int compute_units() {
+    constexpr int kDevices = 64;
+    static std::atomic<int> known[kDevices];
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 256;
+    if (dev < kDevices && (cus = known[dev].load(std::memory_order_relaxed)) > 0) return cus;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) return 256;
+    if (dev < kDevices) known[dev].store(cus, std::memory_order_relaxed);
+    return cus;
 }
 
 // calls f(dt_tag, nt_tag) with integral_constant tags for the problem's classes (up to 64 rows: longer ones run the

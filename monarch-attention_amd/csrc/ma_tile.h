@@ -265,8 +265,8 @@ inline int strip_class(int n) {
 }
 
 // f(integral_constant NWT, integral_constant W, integral_constant PASS) for every launch of a stage of `problems` problems
-// of n rows.  One launch of both passes up to 128 rows, unless there are fewer problems of 6 or 8 strips than compute
-// units: half of their strips per workgroup then (the graph-transformer shape has 120 problems of 128 rows).  Above 128
+// of n rows.  One launch of both passes up to 128 rows, unless there are fewer problems of 6 or 8 strips than the device has
+// compute units: half of their strips per workgroup then (the graph-transformer shape has 120 problems of 128 rows).  Above 128
 // rows half of the strips per workgroup, or four where that would leave compute units without one.
 template <bool F32, class F>
 int each_launch(int n, long long problems, F&& f) {
@@ -276,22 +276,23 @@ int each_launch(int n, long long problems, F&& f) {
     };
     using std::integral_constant;
     constexpr integral_constant<int, 0> one{};
+    const bool fill = problems >= mfma::compute_units();
     switch (strip_class(n)) {
         case 1: return f(integral_constant<int, 1>{}, integral_constant<int, 1>{}, one);
         case 2: return f(integral_constant<int, 2>{}, integral_constant<int, 2>{}, one);
         case 3: return f(integral_constant<int, 3>{}, integral_constant<int, 3>{}, one);
         case 4: return f(integral_constant<int, 4>{}, integral_constant<int, 4>{}, one);
-        case 6: return problems < 256 ? two(integral_constant<int, 6>{}, integral_constant<int, 3>{}, integral_constant<int, 3>{})
-                                      : f(integral_constant<int, 6>{}, integral_constant<int, 6>{}, one);
-        case 8: return problems < 256 ? two(integral_constant<int, 8>{}, integral_constant<int, 4>{}, integral_constant<int, 4>{})
-                                      : f(integral_constant<int, 8>{}, integral_constant<int, 8>{}, one);
+        case 6: return !fill ? two(integral_constant<int, 6>{}, integral_constant<int, 3>{}, integral_constant<int, 3>{})
+                             : f(integral_constant<int, 6>{}, integral_constant<int, 6>{}, one);
+        case 8: return !fill ? two(integral_constant<int, 8>{}, integral_constant<int, 4>{}, integral_constant<int, 4>{})
+                             : f(integral_constant<int, 8>{}, integral_constant<int, 8>{}, one);
         case 12:
             if constexpr (!F32)
-                if (problems >= 256) return two(integral_constant<int, 12>{}, integral_constant<int, 6>{}, integral_constant<int, 6>{});
+                if (fill) return two(integral_constant<int, 12>{}, integral_constant<int, 6>{}, integral_constant<int, 6>{});
             return two(integral_constant<int, 12>{}, integral_constant<int, 4>{}, integral_constant<int, 4>{});
         default:
             if constexpr (!F32)
-                if (problems >= 256) return two(integral_constant<int, 16>{}, integral_constant<int, 4>{}, integral_constant<int, 8>{});
+                if (fill) return two(integral_constant<int, 16>{}, integral_constant<int, 4>{}, integral_constant<int, 8>{});
             return two(integral_constant<int, 16>{}, integral_constant<int, 4>{}, integral_constant<int, 4>{});
     }
 }
