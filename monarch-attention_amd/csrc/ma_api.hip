@@ -424,7 +424,7 @@ bool auto_staged(const ma_fwd_params* p, long long heads, long long M) {
     // tokens on (two launches, 3 - 19 % ahead)
     const bool one_step = p->T == 1 && ((heads % 8 != 0 && p->N >= 4096) || (heads < (p->D > 64 ? 8 : 16) && p->N >= 7168) || (heads <= 4 && p->N >= 1024));
     // launches that leave most of the device empty: the stage kernels run their 6- and 8-strip R and Z problems as two
-    // workgroups each then (halves_pay), which the one-launch kernels do not
+    // workgroups each then (ma_long.h), which the one-launch kernels do not
     const bool rows_halve = p->B > 64 && p->B <= 128, blocks_halve = M > 64 && M <= 128;
     const long long r_problems = heads * M;
     const bool underfilled = (rows_halve && (p->T == 1 ? (r_problems <= 160 || (heads <= 8 && r_problems <= 512))

@@ -24,12 +24,8 @@ inline int nt_class_chain(int n) {
     const int t = (n + 15) / 16;
     return t <= 4 ? (t < 1 ? 1 : t) : t <= 6 ? 6 : 8;
 }
-// (129 .. 256 rows: classes of 12 and 16 strips, per-stage launches only; a head of 32768 tokens in
-// blocks of floor(sqrt(N)) = 181 rows runs in the 12-strip class both ways)
-inline int nt_class(int n) {
-    const int t = (n + 15) / 16;
-    return t <= 4 ? (t < 1 ? 1 : t) : t <= 6 ? 6 : t <= 8 ? 8 : t <= 12 ? 12 : 16;
-}
+// the per-stage launches have up to four strips here; longer problems run the kernels of ma_long.h
+inline int nt_class(int n) { return n <= 16 ? 1 : n <= 32 ? 2 : n <= 48 ? 3 : 4; }
 
 // Raises a kernel's dynamic-LDS limit to `bytes`, once per (kernel, device): the attribute belongs
 // to the device's copy of the code object, so a process that drives several devices needs it on
@@ -87,8 +83,7 @@ inline int compute_units() {
     return cus;
 }
 
-// calls f(dt_tag, nt_tag) with integral_constant tags for the problem's classes (up to 64 rows: longer ones run the
-// kernels of ma_long.h)
+// calls f(dt_tag, nt_tag) with integral_constant tags for the problem's classes
 template <class F>
 int for_classes(int dt, int nt, F&& f) {
 #define MA_NT(DTV)                                                                            \
