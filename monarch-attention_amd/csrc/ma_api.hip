@@ -259,9 +259,9 @@ bool fused_full_width(const ma_fwd_params* p) {
 
 // The variant a problem resolves to.  AUTO: the MFMA kernels when the problem qualifies; among
 // them what a sweep on MI355X says (fp16, E*H = 1 .. 384 heads, N = 256 .. 8192, blocks of 16 .. 128
-// rows, T = 1, 2, 3, head dims 32, 64, 128; every variant that takes a shape timed: the choice
-// below is within 0.0 - 0.7 % of the fastest variant in the geometric mean of each sweep and 18 %
-// at worst):
+// rows, T = 1, 2, 3, head dims 32 .. 128; every variant that takes a shape timed: the choice
+// below is within 0.0 - 1.2 % of the fastest variant in the geometric mean of each sweep, 0.7 - 2.8 %
+// for problems of 65 .. 96 rows at head dims above 64; 115 of 8075 points are more than 10 % off):
 //  * the resident kernel for heads that fit in LDS with their inputs (up to ~256 tokens at d = 64) in
 //    blocks of at most 32 rows: from 128 heads on, and with more than one step for any number of
 //    heads in 16-row blocks; with two or three state tiles for blocks of at most 16 rows from 128
@@ -277,8 +277,8 @@ bool fused_full_width(const ma_fwd_params* p) {
 //    running; everybody else continues down this list;
 //  * one launch per half step where the one-launch kernels are at a disadvantage: 128-row
 //    problems both ways on a head count that does not divide by the 8 XCDs the chained kernel
-//    pins heads to; head dims above 64 with problems of 65 .. 128 rows on many tokens; fewer than 8 heads of thousands of tokens (a head's tasks all run on one
-//    XCD); a single step on an uneven head count from 4096 tokens on, or on 8 heads from ~7000
+//    pins heads to; head dims above 64 with problems of 97 .. 128 rows (D = 96: 65 .. 128) on many tokens;
+//    fewer than 8 heads of thousands of tokens (a head's tasks all run on one XCD); a single step on an uneven head count from 4096 tokens on, or on 8 heads from ~7000
 //    on (two launches against an unbalanced one); few problems of 65 .. 128 rows (a single step:
 //    up to ~160 R problems, or 512 on at most 8 heads; more steps, 97 .. 128 rows only: up to 48,
 //    or at most 4 heads of up to 4096 tokens), which the stage kernels split in halves when a launch would leave the
@@ -404,14 +404,18 @@ bool auto_fused(const ma_fwd_params* p, long long heads, long long M) {
 // 16-bit: do the per-stage launches beat the chained kernel?
 bool auto_staged(const ma_fwd_params* p, long long heads, long long M) {
     const long long heads_bytes = heads * p->N * p->D * 2;   // one tensor
-    // Head dims above 64 (measured at 72, 80, 96, 128), problems of 65 .. 128 rows: the stage kernels of ma_long.h against the
-    // chained kernel.  Of 97 .. 128 rows: 0.69 - 0.94 of its time from 32 MB per tensor on, and from 12 MB on a head count
-    // that does not divide by 8 (8 heads of 12000 tokens, 14 - 25 MB: 0.98 - 1.07); of 65 .. 96 rows from 48 MB on (0.70 -
-    // 1.0, one step of 72-column rows 1.05; D = 96, whose column class only the stage kernels have: from 32 MB; more than 64
-    // short blocks at D = 128: 1.05 - 1.10), below that up to 1.4 (16 heads of 5000 tokens in 72-row blocks, three steps).
+    // Head dims above 64 (measured at 72, 96, 128), problems of 65 .. 128 rows: the stage kernels of ma_long.h in multiples of
+    // the chained kernel's time, by the bytes of one tensor.
+    //  97 .. 128 rows, a head count that 8 does not divide: 0.71 - 1.06 (geometric mean 0.87) from 12 MB on.
+    //  ... else D <= 80: 0.72 - 1.04 from 32 MB on with more than one step, 0.91 - 1.11 (1.05) with a single one; D <= 96: 0.72 -
+    //  1.02 from 32 MB on; wider rows 0.79 - 1.06 (0.94) from 48 MB on, 0.98 - 1.16 at 32 .. 48 MB.
+    //  65 .. 96 rows: D = 96, whose column class only the stage kernels have, 0.87 - 1.07 (0.96) from 32 MB on (shorter blocks, a
+    //  single step: 0.96 - 1.07); D = 72 and 128: 0.92 - 1.23 (1.06) from 48 MB on, they stay with the chained kernel.
     const bool long_rows = p->D > 64 && one_launch_tiles(p) &&
-                           (p->B > 96 || M > 96 ? heads_bytes >= (heads % 8 ? 12ll << 20 : 32ll << 20)
-                                                 : (p->B > 64 || (M > 64 && p->D <= 96)) && heads_bytes >= (p->D > 80 && p->D <= 96 ? 32ll << 20 : 48ll << 20));
+                           (p->B > 96 || M > 96 ? (heads % 8 ? heads_bytes >= (12ll << 20)
+                                                   : p->D <= 80 ? p->T >= 2 && heads_bytes >= (32ll << 20)
+                                                                : heads_bytes >= (p->D <= 96 ? 32ll << 20 : 48ll << 20))
+                                                : p->D > 80 && p->D <= 96 && (p->B > 64 || (M > 64 && p->T >= 2)) && heads_bytes >= (32ll << 20));
     if (long_rows) return true;
     const bool uneven_128 = p->B > 96 && M > 96 && heads % 8 != 0;
     // 128-row blocks in 33 .. 48 blocks (three-strip L / Z problems beside eight-strip R problems) on a head count that

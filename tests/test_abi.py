@@ -298,6 +298,12 @@ def test_auto_variant_policy():
     assert auto(512, 16, 1024, 64, 32) == "staged"      # more heads than the chained kernel has flag words for
     assert auto(2, 16, 8192, 64, 64) == "chained"       # 128 blocks of 64 rows (long documents), head dim 64
     assert auto(2, 16, 8192, 128, 64) == "staged"       # ... but not for wide heads
+    assert auto(1, 16, 8192, 128, 64) == "chained"      # ... under 48 MB a tensor
+    assert auto(8, 8, 8192, 72, 64) == "staged"         # D = 72, 128 blocks, 72 MB a tensor: with more than one step
+    assert auto(8, 8, 8192, 72, 64, T=1) == "chained"
+    assert auto(8, 8, 8192, 72, 96) == "chained"        # 65 .. 96 rows: only at the head dims of the 96-column class
+    assert auto(8, 8, 8192, 96, 96) == "staged"
+    assert auto(4, 8, 8192, 128, 96) == "chained"
     assert auto(2, 16, 5000, 64, 64) == "chained"       # 79 blocks: the 96-row class
     assert auto(1, 2, 8192, 64, 64) == "staged"         # two long heads would run on two of the eight XCDs
     assert auto(2, 2, 197, 64, 16) == "resident"        # few short heads in 16-row blocks, two steps: whole in LDS
