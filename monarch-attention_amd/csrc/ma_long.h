@@ -1,8 +1,9 @@
 // fp16 / bf16 R, L and Z steps of long block problems as per-stage launches: 65 .. 128 rows (*_pair) and 129 .. 256 rows
 // (*_long).  The operand tiles of a problem are in LDS once, its waves walk the 16-row strips.
 //
-// What bounds them: the softmax arithmetic (an R step of 256 rows at D = 64 spends 57 % of its time on the VALU, 25 % on the
-// matrix pipes, and moves its bytes in 66 %) and, at wide head dims, how many waves fit beside the tiles.  So
+// What bounds them: the softmax arithmetic (48 heads of 65536 tokens, D = 64, 256 rows: the R step with V issues vector
+// instructions 45 % of its time, the Z step 58 %, the matrix pipes are busy 19 - 20 %, the traffic runs at 62 - 76 % of a copy's
+// rate) and, at wide head dims, how many waves fit beside the tiles.  So
 //  * problems of up to 128 rows run two strips per wave side by side, so that an operand fragment read from LDS feeds two
 //    matrix instructions (their arithmetic is that of ma_mfma.h to the bit: the chained kernel runs such problems too);
 //  * longer ones loop over their strips, with the next strip's rows loaded ahead, in as many waves as registers and LDS allow
