@@ -1098,7 +1098,8 @@ __global__ __launch_bounds__(NTH) void r_bwd_mfma16(Problem P, BwdBuffers G, int
         }
         for (int jj = threadIdx.x; jj < TJ; jj += NTH) {
             const bool in = j0 + jj < B;
-            c[jj] = 1.0f / (((first || !in) ? 1.0f : cR[j0 + jj]) + P.eps);   // c holds 1 / (cR + eps)
+            const float cr = (first || !in) ? 1.0f : cR[j0 + jj];
+            c[jj] = cr == 0.f ? 0.f : 1.0f / (cr + P.eps);   // c holds 1 / (cR + eps); 0 where no query is live (over_cr in ma_bwd_tile.h)
             gcl[jj] = in ? G.gcL[(eh * B + j0 + jj) * M + k] : 0.f;
         }
         __syncthreads();
