@@ -90,7 +90,7 @@ def test_captured_module_call_replays_like_eager(case):
         return out
 
     side.wait_stream(torch.cuda.current_stream())
-    want = eager()   # warm-up: the call plan and the workspace of this stream exist before the capture
+    want = eager()   # warm-up: the workspace of this stream exists before the capture
     assert_parity(want.cpu(), monarch_attention_oracle(q.cpu(), k.cpu(), v.cpu(), None, T, B, False), dt, f"eager case {case}")
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=side):
