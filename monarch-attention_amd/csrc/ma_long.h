@@ -728,8 +728,10 @@ __global__ __launch_bounds__(64 * W, EU) void l_step_long(Problem P) {
 // ---------------------------------------------------------------- launches
 // Waves per workgroup and waves per SIMD asked of the compiler, by stage (kV: R step with V), 16-column tiles and strips.
 // D <= 64: two workgroups of 256 rows fit the LDS; the R step holds most registers and runs best in 4 waves, the others in 8.
-// Wider rows: the LDS holds one workgroup at 192 / 256 rows, which then takes as many waves as there are strips (an R step
-// without V keeps one tile only: narrow workgroups, more of them).
+// Wider rows: the LDS holds one workgroup at 192 / 256 rows, which then takes many waves - as many as there are strips where
+// registers allow -; an R step without V of up to 192 rows keeps one tile only: narrow workgroups, more of them.  Measured over
+// W = 4 .. 16 and EU = 1 .. 4 on six shapes: within 3 % of the best setting but for an R step without V of 256 wide rows (4
+// waves: 0.89) and one with V of 160 rows at D = 96 (EU = 3: 0.92).
 template <int STAGE, bool kV, int DT, int NWT>
 struct Cfg {
     static constexpr bool kWideRow = DT > 4, k16 = NWT == 16, kR = STAGE == kStageR;
