@@ -1,22 +1,26 @@
 // fp16 / bf16 R, L and Z steps of long block problems as per-stage launches: 65 .. 128 rows (*_pair) and 129 .. 256 rows
 // (*_long).  The operand tiles of a problem are in LDS once, its waves walk the 16-row strips.
 //
-// What bounds them: the softmax arithmetic (48 heads of 65536 tokens, D = 64, 256 rows: the R step with V issues vector
-// instructions 45 % of its time, the Z step 58 %, the matrix pipes are busy 19 - 20 %, the traffic runs at 62 - 76 % of a copy's
-// rate) and, at wide head dims, how many waves fit beside the tiles.  So
+// What bounds them: the softmax arithmetic (48 heads of 65536 tokens, D = 64, 256 rows: vector instructions take half of the
+// cycles, at a clock that the power limit holds at 2 GHz), then the traffic (the Z step moves 1.6 GB at 4.3 TB/s, the R step with V
+// 2.1 GB at 3.9) and, at wide head dims, how many waves fit beside the tiles.  So
 //  * problems of up to 128 rows run two strips per wave side by side, so that an operand fragment read from LDS feeds two
 //    matrix instructions (their arithmetic is that of ma_mfma.h to the bit: the chained kernel runs such problems too);
-//  * longer ones loop over their strips, with the next strip's rows loaded ahead, in as many waves as registers and LDS allow
-//    (Cfg below).  Their logits are packed to 16 bits as they leave the first product (they are rounded to the operand type
-//    there anyway) and the probabilities take their place: half the accumulator registers; probabilities enter the second
-//    product unnormalised, relative to the largest of their row (at most 1, at least as large as the normalised ones), and
-//    its result is divided by their sum - the same relative rounding, one multiplication per entry less -, the exponent is
-//    one FMA from the packed logit;
+//  * longer ones loop over their strips, with the next strips' rows loaded ahead, in as many waves as registers and LDS allow
+//    (Cfg below);
+//  * of those, the R step packs its logits to 16 bits as they leave the first product (the reference rounds them there) and puts
+//    the probabilities in their place, half the accumulator registers; the L and Z steps start the accumulators of the first
+//    product at the bias and keep the sums in fp32, so that an exponent is one FMA and nothing is rounded on the way;
+//  * probabilities enter the second product unnormalised, relative to the largest of their row (at most 1, at least as large as
+//    the normalised ones), and its result is divided by their sum - the same relative rounding, one multiplication per entry less;
 //  * head dims of 81 .. 96 have a column class of their own.
-// Measured before (the kernels of ma_mfma.h) -> after, one launch: 32 heads of 16384, D = 96, 160-row blocks: R step 158 ->
-// 94 us (with V 221 -> 156); 16 heads of 32768, D = 128, 181 rows: L step 259 -> 164, R with V 236 -> 192; 48 heads of
-// 65536, D = 64, 256 rows: Z step 432 -> 403, L step 604 -> 571; 16 heads of 5003, D = 128, 72 rows: R with V 29.5 -> 24.8,
-// L step 24.0 -> 21.5.
+// Vector instructions a strip of 256 rows (D = 64): R step with V 590 -> 467 (packing that the compiler had put off to the second
+// product, maxima that quietened every operand, a branch per tile for masked blocks), Z step 430 -> 317.
+// Measured, one launch, kernels of ma_mfma.h -> two strips / strip loops -> as they stand: 32 heads of 16384, D = 96, 160-row
+// blocks: R step 158 -> 94 -> 90 us (with V 221 -> 156 -> 147); 16 heads of 32768, D = 128, 181 rows: L step 259 -> 169 -> 162, R
+// with V 236 -> 204 -> 193; 16 heads of 65536, D = 128, 256 rows: R with V 423 -> 370, L 345 -> 303, Z 307 -> 265 (the last
+// two); 48 heads of 65536, D = 64, 256 rows: R 478 -> 400, R with V 610 -> 530, L 591 -> 486, Z step 432 -> 408 -> 378; 16 heads of
+// 5003, D = 128, 72 rows: R with V 29.5 -> 24.8, L step 24.0 -> 21.5.
 #pragma once
 
 #include "ma_tile.h"
@@ -45,6 +49,13 @@ struct Pack {
 #pragma unroll
         for (int v = 0; v < 4; ++v) a[v] = mfma::fp32_value(a[v] * f);
         return four(a);
+    }
+    // ... as two registers here and now: left to itself the compiler keeps the four values as they are (twice the registers)
+    // and converts them where they are used
+    static __device__ __forceinline__ V4 four_now(const f32x4& a) {
+        u32x2 p = __builtin_bit_cast(u32x2, four(a));
+        asm("" : "+v"(p));
+        return __builtin_bit_cast(V4, p);
     }
     static __device__ __forceinline__ V8 eight(const V4& a, const V4& b) {
         const u32x2 lo = __builtin_bit_cast(u32x2, a), hi = __builtin_bit_cast(u32x2, b);
@@ -426,39 +437,69 @@ __global__ __launch_bounds__(64 * W) void l_step_pair(Problem P) {
 }
 
 // ================================================================ 129 .. 256 rows: strips one after the other
-// O[dt] += sum_w tile[w][columns of dt] P[w] over NWT tiles
-template <class T, int DT, int NWT>
-__device__ __forceinline__ void gemm2(f32x4 (&O)[DT], const T* tile, const typename Pack<T>::V4 (&Pk)[NWT], int r, int q) {
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) O[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int g = 0; g < NWT / 2; ++g) {
-        const auto p = Pack<T>::eight(Pk[2 * g], Pk[2 * g + 1]);
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) O[dt] = mfma::Ops<T>::mma(mfma::lds_tr8<T, DT, mfma::kTile>(tile, 32 * g + 4 * q, 16, true, dt, r), p, O[dt]);
-    }
+// The largest of five values in two instructions (v_maximum3_f32; fmaxf on a matrix product's result takes one more per operand,
+// which quietens a signalling NaN first)
+__device__ __forceinline__ float max5(float m, const f32x4& a) {
+    return __builtin_elementwise_maximum(__builtin_elementwise_maximum(__builtin_elementwise_maximum(__builtin_elementwise_maximum(m, a[0]), a[1]), a[2]), a[3]);
 }
-// logits of a strip against NWT tiles of rows, rounded to T; per tile f(w, accumulators)
-template <class T, int DT, int NWT, class F>
-__device__ __forceinline__ void gemm1(typename Pack<T>::V4 (&C)[NWT], const T* tile, const typename Mat<T, DT>::Row& x, int r, int q, F&& f) {
+// O[s][dt] = sum_w tile[w][columns of dt] P[s][w] over NWT tiles
+template <class T, int DT, int NWT, int SP>
+__device__ __forceinline__ void gemm2(f32x4 (&O)[SP][DT], const T* tile, const typename Pack<T>::V4 (&Pk)[SP][NWT], int r, int q) {
+    zero(O);
+    gemm2_pair<T, DT, NWT, SP>(O, tile, Pk, r, q);
+}
+// logits of SP strips against NWT tiles of rows, rounded to T; per strip and tile f(s, w, accumulators)
+template <class T, int DT, int NWT, int SP, class F>
+__device__ __forceinline__ void gemm1(typename Pack<T>::V4 (&C)[SP][NWT], const T* tile, const typename Mat<T, DT>::Row (&x)[SP], int r, int q, F&& f) {
+    using MT = Mat<T, DT>;
 #pragma unroll
     for (int w = 0; w < NWT; ++w) {
-        f32x4 a = {0.f, 0.f, 0.f, 0.f};
-        Mat<T, DT>::gemm1(tile, w, r, q, x, a);
-        C[w] = Pack<T>::four(a);
-        f(w, a);
+        f32x4 a[SP];
+#pragma unroll
+        for (int s = 0; s < SP; ++s) a[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < MT::KS; ++ks) {
+            const auto t = mfma::lds_row8<T>(tile + MT::at(16 * w + r, 4 * ks + q));
+#pragma unroll
+            for (int s = 0; s < SP; ++s) a[s] = mfma::Ops<T>::mma(t, x[s].x[ks], a[s]);
+        }
+#pragma unroll
+        for (int s = 0; s < SP; ++s) {
+            C[s][w] = Pack<T>::four_now(a[s]);
+            f(s, w, a[s]);
+        }
         if (w % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // (keeps the tile reads of the whole strip from being hoisted: registers)
     }
 }
 
+// ... in fp32, plus bias[w] (the accumulators start there); per strip and tile f(s, w)
+template <class T, int DT, int NWT, int SP, class F>
+__device__ __forceinline__ void gemm1_biased(f32x4 (&U)[SP][NWT], const T* tile, const float* bias, const typename Mat<T, DT>::Row (&x)[SP], int r, int q, F&& f) {
+    using MT = Mat<T, DT>;
+#pragma unroll
+    for (int w = 0; w < NWT; ++w) {
+#pragma unroll
+        for (int s = 0; s < SP; ++s) U[s][w] = *reinterpret_cast<const f32x4*>(bias + 16 * w + 4 * q);
+#pragma unroll
+        for (int ks = 0; ks < MT::KS; ++ks) {
+            const auto t = mfma::lds_row8<T>(tile + MT::at(16 * w + r, 4 * ks + q));
+#pragma unroll
+            for (int s = 0; s < SP; ++s) U[s][w] = mfma::Ops<T>::mma(t, x[s].x[ks], U[s][w]);
+        }
+#pragma unroll
+        for (int s = 0; s < SP; ++s) f(s, w);
+        if (w % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
 // ---------------------------------------------------------------- R step
-template <class T, int DT, int NWT, int W, int EU, bool kV>
+template <class T, int DT, int NWT, int W, int EU, int SP, bool kV>
 __global__ __launch_bounds__(64 * W, EU) void r_step_long(Problem P, int first) {
     using MT = Mat<T, DT>;
     using PL = typename std::conditional<kV, RPlan<T, DT, NWT>, KPlan<T, DT, NWT>>::type;
     using V4 = typename Pack<T>::V4;
-    constexpr int NTH = 64 * W, ROWS = 16 * NWT, SPW = NWT / W;
-    static_assert(PL::NC1 == 1 && NWT % W == 0, "the problem's tiles fit the LDS");
+    constexpr int NTH = 64 * W, ROWS = 16 * NWT, GROUPS = NWT / (W * SP);
+    static_assert(PL::NC1 == 1 && NWT % (W * SP) == 0, "the problem's tiles fit the LDS");
     extern __shared__ __attribute__((aligned(16))) char lds_raw[];
     T* Kt = reinterpret_cast<T*>(lds_raw);
     T* Vt = Kt + ROWS * MT::LD;
@@ -474,19 +515,23 @@ __global__ __launch_bounds__(64 * W, EU) void r_step_long(Problem P, int first) 
     const bool masked = P.mask != nullptr || B != ROWS || t0 < 0 || t0 + B > P.N;   // uniform: some keys are masked or padding
     const rsrc_t sx = first ? token_slice<T>(P.q, P.qs, e, h, P.N, D) : state_slice(P.aR, eh, np, row_b), scR = state_slice(P.cR, eh, np, 4);
     const unsigned qst = static_cast<unsigned>(P.qs[2]) * sizeof(T);
-    typename MT::Row xn;
-    float cn = 1.f;
-    auto fetch = [&](int j) {   // query row j of the block and its normaliser
-        const unsigned rowid = static_cast<unsigned>(k * B + j);
-        MT::load(xn, sx, j >= B ? kOob : first ? mfma::tok_off(t0 + j, P.N, qst) : rowid * row_b, D, true, q);
-        if (!first) cn = mfma::bloadf<0>(scR, j < B ? rowid * 4u : kOob);
+    typename MT::Row xn[SP];
+    float cn[SP];
+    auto fetch = [&](int g) {   // query rows of the wave's group g of strips and their normalisers
+#pragma unroll
+        for (int s = 0; s < SP; ++s) {
+            const int j = 16 * (SP * (wave + g * W) + s) + r;
+            const unsigned rowid = static_cast<unsigned>(k * B + j);
+            MT::load(xn[s], sx, j >= B ? kOob : first ? mfma::tok_off(t0 + j, P.N, qst) : rowid * row_b, D, true, q);
+            cn[s] = first ? 1.f : mfma::bloadf<0>(scR, j < B ? rowid * 4u : kOob);
+        }
     };
     {
         const rsrc_t sk = token_slice<T>(P.k, P.ks, e, h, P.N, D), sv = token_slice<T>(P.v, P.vs, e, h, P.N, D);
         const unsigned kst = static_cast<unsigned>(P.ks[2]) * sizeof(T), vst = static_cast<unsigned>(P.vs[2]) * sizeof(T);
         TileIn<MT, T, ROWS, NTH> kc, vc;
         kc.issue(sk, D, true, [&](int i) { return i < B ? mfma::tok_off(t0 + i, P.N, kst) : kOob; });
-        fetch(16 * wave + r);
+        fetch(0);
         if (kV) vc.issue(sv, D, true, [&](int i) { return i < B ? mfma::tok_off(t0 + i, P.N, vst) : kOob; });
         if (masked)
             for (int i = threadIdx.x; i < ROWS; i += NTH) kbias[i] = (i < B && token_ok(P, e, t0 + i)) ? 0.f : kNegBig;
@@ -495,81 +540,100 @@ __global__ __launch_bounds__(64 * W, EU) void r_step_long(Problem P, int first) 
     }
     __syncthreads();
 
+    // (One branch around the whole loop: a branch per tile would end the scheduling of its reads and products there.)
+    auto strips = [&](auto has_mask) {
+        constexpr bool kMasked = decltype(has_mask)::value;
 #pragma unroll 1
-    for (int si = 0; si < SPW; ++si) {
-        const int j = 16 * (wave + si * W) + r;
-        const typename MT::Row xb = xn;
-        const float cj = (P.sm_scale * kLog2e) * mfma::rcp(cn + P.eps);   // logits in log2 units
-        if (si + 1 < SPW) fetch(j + 16 * W);
-        V4 C[NWT];
-        float mx = -INFINITY;
-        gemm1<T, DT, NWT>(C, Kt, xb, r, q, [&](int w, f32x4 a) {
-            if (masked) a += *reinterpret_cast<const f32x4*>(kbias + 16 * w + 4 * q);
-            // (rounding is monotonic: the largest rounded logit is the largest logit, rounded)
-            mx = fmaxf(mx, fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3])));
-        });
-        // The row maximum is clamped from below (ma_torch.py:15), so a row whose logits are all negative has probabilities far
-        // below 1, which 16 bits would not hold (fp16: two bits at a maximum of -15, zero below -17).  So p is formed from
-        // the row's own maximum and `shift` octaves are put back per row, in fp32.  60 octaves are enough (eps, at -40, rules
-        // the sum long before) and keep the rows of fully masked blocks at 0.  (A few
-        // instructions a row: 48 heads of 65536 tokens, D = 64, 256 rows, one step: 996.2 us without, 996.3 with.)
-        mx = round_to<T>(mfma::quad_rows_max(mx)) * cj;
-        const float clamped = fmaxf(mx, P.eps * kLog2e);
-        mx = fmaxf(mx, clamped - 60.f);
-        const float shift = mx - clamped, scale = __builtin_amdgcn_exp2f(shift);
-        float sum = 0.f, ent = 0.f;
-        auto softmax = [&](auto has_mask) {
-            constexpr bool kMasked = decltype(has_mask)::value;
+        for (int g = 0; g < GROUPS; ++g) {
+            const int s0 = 16 * SP * (wave + g * W);
+            typename MT::Row xb[SP];
+            float cj[SP];
 #pragma unroll
-            for (int w = 0; w < NWT; ++w) {
-                f32x4 p, b = {-mx, -mx, -mx, -mx};
-                if (kMasked) b += *reinterpret_cast<const f32x4*>(kbias + 16 * w + 4 * q);
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const float d = fmaf(to_f(C[w][v]), cj, b[v]);
-                    p[v] = __builtin_amdgcn_exp2f(d);
-                    sum += p[v];
-                    ent = fmaf(p[v], d, ent);   // sum p log2 p
-                }
-                C[w] = Pack<T>::four(p);
-                if (w % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            for (int s = 0; s < SP; ++s) {
+                xb[s] = xn[s];
+                cj[s] = (P.sm_scale * kLog2e) * mfma::rcp(cn[s] + P.eps);   // logits in log2 units
             }
-        };
-        if (masked) softmax(std::true_type{});
-        else softmax(std::false_type{});
-        sum = mfma::quad_rows_sum(sum);
-        ent = mfma::quad_rows_sum(ent);
-        const float den = fmaf(scale, sum, P.eps), inv = scale * mfma::rcp(den);
-        const unsigned lrow = static_cast<unsigned>(j * M + k);   // row of aL / cL / Y: (j, k)
-        if (q == 0)   // cL = sum_i r log r with r = p scale / den (ma_torch.py:20)
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, kLn2 * (ent * inv + (shift - mfma::log2_normal(den)) * (sum * inv))),
-                                                  state_slice(P.cL, eh, np, 4), j < B ? lrow * 4u : kOob, 0, 0);
-        f32x4 O[DT];
-        gemm2<T, DT, NWT>(O, Kt, C, r, q);
+            if (g + 1 < GROUPS) fetch(g + 1);
+            V4 C[SP][NWT];
+            float mxs[SP], invs[SP];
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+            for (int s = 0; s < SP; ++s) mxs[s] = -INFINITY;
+            gemm1<T, DT, NWT, SP>(C, Kt, xb, r, q, [&](int s, int w, f32x4 a) {
+                // (rounding is monotonic: the largest rounded logit is the largest logit, rounded)
+                mxs[s] = max5(mxs[s], kMasked ? a + *reinterpret_cast<const f32x4*>(kbias + 16 * w + 4 * q) : a);
+            });
 #pragma unroll
-            for (int v = 0; v < 4; ++v) O[dt][v] = P.sm_scale * round_to<T>(O[dt][v] * inv);
-        MT::store(state_slice(P.aL, eh, np, row_b), j < B ? lrow * row_b : kOob, D, O, q, true);
-        if (kV) {
-            gemm2<T, DT, NWT>(O, Vt, C, r, q);
+            for (int s = 0; s < SP; ++s) {
+                const int j = s0 + 16 * s + r;
+                // The row maximum is clamped from below (ma_torch.py:15), so a row whose logits are all negative has probabilities far
+                // below 1, which 16 bits would not hold (fp16: two bits at a maximum of -15, zero below -17).  So p is formed from
+                // the row's own maximum and `shift` octaves are put back per row, in fp32.  60 octaves are enough (eps, at -40, rules
+                // the sum long before) and keep the rows of fully masked blocks at 0.  (A few
+                // instructions a row: 48 heads of 65536 tokens, D = 64, 256 rows, one step: 996.2 us without, 996.3 with.)
+                float mx = round_to<T>(mfma::quad_rows_max(mxs[s])) * cj[s];
+                const float clamped = fmaxf(mx, P.eps * kLog2e);
+                mx = fmaxf(mx, clamped - 60.f);
+                const float shift = mx - clamped, scale = __builtin_amdgcn_exp2f(shift);
+                float sum = 0.f, ent = 0.f;
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
+                    for (int w = 0; w < NWT; ++w) {
+                        f32x4 p, b = {-mx, -mx, -mx, -mx};
+                        if (kMasked) b += *reinterpret_cast<const f32x4*>(kbias + 16 * w + 4 * q);
 #pragma unroll
-                for (int v = 0; v < 4; ++v) O[dt][v] *= inv;
-            MT::store(state_slice(P.Y, eh, np, row_b), j < B ? lrow * row_b : kOob, D, O, q, true);
+                        for (int v = 0; v < 4; ++v) {
+                            const float d = fmaf(to_f(C[s][w][v]), cj[s], b[v]);
+                            p[v] = __builtin_amdgcn_exp2f(d);
+                            sum += p[v];
+                            ent = fmaf(p[v], d, ent);   // sum p log2 p
+                        }
+                        C[s][w] = Pack<T>::four_now(p);
+                        if (w % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                    }
+                sum = mfma::quad_rows_sum(sum);
+                ent = mfma::quad_rows_sum(ent);
+                const float den = fmaf(scale, sum, P.eps);
+                invs[s] = scale * mfma::rcp(den);
+                if (q == 0)   // cL = sum_i r log r with r = p scale / den (ma_torch.py:20); row of aL / cL / Y: (j, k)
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, kLn2 * (ent * invs[s] + (shift - mfma::log2_normal(den)) * (sum * invs[s]))),
+                                                          state_slice(P.cL, eh, np, 4), j < B ? static_cast<unsigned>(j * M + k) * 4u : kOob, 0, 0);
+            }
+            f32x4 O[SP][DT];
+            gemm2<T, DT, NWT, SP>(O, Kt, C, r, q);
+#pragma unroll
+            for (int s = 0; s < SP; ++s) {
+                const int j = s0 + 16 * s + r;
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) O[s][dt][v] = P.sm_scale * round_to<T>(O[s][dt][v] * invs[s]);
+                MT::store(state_slice(P.aL, eh, np, row_b), j < B ? static_cast<unsigned>(j * M + k) * row_b : kOob, D, O[s], q, true);
+            }
+            if (kV) {
+                gemm2<T, DT, NWT, SP>(O, Vt, C, r, q);
+#pragma unroll
+                for (int s = 0; s < SP; ++s) {
+                    const int j = s0 + 16 * s + r;
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) O[s][dt][v] *= invs[s];
+                    MT::store(state_slice(P.Y, eh, np, row_b), j < B ? static_cast<unsigned>(j * M + k) * row_b : kOob, D, O[s], q, true);
+                }
+            }
         }
-    }
+    };
+    if (masked) strips(std::true_type{});
+    else strips(std::false_type{});
 }
 
 // ---------------------------------------------------------------- Z step
-template <class T, int DT, int NWT, int W, int EU>
+template <class T, int DT, int NWT, int W, int EU, int SP>
 __global__ __launch_bounds__(64 * W, EU) void z_step_long(Problem P) {
     using MT = Mat<T, DT>;
     using PL = RPlan<T, DT, NWT>;
     using V4 = typename Pack<T>::V4;
-    constexpr int NTH = 64 * W, ROWS = 16 * NWT, SPW = NWT / W;
-    static_assert(PL::NC1 == 1 && NWT % W == 0, "the problem's tiles fit the LDS");
+    constexpr int NTH = 64 * W, ROWS = 16 * NWT, GROUPS = NWT / (W * SP);
+    static_assert(PL::NC1 == 1 && NWT % (W * SP) == 0, "the problem's tiles fit the LDS");
     extern __shared__ __attribute__((aligned(16))) char lds_raw[];
     T* At = reinterpret_cast<T*>(lds_raw);
     T* Yt = At + ROWS * MT::LD;
@@ -583,68 +647,82 @@ __global__ __launch_bounds__(64 * W, EU) void z_step_long(Problem P) {
     const unsigned row_b = D * static_cast<unsigned>(sizeof(T)), jm = static_cast<unsigned>(j) * M;
     const rsrc_t sq = token_slice<T>(P.q, P.qs, e, h, P.N, D), so = token_slice<T>(P.out, P.os, e, h, P.N, D);
     const unsigned qst = static_cast<unsigned>(P.qs[2]) * sizeof(T), ost = static_cast<unsigned>(P.os[2]) * sizeof(T);
-    typename MT::Row xn;
-    auto fetch = [&](int l) { MT::load(xn, sq, l < M ? mfma::tok_off(l * B + j - P.pad_off, P.N, qst) : kOob, D, true, q); };
+    typename MT::Row xn[SP];
+    auto fetch = [&](int g) {   // query rows of the wave's group g of strips
+#pragma unroll
+        for (int s = 0; s < SP; ++s) {
+            const int l = 16 * (SP * (wave + g * W) + s) + r;
+            MT::load(xn[s], sq, l < M ? mfma::tok_off(l * B + j - P.pad_off, P.N, qst) : kOob, D, true, q);
+        }
+    };
     {
         const rsrc_t scL = state_slice(P.cL, eh, np, 4);
         auto a_off = [&](int k) { return k < M ? (jm + k) * row_b : kOob; };
         TileIn<MT, T, ROWS, NTH> ac, yc;
         ac.issue(state_slice(P.aL, eh, np, row_b), D, true, a_off);
-        fetch(16 * wave + r);
+        fetch(0);
         yc.issue(state_slice(P.Y, eh, np, row_b), D, true, a_off);
-        for (int k = threadIdx.x; k < ROWS; k += NTH) cb[k] = k < M ? -kLog2e * mfma::bloadf<0>(scL, (jm + k) * 4u) : kNegBig;
+        for (int k = threadIdx.x; k < ROWS; k += NTH) cb[k] = k < M ? -mfma::bloadf<0>(scL, (jm + k) * 4u) : kNegBig;
         ac.commit(At);
         yc.commit(Yt);
     }
     __syncthreads();
 
 #pragma unroll 1
-    for (int si = 0; si < SPW; ++si) {
-        const int l = 16 * (wave + si * W) + r;
-        const typename MT::Row xq = xn;
-        if (si + 1 < SPW) fetch(l + 16 * W);
-        V4 C[NWT];
-        float mx = -INFINITY, sum = 0.f;
-        gemm1<T, DT, NWT>(C, At, xq, r, q, [&](int w, f32x4) {
-            const f32x4 b = *reinterpret_cast<const f32x4*>(cb + 16 * w + 4 * q);
+    for (int g = 0; g < GROUPS; ++g) {
+        const int s0 = 16 * SP * (wave + g * W);
+        typename MT::Row xq[SP];
 #pragma unroll
-            for (int v = 0; v < 4; ++v) mx = fmaxf(mx, fmaf(to_f(C[w][v]), kLog2e, b[v]));
-        });
-        mx = mfma::quad_rows_max(mx);
+        for (int s = 0; s < SP; ++s) xq[s] = xn[s];
+        if (g + 1 < GROUPS) fetch(g + 1);
+        V4 C[SP][NWT];
+        float mxs[SP], invs[SP];
 #pragma unroll
-        for (int w = 0; w < NWT; ++w) {
-            const f32x4 b = *reinterpret_cast<const f32x4*>(cb + 16 * w + 4 * q);
-            f32x4 p;
+        for (int s = 0; s < SP; ++s) mxs[s] = -INFINITY;
+        f32x4 U[SP][NWT];
+        gemm1_biased<T, DT, NWT, SP>(U, At, cb, xq, r, q, [&](int s, int w) { mxs[s] = max5(mxs[s], U[s][w]); });
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                p[v] = __builtin_amdgcn_exp2f(fmaf(to_f(C[w][v]), kLog2e, b[v] - mx));
-                sum += p[v];
+        for (int s = 0; s < SP; ++s) {
+            const float mx = kLog2e * mfma::quad_rows_max(mxs[s]);
+            float sum = 0.f;
+#pragma unroll
+            for (int w = 0; w < NWT; ++w) {
+                f32x4 p;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    p[v] = __builtin_amdgcn_exp2f(fmaf(U[s][w][v], kLog2e, -mx));
+                    sum += p[v];
+                }
+                C[s][w] = Pack<T>::four_now(p);
+                if (w % 4 == 3) __builtin_amdgcn_sched_barrier(0);
             }
-            C[w] = Pack<T>::four(p);
-            if (w % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            invs[s] = mfma::rcp(mfma::quad_rows_sum(sum));
         }
-        const float inv = mfma::rcp(mfma::quad_rows_sum(sum));
-        f32x4 O[DT];
-        gemm2<T, DT, NWT>(O, Yt, C, r, q);
+        f32x4 O[SP][DT];
+        gemm2<T, DT, NWT, SP>(O, Yt, C, r, q);
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+        for (int s = 0; s < SP; ++s) {
+            const int l = s0 + 16 * s + r;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) O[dt][v] *= inv;
-        // padded query rows are dropped (ma_torch.py:108)
-        MT::store(so, l < M ? mfma::tok_off(l * B + j - P.pad_off, P.N, ost) : kOob, D, O, q, true);
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) O[s][dt][v] *= invs[s];
+            // padded query rows are dropped (ma_torch.py:108)
+            MT::store(so, l < M ? mfma::tok_off(l * B + j - P.pad_off, P.N, ost) : kOob, D, O[s], q, true);
+        }
     }
 }
 
 // ---------------------------------------------------------------- L step
-// Pass 1, strips of query blocks: c_l = log2(mask / sum) - max of each row, to LDS.  Pass 2, strips of key blocks:
-// L[l,k] = exp2(x log2e + c_l) 2^(-log2e cL_k).
-template <class T, int DT, int NWT, int W, int EU>
+// Pass 1, strips of query blocks: c_l = log(mask / sum) - max of each row, to LDS.  Pass 2, strips of key blocks:
+// L[l,k] = exp(x + c_l - cL_k).
+template <class T, int DT, int NWT, int W, int EU, int SP>
 __global__ __launch_bounds__(64 * W, EU) void l_step_long(Problem P) {
     using MT = Mat<T, DT>;
     using PL = LPlan<T, DT, NWT>;
     using V4 = typename Pack<T>::V4;
-    constexpr int NTH = 64 * W, ROWS = 16 * NWT, SPW = NWT / W;
-    static_assert(PL::NC1 == 1 && NWT % W == 0, "the problem's tiles fit the LDS");
+    constexpr int NTH = 64 * W, ROWS = 16 * NWT, GROUPS = NWT / (W * SP);
+    static_assert(PL::NC1 == 1 && NWT % (W * SP) == 0, "the problem's tiles fit the LDS");
     extern __shared__ __attribute__((aligned(16))) char lds_raw[];
     T* At = reinterpret_cast<T*>(lds_raw);
     T* Qt = At + ROWS * MT::LD;
@@ -664,7 +742,7 @@ __global__ __launch_bounds__(64 * W, EU) void l_step_long(Problem P) {
         ac.issue(state_slice(P.aL, eh, np, row_b), D, true, [&](int k) { return k < M ? (jm + k) * row_b : kOob; });
         qc.issue(sq, D, true, [&](int l) { return l < M ? mfma::tok_off(l * B + j - P.pad_off, P.N, qst) : kOob; });
         for (int k = threadIdx.x; k < ROWS; k += NTH) {
-            cb[k] = k < M ? -kLog2e * mfma::bloadf<0>(scL, (jm + k) * 4u) : kNegBig;
+            cb[k] = k < M ? -mfma::bloadf<0>(scL, (jm + k) * 4u) : kNegBig;
             // padded / masked queries are zeroed after the softmax (ma_torch.py:30)
             cs[k] = (k < M && token_ok(P, e, k * B + j - P.pad_off)) ? 0.f : -INFINITY;
         }
@@ -673,72 +751,81 @@ __global__ __launch_bounds__(64 * W, EU) void l_step_long(Problem P) {
     }
     __syncthreads();
 #pragma unroll 1
-    for (int si = 0; si < SPW; ++si) {
-        const int s0 = 16 * (wave + si * W);
-        typename MT::Row xq;
-        MT::from_tile(xq, Qt, s0 + r, q);
-        V4 C[NWT];
-        float mx = -INFINITY, sum = 0.f;
-        gemm1<T, DT, NWT>(C, At, xq, r, q, [&](int w, f32x4) {
-            const f32x4 b = *reinterpret_cast<const f32x4*>(cb + 16 * w + 4 * q);
+    for (int g = 0; g < GROUPS; ++g) {
+        const int s0 = 16 * SP * (wave + g * W);
+        typename MT::Row xq[SP];
 #pragma unroll
-            for (int v = 0; v < 4; ++v) mx = fmaxf(mx, fmaf(to_f(C[w][v]), kLog2e, b[v]));
-        });
-        mx = mfma::quad_rows_max(mx);
+        for (int s = 0; s < SP; ++s) MT::from_tile(xq[s], Qt, s0 + 16 * s + r, q);
+        f32x4 U[SP][NWT];
+        float mxs[SP];
 #pragma unroll
-        for (int w = 0; w < NWT; ++w) {
-            const f32x4 b = *reinterpret_cast<const f32x4*>(cb + 16 * w + 4 * q);
+        for (int s = 0; s < SP; ++s) mxs[s] = -INFINITY;
+        gemm1_biased<T, DT, NWT, SP>(U, At, cb, xq, r, q, [&](int s, int w) { mxs[s] = max5(mxs[s], U[s][w]); });
 #pragma unroll
-            for (int v = 0; v < 4; ++v) sum += __builtin_amdgcn_exp2f(fmaf(to_f(C[w][v]), kLog2e, b[v] - mx));
-            if (w % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        for (int s = 0; s < SP; ++s) {
+            const float mx = mfma::quad_rows_max(mxs[s]), m2 = kLog2e * mx;
+            float sum = 0.f;
+#pragma unroll
+            for (int w = 0; w < NWT; ++w) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) sum += __builtin_amdgcn_exp2f(fmaf(U[s][w][v], kLog2e, -m2));
+                if (w % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+            const float c = fmaf(kLn2, mfma::log2_normal(mfma::quad_rows_sum(sum)), mx);
+            if (q == 0) cs[s0 + 16 * s + r] -= c;
         }
-        const float c = mfma::log2_normal(mfma::quad_rows_sum(sum)) + mx;
-        if (q == 0) cs[s0 + r] -= c;
     }
     __syncthreads();
 #pragma unroll 1
-    for (int si = 0; si < SPW; ++si) {
-        const int k = 16 * (wave + si * W) + r;
-        typename MT::Row ak;
-        MT::from_tile(ak, At, k, q);
-        const float eb = __builtin_amdgcn_exp2f(cb[k]);   // (cL in [-log B, 0]: 1 .. B; 0 beyond the M key blocks)
-        V4 C[NWT];
-        float cr = 0.f;
-        gemm1<T, DT, NWT>(C, Qt, ak, r, q, [&](int w, f32x4) {
-            const f32x4 c = *reinterpret_cast<const f32x4*>(cs + 16 * w + 4 * q);
+    for (int g = 0; g < GROUPS; ++g) {
+        const int s0 = 16 * SP * (wave + g * W);
+        typename MT::Row ak[SP];
+        float ck[SP], cr[SP];
+#pragma unroll
+        for (int s = 0; s < SP; ++s) {
+            MT::from_tile(ak[s], At, s0 + 16 * s + r, q);
+            ck[s] = kLog2e * cb[s0 + 16 * s + r];
+            cr[s] = 0.f;
+        }
+        V4 C[SP][NWT];
+        f32x4 U[SP][NWT];
+        gemm1_biased<T, DT, NWT, SP>(U, Qt, cs, ak, r, q, [&](int s, int w) {
             f32x4 p;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                p[v] = __builtin_amdgcn_exp2f(fmaf(to_f(C[w][v]), kLog2e, c[v])) * eb;
-                cr += p[v];
+                p[v] = __builtin_amdgcn_exp2f(fmaf(U[s][w][v], kLog2e, ck[s]));
+                cr[s] += p[v];
             }
-            C[w] = Pack<T>::four(p);
+            C[s][w] = Pack<T>::four_now(p);
         });
-        const unsigned arow = static_cast<unsigned>(k * B + j);   // row of aR / cR: (k, j)
-        cr = mfma::quad_rows_sum(cr);
-        if (q == 0)
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, cr), state_slice(P.cR, eh, np, 4), k < M ? arow * 4u : kOob, 0, 0);
-        f32x4 O[DT];
-        gemm2<T, DT, NWT>(O, Qt, C, r, q);
-        MT::store(state_slice(P.aR, eh, np, row_b), k < M ? arow * row_b : kOob, D, O, q, true);
+        f32x4 O[SP][DT];
+        gemm2<T, DT, NWT, SP>(O, Qt, C, r, q);
+#pragma unroll
+        for (int s = 0; s < SP; ++s) {
+            const int k = s0 + 16 * s + r;
+            const unsigned arow = static_cast<unsigned>(k * B + j);   // row of aR / cR: (k, j)
+            const float c = mfma::quad_rows_sum(cr[s]);
+            if (q == 0)
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, c), state_slice(P.cR, eh, np, 4), k < M ? arow * 4u : kOob, 0, 0);
+            MT::store(state_slice(P.aR, eh, np, row_b), k < M ? arow * row_b : kOob, D, O[s], q, true);
+        }
     }
 }
 
-
 // ---------------------------------------------------------------- launches
-// Waves per workgroup and waves per SIMD asked of the compiler, by stage (kV: R step with V), 16-column tiles and strips.
-// D <= 64: two workgroups of 256 rows fit the LDS; the R step holds most registers and runs best in 4 waves, the others in 8.
-// Wider rows: the LDS holds one workgroup at 192 / 256 rows, which then takes many waves - as many as there are strips where
-// registers allow -; an R step without V of up to 192 rows keeps one tile only: narrow workgroups, more of them.  Measured over
-// W = 4 .. 16 and EU = 1 .. 4 on six shapes: within 3 % of the best setting but for an R step without V of 256 wide rows (4
-// waves: 0.89) and one with V of 160 rows at D = 96 (EU = 3: 0.92).
+// Waves per workgroup, strips a wave walks side by side and waves per SIMD asked of the compiler, by stage (kV: R step with V),
+// 16-column tiles and strips.  D <= 64: two workgroups of 256 rows fit the LDS, and four waves per SIMD hide more than an
+// operand read shared by two strips saves.  Wider rows: the LDS holds one workgroup of 193 .. 256 rows, eight waves of two
+// strips each, whose reads of the tiles are what an LDS of that width costs; an R step without V keeps one tile only, so that two
+// workgroups fit (D <= 96: one strip per wave then).  129 .. 192 rows at D > 96: as many waves as strips, or, for an R
+// step without V, narrow workgroups, more of them.  Measured over W = 4 .. 16, one to four strips and EU = 1 .. 4 on six shapes:
+// within 3 % of the best setting.
 template <int STAGE, bool kV, int DT, int NWT>
 struct Cfg {
-    static constexpr bool kWideRow = DT > 4, k16 = NWT == 16, kR = STAGE == kStageR;
-    static constexpr int W = !kWideRow ? (kR || !k16 ? 4 : 8)
-                             : kR ? (k16 ? 8 : kV && DT == 8 ? 12 : 4)
-                                  : (k16 ? (STAGE == kStageL ? 16 : 8) : STAGE == kStageL || DT == 8 ? 12 : 4);
-    static constexpr int EU = kWideRow ? 1 : k16 ? (kR ? 2 : STAGE == kStageL ? 4 : 3) : 3;
+    static constexpr bool kWideRow = DT > 4, k16 = NWT == 16, kKeysOnly = STAGE == kStageR && !kV;
+    static constexpr int W = k16 ? 8 : DT == 8 && !kKeysOnly ? 12 : 4;
+    static constexpr int SP = k16 && kWideRow && !(kKeysOnly && DT == 6) ? 2 : 1;
+    static constexpr int EU = !kWideRow ? 4 : SP == 2 ? 2 : k16 ? 4 : 3;
 };
 
 template <class T, int DT>
@@ -764,10 +851,10 @@ int launch(const Problem& P, int stage, bool first, bool with_v, hipStream_t s) 
         using CZ = Cfg<kStageZ, false, DT, NWT>;
         using CV = Cfg<kStageR, true, DT, NWT>;
         using CK = Cfg<kStageR, false, DT, NWT>;
-        if (stage == kStageL) return run(l_step_long<T, DT, NWT, CL::W, CL::EU>, LPlan<T, DT, NWT>::kLds, problems, 1, CL::W, s, P);
-        if (stage == kStageZ) return run(z_step_long<T, DT, NWT, CZ::W, CZ::EU>, RPlan<T, DT, NWT>::kLds, problems, 1, CZ::W, s, P);
-        if (with_v) return run(r_step_long<T, DT, NWT, CV::W, CV::EU, true>, RPlan<T, DT, NWT>::kLds, problems, 1, CV::W, s, P, first ? 1 : 0);
-        return run(r_step_long<T, DT, NWT, CK::W, CK::EU, false>, KPlan<T, DT, NWT>::kLds, problems, 1, CK::W, s, P, first ? 1 : 0);
+        if (stage == kStageL) return run(l_step_long<T, DT, NWT, CL::W, CL::EU, CL::SP>, LPlan<T, DT, NWT>::kLds, problems, 1, CL::W, s, P);
+        if (stage == kStageZ) return run(z_step_long<T, DT, NWT, CZ::W, CZ::EU, CZ::SP>, RPlan<T, DT, NWT>::kLds, problems, 1, CZ::W, s, P);
+        if (with_v) return run(r_step_long<T, DT, NWT, CV::W, CV::EU, CV::SP, true>, RPlan<T, DT, NWT>::kLds, problems, 1, CV::W, s, P, first ? 1 : 0);
+        return run(r_step_long<T, DT, NWT, CK::W, CK::EU, CK::SP, false>, KPlan<T, DT, NWT>::kLds, problems, 1, CK::W, s, P, first ? 1 : 0);
     };
     switch (strip_class(stage == kStageR ? P.B : P.M)) {
         case 6: return pair(std::integral_constant<int, 6>{});

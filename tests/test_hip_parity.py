@@ -940,6 +940,20 @@ def test_long_stages_at_strip_edges(i, B, M, heads, dt):
         assert_parity(out.cpu(), ref, dt)
 
 
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("B,M,D,dt", [(193, 2, 96, "f16"), (256, 3, 128, "bf16"), (241, 2, 104, "f16"), (2, 200, 128, "f16"), (3, 256, 96, "bf16"),
+                                      (192, 2, 128, "bf16"), (256, 2, 64, "bf16"), (224, 2, 40, "f16")])
+def test_long_stages_with_and_without_masked_keys(B, M, D, dt, masked):
+    """The strip loops of 129 .. 256 rows: whole blocks without a mask (no bias is added to the logits) and ragged, masked ones;
+    wide rows of 193 .. 256 run two strips per wave side by side."""
+    N, T = B * M - 3 * masked, 2
+    q, k, v = seeded_qkv(1, 2, N, D, DT[dt], seed=B + M)
+    mask = block_safe_mask(1, N, B, seed=M) if masked else None
+    ref = monarch_attention_oracle(q, k, v, mask, T, B, masked, upcast=True)
+    out = monarch_attention_hip(*(t.to(DEV) for t in (q, k, v)), None if mask is None else mask.to(DEV), T, B, masked, variant="staged")
+    assert_parity(out.cpu(), ref, dt)
+
+
 @pytest.mark.parametrize("kind", ["plain", "mask", "dead_block", "one_key"])
 @pytest.mark.parametrize("B", [129, 181, 192, 256])
 def test_rows_of_negative_logits_in_long_blocks(B, kind):
