@@ -23,6 +23,11 @@
 // those of the strips - which the waves hold in registers from pass 1 and put over the first pair (LDS per workgroup: 2
 // tiles for L / Z and 3 for R, where all operands at once took 4 and 5).  A strip's accumulators of pass 2 are consumed
 // two tiles at a time, and gradients that are added to are loaded at the start and seed the accumulators.
+// Behind the memory come the vector instructions, so an entry of a pass costs one exponential and about eight others: the
+// biases sit in the accumulators, the row sums are taken of unnormalised values in one sweep, pass 2 forms p from one exponent that
+// holds the normaliser, and nothing branches on an entry (a select on "inside" had become a branch each).  Measured, bf16, T = 2,
+// stages Z / R with V / L / R: 32 heads of 8192 tokens in 64-row blocks 70.3 / 57.7 / 78.3 / 57.7 -> 64.3 / 62.5 / 66.2 / 49.5 us,
+// 192 heads of 512 in 32-row blocks 17.4 / 19.5 / 18.7 / 19.5 -> 18.0 / 20.5 / 18.5 / 18.2 (the two R stages averaged before).
 //
 // Problems of more than 128 rows, and problems of 81 .. 128 rows too few to fill the device, run the two passes as two
 // launches whose workgroups own W strips each (PASS = 1, 2; the statistics go through memory); tiles that exceed the LDS
@@ -36,16 +41,25 @@ namespace bwdt {
 
 using namespace tile;
 
-template <class T, int DT, int NWT, int PASS>
-using RPlan = Plan<T, DT, NWT, PASS, 2, 3, 7>;
+template <class T, int DT, int NWT, int PASS, bool kV>
+using RPlan = Plan<T, DT, NWT, PASS, kV ? 2 : 1, kV ? 3 : 2, 7>;
 template <class T, int DT, int NWT, int PASS, bool kZ>
-using LzPlan = Plan<T, DT, NWT, PASS, 2, kZ ? 2 : 1, 6>;
+using LzPlan = Plan<T, DT, NWT, PASS, 2, kZ ? 2 : 1, 5>;
+
+// A term that a product's sum is shifted by: 16-bit operands start the accumulators at it; fp32 sums, which would then be rounded
+// at its magnitude in every step, take it at the end.
+template <class T>
+__device__ __forceinline__ f32x4 start_at(const f32x4& c) { return sizeof(T) == 2 ? c : f32x4{0.f, 0.f, 0.f, 0.f}; }
+template <class T>
+__device__ __forceinline__ f32x4 shifted(const f32x4& sum, const f32x4& c) { return sizeof(T) == 2 ? sum : sum + c; }
+__device__ __forceinline__ f32x4 lds4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 
 // ---------------------------------------------------------------- R stage
-template <class T, int DT, int NWT, int W, int PASS>
-__global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, int first, int with_v) {
+// kV: the last step's stage, the first of a backward pass (Y and dv)
+template <class T, int DT, int NWT, int W, int PASS, bool kV>
+__global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, int first) {
     using MT = Mat<T, DT>;
-    using PL = RPlan<T, DT, NWT, PASS>;
+    using PL = RPlan<T, DT, NWT, PASS, kV>;
     using mfma::quad_rows_max;
     using mfma::quad_rows_sum;
     constexpr int NTH = 64 * W, ROWS = PL::ROWS, CT1 = PL::CT1, CT2 = PL::CT2;
@@ -53,13 +67,13 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
     static_assert(PASS != 0 || W == NWT, "one launch: every strip of the problem in the workgroup");
     extern __shared__ __attribute__((aligned(16))) char lds_raw[];
     T* tiles = reinterpret_cast<T*>(lds_raw);
-    float* kok = reinterpret_cast<float*>(lds_raw + PL::kTiles);
-    float* cjs = kok + ROWS;
-    float* gcls = cjs + ROWS;
-    float* mxs = gcls + ROWS;
-    float* invs = mxs + ROWS;
-    float* lg1s = invs + ROWS;
-    float* dots = lg1s + ROWS;
+    float* kbias = reinterpret_cast<float*>(lds_raw + PL::kTiles);
+    float* scs = kbias + ROWS;   // per query row, for pass 2: scale, factor, c0, gcL ln2, c1 (see below)
+    float* dfs = scs + ROWS;
+    float* c0s = dfs + ROWS;
+    float* gls = c0s + ROWS;
+    float* c1s = gls + ROWS;
+    float* invs = c1s + ROWS;
 
     const int B = P.B, M = P.M, D = P.D;
     unsigned problem;
@@ -86,24 +100,25 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
     auto x_off = [&](int j) { return j >= B ? kOob : first ? mfma::tok_off(t0 + j, P.N, qst) : static_cast<unsigned>(k * B + j) * row_b; };
     auto g_off = [&](int j) { return j < B ? static_cast<unsigned>(j * M + k) * row_b : kOob; };
     auto cr_of = [&](int j) { return first ? 1.f : mfma::bloadf<0>(scR, j < B ? static_cast<unsigned>(k * B + j) * 4u : kOob); };
-    // 1 / (cR + eps).  A row with cR = 0 (its position's queries are all masked) has aR = 0 too, so its logits are 0 whatever
-    // the factor is, and neither its dDot, which multiplies aR, nor its gaR, which L = 0 multiplies, reaches a gradient: the
-    // factor 0 stands for 1 / eps there, whose products would leave the range of fp16 and come back as 0 * inf.
-    auto over_cr = [&](float c) {
-        const float f = mfma::fp32_value(1.0f / (c + P.eps));   // (a value of its own: no branch around the division)
-        return c == 0.f ? 0.f : f;
-    };
+    // Logits in log2 units are scale(cR) times the product; dDot is p (g - sum g p) times factor(cR) = sm / (cR + eps).  A row with
+    // cR = 0 (its position's queries are all masked) has aR = 0 too, so its logits are 0 whatever the scale is, and neither its
+    // dDot, which multiplies aR, nor its gaR, which L = 0 multiplies, reaches a gradient: the factor 0 stands for sm / eps there,
+    // whose products would leave the range of fp16 and come back as 0 * inf.
+    auto over_cr = [&](float c) { return mfma::fp32_value(1.0f / (c + P.eps)); };   // (a value of its own: no branch around the division)
+    auto scale_of = [&](float c, float over) { return c == 0.f ? 1.f : kLog2e * sm * over; };
+    auto factor_of = [&](float c, float over) { return c == 0.f ? 0.f : sm * over; };
     auto gcl_of = [&](int j) { return mfma::bloadf<0>(sgcL, j < B ? static_cast<unsigned>(j * M + k) * 4u : kOob); };
     auto key_ok = [&](int i) { return i < B && token_ok(P, e, t0 + i); };
 
-    // Probability (clamped, ma_torch.py:18) and gradient of one entry from its logit s (-inf: masked key), the gradient
-    // part gg and its row's statistics: 0 where the clamp acted; log r = (S - max) + log(1 / (sum + eps)).
-    auto prob_grad = [](float s, float gg, bool in, float gcl, float mx, float inv, float lg1, float& rc, float& g) {
-        const float d = s - mx;
-        const float ru = __builtin_amdgcn_exp2f(kLog2e * d) * inv;
-        rc = in ? fmaxf(ru, kTiny) : 0.f;
-        g = (in && ru >= kTiny) ? fmaf(gcl, d + lg1, gg) : 0.f;
-    };
+    // With x the product of a query row and a key, d = scale x - max (log2 units, the maximum clamped, ma_torch.py:15), e = 2^d,
+    // p = e / (sum e + eps) and gg the gradient parts that are products:
+    //   g - sum g p = h - c,  h = gg + gcL ln2 d,  c = sum h p - gcL (ln(1 / (sum e + eps)) + 1) eps / (sum e + eps),
+    // so one exponential per entry gives every sum of a row.  In pass 2 log2 p = scale x + c0 and g - sum g p = (gg + c1) + gcL ln2
+    // log2 p.  Entries clamped to `tiny` (ma_torch.py:18) carry 1e-38 of a gradient and are not singled out; the exponent of a
+    // masked key is kFloor: p = 0 and everything that multiplies it is finite.
+    // (fp32: log2 p is not exact enough; there p = 2^(scale x + c0) / (sum e + eps) with c0 = -max, and c1 goes with it.)
+    constexpr float kFloor = -200.f;
+    constexpr bool kF32 = sizeof(T) == 4;
 
     typename MT::Row kb, vb;   // pass 2: this lane's key
     if constexpr (PASS != 2) {
@@ -111,33 +126,32 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
         T* Vt = tiles + 16 * CT1 * MT::LD;
         typename MT::Row xb, ga, gy;
         f32x4 S[NWT], Gg[NWT], O[DT];
-        float cr, cj, gcl;
+        float cr, gcl;
         for (int c = 0; c < PL::NC1; ++c) {   // (one chunk but for the largest fp32 problems)
             TileIn<MT, T, 16 * CT1, NTH> kc, vc;
             kc.issue(sk, D, wide, [&](int i) { return k_off(16 * CT1 * c + i); });
-            if (with_v) vc.issue(sv, D, wide, [&](int i) { return v_off(16 * CT1 * c + i); });
+            if (kV) vc.issue(sv, D, wide, [&](int i) { return v_off(16 * CT1 * c + i); });
             if (c == 0) {
                 MT::load(xb, sx, x_off(own), D, wide, q);
                 MT::load(ga, sga, g_off(own), D, wide, q);
-                if (with_v) MT::load(gy, sgy, g_off(own), D, wide, q);
+                if (kV) MT::load(gy, sgy, g_off(own), D, wide, q);
                 cr = cr_of(own);
                 gcl = gcl_of(own);
-                for (int i = threadIdx.x; i < ROWS; i += NTH) kok[i] = key_ok(i) ? 1.f : 0.f;
+                for (int i = threadIdx.x; i < ROWS; i += NTH) kbias[i] = key_ok(i) ? 0.f : -INFINITY;
             } else {
                 __syncthreads();
             }
             kc.commit(Kt);
-            if (with_v) vc.commit(Vt);
+            if (kV) vc.commit(Vt);
             __syncthreads();
-            if (c == 0) cj = over_cr(cr);   // (not where it is loaded: the tiles would wait for it)
 #pragma unroll
             for (int w = 0; w < CT1; ++w) {
-                f32x4 a = {0.f, 0.f, 0.f, 0.f}, g = {0.f, 0.f, 0.f, 0.f};
+                const f32x4 kb4 = lds4(kbias + 16 * (CT1 * c + w) + 4 * q);
+                f32x4 a = start_at<T>(kb4), g = {0.f, 0.f, 0.f, 0.f};
                 MT::gemm1(Kt, w, r, q, xb, a, ga, g);
-                if (with_v) MT::gemm1(Vt, w, r, q, gy, g);
-                const f32x4 ok = *reinterpret_cast<const f32x4*>(kok + 16 * (CT1 * c + w) + 4 * q);
-#pragma unroll
-                for (int v = 0; v < 4; ++v) a[v] = ok[v] != 0.f ? sm * round_to<T>(a[v]) * cj : -INFINITY;   // S, -inf for masked / padded keys
+                a = shifted<T>(a, kb4);
+                if (kV) MT::gemm1(Vt, w, r, q, gy, g);
+                if (NWT > 4 && w % 2 == 1) __builtin_amdgcn_sched_barrier(0);   // (keeps the tile reads from being hoisted: registers)
                 if constexpr (PL::NC1 == 1) {
                     S[w] = a;
                     Gg[w] = g;
@@ -151,45 +165,57 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
                 }
             }
         }
-        // row statistics: clamped maximum, 1 / (sum + eps)   (ma_torch.py:14-17)
+        const float over = over_cr(cr), scale = scale_of(cr, over), factor = factor_of(cr, over), gl = mfma::kLn2 * gcl;
         float mx = -INFINITY;
 #pragma unroll
         for (int w = 0; w < NWT; ++w)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) mx = fmaxf(mx, S[w][v]);
-        mx = fmaxf(quad_rows_max(mx), P.eps);
-        float sum = 0.f;
+            for (int v = 0; v < 4; ++v) mx = __builtin_elementwise_maximum(mx, S[w][v]);
+        mx = fmaxf(quad_rows_max(mx) * scale, P.eps * kLog2e);
+        float sum = 0.f, hs = 0.f, es = 0.f, ehs = 0.f;   // of e, e h, e d, e h d
+        auto sums = [&](auto with_gcr) {   // (S becomes e and Gg h; fp32 keeps S and forms e again)
 #pragma unroll
-        for (int w = 0; w < NWT; ++w)
+            for (int w = 0; w < NWT; ++w)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) sum += __builtin_amdgcn_exp2f(kLog2e * (S[w][v] - mx));
-        const float inv = mfma::rcp(quad_rows_sum(sum) + P.eps);
-        const float lg1 = __logf(inv) + 1.0f;
-        float dot = 0.f;   // sum_i g r
-#pragma unroll
-        for (int w = 0; w < NWT; ++w)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                float rc, g;
-                prob_grad(S[w][v], Gg[w][v], 16 * w + 4 * q + v < B, gcl, mx, inv, lg1, rc, g);
-                Gg[w][v] = g;
-                dot = fmaf(g, rc, dot);
-            }
-        dot = quad_rows_sum(dot);
-        // dS = r (g - dot), gcR = -sum_i dS S / (cR + eps), dDot = dS sm / (cR + eps); r once more from S: a third array
-        // of NWT accumulators would cost a wave per SIMD
+                for (int v = 0; v < 4; ++v) {
+                    const float d = fmaxf(fmaf(S[w][v], scale, -mx), kFloor), e = __builtin_amdgcn_exp2f(d);
+                    const float h = fmaf(gl, d, Gg[w][v]), eh = e * h;
+                    sum += e;
+                    hs += eh;
+                    if (!kF32 && decltype(with_gcr)::value) {
+                        es = fmaf(e, d, es);
+                        ehs = fmaf(eh, d, ehs);
+                    }
+                    if (!kF32) S[w][v] = e;
+                    Gg[w][v] = h;
+                }
+        };
+        if (first) sums(std::false_type{});
+        else sums(std::true_type{});
+        sum = quad_rows_sum(sum);
+        const float inv = mfma::rcp(sum + P.eps), lg = mfma::log2_normal(inv), k1 = gcl * fmaf(mfma::kLn2, lg, 1.f);
+        const float dot = inv * quad_rows_sum(hs), ctr = dot - k1 * (P.eps * inv);
         float gc = 0.f;
+        if (!kF32 && !first) {   // gcR = -sum_i dS S / (cR + eps)
+            es = inv * quad_rows_sum(es);
+            ehs = inv * quad_rows_sum(ehs);
+            gc = -mfma::kLn2 * over * (ehs - ctr * es + mx * (dot - ctr * (sum * inv)));
+        }
+        const float f = inv * factor;
 #pragma unroll
         for (int w = 0; w < NWT; ++w)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const bool live = S[w][v] != -INFINITY;
-                const float rc = fmaxf(__builtin_amdgcn_exp2f(kLog2e * (S[w][v] - mx)) * inv, kTiny);
-                const float ds = live ? rc * (Gg[w][v] - dot) : 0.f;
-                gc = live ? fmaf(-ds, S[w][v] * cj, gc) : gc;
-                S[w][v] = ds * (sm * cj);
+            for (int v = 0; v < 4; ++v) {   // dDot
+                if (kF32) {
+                    const float d = fmaxf(fmaf(S[w][v], scale, -mx), kFloor), ds = inv * __builtin_amdgcn_exp2f(d) * (Gg[w][v] - ctr);
+                    gc = fmaf(-ds, (d + mx) * (mfma::kLn2 * over), gc);
+                    S[w][v] = ds * factor;
+                } else {
+                    S[w][v] *= (Gg[w][v] - ctr) * f;
+                }
             }
-        gc = quad_rows_sum(gc);
+        if (kF32) gc = quad_rows_sum(gc);
+        if (cr == 0.f) gc = 0.f;
         // first step: aR is q itself, and dq is complete with this stage's part (loaded here, where Gg is done with, to
         // arrive behind the product)
         f32x4 dq0[DT];
@@ -197,15 +223,16 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) O[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (q == 0) {
+            const float c0 = kF32 ? -mx : lg - mx, c1 = kF32 ? -ctr : gcl - dot - k1 * (sum * inv);
             if constexpr (PASS == 0) {
-                cjs[own] = cj;
-                gcls[own] = gcl;
-                mxs[own] = mx;
+                scs[own] = scale;
+                dfs[own] = factor;
+                c0s[own] = c0;
+                gls[own] = gl;
+                c1s[own] = c1;
                 invs[own] = inv;
-                lg1s[own] = lg1;
-                dots[own] = dot;
             } else if (own_in) {
-                *reinterpret_cast<f32x4*>(G.stat + 4 * (eh * np + k * B + own)) = f32x4{mx, inv, dot, 0.f};
+                *reinterpret_cast<f32x4*>(G.stat + 4 * (eh * np + k * B + own)) = f32x4{c0, c1, inv, 0.f};
             }
             if (!first && own_in) G.gcR[eh * np + k * B + own] = gc;
         }
@@ -233,11 +260,11 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
         else MT::store(state_slice(G.gaR, eh, np, row_b), own_in ? static_cast<unsigned>(k * B + own) * row_b : kOob, D, O, q, D % 8 == 0);
         if constexpr (PASS == 0) {   // the strip's rows take the place of the key / value tiles
             MT::from_tile(kb, Kt, own, q);
-            if (with_v) MT::from_tile(vb, Vt, own, q);
+            if (kV) MT::from_tile(vb, Vt, own, q);
             __syncthreads();
             MT::to_tile(xb, tiles, own, q);
             MT::to_tile(ga, tiles + 16 * CT2 * MT::LD, own, q);
-            if (with_v) MT::to_tile(gy, tiles + 32 * CT2 * MT::LD, own, q);
+            if (kV) MT::to_tile(gy, tiles + 32 * CT2 * MT::LD, own, q);
         }
     }
 
@@ -248,76 +275,91 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
         const bool done = first != 0;   // dk is complete with this stage: it goes to the caller's tensor
         const rsrc_t sdk = state_slice(G.dk, eh, np, D * 4u);
         f32x4 Ok[DT], Ov[DT];
-        // the stage that also forms dv is the first R stage of a backward pass: it starts dk's sums
-        load_acc<MT, DT>(Ok, sdk, static_cast<unsigned>(k * B + own), D, q, !with_v && own_in);
+        // the stage that also forms dv is the first R stage of a backward pass: it starts dk's sums.  Between the R stages dk is read and
+        // written by the same strips: see load_strip (bf16, 192 heads of 512: 24.0 -> 21.8 us in the stage that writes,
+        // 32 heads of 8192: 57.2 -> 52.6 in the one that reads)
+        const int strip0 = 16 * (group * W + wave);
+        const bool whole = strip0 + 16 <= B && D == 16 * DT;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) Ok[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (!kV) {
+            if (whole) load_strip(Ok, sdk, static_cast<unsigned>(k * B + strip0));
+            else load_acc<MT, DT>(Ok, sdk, static_cast<unsigned>(k * B + own), D, q, own_in);
+        }
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) Ov[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
         bool ok = false;
         if constexpr (PASS == 2) {
             MT::load(kb, sk, k_off(own), D, wide, q);
-            if (with_v) MT::load(vb, sv, v_off(own), D, wide, q);
+            if (kV) MT::load(vb, sv, v_off(own), D, wide, q);
             ok = key_ok(own);
         }
         for (int c = 0; c < PL::NC2; ++c) {
             if constexpr (PASS == 2) {
                 TileIn<MT, T, 16 * CT2, NTH> xc, ac, yc;
+                constexpr bool kLate = 3 * 4 * decltype(xc)::CNT > 128;   // three tiles on their way at once would take most registers
                 xc.issue(sx, D, wide, [&](int j) { return x_off(16 * CT2 * c + j); });
                 ac.issue(sga, D, wide, [&](int j) { return g_off(16 * CT2 * c + j); });
-                if (with_v) yc.issue(sgy, D, wide, [&](int j) { return g_off(16 * CT2 * c + j); });
+                if (kV && !kLate) yc.issue(sgy, D, wide, [&](int j) { return g_off(16 * CT2 * c + j); });
                 if (c == 0) {
                     for (int j = threadIdx.x; j < ROWS; j += NTH) {
-                        cjs[j] = over_cr(cr_of(j));
-                        gcls[j] = gcl_of(j);
-                        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+                        const float cr = cr_of(j), over = over_cr(cr);
+                        f32x4 s = {kFloor, 0.f, 0.f, 0.f};
                         if (j < B) s = *reinterpret_cast<const f32x4*>(G.stat + 4 * (eh * np + k * B + j));
-                        mxs[j] = s[0];
-                        invs[j] = s[1];
-                        lg1s[j] = __logf(s[1]) + 1.0f;
-                        dots[j] = s[2];
+                        scs[j] = scale_of(cr, over);
+                        dfs[j] = factor_of(cr, over);
+                        c0s[j] = s[0];
+                        gls[j] = mfma::kLn2 * gcl_of(j);
+                        c1s[j] = s[1];
+                        invs[j] = s[2];
                     }
                 } else {
                     __syncthreads();
                 }
                 xc.commit(Xt);
                 ac.commit(Gat);
-                if (with_v) yc.commit(Gyt);
+                if (kV && kLate) yc.issue(sgy, D, wide, [&](int j) { return g_off(16 * CT2 * c + j); });
+                if (kV) yc.commit(Gyt);
             }
             __syncthreads();
-            if constexpr (PASS == 0) ok = kok[own] != 0.f;
+            if constexpr (PASS == 0) ok = kbias[own] == 0.f;
+            const float most = ok ? INFINITY : kFloor;
             constexpr int ST = CT2 == 1 ? 1 : 2;   // strips per step
 #pragma unroll 2
             for (int s = 0; s < CT2; s += ST) {
                 f32x4 PR[ST], DD[ST];
 #pragma unroll
                 for (int u = 0; u < ST; ++u) {
-                    f32x4 a = {0.f, 0.f, 0.f, 0.f}, g = {0.f, 0.f, 0.f, 0.f};
+                    const int j0 = 16 * (CT2 * c + s + u) + 4 * q;
+                    f32x4 a = {0.f, 0.f, 0.f, 0.f};
                     PR[u] = a;
                     DD[u] = a;
                     if (CT2 % 2 == 1 && s + u >= CT2) continue;
+                    const f32x4 c14 = lds4(c1s + j0);
+                    f32x4 g = start_at<T>(c14);
                     MT::gemm1(Xt, s + u, r, q, kb, a);
                     MT::gemm1(Gat, s + u, r, q, kb, g);
-                    if (with_v) MT::gemm1(Gyt, s + u, r, q, vb, g);
-                    const int j0 = 16 * (CT2 * c + s + u) + 4 * q;
-                    const f32x4 cj4 = *reinterpret_cast<const f32x4*>(cjs + j0), gcl4 = *reinterpret_cast<const f32x4*>(gcls + j0);
-                    const f32x4 mx4 = *reinterpret_cast<const f32x4*>(mxs + j0), inv4 = *reinterpret_cast<const f32x4*>(invs + j0);
-                    const f32x4 lg4 = *reinterpret_cast<const f32x4*>(lg1s + j0), dot4 = *reinterpret_cast<const f32x4*>(dots + j0);
+                    if (kV) MT::gemm1(Gyt, s + u, r, q, vb, g);
+                    g = shifted<T>(g, c14);
+                    const f32x4 sc4 = lds4(scs + j0), c04 = lds4(c0s + j0), gl4 = lds4(gls + j0), df4 = lds4(dfs + j0);
+                    const f32x4 inv4 = kF32 ? lds4(invs + j0) : f32x4{1.f, 1.f, 1.f, 1.f};
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
-                        const float sv1 = ok ? sm * round_to<T>(a[v]) * cj4[v] : -INFINITY;
-                        float rc, gv;
-                        prob_grad(sv1, g[v], own_in, gcl4[v], mx4[v], inv4[v], lg4[v], rc, gv);
-                        PR[u][v] = rc;
-                        DD[u][v] = ok ? rc * (gv - dot4[v]) * (sm * cj4[v]) : 0.f;
+                        const float lp = fminf(fmaf(a[v], sc4[v], c04[v]), most);
+                        const float p = kF32 ? __builtin_amdgcn_exp2f(lp) * inv4[v] : __builtin_amdgcn_exp2f(lp);
+                        PR[u][v] = p;
+                        DD[u][v] = p * fmaf(gl4[v], lp, g[v]) * df4[v];
                     }
                 }
                 auto products = [&](auto n) {
                     constexpr int NT = decltype(n)::value;
                     MT::template gemm2<NT>(Ok, Gat + 16 * s * MT::LD, PR, r, q);
                     MT::template gemm2<NT>(Ok, Xt + 16 * s * MT::LD, DD, r, q);
-                    if (with_v) MT::template gemm2<NT>(Ov, Gyt + 16 * s * MT::LD, PR, r, q);
+                    if (kV) MT::template gemm2<NT>(Ov, Gyt + 16 * s * MT::LD, PR, r, q);
                 };
                 if (CT2 % 2 == 1 && s + ST > CT2) products(std::integral_constant<int, 1>{});
                 else products(std::integral_constant<int, ST>{});
+                if (NWT > 4) __builtin_amdgcn_sched_barrier(0);
             }
         }
         auto emit = [&](int which_out, const f32x4 (&O)[DT]) {
@@ -325,29 +367,32 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
                       own_in ? mfma::tok_off(own_t, P.N, static_cast<unsigned>(G.outs[which_out][2]) * sizeof(T)) : kOob, D, O, q, wide);
         };
         if (done) emit(1, Ok);
+        else if (whole) store_strip(sdk, static_cast<unsigned>(k * B + strip0), Ok);
         else store_acc<MT, DT>(sdk, static_cast<unsigned>(k * B + own), D, Ok, q, own_in);
-        if (with_v) emit(2, Ov);
+        if (kV) emit(2, Ov);
     }
 }
 
 // ---------------------------------------------------------------- L and Z stages
+// (Eight strips of up to 64 columns: two workgroups of eight waves share a compute unit as long as a wave keeps to 128 registers.  The
+// L stage of 32 heads of 8192 tokens takes 66 us at 128 and 87 above.)
 template <class T, int DT, int NWT, int W, int PASS, bool kZ>
-__global__ __launch_bounds__(64 * W) void lz_bwd_tile(Problem P, BwdBuffers G) {
+__global__ __launch_bounds__(64 * W, sizeof(T) == 2 && DT <= 4 && NWT == 8 && PASS == 0 ? 4 : 1) void lz_bwd_tile(Problem P, BwdBuffers G) {
     using MT = Mat<T, DT>;
     using PL = LzPlan<T, DT, NWT, PASS, kZ>;
     using mfma::quad_rows_max;
     using mfma::quad_rows_sum;
     constexpr int NTH = 64 * W, ROWS = PL::ROWS, CT1 = PL::CT1, CT2 = PL::CT2;
     constexpr float kLog2e = mfma::kLog2e;
+    constexpr bool kF32 = sizeof(T) == 4;
     static_assert(PASS != 0 || W == NWT, "one launch: every strip of the problem in the workgroup");
     extern __shared__ __attribute__((aligned(16))) char lds_raw[];
     T* tiles = reinterpret_cast<T*>(lds_raw);
-    float* cl = reinterpret_cast<float*>(lds_raw + PL::kTiles);
-    float* cw = cl + ROWS;
-    float* qok = cw + ROWS;
-    float* mxs = qok + ROWS;
-    float* invs = mxs + ROWS;
-    float* dots = invs + ROWS;
+    float* ncl = reinterpret_cast<float*>(lds_raw + PL::kTiles);   // per key block: -cL (-inf beyond the last), gcR
+    float* cw = ncl + ROWS;
+    float* c0s = cw + ROWS;                                         // per query block, for pass 2: log(mask / sum) - max, -sum g p
+    float* nds = c0s + ROWS;
+    float* pks = nds + ROWS;                                        // (fp32: c0 = -max, and mask / sum apart)
 
     const int M = P.M, D = P.D, B = P.B;
     unsigned problem;
@@ -372,7 +417,10 @@ __global__ __launch_bounds__(64 * W) void lz_bwd_tile(Problem P, BwdBuffers G) {
     auto q_off = [&](int l) { return l < M ? mfma::tok_off(tok(l), P.N, qst) : kOob; };
     auto o_off = [&](int l) { return l < M ? mfma::tok_off(tok(l), P.N, ost) : kOob; };
     auto keep_of = [&](int l) { return (l < M && token_ok(P, e, tok(l))) ? 1.f : 0.f; };
-    auto cl_of = [&](int k) { return mfma::bloadf<0>(scL, k < M ? (jm + k) * 4u : kOob); };
+    auto ncl_of = [&](int k) {
+        const float c = mfma::bloadf<0>(scL, k < M ? (jm + k) * 4u : kOob);
+        return k < M ? -c : -INFINITY;
+    };
     auto cw_of = [&](int k) { return mfma::bloadf<0>(sgcR, k < M ? static_cast<unsigned>(k * B + j) * 4u : kOob); };
 
     typename MT::Row ak, wk;   // pass 2: this lane's key block
@@ -393,7 +441,7 @@ __global__ __launch_bounds__(64 * W) void lz_bwd_tile(Problem P, BwdBuffers G) {
                 if (kZ) MT::load(xo, so, o_off(own), D, wide, q);
                 if (!kZ) keep = keep_of(own);
                 for (int k = threadIdx.x; k < ROWS; k += NTH) {
-                    cl[k] = cl_of(k);
+                    ncl[k] = ncl_of(k);
                     if (!kZ) cw[k] = cw_of(k);
                 }
                 // the Z stage runs first and every dq row belongs to one workgroup: it is written, not added to
@@ -411,17 +459,13 @@ __global__ __launch_bounds__(64 * W) void lz_bwd_tile(Problem P, BwdBuffers G) {
             __syncthreads();
 #pragma unroll
             for (int w = 0; w < CT1; ++w) {
-                f32x4 a = {0.f, 0.f, 0.f, 0.f}, g = {0.f, 0.f, 0.f, 0.f};
-                MT::gemm1(At, w, r, q, xq, a);
-                MT::gemm1(Wt, w, r, q, kZ ? xo : xq, g);
                 const int k0 = 16 * (CT1 * c + w) + 4 * q;
-                const f32x4 cl4 = *reinterpret_cast<const f32x4*>(cl + k0), cw4 = *reinterpret_cast<const f32x4*>(cw + k0);
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const bool in = k0 + v < M;
-                    a[v] = in ? round_to<T>(a[v]) - cl4[v] : -INFINITY;   // U, -inf beyond the M key blocks
-                    if (!kZ) g[v] = in ? keep * (g[v] + cw4[v]) : 0.f;     // gLm = mask_q (Q gaR^T + gcR)
-                }
+                const f32x4 ncl4 = lds4(ncl + k0), cw4 = kZ ? f32x4{0.f, 0.f, 0.f, 0.f} : lds4(cw + k0);
+                f32x4 a = start_at<T>(ncl4), g = start_at<T>(cw4);
+                MT::gemm1(At, w, r, q, xq, a);                   // U
+                MT::gemm1(Wt, w, r, q, kZ ? xo : xq, g);         // gL = Q gaR^T + gcR (mask_q: see keep)
+                a = shifted<T>(a, ncl4);
+                if (!kZ) g = shifted<T>(g, cw4);
                 if constexpr (PL::NC1 == 1) {
                     U[w] = a;
                     Gg[w] = g;
@@ -439,42 +483,38 @@ __global__ __launch_bounds__(64 * W) void lz_bwd_tile(Problem P, BwdBuffers G) {
 #pragma unroll
         for (int w = 0; w < NWT; ++w)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) mx = fmaxf(mx, U[w][v]);
+            for (int v = 0; v < 4; ++v) mx = __builtin_elementwise_maximum(mx, U[w][v]);
         mx = quad_rows_max(mx);
-        float sum = 0.f;
+        const float m2 = kLog2e * mx;
+        float sum = 0.f, dot = 0.f;
 #pragma unroll
         for (int w = 0; w < NWT; ++w)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                U[w][v] = __builtin_amdgcn_exp2f(kLog2e * (U[w][v] - mx));
+                U[w][v] = __builtin_amdgcn_exp2f(kF32 ? kLog2e * (U[w][v] - mx) : fmaf(U[w][v], kLog2e, -m2));
                 sum += U[w][v];
-            }
-        const float inv = mfma::rcp(quad_rows_sum(sum));
-        float dot = 0.f;
-#pragma unroll
-        for (int w = 0; w < NWT; ++w)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                U[w][v] *= inv;
                 dot = fmaf(Gg[w][v], U[w][v], dot);
             }
-        dot = quad_rows_sum(dot);
+        const float inv = mfma::rcp(quad_rows_sum(sum));
+        dot = inv * quad_rows_sum(dot);
+        // Lm = mask_q Lp and dU = mask_q Lp (gL - sum gL Lp): a masked query block is one whose probabilities count 0 times
+        const float pk = inv * keep;
         if (q == 0) {
+            const float c0 = kF32 ? -mx : fmaf(mfma::kLn2, mfma::log2_normal(pk), -mx);
             if constexpr (PASS == 0) {
-                qok[own] = keep;
-                mxs[own] = mx;
-                invs[own] = inv;
-                dots[own] = dot;
+                c0s[own] = c0;
+                nds[own] = -dot;
+                pks[own] = pk;
             } else if (own_in) {
-                *reinterpret_cast<f32x4*>(G.stat + 4 * (eh * np + jm + own)) = f32x4{mx, inv, dot, keep};
+                *reinterpret_cast<f32x4*>(G.stat + 4 * (eh * np + jm + own)) = f32x4{c0, -dot, pk, 0.f};
             }
         }
 #pragma unroll
         for (int w = 0; w < NWT; ++w)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
+                U[w][v] *= pk;
                 Gg[w][v] = U[w][v] * (Gg[w][v] - dot);   // dU
-                if (!kZ) U[w][v] *= keep;                 // Lm = mask_q Lp
             }
         // dq rows (l, j) (+)= dU aL  (L: + round(Lm) gaR)
         for (int c = PL::NC1 - 1; c >= 0; --c) {
@@ -519,9 +559,9 @@ __global__ __launch_bounds__(64 * W) void lz_bwd_tile(Problem P, BwdBuffers G) {
             MT::load(ak, saL, a_off(own), D, wide_s, q);
             MT::load(wk, sw, w_off(own), D, wide_s, q);
         }
-        float clk = 0.f, cwk = 0.f, gcl = 0.f;
+        float nck = 0.f, cwk = 0.f, gcl = 0.f;
         if constexpr (PASS == 2) {
-            clk = cl_of(own);
+            nck = ncl_of(own);
             if (!kZ) cwk = cw_of(own);
         }
         for (int c = 0; c < PL::NC2; ++c) {
@@ -531,12 +571,11 @@ __global__ __launch_bounds__(64 * W) void lz_bwd_tile(Problem P, BwdBuffers G) {
                 if (kZ) oc.issue(so, D, wide, [&](int l) { return o_off(16 * CT2 * c + l); });
                 if (c == 0) {
                     for (int l = threadIdx.x; l < ROWS; l += NTH) {
-                        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+                        f32x4 s = {kF32 ? 0.f : -INFINITY, 0.f, 0.f, 0.f};
                         if (l < M) s = *reinterpret_cast<const f32x4*>(G.stat + 4 * (eh * np + jm + l));
-                        mxs[l] = s[0];
-                        invs[l] = s[1];
-                        dots[l] = s[2];
-                        qok[l] = s[3];
+                        c0s[l] = s[0];
+                        nds[l] = s[1];
+                        pks[l] = s[2];
                     }
                 } else {
                     __syncthreads();
@@ -546,34 +585,32 @@ __global__ __launch_bounds__(64 * W) void lz_bwd_tile(Problem P, BwdBuffers G) {
             }
             __syncthreads();
             if constexpr (PASS == 0) {
-                clk = cl[own];
+                nck = ncl[own];
                 if (!kZ) cwk = cw[own];
             }
+            const float n2 = kLog2e * nck;
             constexpr int ST = CT2 == 1 ? 1 : 2;
 #pragma unroll 2
             for (int s = 0; s < CT2; s += ST) {
                 f32x4 PR[ST], DU[ST];
 #pragma unroll
                 for (int u = 0; u < ST; ++u) {
-                    f32x4 a = {0.f, 0.f, 0.f, 0.f}, g = {0.f, 0.f, 0.f, 0.f};
-                    PR[u] = a;
-                    DU[u] = a;
+                    const int l0 = 16 * (CT2 * c + s + u) + 4 * q;
+                    PR[u] = DU[u] = f32x4{0.f, 0.f, 0.f, 0.f};
                     if (CT2 % 2 == 1 && s + u >= CT2) continue;
+                    const f32x4 c04 = lds4(c0s + l0), nd4 = lds4(nds + l0), pk4 = kF32 ? lds4(pks + l0) : f32x4{1.f, 1.f, 1.f, 1.f};
+                    f32x4 a = start_at<T>(c04), g = start_at<T>(nd4);
                     if (kZ) {
                         MT::gemm1(Qt, s + u, r, q, ak, a);
                         MT::gemm1(dOt, s + u, r, q, wk, g);
                     } else {
                         MT::gemm1(Qt, s + u, r, q, ak, a, wk, g);
                     }
-                    const int l0 = 16 * (CT2 * c + s + u) + 4 * q;
-                    const f32x4 mx4 = *reinterpret_cast<const f32x4*>(mxs + l0), inv4 = *reinterpret_cast<const f32x4*>(invs + l0);
-                    const f32x4 dot4 = *reinterpret_cast<const f32x4*>(dots + l0), keep4 = *reinterpret_cast<const f32x4*>(qok + l0);
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
-                        const float x = own_in ? round_to<T>(a[v]) - clk : -INFINITY;
-                        const float p = __builtin_amdgcn_exp2f(kLog2e * (x - mx4[v])) * inv4[v];
-                        const float gv = kZ ? g[v] : (own_in ? keep4[v] * (g[v] + cwk) : 0.f);
-                        const float du = p * (gv - dot4[v]);
+                        const float p = kF32 ? __builtin_amdgcn_exp2f(kLog2e * (a[v] + nck + c04[v])) * pk4[v]
+                                             : __builtin_amdgcn_exp2f(fmaf(a[v], kLog2e, n2));
+                        const float gd = kF32 ? (kZ ? g[v] : g[v] + cwk) + nd4[v] : kZ ? g[v] : g[v] + cwk, du = p * gd;
                         PR[u][v] = p;
                         DU[u][v] = du;
                         gcl -= du;
@@ -600,17 +637,17 @@ __global__ __launch_bounds__(64 * W) void lz_bwd_tile(Problem P, BwdBuffers G) {
 }
 
 // ---------------------------------------------------------------- launches
-template <class T, int DT>
-int launch_r(const Problem& P, const BwdBuffers& G, bool first, bool with_v, hipStream_t s) {
+template <class T, int DT, bool kV>
+int launch_r(const Problem& P, const BwdBuffers& G, bool first, hipStream_t s) {
     const long long problems = static_cast<long long>(P.E) * P.H * P.M;
     return each_launch<sizeof(T) == 4>(P.B, problems, [&](auto nwt, auto w, auto pass) {
         constexpr int NWT = decltype(nwt)::value, W = decltype(w)::value, PASS = decltype(pass)::value;
-        if constexpr (PASS == 0 && !RPlan<T, DT, NWT, 0>::kFits) {   // three fp32 tiles of 128 rows: the passes one after the other
+        if constexpr (PASS == 0 && !RPlan<T, DT, NWT, 0, kV>::kFits) {   // three fp32 tiles of 128 rows: the passes one after the other
             static_assert(NWT > 4, "the statistics of problems of up to 64 rows have no room in the workspace");
-            const int st = run(r_bwd_tile<T, DT, NWT, NWT / 2, 1>, RPlan<T, DT, NWT, 1>::kLds, problems, 2, NWT / 2, s, P, G, first ? 1 : 0, with_v ? 1 : 0);
-            return st ? st : run(r_bwd_tile<T, DT, NWT, NWT / 2, 2>, RPlan<T, DT, NWT, 2>::kLds, problems, 2, NWT / 2, s, P, G, first ? 1 : 0, with_v ? 1 : 0);
+            const int st = run(r_bwd_tile<T, DT, NWT, NWT / 2, 1, kV>, RPlan<T, DT, NWT, 1, kV>::kLds, problems, 2, NWT / 2, s, P, G, first ? 1 : 0);
+            return st ? st : run(r_bwd_tile<T, DT, NWT, NWT / 2, 2, kV>, RPlan<T, DT, NWT, 2, kV>::kLds, problems, 2, NWT / 2, s, P, G, first ? 1 : 0);
         } else {
-            return run(r_bwd_tile<T, DT, NWT, W, PASS>, RPlan<T, DT, NWT, PASS>::kLds, problems, NWT / W, W, s, P, G, first ? 1 : 0, with_v ? 1 : 0);
+            return run(r_bwd_tile<T, DT, NWT, W, PASS, kV>, RPlan<T, DT, NWT, PASS, kV>::kLds, problems, NWT / W, W, s, P, G, first ? 1 : 0);
         }
     });
 }
@@ -628,7 +665,7 @@ int launch_lz(const Problem& P, const BwdBuffers& G, hipStream_t s) {
 template <class T, int DT>
 int launch(const Problem& P, const BwdBuffers& G, int stage, bool first, bool with_v, hipStream_t s) {
     switch (stage) {
-        case kStageR: return launch_r<T, DT>(P, G, first, with_v, s);
+        case kStageR: return with_v ? launch_r<T, DT, true>(P, G, first, s) : launch_r<T, DT, false>(P, G, first, s);
         case kStageL: return launch_lz<T, DT, false>(P, G, s);
         default: return launch_lz<T, DT, true>(P, G, s);
     }

@@ -189,6 +189,21 @@ __device__ __forceinline__ void store_acc(rsrc_t s, unsigned row, int D, const f
     for (int dt = 0; dt < DT; ++dt)
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, O[dt]), s, want && MT::col(q, dt) < D ? (row * D + MT::col(q, dt)) * 4u : kOob, 0, 0);
 }
+// ... of a strip that only waves with this very strip read again: as the accumulators lie in the registers, 1 KB contiguous per
+// instruction (rows: 16 pieces of 64 bytes).  Needs a whole strip and D = 16 DT; row0: the strip's first row; the bytes are those
+// of its 16 rows.
+template <int DT>
+__device__ __forceinline__ void load_strip(f32x4 (&O)[DT], rsrc_t s, unsigned row0) {
+    const unsigned at = row0 * (64u * DT) + (threadIdx.x & 63) * 16u;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) O[dt] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(s, at + 1024u * dt, 0, 0));
+}
+template <int DT>
+__device__ __forceinline__ void store_strip(rsrc_t s, unsigned row0, const f32x4 (&O)[DT]) {
+    const unsigned at = row0 * (64u * DT) + (threadIdx.x & 63) * 16u;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, O[dt]), s, at + 1024u * dt, 0, 0);
+}
 
 // ROWS rows on their way from memory to an LDS tile: issue() starts the loads, commit() writes the tile
 template <class MT, class T, int ROWS, int NTH>
