@@ -194,7 +194,7 @@ __global__ __launch_bounds__(64 * W) void r_step_pair(Problem P, int first) {
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int v = 0; v < 4; ++v) O[s][dt][v] = P.sm_scale * round_to<T>(O[s][dt][v]);
-        MT::store(state_slice(P.aL, eh, np, row_b), j < B ? static_cast<unsigned>(j * M + k) * row_b : kOob, D, O[s], q, true, stream_rows(P, row_b));
+        MT::template store<false>(state_slice(P.aL, eh, np, row_b), j < B ? static_cast<unsigned>(j * M + k) * row_b : kOob, D, O[s], q, true, stream_rows(P, row_b));
     }
     if (kV) {
         zero(O);
@@ -202,7 +202,7 @@ __global__ __launch_bounds__(64 * W) void r_step_pair(Problem P, int first) {
 #pragma unroll
         for (int s = 0; s < SP; ++s) {
             const int j = 16 * ((group * W + wave) * SP + s) + r;
-            MT::store(state_slice(P.Y, eh, np, row_b), j < B ? static_cast<unsigned>(j * M + k) * row_b : kOob, D, O[s], q, true, stream_rows(P, row_b));
+            MT::template store<false>(state_slice(P.Y, eh, np, row_b), j < B ? static_cast<unsigned>(j * M + k) * row_b : kOob, D, O[s], q, true, stream_rows(P, row_b));
         }
     }
 }
@@ -295,7 +295,7 @@ __global__ __launch_bounds__(64 * W) void z_step_pair(Problem P) {
     for (int s = 0; s < SP; ++s) {
         const int l = 16 * ((group * W + wave) * SP + s) + r;
         // padded query rows are dropped (ma_torch.py:108)
-        MT::store(so, l < M ? mfma::tok_off(l * B + j - P.pad_off, P.N, ost) : kOob, D, O[s], q, true,
+        MT::template store<false>(so, l < M ? mfma::tok_off(l * B + j - P.pad_off, P.N, ost) : kOob, D, O[s], q, true,
                   stream_rows(P, row_b) && ost % 128u == 0 && (reinterpret_cast<unsigned long long>(P.out) + static_cast<unsigned long long>(e * P.os[0] + h * P.os[1]) * sizeof(T)) % 128u == 0);
     }
 }
@@ -431,7 +431,7 @@ __global__ __launch_bounds__(64 * W) void l_step_pair(Problem P) {
             const float c = mfma::quad_rows_sum(cr[s]);
             if (q == 0)
                 __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, c), state_slice(P.cR, eh, np, 4), k < M ? arow * 4u : kOob, 0, 0);
-            MT::store(state_slice(P.aR, eh, np, row_b), k < M ? arow * row_b : kOob, D, O[s], q, true, stream_rows(P, row_b));
+            MT::template store<false>(state_slice(P.aR, eh, np, row_b), k < M ? arow * row_b : kOob, D, O[s], q, true, stream_rows(P, row_b));
         }
     }
 }

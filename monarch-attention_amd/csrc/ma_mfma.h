@@ -284,6 +284,29 @@ __device__ __forceinline__ u32x4 pair_piece(u32x2 a, u32x2 b) {
     return u32x4{a[0], a[1], b[0], b[1]};
 }
 
+// Two 16-byte pieces of a lane's row - the four lanes of a row hold 64 contiguous bytes with each - stored so that either
+// instruction writes 128 contiguous bytes of 8 rows instead of 64 of 16: neighbouring lanes exchange a piece (the even lane's
+// second for the odd lane's first) and its offset.  Every lane of the wave takes part.  For rows of one 128-byte line (64
+// columns) in the head-resident kernels (192 heads of 512: 27.0 -> 26.3 us) and the kernels of ma_tile.h (training on
+// them 121.5 -> 118.2); rows of 144 and 256 bytes gain nothing or lose 1 %, and neither do the chained kernel's problems, whose
+// chain the exchange lengthens (16 heads of 5824 28.1 -> 28.7 us).
+template <int AUX>
+__device__ __forceinline__ void store_pieces(rsrc_t dst, const u32x4& a, unsigned off_a, const u32x4& b, unsigned off_b) {
+    const bool odd = (threadIdx.x & 1) != 0;
+    u32x4 x;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(odd ? a[i] : b[i]), 0xB1, 0xf, 0xf, true));
+    const unsigned off_x = static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(odd ? off_a : off_b), 0xB1, 0xf, 0xf, true));
+    u32x4 even_row, odd_row;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        even_row[i] = odd ? x[i] : a[i];
+        odd_row[i] = odd ? b[i] : x[i];
+    }
+    __builtin_amdgcn_raw_buffer_store_b128(even_row, dst, odd ? off_x : off_a, 0, AUX);
+    __builtin_amdgcn_raw_buffer_store_b128(odd_row, dst, odd ? off_b : off_x, 0, AUX);
+}
+
 // P (fp32, C layout, NWT tiles) -> B operands of GEMM2, rounded to T.  k slot s of
 // step g is row w = 32g + 16(s/4) + 4q + s%4: slots 0-3 from C tile 2g, 4-7 from 2g+1.
 template <class T, int NWT>
@@ -325,7 +348,7 @@ __device__ __forceinline__ void gemm2(f32x4 (&O)[DT], const T* tile, const typen
 // (measured: 5 us after an R step that wrote 17 MB, against 2 us with streaming stores).
 // Rows that share lines with other writers keep the plain policy (partial streaming
 // writes are several times slower).
-template <class T, int DT, int MODE>
+template <class T, int DT, int MODE, bool LINES = false>
 __device__ __forceinline__ void store_row(rsrc_t dst, unsigned ro, int D, const f32x4 (&O)[DT], int q, bool stream = false) {
     typedef typename Ops<T>::v4 V4;
     const bool whole = D == 16 * DT;   // no piece lies beyond the row
@@ -335,14 +358,27 @@ __device__ __forceinline__ void store_row(rsrc_t dst, unsigned ro, int D, const 
     if (MODE != kRun || (DT % 2 == 0 && whole)) {
         const int col0 = MODE == kRun ? 4 * DT * q : 8 * q;   // the pieces sit at fixed distances from this column
         const unsigned base = ro + 2 * col0;
+        u32x4 x[DT / 2 + 1];
+        unsigned off[DT / 2 + 1];
 #pragma unroll
         for (int p = 0; p < DT / 2; ++p) {
             const u32x2 lo = __builtin_bit_cast(u32x2, v[2 * p]), hi = __builtin_bit_cast(u32x2, v[2 * p + 1]);
-            const u32x4 x = MODE == kTile ? pair_piece(lo, hi) : u32x4{lo[0], lo[1], hi[0], hi[1]};
-            unsigned off = base + (MODE == kRun ? 16 : 64) * p;
-            if (!whole) off = 32 * p + 8 * q < D ? off : kOob;   // (kRun: whole rows only here)
-            if (stream) __builtin_amdgcn_raw_buffer_store_b128(x, dst, off, 0, 2);
-            else __builtin_amdgcn_raw_buffer_store_b128(x, dst, off, 0, 0);
+            x[p] = MODE == kTile ? pair_piece(lo, hi) : u32x4{lo[0], lo[1], hi[0], hi[1]};
+            off[p] = base + (MODE == kRun ? 16 : 64) * p;
+            if (!whole) off[p] = 32 * p + 8 * q < D ? off[p] : kOob;   // (kRun: whole rows only here)
+        }
+#pragma unroll
+        for (int p = 0; p < DT / 2; p += 2) {
+            if (LINES && MODE != kRun && DT == 4 && whole) {
+                if (stream) store_pieces<2>(dst, x[p], off[p], x[p + 1], off[p + 1]);
+                else store_pieces<0>(dst, x[p], off[p], x[p + 1], off[p + 1]);
+            } else {
+#pragma unroll
+                for (int s = p; s < p + 2 && s < DT / 2; ++s) {
+                    if (stream) __builtin_amdgcn_raw_buffer_store_b128(x[s], dst, off[s], 0, 2);
+                    else __builtin_amdgcn_raw_buffer_store_b128(x[s], dst, off[s], 0, 0);
+                }
+            }
         }
         if (DT % 2 == 1) {
             const int d0 = chunk_col<DT, MODE>(q, DT - 1);

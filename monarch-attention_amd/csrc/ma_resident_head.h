@@ -559,7 +559,7 @@ struct HeadRes {
         f32x4 O[DT];
         gemm2_rows<NTM, false>(O, c, c.row(c.L.V, 0, j), c.BP, M, pb);   // Y(j, k) sits in V's row j of block k
         const int t = l * B + j - P.pad_off;
-        store_row<T, DT, kSmall>(hd.out, l < M ? tok_off(t, P.N, c.ost) : kOob, P.D, O, q, false);   // padded query rows are dropped
+        store_row<T, DT, kSmall, true>(hd.out, l < M ? tok_off(t, P.N, c.ost) : kOob, P.D, O, q, false);   // padded query rows are dropped
     }
 };
 

@@ -87,17 +87,33 @@ struct Mat {   // 16-bit
                 O[dt] = mfma::Ops<T>::mma(mfma::lds_tr8<T, DT, mfma::kTile>(tile, 32 * g + 4 * q, 16, 2 * g + 1 < NT, dt, r), p, O[dt]);
         }
     }
+    // LINES: see mfma::store_pieces (not for problems whose chain of latencies is what counts)
+    template <bool LINES = true>
     static __device__ __forceinline__ void store(rsrc_t s, unsigned ro, int D, const f32x4 (&O)[DT], int q, bool wide, bool stream = false) {
         V4 v[DT];
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) v[dt] = V4{from_f<T>(O[dt][0]), from_f<T>(O[dt][1]), from_f<T>(O[dt][2]), from_f<T>(O[dt][3])};
         if (wide) {   // tiles 2 p and 2 p + 1: one 16-byte piece, wholly inside or beyond a row of a multiple of 8 columns
+            u32x4 x[DT / 2 + 1];
+            unsigned off[DT / 2 + 1];
 #pragma unroll
             for (int p = 0; p < DT / 2; ++p) {
                 const int c = 32 * p + 8 * q;
-                const u32x4 x = mfma::pair_piece(__builtin_bit_cast(u32x2, v[2 * p]), __builtin_bit_cast(u32x2, v[2 * p + 1]));
-                if (stream) __builtin_amdgcn_raw_buffer_store_b128(x, s, c < D ? ro + 2 * c : kOob, 0, 2);
-                else __builtin_amdgcn_raw_buffer_store_b128(x, s, c < D ? ro + 2 * c : kOob, 0, 0);
+                x[p] = mfma::pair_piece(__builtin_bit_cast(u32x2, v[2 * p]), __builtin_bit_cast(u32x2, v[2 * p + 1]));
+                off[p] = c < D ? ro + 2 * c : kOob;
+            }
+#pragma unroll
+            for (int p = 0; p < DT / 2; p += 2) {
+                if (LINES && DT == 4 && D == 64) {
+                    if (stream) mfma::store_pieces<2>(s, x[p], off[p], x[p + 1], off[p + 1]);
+                    else mfma::store_pieces<0>(s, x[p], off[p], x[p + 1], off[p + 1]);
+                } else {
+#pragma unroll
+                    for (int i = p; i < p + 2 && i < DT / 2; ++i) {
+                        if (stream) __builtin_amdgcn_raw_buffer_store_b128(x[i], s, off[i], 0, 2);
+                        else __builtin_amdgcn_raw_buffer_store_b128(x[i], s, off[i], 0, 0);
+                    }
+                }
             }
         } else {
 #pragma unroll
@@ -169,6 +185,7 @@ struct Mat<float, DT> {   // fp32: k slot q of step (t, u) is column 16 t + 4 q 
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt) O[dt] = mma4(tile[(16 * t + 4 * q + v) * LD + 16 * dt + r], C[t][v], O[dt]);
     }
+    template <bool LINES = true>
     static __device__ __forceinline__ void store(rsrc_t s, unsigned ro, int D, const f32x4 (&O)[DT], int q, bool) {
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
