@@ -189,7 +189,9 @@ uint64_t ma_fwd_workspace_bytes(const ma_fwd_params* p);
 int ma_workspace_init(const ma_fwd_params* p, void* stream);
 
 /* The variant MA_VARIANT_AUTO resolves to for this problem (a ma_variant), or
- * a negative ma_status. */
+ * a negative ma_status.  Where AUTO resolves to CHAINED or RESIDENT, it may run a kernel that
+ * no explicit variant does: 16 positions of a head per workgroup, without exchange between
+ * workgroups ("resident_slice_mfma" by ma_fwd_kernel_name).  The workspace is the same. */
 int ma_fwd_select_variant(const ma_fwd_params* p);
 
 /* Name of the kernel that does the bulk of the work for this problem under the variant it resolves to

@@ -171,6 +171,16 @@ bool mfma32_supported(const ma_fwd_params* p) {
     return true;
 }
 
+int run_slice(const Problem& P, int dtype_qk, bool dry_run, hipStream_t s) {
+    const bool h = dtype_qk == MA_F16;
+    const int D = P.D;
+    if (D <= 32) return h ? launch_slice_f16_d2(P, dry_run, s) : launch_slice_bf16_d2(P, dry_run, s);
+    if (D <= 48) return h ? launch_slice_f16_d3(P, dry_run, s) : launch_slice_bf16_d3(P, dry_run, s);
+    if (D <= 64) return h ? launch_slice_f16_d4(P, dry_run, s) : launch_slice_bf16_d4(P, dry_run, s);
+    if (D <= 80) return h ? launch_slice_f16_d5(P, dry_run, s) : launch_slice_bf16_d5(P, dry_run, s);
+    return MA_ERR_UNSUPPORTED;
+}
+
 int run_resident(const Problem& P, int dtype_qk, bool dry_run, hipStream_t s) {
     if (dtype_qk == MA_F32) return launch_head32(P, dry_run, s);
     const bool h = dtype_qk == MA_F16;
@@ -181,13 +191,18 @@ int run_resident(const Problem& P, int dtype_qk, bool dry_run, hipStream_t s) {
     return h ? launch_resident_f16_d8(P, dry_run, s) : launch_resident_bf16_d8(P, dry_run, s);
 }
 
-// Does a head's state fit in LDS (the resident kernel's condition)?  one_tile: also count the form that
-// keeps aL and aR in one tile and passes Y through the workspace.
-bool resident_fits(const ma_fwd_params* p, bool one_tile) {
+Problem sizes_of(const ma_fwd_params* p) {
     Problem P;
     std::memset(&P, 0, sizeof(P));
     P.E = p->E; P.H = p->H; P.N = p->N; P.D = p->D; P.Dv = p->Dv; P.B = p->B; P.T = p->T;
     P.M = (p->N + p->B - 1) / p->B;
+    return P;
+}
+
+// Does a head's state fit in LDS (the resident kernel's condition)?  one_tile: also count the form that
+// keeps aL and aR in one tile and passes Y through the workspace.
+bool resident_fits(const ma_fwd_params* p, bool one_tile) {
+    Problem P = sizes_of(p);
     P.one_tile_ok = one_tile ? 1 : 0;
     return run_resident(P, p->dtype_qk, true, nullptr) == MA_OK;
 }
@@ -197,12 +212,53 @@ bool resident_fits(const ma_fwd_params* p, bool one_tile) {
 // launch run a head-resident form (4: the four-tile one) in workgroups of 4 or 8 waves, several of them per compute
 // unit (more short heads than compute units)?
 bool resident_head_fits(const ma_fwd_params* p, int forms = 1) {
-    Problem P;
-    std::memset(&P, 0, sizeof(P));
-    P.E = p->E; P.H = p->H; P.N = p->N; P.D = p->D; P.Dv = p->Dv; P.B = p->B; P.T = p->T;
-    P.M = (p->N + p->B - 1) / p->B;
+    Problem P = sizes_of(p);
     P.resident_head_only = forms;
     return p->dtype_qk != MA_F32 && run_resident(P, p->dtype_qk, true, nullptr) == MA_OK;
+}
+
+// AUTO, 16-bit: is the slice-resident kernel (ma_resident_slice.h: a workgroup per 16 positions of a head) ahead of the kernel that
+// variant v would run?  A slice has a compute unit, or half of one, to itself, so the rules are about how well heads x slices fill
+// whole passes over the 256 compute units they were measured on, and how many of a slice's 16 positions exist.  Heads that fit in
+// LDS whole stay with the head-resident kernels where those are chosen, but for blocks of 14 and 15 rows and for a single pass of
+// slices: beyond, which of the two is ahead turns on how the last pass ends (0.6 - 1.4).  In the comments: multiples of the time of the kernel
+// it replaces, at D = 32 .. 80, 64 .. 4096 tokens, 8 .. 768 heads, T = 1, 2, 3 (profiles/slice_resident_sweep.md).
+bool slice_pays(const ma_fwd_params* p, int v) {
+    if (p->dtype_qk == MA_F32 || (v != MA_VARIANT_CHAINED && v != MA_VARIANT_RESIDENT)) return false;
+    Problem P = sizes_of(p);
+    P.one_tile_ok = 1;
+    if (P.B > 64 || P.M > 64 || run_slice(P, p->dtype_qk, true, nullptr) != MA_OK) return false;
+    const long long heads = static_cast<long long>(P.E) * P.H, slices = heads * ((P.B + 15) / 16);
+    const int B = P.B, M = P.M, D = P.D;
+    const bool multi = P.T >= 2, wide = D > 64;
+    if (B <= 16) {   // one slice a head: beside the head-resident kernels, which lose to padding where blocks are a little short of 16 rows
+        if (B == 16 || B < 14 || M < 12) return false;
+        if (M > 32) return multi && heads >= 192;                                             // 0.6 - 0.85
+        if (M > 16) return heads >= 112 && heads <= 288 && (multi || D <= 32);              // 0.83 - 1.0
+        if (!multi) return heads >= 96 && heads <= (wide ? 400 : 256);                       // 0.78 - 0.91
+        return wide ? heads >= (P.T == 2 ? 64 : 8) && heads <= 400                            // 0.80 - 0.94
+                    : heads <= 256 && (P.T == 2 || B == 15);                                  // 0.85 - 0.99 (others 0.96 - 1.02)
+    }
+    if (v == MA_VARIANT_RESIDENT && heads > 128 && resident_head_fits(p, 2)) return false;
+    const bool most = slices >= 192 && multi && B <= 32 && M > 16 && M <= 32 && (wide ? B >= 30 && M >= 28 : B >= 24);   // 0.79 - 0.98
+    if (slices < 224 && !most) return false;              // less than most of one pass
+    if (B <= 32) {
+        if (M <= 16) return heads <= 128 || (B >= 30 && (multi || heads >= 224));             // 0.65 - 0.94; 0.6 - 0.95
+        if (M <= 32) {
+            if (heads <= 128) return multi || B >= 24;                                        // 0.64 - 0.99
+            if (heads < 224) return multi && B >= 28 && M >= 28;                              // 0.76 - 0.98 (shorter: 0.87 - 1.03)
+            return multi || B >= (wide ? 28 : 24);                                            // 0.5 - 0.9; 0.7 - 0.97
+        }
+        if (B < 20 || (heads > 128 && heads < 224)) return false;                             // (0.89 - 1.14)
+        return multi || (B >= 28 && M <= 48);                                                 // 0.6 - 0.97; 0.8 - 1.0
+    }
+    if (B <= 48) {
+        if (D <= 32) return heads <= 85 || heads >= 224 || (multi && heads >= 112);           // 0.55 - 0.99
+        if (D <= 48) return multi && heads >= 224 && M > 20;                                  // 0.74 - 0.94
+        if (D <= 64) return multi && M > 16 && (heads >= 224 || (heads <= 85 && B >= 44));    // 0.75 - 0.97; 0.84 - 0.98
+        return multi && heads >= 512 && M > 16;                                               // 0.76 - 0.97
+    }
+    return D <= 32 && multi && B >= 56 && (heads <= 64 || (heads >= 112 && M >= 30));         // 0.63 - 0.94
 }
 
 // The fused, chained and resident kernels are built for block problems of at most 128 rows.
@@ -465,6 +521,7 @@ __global__ void zero_sync_kernel(uint4* sync, int chunks) {
 struct Prepared {
     Problem P;
     int variant;
+    bool slice = false;   // AUTO: the slice-resident kernel in place of the variant's own
 };
 
 int run_fused(const Prepared& pr, const ma_fwd_params* p, hipStream_t s) {
@@ -558,6 +615,7 @@ int prepare(const ma_fwd_params* p, Prepared* out) {
     if (v < 0) return v;
     out->P = make_problem(p, L);
     out->variant = v;
+    out->slice = p->variant == MA_VARIANT_AUTO && slice_pays(p, v);
     set_policies(p, out);
     out->P.one_tile_ok = 1;   // a problem that resolves to the resident kernel may use any of its forms
     return MA_OK;
@@ -901,7 +959,9 @@ int ma_fwd_select_variant(const ma_fwd_params* p) {
 const char* ma_fwd_kernel_name(const ma_fwd_params* p) {
     if (check_shape(p) != MA_OK) return nullptr;
     const bool f32 = p->dtype_qk == MA_F32;
-    switch (select_variant(p)) {
+    const int v = select_variant(p);
+    if (p->variant == MA_VARIANT_AUTO && slice_pays(p, v)) return "resident_slice_mfma";
+    switch (v) {
         case MA_VARIANT_GENERIC: return "r_step_kernel";
         case MA_VARIANT_STAGED: return f32 ? "r_step_f32" : p->B > 128 ? "r_step_long" : p->B > 64 ? "r_step_pair" : "r_step_mfma";   // (see runs_long)
         case MA_VARIANT_FUSED: return "fused_fwd_mfma";
@@ -910,11 +970,7 @@ const char* ma_fwd_kernel_name(const ma_fwd_params* p) {
             if (!f32)
                 return resident_head_fits(p, 4) ? "resident_head_mfma" : resident_head_fits(p, 3) ? "resident_head2_mfma"
                        : resident_head_fits(p, 1) ? "resident_head_mfma" : resident_head_fits(p, 2) ? "resident_head2_mfma" : "resident_fwd_mfma";
-            Problem P;
-            std::memset(&P, 0, sizeof(P));
-            P.E = p->E; P.H = p->H; P.N = p->N; P.D = p->D; P.Dv = p->Dv; P.B = p->B; P.T = p->T;
-            P.M = (p->N + p->B - 1) / p->B;
-            return head32_single_step(P) ? "head_t1_f32" : "head_fwd_f32";
+            return head32_single_step(sizes_of(p)) ? "head_t1_f32" : "head_fwd_f32";
         }
         default: return nullptr;
     }
@@ -949,6 +1005,7 @@ int ma_fwd(const ma_fwd_params* p, void* stream) {
     int st = prepare(p, &pr);
     if (st != MA_OK) return st;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (pr.slice) return run_slice(pr.P, p->dtype_qk, false, s);
     if (pr.variant == MA_VARIANT_FUSED) return run_fused(pr, p, s);
     if (pr.variant == MA_VARIANT_CHAINED) return run_chain(pr, p, s);
     if (pr.variant == MA_VARIANT_RESIDENT) return run_resident(pr.P, p->dtype_qk, false, s);

@@ -244,6 +244,14 @@ int launch_fused_bf16_d8(const Problem& P, bool sync_ready, hipStream_t s);
 
 // Resident forward (one launch, per-head state kept in LDS).  dry_run: only report
 // whether the problem fits (MA_OK / MA_ERR_UNSUPPORTED), launch nothing.
+int launch_slice_f16_d2(const Problem& P, bool dry_run, hipStream_t s);
+int launch_slice_f16_d3(const Problem& P, bool dry_run, hipStream_t s);
+int launch_slice_f16_d4(const Problem& P, bool dry_run, hipStream_t s);
+int launch_slice_f16_d5(const Problem& P, bool dry_run, hipStream_t s);
+int launch_slice_bf16_d2(const Problem& P, bool dry_run, hipStream_t s);
+int launch_slice_bf16_d3(const Problem& P, bool dry_run, hipStream_t s);
+int launch_slice_bf16_d4(const Problem& P, bool dry_run, hipStream_t s);
+int launch_slice_bf16_d5(const Problem& P, bool dry_run, hipStream_t s);
 int launch_resident_f16_d2(const Problem& P, bool dry_run, hipStream_t s);
 int launch_resident_f16_d4(const Problem& P, bool dry_run, hipStream_t s);
 int launch_resident_f16_d5(const Problem& P, bool dry_run, hipStream_t s);

@@ -131,8 +131,9 @@ __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x);
 __device__ __forceinline__ float log2_normal(float x) { return __builtin_amdgcn_logf(x); }
 
 // x as an fp32 value of its own: keeps the compiler from rounding a product once, to 16 bits, where the kernels round it to
-// fp32 and then to 16 bits (it does so for a few values of some kernels).  Problems of more than 64 rows run in kernels that
-// differ by launch (chained, per stage), and a head's result must not depend on which.
+// fp32 and then to 16 bits (it does so for a few values of some kernels).  R problems of more than 32 rows and others
+// of more than 64 run in kernels that differ by launch (chained, per stage, slices of a head), and a head's result must not depend
+// on which.
 __device__ __forceinline__ float fp32_value(float x) {
     asm("" : "+v"(x));
     return x;
@@ -659,7 +660,7 @@ struct RProb {
 #pragma unroll
             for (int wt = 0; wt < NWT; ++wt)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) C[wt][v] = NWT > 4 ? fp32_value(C[wt][v] * inv) : C[wt][v] * inv;
+                for (int v = 0; v < 4; ++v) C[wt][v] = NWT > 2 ? fp32_value(C[wt][v] * inv) : C[wt][v] * inv;
             // cL = sum_i r log r with r = p / den (ma_torch.py:20); rows of tiny r add ~1e-36
             lrow = static_cast<unsigned>(j * M + m);   // row of aL / cL / Y: (j, m)
             if (q == 0)

@@ -1,0 +1,6 @@
+// Slice-resident forward kernels, bf16 operands, head-dim class 5 (see ma_resident_slice.h).
+#include "ma_slice_launch.h"
+
+namespace ma {
+int launch_slice_bf16_d5(const Problem& P, bool dry_run, hipStream_t s) { return mfma::launch_slice<bf16, 5>(P, dry_run, s); }
+}  // namespace ma

@@ -1,0 +1,6 @@
+// Slice-resident forward kernels, f16 operands, head-dim class 2 (see ma_resident_slice.h).
+#include "ma_slice_launch.h"
+
+namespace ma {
+int launch_slice_f16_d2(const Problem& P, bool dry_run, hipStream_t s) { return mfma::launch_slice<f16, 2>(P, dry_run, s); }
+}  // namespace ma

@@ -1,0 +1,6 @@
+// Slice-resident forward kernels, f16 operands, head-dim class 3 (see ma_resident_slice.h).
+#include "ma_slice_launch.h"
+
+namespace ma {
+int launch_slice_f16_d3(const Problem& P, bool dry_run, hipStream_t s) { return mfma::launch_slice<f16, 3>(P, dry_run, s); }
+}  // namespace ma

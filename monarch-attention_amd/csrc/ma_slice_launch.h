@@ -1,0 +1,64 @@
+// Host-side dispatch of the slice-resident forward kernel.  Included by one .hip file per (dtype, head-dim class).
+#pragma once
+
+#include "ma_mfma_launch.h"
+#include "ma_resident_slice.h"
+
+namespace ma {
+namespace mfma {
+
+constexpr size_t kSliceLds = 160 * 1024;
+
+template <class T, int DT, int NTB, int NTM, int W>
+int launch_slice_w(const Problem& P, hipStream_t s) {
+    using SL = Slice<T, DT, NTB, NTM, W>;
+    if (!SL::takes(P.D, P.M, P.B, kSliceLds)) return MA_ERR_UNSUPPORTED;
+    const int lds_err = set_lds_limit(resident_slice_mfma<T, DT, NTB, NTM, W>, kSliceLds);
+    if (lds_err) return lds_err;
+    const long long heads = static_cast<long long>(P.E) * P.H, grid = (heads + 7) / 8 * 8 * ((P.B + 15) / 16);
+    hipLaunchKernelGGL((resident_slice_mfma<T, DT, NTB, NTM, W>), dim3(static_cast<unsigned>(grid)), dim3(64 * W), SL::layout(P.D, P.M).total, s, P);
+    return static_cast<int>(hipGetLastError());
+}
+
+// As many waves as the LDS has tiles for: 16 or 8, 12 or 8 for problems of more than two strips (256 heads of 1024, 48-row blocks, T =
+// 2: 0.77 of the chained kernel's time in 12 waves, 0.85 in 8).  Eight where two slices share a compute unit and there are more
+// slices than compute units (192 heads of 512, T = 2: 24.7 us, 26.8 in 16).
+template <class T, int DT, int NTB, int NTM>
+int launch_slice_one(const Problem& P, bool dry_run, hipStream_t s) {
+    using Narrow = Slice<T, DT, NTB, NTM, 8>;
+    if (dry_run) return Narrow::takes(P.D, P.M, P.B, kSliceLds) ? MA_OK : MA_ERR_UNSUPPORTED;
+    if constexpr (NTB <= 2 && NTM <= 2) {
+        const long long slices = static_cast<long long>(P.E) * P.H * ((P.B + 15) / 16);
+        if (slices <= compute_units() || 2 * Narrow::layout(P.D, P.M).total > kSliceLds) {
+            const int err = launch_slice_w<T, DT, NTB, NTM, 16>(P, s);
+            if (err != MA_ERR_UNSUPPORTED) return err;
+        }
+    } else {
+        const int err = launch_slice_w<T, DT, NTB, NTM, 12>(P, s);
+        if (err != MA_ERR_UNSUPPORTED) return err;
+    }
+    return launch_slice_w<T, DT, NTB, NTM, 8>(P, s);
+}
+
+template <class T, int DT>
+int launch_slice(const Problem& P, bool dry_run, hipStream_t s) {
+    if (P.B > 64 || P.M > 64 || !P.one_tile_ok) return MA_ERR_UNSUPPORTED;
+    auto blocks = [&](auto ntb) {
+        constexpr int NTB = decltype(ntb)::value;
+        switch ((P.M + 15) / 16) {
+            case 1: return launch_slice_one<T, DT, NTB, 1>(P, dry_run, s);
+            case 2: return launch_slice_one<T, DT, NTB, 2>(P, dry_run, s);
+            case 3: return launch_slice_one<T, DT, NTB, 3>(P, dry_run, s);
+            default: return launch_slice_one<T, DT, NTB, 4>(P, dry_run, s);
+        }
+    };
+    switch ((P.B + 15) / 16) {
+        case 1: return blocks(std::integral_constant<int, 1>{});
+        case 2: return blocks(std::integral_constant<int, 2>{});
+        case 3: return blocks(std::integral_constant<int, 3>{});
+        default: return blocks(std::integral_constant<int, 4>{});
+    }
+}
+
+}  // namespace mfma
+}  // namespace ma

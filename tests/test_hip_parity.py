@@ -325,6 +325,36 @@ def test_resident_kernel_with_one_state_tile(E, H, N, D, B, T, pre, dt, masked):
     assert torch.equal(out, again)
 
 
+SLICES = [  # 14 / 15, 17 .. 32, 33 .. 48 and 49 .. 64 rows a block; every class of block counts; head dims with and without a half step
+    (2, 4, 197, 64, 14, 2, True, "f16", False), (3, 3, 225, 72, 15, 3, False, "bf16", True), (4, 32, 400, 32, 15, 1, True, "f16", True),
+    (7, 16, 512, 64, 32, 2, False, "f16", True), (8, 14, 300, 40, 20, 1, True, "bf16", False), (7, 16, 1024, 72, 32, 3, False, "f16", False),
+    (8, 14, 900, 80, 30, 2, True, "f16", True), (30, 12, 700, 64, 28, 2, False, "bf16", True), (8, 14, 1300, 32, 25, 2, False, "f16", True),
+    (8, 14, 1300, 32, 28, 1, True, "f16", True), (5, 15, 1500, 32, 40, 2, False, "f16", True), (16, 14, 1000, 64, 44, 2, True, "f16", True),
+    (16, 14, 1600, 48, 40, 3, False, "bf16", True), (4, 14, 2500, 32, 60, 2, True, "f16", True), (4, 14, 3200, 32, 64, 3, False, "bf16", False),
+    (16, 12, 600, 32, 15, 2, True, "f16", True), (8, 12, 800, 64, 32, 3, False, "f16", True),
+]
+
+
+@pytest.mark.parametrize("E,H,N,D,B,T,pre,dt,masked", SLICES)
+def test_slice_resident_kernel(E, H, N, D, B, T, pre, dt, masked):
+    """Where AUTO runs the kernel that keeps 16 positions of a head per workgroup: every head bit-equal to the chained
+    kernel's (a head's result does not depend on the size of the batch), two batch entries against the oracle.  Masks end
+    mid-block and leave whole blocks without keys."""
+    q, k, v = seeded_qkv(E, H, N, D, DT[dt], seed=N + B)
+    mask = None
+    if masked:
+        mask = block_safe_mask(E, N, B, seed=B)
+        mask[E - 1, N // 2 + 3:] = False
+    dev = to_dev(q, k, v, mask)
+    p = make_params(*dev[:3], dev[3], torch.empty_like(dev[2]), T, B, pre, "auto")
+    assert L.load().ma_fwd_kernel_name(p).decode() == "resident_slice_mfma"
+    out = monarch_attention_hip(*dev, T, B, pre)
+    assert torch.equal(out, monarch_attention_hip(*dev, T, B, pre, variant="chained"))
+    few = [0, E - 1] if E > 1 else [0]
+    ref = monarch_attention_oracle(q[few, :2], k[few, :2], v[few, :2], None if mask is None else mask[few], T, B, pre, upcast=True)
+    assert_parity(out[few, :2].cpu(), ref, dt, f"slices {(E, H, N, D, B, T)}")
+
+
 SMALL_F32 = [  # E, H, N, D, B, T, pre, masked: fp32 heads of at most 16 blocks of at most 16 rows
     (1, 1, 256, 64, 16, 1, False, False),      # the reference's CPU-sized case
     (2, 3, 197, 64, 16, 1, True, True), (1, 4, 100, 32, 8, 1, False, True), (3, 2, 250, 48, 16, 1, True, False),   # a single step, few heads
