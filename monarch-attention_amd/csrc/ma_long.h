@@ -820,12 +820,16 @@ __global__ __launch_bounds__(64 * W, EU) void l_step_long(Problem P) {
 // workgroups fit (D <= 96: one strip per wave then).  129 .. 192 rows at D > 96: as many waves as strips, or, for an R
 // step without V, narrow workgroups, more of them.  Measured over W = 4 .. 16, one to four strips and EU = 1 .. 4 on six shapes:
 // within 3 % of the best setting.
-template <int STAGE, bool kV, int DT, int NWT>
+// At most one problem per compute unit (FEW): as many waves as strips, since a wave's strips then run one after the other while
+// most of the compute unit is idle.  A head of 10672 tokens, D = 72, 64-row blocks, two steps: 34.5 -> 28.6 us; of 40000, D = 64,
+// 200-row blocks: 54.3 -> 51.0; of 30000, D = 96: 59.1 -> 53.1; four heads of 10672, D = 64, 64-row blocks: 36.0 -> 31.4.
+template <int STAGE, bool kV, int DT, int NWT, bool FEW>
 struct Cfg {
     static constexpr bool kWideRow = DT > 4, k16 = NWT == 16, kKeysOnly = STAGE == kStageR && !kV;
-    static constexpr int W = k16 ? 8 : DT == 8 && !kKeysOnly ? 12 : 4;
-    static constexpr int SP = k16 && kWideRow && !(kKeysOnly && DT == 6) ? 2 : 1;
-    static constexpr int EU = !kWideRow ? 4 : SP == 2 ? 2 : k16 ? 4 : 3;
+    static constexpr bool kOne = FEW && !(STAGE == kStageR && k16 && kWideRow);   // (there the registers of 16 waves do not hold a strip)
+    static constexpr int W = kOne ? NWT : k16 ? 8 : DT == 8 && !kKeysOnly ? 12 : 4;
+    static constexpr int SP = k16 && kWideRow && !kOne && !(kKeysOnly && DT == 6) ? 2 : 1;
+    static constexpr int EU = kOne ? NWT / 4 : !kWideRow ? 4 : SP == 2 ? 2 : k16 ? 4 : 3;
 };
 
 template <class T, int DT>
@@ -847,14 +851,19 @@ int launch(const Problem& P, int stage, bool first, bool with_v, hipStream_t s) 
     };
     auto whole = [&](auto nwt) {
         constexpr int NWT = decltype(nwt)::value;
-        using CL = Cfg<kStageL, false, DT, NWT>;
-        using CZ = Cfg<kStageZ, false, DT, NWT>;
-        using CV = Cfg<kStageR, true, DT, NWT>;
-        using CK = Cfg<kStageR, false, DT, NWT>;
-        if (stage == kStageL) return run(l_step_long<T, DT, NWT, CL::W, CL::EU, CL::SP>, LPlan<T, DT, NWT>::kLds, problems, 1, CL::W, s, P);
-        if (stage == kStageZ) return run(z_step_long<T, DT, NWT, CZ::W, CZ::EU, CZ::SP>, RPlan<T, DT, NWT>::kLds, problems, 1, CZ::W, s, P);
-        if (with_v) return run(r_step_long<T, DT, NWT, CV::W, CV::EU, CV::SP, true>, RPlan<T, DT, NWT>::kLds, problems, 1, CV::W, s, P, first ? 1 : 0);
-        return run(r_step_long<T, DT, NWT, CK::W, CK::EU, CK::SP, false>, KPlan<T, DT, NWT>::kLds, problems, 1, CK::W, s, P, first ? 1 : 0);
+        auto go = [&](auto few) {
+            constexpr bool FEW = decltype(few)::value;
+            using CL = Cfg<kStageL, false, DT, NWT, FEW>;
+            using CZ = Cfg<kStageZ, false, DT, NWT, FEW>;
+            using CV = Cfg<kStageR, true, DT, NWT, FEW>;
+            using CK = Cfg<kStageR, false, DT, NWT, FEW>;
+            if (stage == kStageL) return run(l_step_long<T, DT, NWT, CL::W, CL::EU, CL::SP>, LPlan<T, DT, NWT>::kLds, problems, 1, CL::W, s, P);
+            if (stage == kStageZ) return run(z_step_long<T, DT, NWT, CZ::W, CZ::EU, CZ::SP>, RPlan<T, DT, NWT>::kLds, problems, 1, CZ::W, s, P);
+            if (with_v) return run(r_step_long<T, DT, NWT, CV::W, CV::EU, CV::SP, true>, RPlan<T, DT, NWT>::kLds, problems, 1, CV::W, s, P, first ? 1 : 0);
+            return run(r_step_long<T, DT, NWT, CK::W, CK::EU, CK::SP, false>, KPlan<T, DT, NWT>::kLds, problems, 1, CK::W, s, P, first ? 1 : 0);
+        };
+        if (problems <= mfma::compute_units()) return go(std::true_type{});
+        return go(std::false_type{});
     };
     switch (strip_class(stage == kStageR ? P.B : P.M)) {
         case 6: return pair(std::integral_constant<int, 6>{});
