@@ -608,8 +608,13 @@ struct RProb {
             if (tix < ROWS) kbias[tix] = (tix < P.B && token_kept(P, m * P.B - P.pad_off + tix, pre.km)) ? 0.f : kNegBig;
         }
         problem_sync<WPP>();
+        // The last strip has rows (uniform).  65 - 80 and 97 - 112 rows leave it empty in the classes of 6 and 8 strips: as a strip
+        // of queries and as a tile of keys it is passed over (16 heads of 5003, 72-row blocks, two steps: D = 64 44.8 -> 40.3 us,
+        // D = 128 74 -> 70; 104-row blocks, 10600 tokens, D = 64: 78.7 -> 74; full classes unchanged).
+        const bool full = NWT <= 4 || 16 * (NWT - 1) < B;
 #pragma unroll
         for (int si = 0; si < SPW; ++si) {
+          if (!full && strip_of(wig, si) == NWT - 1) continue;
           f32x4 OY[DT];
           V8 pb[(NWT + 1) / 2];
           bool jv = false;
@@ -627,6 +632,10 @@ struct RProb {
             f32x4 C[NWT];
 #pragma unroll
             for (int wt = 0; wt < NWT; ++wt) {
+                if (wt == NWT - 1 && !full) {
+                    C[wt] = f32x4{kNegBig, kNegBig, kNegBig, kNegBig};
+                    break;
+                }
                 f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int ks = 0; ks < G::KS; ++ks) acc = Ops<T>::mma(lds_row8<T>(Kt + G::at(16 * wt + r, 4 * ks + q)), xb[ks], acc);
@@ -644,7 +653,11 @@ struct RProb {
             mx = fmaxf(quad_rows_max(mx), P.eps * kLog2e);
             float sum = 0.f, ent = 0.f;
 #pragma unroll
-            for (int wt = 0; wt < NWT; ++wt)
+            for (int wt = 0; wt < NWT; ++wt) {
+                if (wt == NWT - 1 && !full) {
+                    C[wt] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    break;
+                }
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const float d = C[wt][v] - mx;
@@ -653,6 +666,7 @@ struct RProb {
                     ent = fmaf(p, d, ent);  // sum p * log2(p)
                     C[wt][v] = p;
                 }
+            }
             sum = quad_rows_sum(sum);
             ent = quad_rows_sum(ent);
             const float den = sum + P.eps;
@@ -774,8 +788,10 @@ struct ZProb {
             if (tix < ROWS) cb[tix] = st.cbv;
         }
         problem_sync<WPP>();
+        const bool full = NWT <= 4 || 16 * (NWT - 1) < P.M;   // (as in RProb)
 #pragma unroll
         for (int si = 0; si < SPW; ++si) {
+          if (!full && strip_of(wig, si) == NWT - 1) continue;
           V8 pb[(NWT + 1) / 2];
           if (active) {
             const int strip = strip_of(wig, si);
@@ -785,6 +801,10 @@ struct ZProb {
             f32x4 C[NWT];
 #pragma unroll
             for (int wt = 0; wt < NWT; ++wt) {
+                if (wt == NWT - 1 && !full) {
+                    C[wt] = f32x4{kNegBig, kNegBig, kNegBig, kNegBig};
+                    break;
+                }
                 f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int ks = 0; ks < G::KS; ++ks) acc = Ops<T>::mma(lds_row8<T>(At + G::at(16 * wt + r, 4 * ks + q)), xb[ks], acc);
@@ -802,13 +822,18 @@ struct ZProb {
             mx = quad_rows_max(mx);
             float sum = 0.f;
 #pragma unroll
-            for (int wt = 0; wt < NWT; ++wt)
+            for (int wt = 0; wt < NWT; ++wt) {
+                if (wt == NWT - 1 && !full) {
+                    C[wt] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    break;
+                }
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const float p = __builtin_amdgcn_exp2f(C[wt][v] - mx);
                     sum += p;
                     C[wt][v] = p;
                 }
+            }
             const float inv = rcp(quad_rows_sum(sum));
 #pragma unroll
             for (int wt = 0; wt < NWT; ++wt)
@@ -927,11 +952,13 @@ struct LProb {
             if (tix < ROWS) cb[tix] = st.cbv;
         }
         problem_sync<WPP>();
+        const bool full = NWT <= 4 || 16 * (NWT - 1) < P.M;   // (as in RProb)
         if (active) {
             // pass 1: lane holds query block l = l0 + r, rows = key blocks 16kt + 4q + v
 #pragma unroll
             for (int si = 0; si < SPW; ++si) {
                 const int l = 16 * (wig + si * WPP) + r;
+                if (!full && wig + si * WPP == NWT - 1) continue;
                 V8 xq[G::KS];
 #pragma unroll
                 for (int ks = 0; ks < G::KS; ++ks) xq[ks] = lds_row8<T>(Qt + G::at(l, 4 * ks + q));
@@ -939,6 +966,7 @@ struct LProb {
                 float mx = kNegBig;
 #pragma unroll
                 for (int kt = 0; kt < NWT; ++kt) {
+                    if (kt == NWT - 1 && !full) break;
                     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                     for (int ks = 0; ks < G::KS; ++ks) acc = Ops<T>::mma(lds_row8<T>(At + G::at(16 * kt + r, 4 * ks + q)), xq[ks], acc);
@@ -953,9 +981,11 @@ struct LProb {
                 mx = quad_rows_max(mx);
                 float sum = 0.f;
 #pragma unroll
-                for (int kt = 0; kt < NWT; ++kt)
+                for (int kt = 0; kt < NWT; ++kt) {
+                    if (kt == NWT - 1 && !full) break;
 #pragma unroll
                     for (int v = 0; v < 4; ++v) sum += __builtin_amdgcn_exp2f(C[kt][v] - mx);
+                }
                 sum = quad_rows_sum(sum);
                 if (q == 0) {
                     mxs[l] = mx;
@@ -970,6 +1000,7 @@ struct LProb {
 #pragma unroll
             for (int si = 0; si < SPW; ++si) {
                 const int k = 16 * (wig + si * WPP) + r;
+                if (!full && wig + si * WPP == NWT - 1) continue;
                 const bool kv = ti.ok(P, k);
                 V8 xk[G::KS];
 #pragma unroll
@@ -979,6 +1010,10 @@ struct LProb {
                 float crs = 0.f;
 #pragma unroll
                 for (int lt = 0; lt < NWT; ++lt) {
+                    if (lt == NWT - 1 && !full) {
+                        C[lt] = f32x4{0.f, 0.f, 0.f, 0.f};
+                        break;
+                    }
                     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                     for (int ks = 0; ks < G::KS; ++ks) acc = Ops<T>::mma(lds_row8<T>(Qt + G::at(16 * lt + r, 4 * ks + q)), xk[ks], acc);

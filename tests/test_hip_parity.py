@@ -355,6 +355,19 @@ def test_slice_resident_kernel(E, H, N, D, B, T, pre, dt, masked):
     assert_parity(out[few, :2].cpu(), ref, dt, f"slices {(E, H, N, D, B, T)}")
 
 
+@pytest.mark.parametrize("variant", ["chained", "fused"])
+@pytest.mark.parametrize("B,M,D,T,dt", [(65, 96, 64, 2, "f16"), (80, 65, 72, 1, "bf16"), (81, 80, 128, 2, "f16"), (97, 112, 32, 2, "bf16"),
+                                        (112, 128, 64, 1, "f16"), (113, 72, 96, 2, "f16"), (40, 104, 64, 3, "f16")])
+def test_classes_whose_last_strip_is_empty(B, M, D, T, dt, variant):
+    """65 .. 80 and 97 .. 112 rows or blocks in the 6- and 8-strip kernels: nothing of the last strip exists."""
+    N = B * M - 5
+    q, k, v = seeded_qkv(1, 2, N, D, DT[dt], seed=B + M)
+    mask = block_safe_mask(1, N, B, seed=M)
+    ref = monarch_attention_oracle(q, k, v, mask, T, B, True, upcast=True)
+    out = run_hip(*to_dev(q, k, v, mask), T, B, True, variant)
+    assert_parity(out.cpu(), ref, dt, f"empty strip {(B, M, D, T, dt)}")
+
+
 SMALL_F32 = [  # E, H, N, D, B, T, pre, masked: fp32 heads of at most 16 blocks of at most 16 rows
     (1, 1, 256, 64, 16, 1, False, False),      # the reference's CPU-sized case
     (2, 3, 197, 64, 16, 1, True, True), (1, 4, 100, 32, 8, 1, False, True), (3, 2, 250, 48, 16, 1, True, False),   # a single step, few heads
