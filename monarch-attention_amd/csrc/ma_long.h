@@ -498,8 +498,8 @@ __global__ __launch_bounds__(64 * W, EU) void r_step_long(Problem P, int first) 
     using MT = Mat<T, DT>;
     using PL = typename std::conditional<kV, RPlan<T, DT, NWT>, KPlan<T, DT, NWT>>::type;
     using V4 = typename Pack<T>::V4;
-    constexpr int NTH = 64 * W, ROWS = 16 * NWT, GROUPS = NWT / (W * SP);
-    static_assert(PL::NC1 == 1 && NWT % (W * SP) == 0, "the problem's tiles fit the LDS");
+    constexpr int NTH = 64 * W, ROWS = 16 * NWT, GROUPS = (NWT + W * SP - 1) / (W * SP);
+    static_assert(PL::NC1 == 1 && NWT % SP == 0, "the problem's tiles fit the LDS");
     extern __shared__ __attribute__((aligned(16))) char lds_raw[];
     T* Kt = reinterpret_cast<T*>(lds_raw);
     T* Vt = Kt + ROWS * MT::LD;
@@ -546,6 +546,7 @@ __global__ __launch_bounds__(64 * W, EU) void r_step_long(Problem P, int first) 
 #pragma unroll 1
         for (int g = 0; g < GROUPS; ++g) {
             const int s0 = 16 * SP * (wave + g * W);
+            if (s0 >= B) break;   // (strips of which nothing exists)
             typename MT::Row xb[SP];
             float cj[SP];
 #pragma unroll
@@ -632,8 +633,8 @@ __global__ __launch_bounds__(64 * W, EU) void z_step_long(Problem P) {
     using MT = Mat<T, DT>;
     using PL = RPlan<T, DT, NWT>;
     using V4 = typename Pack<T>::V4;
-    constexpr int NTH = 64 * W, ROWS = 16 * NWT, GROUPS = NWT / (W * SP);
-    static_assert(PL::NC1 == 1 && NWT % (W * SP) == 0, "the problem's tiles fit the LDS");
+    constexpr int NTH = 64 * W, ROWS = 16 * NWT, GROUPS = (NWT + W * SP - 1) / (W * SP);
+    static_assert(PL::NC1 == 1 && NWT % SP == 0, "the problem's tiles fit the LDS");
     extern __shared__ __attribute__((aligned(16))) char lds_raw[];
     T* At = reinterpret_cast<T*>(lds_raw);
     T* Yt = At + ROWS * MT::LD;
@@ -671,6 +672,7 @@ __global__ __launch_bounds__(64 * W, EU) void z_step_long(Problem P) {
 #pragma unroll 1
     for (int g = 0; g < GROUPS; ++g) {
         const int s0 = 16 * SP * (wave + g * W);
+        if (s0 >= M) break;
         typename MT::Row xq[SP];
 #pragma unroll
         for (int s = 0; s < SP; ++s) xq[s] = xn[s];
@@ -721,8 +723,8 @@ __global__ __launch_bounds__(64 * W, EU) void l_step_long(Problem P) {
     using MT = Mat<T, DT>;
     using PL = LPlan<T, DT, NWT>;
     using V4 = typename Pack<T>::V4;
-    constexpr int NTH = 64 * W, ROWS = 16 * NWT, GROUPS = NWT / (W * SP);
-    static_assert(PL::NC1 == 1 && NWT % (W * SP) == 0, "the problem's tiles fit the LDS");
+    constexpr int NTH = 64 * W, ROWS = 16 * NWT, GROUPS = (NWT + W * SP - 1) / (W * SP);
+    static_assert(PL::NC1 == 1 && NWT % SP == 0, "the problem's tiles fit the LDS");
     extern __shared__ __attribute__((aligned(16))) char lds_raw[];
     T* At = reinterpret_cast<T*>(lds_raw);
     T* Qt = At + ROWS * MT::LD;
@@ -753,6 +755,7 @@ __global__ __launch_bounds__(64 * W, EU) void l_step_long(Problem P) {
 #pragma unroll 1
     for (int g = 0; g < GROUPS; ++g) {
         const int s0 = 16 * SP * (wave + g * W);
+        if (s0 >= M) break;
         typename MT::Row xq[SP];
 #pragma unroll
         for (int s = 0; s < SP; ++s) MT::from_tile(xq[s], Qt, s0 + 16 * s + r, q);
@@ -779,6 +782,7 @@ __global__ __launch_bounds__(64 * W, EU) void l_step_long(Problem P) {
 #pragma unroll 1
     for (int g = 0; g < GROUPS; ++g) {
         const int s0 = 16 * SP * (wave + g * W);
+        if (s0 >= M) break;
         typename MT::Row ak[SP];
         float ck[SP], cr[SP];
 #pragma unroll
@@ -820,16 +824,22 @@ __global__ __launch_bounds__(64 * W, EU) void l_step_long(Problem P) {
 // workgroups fit (D <= 96: one strip per wave then).  129 .. 192 rows at D > 96: as many waves as strips, or, for an R
 // step without V, narrow workgroups, more of them.  Measured over W = 4 .. 16, one to four strips and EU = 1 .. 4 on six shapes:
 // within 3 % of the best setting.
-// At most one problem per compute unit (FEW): as many waves as strips, since a wave's strips then run one after the other while
-// most of the compute unit is idle.  A head of 10672 tokens, D = 72, 64-row blocks, two steps: 34.5 -> 28.6 us; of 40000, D = 64,
-// 200-row blocks: 54.3 -> 51.0; of 30000, D = 96: 59.1 -> 53.1; four heads of 10672, D = 64, 64-row blocks: 36.0 -> 31.4.
+// FEW problems: at most one per compute unit, or two where two such workgroups share one (129 .. 192 rows of D <= 64; wider or
+// longer ones lose 2 - 12 % there).  As many waves as strips, since a wave's strips would run one after the other while most of the
+// compute unit is idle.  One head of 10672 tokens, D = 72, 64-row blocks, two steps: 34.5 -> 28.6 us; of 40000, D = 64, 200-row
+// blocks: 54.3 -> 51.0; of 30000, D = 96: 59.1 -> 53.1; two heads of 22000, D = 64, 140 rows: 54.4 -> 48.3; eight of 10672, 64 rows:
+// 55.4 -> 51.1.
+// Classes of 10, 12, 14 and 16 strips; strips beyond the last row are passed over.  Measured without the classes of 10 and 14 ->
+// with them: 32 heads of 22000, D = 64, 140-row blocks, two steps 414 -> 345 us; 16 of 40000, D = 64, 200 rows 450 -> 382;
+// 16 of 48000, D = 96, 220 rows, one step 419 -> 390; 16 of 40000, D = 128, 200 rows 454 -> 429.  (Workgroups of 5 and 7 waves,
+// which the strips fill evenly, lose 1 - 4 % to those of 4 and 8.)
 template <int STAGE, bool kV, int DT, int NWT, bool FEW>
 struct Cfg {
-    static constexpr bool kWideRow = DT > 4, k16 = NWT == 16, kKeysOnly = STAGE == kStageR && !kV;
+    static constexpr bool kWideRow = DT > 4, k16 = NWT > 12, kKeysOnly = STAGE == kStageR && !kV;
     static constexpr bool kOne = FEW && !(STAGE == kStageR && k16 && kWideRow);   // (there the registers of 16 waves do not hold a strip)
-    static constexpr int W = kOne ? NWT : k16 ? 8 : DT == 8 && !kKeysOnly ? 12 : 4;
+    static constexpr int W = kOne ? NWT : k16 ? 8 : DT == 8 && !kKeysOnly ? NWT : 4;
     static constexpr int SP = k16 && kWideRow && !kOne && !(kKeysOnly && DT == 6) ? 2 : 1;
-    static constexpr int EU = kOne ? NWT / 4 : !kWideRow ? 4 : SP == 2 ? 2 : k16 ? 4 : 3;
+    static constexpr int EU = kOne ? (NWT + 3) / 4 : !kWideRow ? 4 : SP == 2 ? 2 : k16 ? 4 : 3;
 };
 
 template <class T, int DT>
@@ -862,15 +872,16 @@ int launch(const Problem& P, int stage, bool first, bool with_v, hipStream_t s) 
             if (with_v) return run(r_step_long<T, DT, NWT, CV::W, CV::EU, CV::SP, true>, RPlan<T, DT, NWT>::kLds, problems, 1, CV::W, s, P, first ? 1 : 0);
             return run(r_step_long<T, DT, NWT, CK::W, CK::EU, CK::SP, false>, KPlan<T, DT, NWT>::kLds, problems, 1, CK::W, s, P, first ? 1 : 0);
         };
-        if (problems <= mfma::compute_units()) return go(std::true_type{});
+        if (problems <= (DT <= 4 && NWT <= 12 ? 2 : 1) * mfma::compute_units()) return go(std::true_type{});
         return go(std::false_type{});
     };
-    switch (strip_class(stage == kStageR ? P.B : P.M)) {
-        case 6: return pair(std::integral_constant<int, 6>{});
-        case 8: return pair(std::integral_constant<int, 8>{});
-        case 12: return whole(std::integral_constant<int, 12>{});
-        default: return whole(std::integral_constant<int, 16>{});
-    }
+    const int strips = ((stage == kStageR ? P.B : P.M) + 15) / 16;
+    if (strips <= 6) return pair(std::integral_constant<int, 6>{});
+    if (strips <= 8) return pair(std::integral_constant<int, 8>{});
+    if (strips <= 10) return whole(std::integral_constant<int, 10>{});
+    if (strips <= 12) return whole(std::integral_constant<int, 12>{});
+    if (strips <= 14) return whole(std::integral_constant<int, 14>{});
+    return whole(std::integral_constant<int, 16>{});
 }
 
 }  // namespace lng

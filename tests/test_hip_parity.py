@@ -999,15 +999,16 @@ def test_long_stages_with_and_without_masked_keys(B, M, D, dt, masked):
 
 @pytest.mark.parametrize("N,D,B,T,dt,masked", [
     (140 * 150, 64, 140, 2, "f16", True), (230 * 210, 40, 210, 1, "bf16", False), (180 * 250, 96, 180, 2, "bf16", True), (256 * 190, 128, 256, 2, "f16", False),
+    (129 * 208, 64, 129, 2, "bf16", False), (160 * 193, 32, 160, 2, "f16", True), (144 * 224, 128, 144, 1, "f16", True), (161 * 225, 48, 161, 2, "f16", False),
 ])
 def test_long_stages_of_few_and_of_more_problems(N, D, B, T, dt, masked):
-    """129 .. 256 rows: one head has at most one problem per compute unit, which takes as many waves as strips; three heads have
-    more, in narrower workgroups.  A head's result is the same in both."""
-    q, k, v = seeded_qkv(1, 3, N, D, DT[dt], seed=N + B)
+    """129 .. 256 rows: the problems of one head fit the compute units side by side and take as many waves as strips; those of five
+    do not and run in narrower workgroups.  A head's result is the same in both."""
+    q, k, v = seeded_qkv(1, 5, N, D, DT[dt], seed=N + B)
     mask = block_safe_mask(1, N, B, seed=B) if masked else None
     q, k, v, mask = to_dev(q, k, v, mask)
     out = monarch_attention_hip(q, k, v, mask, T, B, False)
-    for h in (0, 2):
+    for h in (0, 4):
         one = monarch_attention_hip(q[:, h:h + 1], k[:, h:h + 1], v[:, h:h + 1], mask, T, B, False)
         assert torch.equal(one[:, 0], out[:, h])
     gen = monarch_attention_hip(q[:, :1], k[:, :1], v[:, :1], mask, T, B, False, variant="generic")
