@@ -223,21 +223,19 @@ bool resident_head_fits(const ma_fwd_params* p, int forms = 1) {
 // LDS whole stay with the head-resident kernels where those are chosen, but for blocks of 14 and 15 rows and for a single pass of
 // slices: beyond, which of the two is ahead turns on how the last pass ends (0.6 - 1.4).  In the comments: multiples of the time of the kernel
 // it replaces, at D = 32 .. 80, 64 .. 4096 tokens, 8 .. 768 heads, T = 1, 2, 3 (profiles/slice_resident_sweep.md).
-bool slice_pays(const ma_fwd_params* p, int v) {
+bool slice_is_ahead(const ma_fwd_params* p, int v) {
     if (p->dtype_qk == MA_F32 || (v != MA_VARIANT_CHAINED && v != MA_VARIANT_RESIDENT)) return false;
-    Problem P = sizes_of(p);
-    P.one_tile_ok = 1;
-    if (P.B > 64 || P.M > 64 || run_slice(P, p->dtype_qk, true, nullptr) != MA_OK) return false;
-    const long long heads = static_cast<long long>(P.E) * P.H, slices = heads * ((P.B + 15) / 16);
-    const int B = P.B, M = P.M, D = P.D;
-    const bool multi = P.T >= 2, wide = D > 64;
+    const int B = p->B, M = (p->N + p->B - 1) / p->B, D = p->D;
+    if (B > 64 || M > 64) return false;
+    const long long heads = static_cast<long long>(p->E) * p->H, slices = heads * ((B + 15) / 16);
+    const bool multi = p->T >= 2, wide = D > 64;
     if (B <= 16) {   // one slice a head: beside the head-resident kernels, which lose to padding where blocks are a little short of 16 rows
         if (B == 16 || B < 14 || M < 12) return false;
         if (M > 32) return multi && heads >= 192;                                             // 0.6 - 0.85
         if (M > 16) return heads >= 112 && heads <= 288 && (multi || D <= 32);              // 0.83 - 1.0
         if (!multi) return heads >= 96 && heads <= (wide ? 400 : 256);                       // 0.78 - 0.91
-        return wide ? heads >= (P.T == 2 ? 64 : 8) && heads <= 400                            // 0.80 - 0.94
-                    : heads <= 256 && (P.T == 2 || B == 15);                                  // 0.85 - 0.99 (others 0.96 - 1.02)
+        return wide ? heads >= (p->T == 2 ? 64 : 8) && heads <= 400                            // 0.80 - 0.94
+                    : heads <= 256 && (p->T == 2 || B == 15);                                  // 0.85 - 0.99 (others 0.96 - 1.02)
     }
     if (v == MA_VARIANT_RESIDENT && heads > 128 && resident_head_fits(p, 2)) return false;
     const bool most = slices >= 192 && multi && B <= 32 && M > 16 && M <= 32 && (wide ? B >= 30 && M >= 28 : B >= 24);   // 0.79 - 0.98
@@ -259,6 +257,12 @@ bool slice_pays(const ma_fwd_params* p, int v) {
         return multi && heads >= 512 && M > 16;                                               // 0.76 - 0.97
     }
     return D <= 32 && multi && B >= 56 && (heads <= 64 || (heads >= 112 && M >= 30));         // 0.63 - 0.94
+}
+bool slice_pays(const ma_fwd_params* p, int v) {
+    if (!slice_is_ahead(p, v)) return false;   // (first: it costs a few comparisons of the host's time, 6 us calls lost 1 % otherwise)
+    Problem P = sizes_of(p);
+    P.one_tile_ok = 1;
+    return run_slice(P, p->dtype_qk, true, nullptr) == MA_OK;   // the state fits in LDS
 }
 
 // The fused, chained and resident kernels are built for block problems of at most 128 rows.
