@@ -359,26 +359,26 @@ __device__ __forceinline__ void store_row(rsrc_t dst, unsigned ro, int D, const 
     if (MODE != kRun || (DT % 2 == 0 && whole)) {
         const int col0 = MODE == kRun ? 4 * DT * q : 8 * q;   // the pieces sit at fixed distances from this column
         const unsigned base = ro + 2 * col0;
-        u32x4 x[DT / 2 + 1];
-        unsigned off[DT / 2 + 1];
-#pragma unroll
-        for (int p = 0; p < DT / 2; ++p) {
+        auto piece = [&](int p) {
             const u32x2 lo = __builtin_bit_cast(u32x2, v[2 * p]), hi = __builtin_bit_cast(u32x2, v[2 * p + 1]);
-            x[p] = MODE == kTile ? pair_piece(lo, hi) : u32x4{lo[0], lo[1], hi[0], hi[1]};
-            off[p] = base + (MODE == kRun ? 16 : 64) * p;
-            if (!whole) off[p] = 32 * p + 8 * q < D ? off[p] : kOob;   // (kRun: whole rows only here)
+            return MODE == kTile ? pair_piece(lo, hi) : u32x4{lo[0], lo[1], hi[0], hi[1]};
+        };
+        bool stored = false;
+        if constexpr (LINES && MODE != kRun && DT == 4) {
+            if (whole) {
+                if (stream) store_pieces<2>(dst, piece(0), base, piece(1), base + 64);
+                else store_pieces<0>(dst, piece(0), base, piece(1), base + 64);
+                stored = true;
+            }
         }
+        if (!stored) {
 #pragma unroll
-        for (int p = 0; p < DT / 2; p += 2) {
-            if (LINES && MODE != kRun && DT == 4 && whole) {
-                if (stream) store_pieces<2>(dst, x[p], off[p], x[p + 1], off[p + 1]);
-                else store_pieces<0>(dst, x[p], off[p], x[p + 1], off[p + 1]);
-            } else {
-#pragma unroll
-                for (int s = p; s < p + 2 && s < DT / 2; ++s) {
-                    if (stream) __builtin_amdgcn_raw_buffer_store_b128(x[s], dst, off[s], 0, 2);
-                    else __builtin_amdgcn_raw_buffer_store_b128(x[s], dst, off[s], 0, 0);
-                }
+            for (int p = 0; p < DT / 2; ++p) {
+                const u32x4 x = piece(p);
+                unsigned off = base + (MODE == kRun ? 16 : 64) * p;
+                if (!whole) off = 32 * p + 8 * q < D ? off : kOob;   // (kRun: whole rows only here)
+                if (stream) __builtin_amdgcn_raw_buffer_store_b128(x, dst, off, 0, 2);
+                else __builtin_amdgcn_raw_buffer_store_b128(x, dst, off, 0, 0);
             }
         }
         if (DT % 2 == 1) {
@@ -608,10 +608,10 @@ struct RProb {
             if (tix < ROWS) kbias[tix] = (tix < P.B && token_kept(P, m * P.B - P.pad_off + tix, pre.km)) ? 0.f : kNegBig;
         }
         problem_sync<WPP>();
-        // The last strip has rows (uniform).  65 - 80 and 97 - 112 rows leave it empty in the classes of 6 and 8 strips: as a strip
-        // of queries and as a tile of keys it is passed over (16 heads of 5003, 72-row blocks, two steps: D = 64 44.8 -> 40.3 us,
-        // D = 128 74 -> 70; 104-row blocks, 10600 tokens, D = 64: 78.7 -> 74; full classes unchanged).
-        const bool full = NWT <= 4 || 16 * (NWT - 1) < B;
+        // The last strip has rows (uniform).  65 - 80 rows leave it empty in the class of 6 strips: it is passed over (16 heads of 5003,
+        // 72-row blocks, two steps: D = 64 45.2 -> 42.9 us, D = 128 75.1 -> 72.3; full classes unchanged).  Passing over its tile of
+        // keys too gives as much again, but takes 16 registers, and full strips lose 1 - 2 %; so do 8 strips with either.
+        const bool full = NWT != 6 || 16 * (NWT - 1) < B;
 #pragma unroll
         for (int si = 0; si < SPW; ++si) {
           if (!full && strip_of(wig, si) == NWT - 1) continue;
@@ -632,10 +632,6 @@ struct RProb {
             f32x4 C[NWT];
 #pragma unroll
             for (int wt = 0; wt < NWT; ++wt) {
-                if (wt == NWT - 1 && !full) {
-                    C[wt] = f32x4{kNegBig, kNegBig, kNegBig, kNegBig};
-                    break;
-                }
                 f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int ks = 0; ks < G::KS; ++ks) acc = Ops<T>::mma(lds_row8<T>(Kt + G::at(16 * wt + r, 4 * ks + q)), xb[ks], acc);
@@ -654,10 +650,6 @@ struct RProb {
             float sum = 0.f, ent = 0.f;
 #pragma unroll
             for (int wt = 0; wt < NWT; ++wt) {
-                if (wt == NWT - 1 && !full) {
-                    C[wt] = f32x4{0.f, 0.f, 0.f, 0.f};
-                    break;
-                }
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const float d = C[wt][v] - mx;
@@ -788,7 +780,7 @@ struct ZProb {
             if (tix < ROWS) cb[tix] = st.cbv;
         }
         problem_sync<WPP>();
-        const bool full = NWT <= 4 || 16 * (NWT - 1) < P.M;   // (as in RProb)
+        const bool full = NWT != 6 || 16 * (NWT - 1) < P.M;   // (as in RProb)
 #pragma unroll
         for (int si = 0; si < SPW; ++si) {
           if (!full && strip_of(wig, si) == NWT - 1) continue;
@@ -801,10 +793,6 @@ struct ZProb {
             f32x4 C[NWT];
 #pragma unroll
             for (int wt = 0; wt < NWT; ++wt) {
-                if (wt == NWT - 1 && !full) {
-                    C[wt] = f32x4{kNegBig, kNegBig, kNegBig, kNegBig};
-                    break;
-                }
                 f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int ks = 0; ks < G::KS; ++ks) acc = Ops<T>::mma(lds_row8<T>(At + G::at(16 * wt + r, 4 * ks + q)), xb[ks], acc);
@@ -823,10 +811,6 @@ struct ZProb {
             float sum = 0.f;
 #pragma unroll
             for (int wt = 0; wt < NWT; ++wt) {
-                if (wt == NWT - 1 && !full) {
-                    C[wt] = f32x4{0.f, 0.f, 0.f, 0.f};
-                    break;
-                }
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const float p = __builtin_amdgcn_exp2f(C[wt][v] - mx);
@@ -952,13 +936,16 @@ struct LProb {
             if (tix < ROWS) cb[tix] = st.cbv;
         }
         problem_sync<WPP>();
-        const bool full = NWT <= 4 || 16 * (NWT - 1) < P.M;   // (as in RProb)
+        const bool full = NWT != 6 || 16 * (NWT - 1) < P.M;   // (as in RProb)
         if (active) {
             // pass 1: lane holds query block l = l0 + r, rows = key blocks 16kt + 4q + v
 #pragma unroll
             for (int si = 0; si < SPW; ++si) {
                 const int l = 16 * (wig + si * WPP) + r;
-                if (!full && wig + si * WPP == NWT - 1) continue;
+                if (!full && wig + si * WPP == NWT - 1) {   // (pass 2 reads its statistics)
+                    if (q == 0) mxs[l] = invs[l] = 0.f;
+                    continue;
+                }
                 V8 xq[G::KS];
 #pragma unroll
                 for (int ks = 0; ks < G::KS; ++ks) xq[ks] = lds_row8<T>(Qt + G::at(l, 4 * ks + q));
@@ -966,7 +953,6 @@ struct LProb {
                 float mx = kNegBig;
 #pragma unroll
                 for (int kt = 0; kt < NWT; ++kt) {
-                    if (kt == NWT - 1 && !full) break;
                     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                     for (int ks = 0; ks < G::KS; ++ks) acc = Ops<T>::mma(lds_row8<T>(At + G::at(16 * kt + r, 4 * ks + q)), xq[ks], acc);
@@ -982,7 +968,6 @@ struct LProb {
                 float sum = 0.f;
 #pragma unroll
                 for (int kt = 0; kt < NWT; ++kt) {
-                    if (kt == NWT - 1 && !full) break;
 #pragma unroll
                     for (int v = 0; v < 4; ++v) sum += __builtin_amdgcn_exp2f(C[kt][v] - mx);
                 }
@@ -1010,10 +995,6 @@ struct LProb {
                 float crs = 0.f;
 #pragma unroll
                 for (int lt = 0; lt < NWT; ++lt) {
-                    if (lt == NWT - 1 && !full) {
-                        C[lt] = f32x4{0.f, 0.f, 0.f, 0.f};
-                        break;
-                    }
                     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                     for (int ks = 0; ks < G::KS; ++ks) acc = Ops<T>::mma(lds_row8<T>(Qt + G::at(16 * lt + r, 4 * ks + q)), xk[ks], acc);
