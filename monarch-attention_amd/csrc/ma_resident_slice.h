@@ -21,8 +21,8 @@
 //
 // What bounds it: the chain of a wave's problems (2 T phases of M / W and 16 / W problems) behind the arrival of the first tiles.
 // The keys of a head are read by each of its slices, from the XCD's L2 (slices of a head run on one XCD, next to each other).
-// 128 heads of 1024 tokens, D = 72, 32-row blocks (256 workgroups of 16 waves), T = 3: 53 us, 77.5 in the chained kernel
-// (vector instructions issue in half of the cycles; 175 MB of memory traffic, 404 MB chained); T = 1: 26 us, 31.  Where it is
+// 128 heads of 1024 tokens, D = 72, 32-row blocks (256 workgroups of 16 waves), T = 3: 46.4 us, 77.5 in the chained kernel
+// (vector instructions issue in half of the cycles; 188 MB of memory traffic, 404 MB chained); T = 1: 26 us, 31.  Where it is
 // chosen: slice_pays in ma_api.hip; in how many waves: ma_slice_launch.h.
 //
 // Sums, roundings and their order are those of RProb, LProb and ZProb (ma_mfma.h): a head's result does not depend on how many
@@ -323,7 +323,9 @@ struct Slice {
     }
 };
 
-// Workgroup id -> head and slice: the slices of a head are 8 ids apart (one XCD, dispatched one after the other).
+// Workgroup id -> head and slice: the slices of a head are 8 ids apart (one XCD, dispatched one after the other), and an XCD takes
+// heads that follow each other: rows that are no whole lines share them with the next head's where a token's heads lie side by side
+// (128 heads of 1024, D = 72, T = 3, (E, N, H, D): 312 -> 188 MB of traffic, 53.2 -> 46.4 us; D = 80, T = 1 31.7 -> 28.4; D = 64 unchanged).
 // 128 registers where two workgroups of 8 waves or one of 16 share a compute unit, else 256.
 template <class T, int DT, int NTB, int NTM, int W>
 __global__ __launch_bounds__(64 * W, W == 16 || (NTB <= 2 && NTM <= 2) ? 4 : W == 12 ? 3 : 2) void resident_slice_mfma(Problem P) {
@@ -332,7 +334,8 @@ __global__ __launch_bounds__(64 * W, W == 16 || (NTB <= 2 && NTM <= 2) ? 4 : W =
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int B = P.B, M = P.M, heads = P.E * P.H, slices = (B + 15) / 16;
     const unsigned id = blockIdx.x;
-    const int head = static_cast<int>(id / (8u * slices) * 8u + id % 8u), j0 = 16 * static_cast<int>(id / 8u % static_cast<unsigned>(slices));
+    const int per_xcd = (heads + 7) / 8, in_xcd = static_cast<int>(id / (8u * slices)), head = static_cast<int>(id % 8u) * per_xcd + in_xcd;
+    const int j0 = 16 * static_cast<int>(id / 8u % static_cast<unsigned>(slices));
     if (head >= heads) return;
     const int e = static_cast<unsigned>(head) / static_cast<unsigned>(P.H), h = static_cast<unsigned>(head) % static_cast<unsigned>(P.H);
     const Slices S = make_slices<T>(P, e, h, head);
