@@ -22,7 +22,7 @@
 // producers are still writing slows the whole memory channel of that line down.)
 //
 // Coherence: workgroup ids are dealt round-robin to the 8 XCDs, and head h only
-// uses ids with id % 8 == h % 8, so producers and consumers of a head share one
+// uses ids of one remainder by 8, so producers and consumers of a head share one
 // L2: publishing needs only "my stores are acknowledged" (vmcnt(0)), reading uses
 // streaming loads that never hit in L1 - no L2 write-back, no invalidate.  The
 // arrivals carry the XCC id of their workgroup (sum and sum of squares, which
@@ -48,7 +48,8 @@ namespace ma {
 namespace mfma {
 
 struct ChainPlan {
-    int hx;        // heads per XCD (heads xcd, xcd + 8, ...)
+    int hx;        // heads per XCD: heads hs * xcd, + hk, + 2 hk, ...
+    int hs, hk;
     int tR, tL;    // tasks per head in an R phase / an L or Z phase
     int stride;    // sync words per head (see chain_stride)
     int go_off;    // offset of the release words inside a head's words
@@ -118,7 +119,7 @@ __global__ __launch_bounds__(64 * W) void chain_fwd_mfma(Problem P, ChainPlan pl
     const int p = 2 * step + (odd ? 1 : 0);
     const unsigned tasks = odd ? plan.tL : plan.tR;
     const unsigned idx = odd ? rem - perR : rem;
-    const int head = xcd + 8 * (idx / tasks);
+    const int head = xcd * plan.hs + (idx / tasks) * plan.hk;
     const int task = idx % tasks;
     if (p >= nph || head >= heads) return;
     const int e = static_cast<unsigned>(head) / static_cast<unsigned>(P.H), h = static_cast<unsigned>(head) % static_cast<unsigned>(P.H);
