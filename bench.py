@@ -2,9 +2,9 @@
 """Benchmark of the MonarchAttention forward pass on one MI355X.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--config cM] [--T 1]
-                    [--variant auto|generic|staged|fused|resident|chained] [--no-cpu] [--no-sdpa] [--no-sweep]
+                    [--variant auto|generic|staged|fused|resident|chained|sliced] [--no-cpu] [--no-sdpa] [--no-sweep]
     python bench.py --sweep-n | --sweep-e        # the reference's own sweep protocol, against dense SDPA
-    python bench.py --sweep-variants [--T 2] [--head-dim 64] [--sweep-grid class96|fewheads|ragged|mid|short]   # every variant over a grid of shapes: AUTO's choice vs the fastest
+    python bench.py --sweep-variants [--T 2] [--head-dim 64] [--sweep-grid class96|fewheads|ragged|mid|short|slices] [--sweep-layout heads|tokens]   # every variant over a grid of shapes: AUTO's choice vs the fastest
     python bench.py --record-traffic FETCH.csv WRITE.csv [--config cM --T 1 --variant auto]
 
 A step is ONE forward call of the hot path (monarch_attention, all T steps)
@@ -67,7 +67,7 @@ MFMA_PEAK_TFLOPS_F32 = 157.3   # dense fp32
 FETCH_SIZE_FACTOR = 2.00       # FETCH_SIZE under-reports a plain copy of known size by this factor (profiles/traffic_forward_kernels.md)
 TRAFFIC_JSON = os.path.join(ROOT, "profiles", "traffic.json")
 KERNEL_DIR = os.path.join(ROOT, "monarch-attention_amd", "csrc")
-ONE_LAUNCH = ("fused", "resident", "chained")   # variants that are one kernel launch per forward (its name: ma_fwd_kernel_name)
+ONE_LAUNCH = ("fused", "resident", "chained", "sliced")   # variants that are one kernel launch per forward (its name: ma_fwd_kernel_name)
 
 
 def kernel_source_hash() -> str:
@@ -101,6 +101,7 @@ def record_traffic(args) -> None:
     fetch_csv, write_csv = args.record_traffic
 
     names = ("r_step_mfma", "l_step_mfma", "z_step_mfma", "fused_fwd_mfma", "chain_fwd_mfma", "resident_fwd_mfma", "resident_head_mfma", "resident_head2_mfma",
+             "resident_slice_mfma",
              "r_step_f32", "l_step_f32", "z_step_f32", "head_fwd_f32", "head_t1_f32",
              "r_step_pair", "l_step_pair", "z_step_pair", "r_step_long", "l_step_long", "z_step_long")
 
@@ -120,7 +121,7 @@ def record_traffic(args) -> None:
     T = args.T or T
     # launches of each kernel in one forward (the bench also launches single stages for the per-stage timings:
     # the per-dispatch means make that irrelevant)
-    per_fwd = {"r_step_mfma": T, "l_step_mfma": T - 1, "z_step_mfma": 1, "fused_fwd_mfma": 1, "chain_fwd_mfma": 1, "resident_fwd_mfma": 1,
+    per_fwd = {"r_step_mfma": T, "l_step_mfma": T - 1, "z_step_mfma": 1, "fused_fwd_mfma": 1, "chain_fwd_mfma": 1, "resident_fwd_mfma": 1, "resident_slice_mfma": 1,
                "resident_head_mfma": 1, "resident_head2_mfma": 1, "r_step_f32": T, "l_step_f32": T - 1, "z_step_f32": 1, "head_fwd_f32": 1, "head_t1_f32": 1,
                "r_step_pair": T, "l_step_pair": T - 1, "z_step_pair": 1, "r_step_long": T, "l_step_long": T - 1, "z_step_long": 1}
     kernels, total = {}, 0.0
@@ -151,7 +152,7 @@ def main():
     ap.add_argument("--warmup", type=int, default=40)
     ap.add_argument("--config", default="cM", choices=sorted(CONFIGS))
     ap.add_argument("--T", type=int, default=None, help="override the number of alternating steps")
-    ap.add_argument("--variant", default="auto", choices=["auto", "generic", "staged", "fused", "resident", "chained"])
+    ap.add_argument("--variant", default="auto", choices=["auto", "generic", "staged", "fused", "resident", "chained", "sliced"])
     ap.add_argument("--rotate-workspaces", action="store_true",
                     help="a workspace per input set (default: all sets share one, like the calls of a model)")
     ap.add_argument("--shared-device", action="store_true",
@@ -170,10 +171,13 @@ def main():
                          "N = 256 .. 8192, blocks of 16 .. 128 rows (T from --T, default 2; head dim from --head-dim); prints the rows "
                          "and how far AUTO's choice is from the fastest variant")
     ap.add_argument("--head-dim", type=int, default=64, help="head dim of --sweep-variants")
-    ap.add_argument("--sweep-grid", default="pow2", choices=["pow2", "class96", "fewheads", "ragged", "mid", "short"],
+    ap.add_argument("--sweep-grid", default="pow2", choices=["pow2", "class96", "fewheads", "ragged", "mid", "short", "slices"],
                     help="shapes of --sweep-variants: power-of-two lengths and blocks, blocks / block counts in the 96-row tile class, "
                          "few heads of thousands of tokens, lengths that are no multiple of the block (197, 500, 1000, 3000, 5000, 7600), "
-                         "heads of 256 .. 1000 tokens, or up to thousands of heads of at most 256 tokens")
+                         "heads of 256 .. 1000 tokens, up to thousands of heads of at most 256 tokens, or heads of blocks and block "
+                         "counts of up to 64 (the sizes of the slice-resident kernel)")
+    ap.add_argument("--sweep-layout", default="heads", choices=["heads", "tokens"],
+                    help="layout of --sweep-variants: contiguous (E, H, N, D), or views of (E, N, H, D)")
     ap.add_argument("--sweep-dtype", default="f16", choices=["f16", "bf16", "f32"], help="operand dtype of --sweep-variants")
     ap.add_argument("--sweep-mask", action="store_true", help="--sweep-variants with a key / query mask (int64, ~10 %% of the tokens masked out in whole runs)")
     ap.add_argument("--sweep-pre-pad", action="store_true", help="--sweep-variants with the padding at the front")
@@ -296,7 +300,7 @@ def main():
         T_, D = args.T or 2, args.head_dim
         # without the statement that the benchmark owns the device AUTO may not choose the team kernel: it is
         # then judged against the variants it may choose
-        names = ("staged", "chained", "resident") if args.shared_device else ("staged", "chained", "fused", "resident")
+        names = ("staged", "chained", "resident", "sliced") if args.shared_device else ("staged", "chained", "fused", "resident", "sliced")
         sdt = DT[args.sweep_dtype]
         selt = torch.empty((), dtype=sdt).element_size()
         rows, logsum, worst = [], 0.0, None
@@ -313,6 +317,14 @@ def main():
         elif args.sweep_grid == "short":      # hundreds to thousands of heads of at most 256 tokens (windows, patches): the narrow-workgroup forms
             grid = [(h, N, B) for h in (64, 128, 256, 384, 512, 768, 1024, 1536, 3072)
                     for (N, B) in ((49, 7), (64, 16), (96, 16), (128, 16), (128, 32), (160, 32), (197, 16), (224, 32), (256, 16))]
+        elif args.sweep_grid == "slices":     # heads of blocks and block counts of up to 64: 16 positions a workgroup against the rest
+            grid = [(h, N, B) for h in (8, 16, 32, 48, 64, 80, 96, 112, 128, 160, 192, 224, 256, 320, 384, 512, 768)
+                    for (N, B) in ((64, 8), (100, 10), (150, 12), (180, 13), (197, 14), (225, 15), (300, 15), (400, 15), (700, 15), (256, 16),
+                                   (128, 32), (150, 18), (200, 20), (256, 24), (256, 32), (300, 20), (350, 24), (400, 25), (400, 32), (480, 28),
+                                   (512, 32), (576, 24), (600, 30), (640, 20), (700, 27), (768, 32), (900, 30), (1024, 32), (1200, 20), (1200, 30),
+                                   (1500, 30), (2000, 32), (500, 40), (600, 40), (700, 48), (800, 40), (1024, 48), (1300, 36), (1500, 44),
+                                   (2000, 45), (2304, 48), (1024, 64), (1500, 50), (2304, 64), (3000, 60), (4096, 64))
+                    if h * N * D <= 60e6]
         elif args.sweep_grid == "fewheads":   # 8, 16, 24 heads of thousands of tokens: where the team kernel competes
             grid = [(h, N, B) for h in (8, 16, 24) for N in (2048, 4096, 5000, 6144, 8000, 8192) for B in (32, 64, 128)]
         else:   # blocks and / or block counts of 65 .. 96 rows (and two 128-row shapes with ragged block counts)
@@ -320,17 +332,21 @@ def main():
                     for (N, B) in ((8192, 96), (6000, 64), (4096, 48), (2048, 24), (1000, 80), (512, 96), (9000, 96), (5500, 80),
                                    (7000, 128), (12000, 128), (768, 96))]
         for (heads, N, B) in grid:
+            if len(rows) % 100 == 99:
+                print(f"{len(rows)} points", file=sys.stderr, flush=True)
             M = -(-N // B)
             set_bytes = 4 * heads * N * D * selt
             if M > 128 or M < 2 or set_bytes > (1.2e9 if args.sweep_grid == "pow2" else 0.6e9):
                 continue
             E, H = (heads // 4, 4) if heads % 4 == 0 else (1, heads)
-            gen = torch.Generator().manual_seed(0)
+            gen = torch.Generator(device=dev).manual_seed(0)
             nbuf = max(2, min(8, -(-400 * 2 ** 20 // set_bytes)))
-            base = [torch.randn(E, H, N, D, generator=gen).to(sdt) for _ in range(3)]
+            base = [torch.randn(E, H, N, D, generator=gen, device=dev).to(sdt) for _ in range(3)]
             sets = []
             for i in range(nbuf):
-                q, k, v = (t.to(dev).roll(i, dims=2).contiguous() for t in base)
+                q, k, v = (t.roll(i, dims=2).contiguous() for t in base)
+                if args.sweep_layout == "tokens":   # (E, H, N, D) views of (E, N, H, D), as models pass them
+                    q, k, v = (t.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3) for t in (q, k, v))
                 sets.append((q, k, v, torch.empty_like(q)))
             mask = None
             if args.sweep_mask:   # a tokenizer-style int64 mask: the tail of every sequence masked out, at most 10 % of it
@@ -342,6 +358,8 @@ def main():
                 sel = lib.ma_fwd_select_variant(ps[0])
                 if variant == "auto":
                     row["auto"] = L.VARIANT_NAMES[sel]
+                    if lib.ma_fwd_kernel_name(ps[0]) == b"resident_slice_mfma":   # (in place of the kernel that AUTO resolves to)
+                        row["auto"], row["in_place_of"] = "sliced", row["auto"]
                     continue
                 if sel < 0:
                     continue

@@ -81,11 +81,17 @@ typedef enum ma_variant {
                             /* inputs streamed (and Y through the workspace) up to   */
                             /* ~1000; several narrow workgroups per compute unit     */
                             /* when there are more short heads than compute units    */
-    MA_VARIANT_CHAINED = 5  /* MFMA, ONE launch, one workgroup per block problem of  */
+    MA_VARIANT_CHAINED = 5, /* MFMA, ONE launch, one workgroup per block problem of  */
                             /* every phase; a problem starts when its head's         */
                             /* previous phase has released it through the workspace. */
                             /* Producers are always dispatched before consumers: no  */
                             /* co-residency requirement, safe beside other kernels   */
+    MA_VARIANT_SLICED = 6   /* MFMA, ONE launch, a workgroup runs 16 in-block        */
+                            /* positions of a head through all T steps with their    */
+                            /* state in LDS: no exchange between workgroups.  16-bit, */
+                            /* d <= 80, blocks and block counts of at most 64 whose   */
+                            /* state fits beside the waves' tiles (else               */
+                            /* MA_ERR_UNSUPPORTED).  Same results as CHAINED          */
 } ma_variant;
 
 typedef enum ma_status {
@@ -189,9 +195,9 @@ uint64_t ma_fwd_workspace_bytes(const ma_fwd_params* p);
 int ma_workspace_init(const ma_fwd_params* p, void* stream);
 
 /* The variant MA_VARIANT_AUTO resolves to for this problem (a ma_variant), or
- * a negative ma_status.  Where AUTO resolves to CHAINED or RESIDENT, it may run a kernel that
- * no explicit variant does: 16 positions of a head per workgroup, without exchange between
- * workgroups ("resident_slice_mfma" by ma_fwd_kernel_name).  The workspace is the same. */
+ * a negative ma_status.  Where AUTO resolves to CHAINED or RESIDENT, it runs the kernel of SLICED
+ * in its place where that is faster ("resident_slice_mfma" by ma_fwd_kernel_name).  The
+ * workspace and the results are the same. */
 int ma_fwd_select_variant(const ma_fwd_params* p);
 
 /* Name of the kernel that does the bulk of the work for this problem under the variant it resolves to

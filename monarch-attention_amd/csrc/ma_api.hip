@@ -30,7 +30,7 @@ int check_shape(const ma_fwd_params* p) {
     if (p == nullptr) return MA_ERR_NULL;
     if (p->E < 1 || p->H < 1 || p->N < 1 || p->D < 1 || p->Dv < 1 || p->B < 1 || p->T < 1) return MA_ERR_SHAPE;
     if (!dtype_ok(p->dtype_qk) || !dtype_ok(p->dtype_v)) return MA_ERR_DTYPE;
-    if (p->variant < MA_VARIANT_AUTO || p->variant > MA_VARIANT_CHAINED) return MA_ERR_VARIANT;
+    if (p->variant < MA_VARIANT_AUTO || p->variant > MA_VARIANT_SLICED) return MA_ERR_VARIANT;
     if (p->flags & ~(MA_FLAG_SYNC_READY | MA_FLAG_TEST_NO_SPIN | MA_FLAG_DEVICE_EXCLUSIVE)) return MA_ERR_SHAPE;
     const long long M = (static_cast<long long>(p->N) + p->B - 1) / p->B;
     const long long Np = M * p->B;
@@ -258,12 +258,14 @@ bool slice_is_ahead(const ma_fwd_params* p, int v) {
     }
     return D <= 32 && multi && B >= 56 && (heads <= 64 || (heads >= 112 && M >= 30));         // 0.63 - 0.94
 }
-bool slice_pays(const ma_fwd_params* p, int v) {
-    if (!slice_is_ahead(p, v)) return false;   // (first: it costs a few comparisons of the host's time, 6 us calls lost 1 % otherwise)
+// Does the slice-resident kernel take the problem: a class of its strips and columns, the state in LDS?  (16-bit operands)
+bool slice_fits(const ma_fwd_params* p) {
     Problem P = sizes_of(p);
     P.one_tile_ok = 1;
-    return run_slice(P, p->dtype_qk, true, nullptr) == MA_OK;   // the state fits in LDS
+    return run_slice(P, p->dtype_qk, true, nullptr) == MA_OK;
 }
+// (the rule first: it costs a few comparisons of the host's time, 6 us calls lost 1 % otherwise)
+bool slice_pays(const ma_fwd_params* p, int v) { return slice_is_ahead(p, v) && slice_fits(p); }
 
 // The fused, chained and resident kernels are built for block problems of at most 128 rows.
 bool one_launch_tiles(const ma_fwd_params* p) {
@@ -508,6 +510,7 @@ int select_variant(const ma_fwd_params* p) {
         case MA_VARIANT_FUSED: return fast && one_launch_tiles(p) ? MA_VARIANT_FUSED : MA_ERR_UNSUPPORTED;
         case MA_VARIANT_CHAINED: return fast && chain_fits(p) ? MA_VARIANT_CHAINED : MA_ERR_UNSUPPORTED;
         case MA_VARIANT_RESIDENT: return (fast || fast32) && resident_fits(p, true) ? MA_VARIANT_RESIDENT : MA_ERR_UNSUPPORTED;
+        case MA_VARIANT_SLICED: return fast && slice_fits(p) ? MA_VARIANT_SLICED : MA_ERR_UNSUPPORTED;
         default:
             if (fast32) return auto_fp32(p, heads, M);
             if (!fast) return MA_VARIANT_GENERIC;
@@ -517,6 +520,10 @@ int select_variant(const ma_fwd_params* p) {
     }
 }
 
+// Does a call that resolves to variant v run the slice-resident kernel?  AUTO names the kernel that it replaces (its results are the
+// same to the bit), so that what AUTO resolves to does not say which of the two runs; ma_fwd_kernel_name does.
+bool runs_slices(const ma_fwd_params* p, int v) { return v == MA_VARIANT_SLICED || (p->variant == MA_VARIANT_AUTO && slice_pays(p, v)); }
+
 // 16 bytes per lane and store, one workgroup per compute unit or so: the 2 MiB area is gone in two passes
 __global__ void zero_sync_kernel(uint4* sync, int chunks) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < chunks; i += gridDim.x * blockDim.x) sync[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -525,7 +532,7 @@ __global__ void zero_sync_kernel(uint4* sync, int chunks) {
 struct Prepared {
     Problem P;
     int variant;
-    bool slice = false;   // AUTO: the slice-resident kernel in place of the variant's own
+    bool slice = false;   // the slice-resident kernel: by name, or under AUTO in place of the variant's own
 };
 
 int run_fused(const Prepared& pr, const ma_fwd_params* p, hipStream_t s) {
@@ -601,7 +608,7 @@ void set_policies(const ma_fwd_params* p, Prepared* pr) {
 
 // The variant that runs a forward call whose states are kept: the ones that hold every step's state in memory.
 int select_keep_variant(const ma_fwd_params* p) {
-    if (p->variant == MA_VARIANT_FUSED || p->variant == MA_VARIANT_RESIDENT) return MA_ERR_UNSUPPORTED;
+    if (p->variant == MA_VARIANT_FUSED || p->variant == MA_VARIANT_RESIDENT || p->variant == MA_VARIANT_SLICED) return MA_ERR_UNSUPPORTED;
     if (p->variant != MA_VARIANT_AUTO) return select_variant(p);
     if (mfma32_supported(p)) return MA_VARIANT_STAGED;
     if (!mfma_supported(p)) return MA_VARIANT_GENERIC;
@@ -619,7 +626,7 @@ int prepare(const ma_fwd_params* p, Prepared* out) {
     if (v < 0) return v;
     out->P = make_problem(p, L);
     out->variant = v;
-    out->slice = p->variant == MA_VARIANT_AUTO && slice_pays(p, v);
+    out->slice = runs_slices(p, v);
     set_policies(p, out);
     out->P.one_tile_ok = 1;   // a problem that resolves to the resident kernel may use any of its forms
     return MA_OK;
@@ -964,7 +971,7 @@ const char* ma_fwd_kernel_name(const ma_fwd_params* p) {
     if (check_shape(p) != MA_OK) return nullptr;
     const bool f32 = p->dtype_qk == MA_F32;
     const int v = select_variant(p);
-    if (p->variant == MA_VARIANT_AUTO && slice_pays(p, v)) return "resident_slice_mfma";
+    if (v >= 0 && runs_slices(p, v)) return "resident_slice_mfma";
     switch (v) {
         case MA_VARIANT_GENERIC: return "r_step_kernel";
         case MA_VARIANT_STAGED: return f32 ? "r_step_f32" : p->B > 128 ? "r_step_long" : p->B > 64 ? "r_step_pair" : "r_step_mfma";   // (see runs_long)
@@ -1099,7 +1106,7 @@ int ma_matrix(const ma_fwd_params* p, float* A, void* stream) {
     if (pp.E > 1 && pp.out_stride[0] == 0) pp.out_stride[0] = 1;   // q may be broadcast; the stand-in
     if (pp.H > 1 && pp.out_stride[1] == 0) pp.out_stride[1] = 1;   // output must pass the overlap check
     if (pp.variant != MA_VARIANT_AUTO && pp.variant != MA_VARIANT_GENERIC && pp.variant != MA_VARIANT_STAGED)
-        return pp.variant < MA_VARIANT_AUTO || pp.variant > MA_VARIANT_CHAINED ? MA_ERR_VARIANT : MA_ERR_UNSUPPORTED;
+        return pp.variant < MA_VARIANT_AUTO || pp.variant > MA_VARIANT_SLICED ? MA_ERR_VARIANT : MA_ERR_UNSUPPORTED;
     if (pp.variant == MA_VARIANT_AUTO) {
         const int st = check_shape(&pp);
         if (st != MA_OK) return st;

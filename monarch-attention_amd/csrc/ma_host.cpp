@@ -406,7 +406,7 @@ struct MonarchAttentionHipBackward : public torch::autograd::Node {
 Tensor run_recorded(const Call& c, bool keep) {
     auto node = std::shared_ptr<MonarchAttentionHipBackward>(new MonarchAttentionHipBackward(), torch::autograd::deleteNode);
     node->set_next_edges(torch::autograd::collect_next_edges(c.q, c.k, c.v));
-    const bool keeps = keep && c.variant != MA_VARIANT_FUSED && c.variant != MA_VARIANT_RESIDENT;
+    const bool keeps = keep && c.variant != MA_VARIANT_FUSED && c.variant != MA_VARIANT_RESIDENT && c.variant != MA_VARIANT_SLICED;
     Tensor out, state;
     {
         const c10::AutoGradMode no_grad(false);

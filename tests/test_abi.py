@@ -215,6 +215,49 @@ def test_kernel_name_follows_the_resolved_variant():
     assert name(1, 16, 0, 64, 64) is None                         # invalid problem
 
 
+def test_sliced_by_name():
+    """The slice-resident kernel by name: wherever AUTO runs it, and beyond; refused outside of its sizes, by the paths that keep
+    the state of the steps or run them as stages, and with operands of 32 bits."""
+    lib = L.load()
+
+    def params(heads, N, D, B, T=2, variant="sliced", dt=L.MA_F16):
+        p = good_params()
+        p.E, p.H, p.N, p.D, p.Dv, p.B, p.T, p.variant = heads, 1, N, D, D, B, T, L.VARIANTS[variant]
+        p.dtype_qk = p.dtype_v = dt
+        for field in ("q_stride", "k_stride", "v_stride", "out_stride"):
+            setattr(p, field, (C.c_int64 * 3)(N * D, N * D, D))
+        return p
+
+    ran = 0
+    for heads in (8, 64, 128, 192, 256, 512):
+        for N, B in ((197, 14), (400, 20), (512, 32), (1024, 32), (1500, 40), (2304, 48), (3000, 60)):
+            for D in (32, 48, 64, 72, 80):
+                for T in (1, 2, 3):
+                    if lib.ma_fwd_kernel_name(params(heads, N, D, B, T, "auto")) != b"resident_slice_mfma":
+                        continue
+                    ran += 1
+                    p = params(heads, N, D, B, T)
+                    assert lib.ma_fwd_select_variant(p) == L.VARIANTS["sliced"], (heads, N, D, B, T)
+                    assert lib.ma_fwd_kernel_name(p) == b"resident_slice_mfma"
+                    assert lib.ma_fwd_workspace_bytes(p) == lib.ma_fwd_workspace_bytes(params(heads, N, D, B, T, "chained"))
+    assert ran > 100
+    assert lib.ma_fwd_select_variant(params(1, 512, 64, 32)) == L.VARIANTS["sliced"]      # one head: AUTO would not
+    for refused in (params(64, 1024, 96, 32), params(64, 1024, 64, 65), params(64, 2080, 64, 32), params(64, 1000, 60, 32),
+                    params(64, 4096, 80, 64), params(64, 512, 64, 32, dt=L.MA_F32)):
+        assert lib.ma_fwd_select_variant(refused) == L.MA_ERR_UNSUPPORTED
+        assert lib.ma_fwd_kernel_name(refused) is None
+    p = params(1, 512, 64, 32)
+    p.q = p.k = p.v = p.out = p.workspace = 0x100000
+    p.workspace_bytes = 1 << 40
+    assert lib.ma_matrix(p, 0x20000, None) == L.MA_ERR_UNSUPPORTED
+    assert lib.ma_fwd_keep(p, 0x100000, 1 << 40, None) == L.MA_ERR_UNSUPPORTED
+    assert lib.ma_r_step(p, 1, 0, None) == L.MA_ERR_UNSUPPORTED
+    b = L.BwdParams()
+    b.fwd = p
+    b.dq_stride = b.dk_stride = b.dv_stride = b.dout_stride = (C.c_int64 * 3)(512 * 64, 512 * 64, 64)
+    assert lib.ma_bwd_workspace_bytes(b) == 0
+
+
 def test_check_maps_status_to_python_exceptions():
     with pytest.raises(ValueError):
         L.check(L.MA_ERR_SHAPE, "x")

@@ -355,6 +355,38 @@ def test_slice_resident_kernel(E, H, N, D, B, T, pre, dt, masked):
     assert_parity(out[few, :2].cpu(), ref, dt, f"slices {(E, H, N, D, B, T)}")
 
 
+# E, H, N, D, B, T, pre, dt, masked: every class of strips of blocks and of block counts; one head, heads that 8 divides and
+# that it does not; up to 8 blocks (the chained kernel packs their L / Z problems); rows that are no whole 128-byte lines
+SLICED = [
+    (1, 1, 7, 64, 7, 2, False, "f16", False), (2, 4, 100, 40, 13, 2, True, "bf16", True), (3, 3, 225, 72, 15, 3, False, "f16", True),
+    (2, 8, 256, 80, 32, 2, False, "f16", True), (1, 5, 130, 48, 28, 3, True, "f16", False), (2, 4, 512, 72, 32, 3, False, "bf16", True),
+    (1, 16, 600, 80, 20, 1, True, "f16", True), (2, 4, 1000, 40, 32, 2, False, "f16", True), (1, 8, 500, 72, 40, 2, True, "f16", False),
+    (3, 2, 1000, 32, 40, 2, False, "bf16", True), (1, 8, 1500, 40, 33, 1, False, "f16", True), (2, 4, 700, 48, 16, 2, True, "f16", True),
+    (1, 3, 1900, 32, 30, 2, False, "f16", True), (1, 8, 1024, 64, 48, 2, False, "bf16", True), (1, 2, 2500, 32, 60, 2, True, "f16", True),
+]
+
+
+def in_layout(t, layout):
+    """The same values as a contiguous tensor, or as an (E, H, N, D) view of an (E, N, H, D) one."""
+    return t.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3) if layout == "tokens" else t.contiguous()
+
+
+@pytest.mark.parametrize("layout", ["heads", "tokens"])
+@pytest.mark.parametrize("E,H,N,D,B,T,pre,dt,masked", SLICED)
+def test_sliced_by_name(E, H, N, D, B, T, pre, dt, masked, layout):
+    """The slice-resident kernel by name, in both layouts of its operands and its output: bit-equal to the chained kernel on
+    contiguous heads, and within the gate of the oracle."""
+    q, k, v = seeded_qkv(E, H, N, D, DT[dt], seed=N + B)
+    mask = block_safe_mask(E, N, B, seed=B) if masked else None
+    dq, dk, dv, dm = to_dev(q, k, v, mask)
+    chained = monarch_attention_hip(dq, dk, dv, dm, T, B, pre, variant="chained")
+    out = monarch_attention_hip(*(in_layout(t, layout) for t in (dq, dk, dv)), dm, T, B, pre, variant="sliced")
+    assert out.stride() == in_layout(dv, layout).stride()
+    assert torch.equal(out, chained)
+    ref = monarch_attention_oracle(q, k, v, mask, T, B, pre, upcast=True)
+    assert_parity(out.cpu(), ref, dt, f"sliced {(E, H, N, D, B, T, pre, dt, masked, layout)}")
+
+
 @pytest.mark.parametrize("variant", ["chained", "fused"])
 @pytest.mark.parametrize("B,M,D,T,dt", [(65, 96, 64, 2, "f16"), (80, 65, 72, 1, "bf16"), (81, 80, 128, 2, "f16"), (97, 112, 32, 2, "bf16"),
                                         (112, 128, 64, 1, "f16"), (113, 72, 96, 2, "f16"), (40, 104, 64, 3, "f16")])
