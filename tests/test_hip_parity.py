@@ -387,6 +387,26 @@ def test_sliced_by_name(E, H, N, D, B, T, pre, dt, masked, layout):
     assert_parity(out.cpu(), ref, dt, f"sliced {(E, H, N, D, B, T, pre, dt, masked, layout)}")
 
 
+@pytest.mark.parametrize("layouts", [("tokens", "tokens", "tokens"), ("heads", "tokens", "heads"), ("tokens", "heads", "tokens")])
+@pytest.mark.parametrize("E,H,N,D,B,T,pre,dt", [
+    (2, 4, 100, 40, 16, 2, False, "f16"), (1, 8, 500, 72, 32, 2, True, "bf16"), (1, 16, 700, 80, 24, 3, False, "f16"),
+    (2, 8, 300, 72, 64, 1, False, "f16"), (3, 8, 2000, 96, 70, 2, True, "bf16"), (1, 8, 3000, 48, 48, 1, False, "f16"),
+    (1, 12, 500, 72, 32, 2, False, "f16"), (2, 4, 500, 64, 32, 2, False, "f16"),
+])
+def test_chained_kernel_takes_heads_in_either_order(E, H, N, D, B, T, pre, dt, layouts):
+    """Heads that follow each other run on one XCD where a token's heads lie side by side in rows that are no whole lines and 8
+    divides the heads (all but the last two shapes with k in (E, N, H, D)), else heads 8 apart: the result does not depend on it."""
+    q, k, v = seeded_qkv(E, H, N, D, DT[dt], seed=N + B)
+    mask = block_safe_mask(E, N, B, seed=B)
+    dq, dk, dv, dm = to_dev(q, k, v, mask)
+    plain = monarch_attention_hip(dq, dk, dv, dm, T, B, pre, variant="chained")
+    out = monarch_attention_hip(*(in_layout(t, lay) for t, lay in zip((dq, dk, dv), layouts)), dm, T, B, pre, variant="chained")
+    assert torch.equal(out, plain)
+    ref = monarch_attention_oracle(q, k, v, mask, T, B, pre, upcast=True)
+    assert_parity(out.cpu(), ref, dt, f"chained {(E, H, N, D, B, T, pre, dt, layouts)}")
+    assert sync_status() == 0
+
+
 @pytest.mark.parametrize("variant", ["chained", "fused"])
 @pytest.mark.parametrize("B,M,D,T,dt", [(65, 96, 64, 2, "f16"), (80, 65, 72, 1, "bf16"), (81, 80, 128, 2, "f16"), (97, 112, 32, 2, "bf16"),
                                         (112, 128, 64, 1, "f16"), (113, 72, 96, 2, "f16"), (40, 104, 64, 3, "f16")])
