@@ -179,7 +179,7 @@ __global__ __launch_bounds__(64 * W) void r_step_pair(Problem P, int first) {
         ent = mfma::quad_rows_sum(ent);
         const float den = sum + P.eps, inv = mfma::rcp(den);
         if (q == 0)   // cL = sum_i r log r with r = p / den (ma_torch.py:20)
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, kLn2 * (ent * inv - mfma::log2_normal(den) * (sum * inv))),
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, mfma::row_entropy(ent, sum, den, inv)),
                                                   state_slice(P.cL, eh, np, 4), j < B ? static_cast<unsigned>(j * M + k) * 4u : kOob, 0, 0);
 #pragma unroll
         for (int w = 0; w < NWT; ++w) Pk[s][w] = Pack<T>::four_of(C[s][w], inv);

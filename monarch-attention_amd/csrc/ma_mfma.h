@@ -131,12 +131,17 @@ __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x);
 __device__ __forceinline__ float log2_normal(float x) { return __builtin_amdgcn_logf(x); }
 
 // x as an fp32 value of its own: keeps the compiler from rounding a product once, to 16 bits, where the kernels round it to
-// fp32 and then to 16 bits (it does so for a few values of some kernels).  R problems of more than 32 rows and others
-// of more than 64 run in kernels that differ by launch (chained, per stage, slices of a head), and a head's result must not depend
-// on which.
+// fp32 and then to 16 bits (it does so for a few values of some kernels).  A block problem of any size runs in kernels that differ
+// by launch (chained, per stage, whole heads, slices of a head), and a head's result must not depend on which: they all keep the
+// probabilities in fp32 first, and where a product enters a sum it is spelled out which of the two is rounded.
 __device__ __forceinline__ float fp32_value(float x) {
     asm("" : "+v"(x));
     return x;
+}
+
+// cL = sum_i r log r with r = p / den (ma_torch.py:20), from sum p log2 p and sum p; rows of tiny r add ~1e-36
+__device__ __forceinline__ float row_entropy(float ent, float sum, float den, float inv) {
+    return fp32_value(kLn2 * fmaf(ent, inv, -(log2_normal(den) * (sum * inv))));
 }
 
 // ---- global memory through buffer resources ---------------------------------
@@ -666,11 +671,10 @@ struct RProb {
 #pragma unroll
             for (int wt = 0; wt < NWT; ++wt)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) C[wt][v] = NWT > 2 ? fp32_value(C[wt][v] * inv) : C[wt][v] * inv;
-            // cL = sum_i r log r with r = p / den (ma_torch.py:20); rows of tiny r add ~1e-36
+                for (int v = 0; v < 4; ++v) C[wt][v] = fp32_value(C[wt][v] * inv);
             lrow = static_cast<unsigned>(j * M + m);   // row of aL / cL / Y: (j, m)
             if (q == 0)
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, kLn2 * (ent * inv - log2_normal(den) * (sum * inv))),
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, row_entropy(ent, sum, den, inv)),
                                                       S.cL, jv ? lrow * 4u : kOob, 0, 0);
 
             pack_p<T, NWT>(pb, C);
@@ -822,7 +826,7 @@ struct ZProb {
 #pragma unroll
             for (int wt = 0; wt < NWT; ++wt)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) C[wt][v] = NWT > 4 ? fp32_value(C[wt][v] * inv) : C[wt][v] * inv;
+                for (int v = 0; v < 4; ++v) C[wt][v] = fp32_value(C[wt][v] * inv);
             pack_p<T, NWT>(pb, C);
           }
           if (active) {
@@ -1003,9 +1007,9 @@ struct LProb {
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
                         const float u = ti.same(16 * lt + 4 * q + v, k) ? fmaf(round_to<T>(acc[v]), kLog2e, cbk) : kNegBig;
-                        const float ex = __builtin_amdgcn_exp2f(u - mx4[v]), lv = ex * inv4[v];
-                        crs = NWT > 4 ? fmaf(ex, inv4[v], crs) : crs + lv;   // (spelled out: see fp32_value)
-                        acc[v] = NWT > 4 ? fp32_value(lv) : lv;
+                        const float ex = __builtin_amdgcn_exp2f(u - mx4[v]);
+                        crs = fmaf(ex, inv4[v], crs);
+                        acc[v] = fp32_value(ex * inv4[v]);
                     }
                     C[lt] = acc;
                 }

@@ -362,10 +362,9 @@ struct HeadRes {
 #pragma unroll
             for (int wt = 0; wt < NTB; ++wt)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) C[wt][v] *= inv;
-            // cL = sum_i r log r with r = p / den (ma_torch.py:20), kept as the softmax bias -log2(e) * cL of the
-            // L and Z problems of position j; the four lanes of a row all hold it
-            *(ok ? c.fat(c.L.cb) + j * ROWSM + m : c.fat(c.L.trash)) = -kLog2e * (kLn2 * (ent * inv - log2_normal(den) * (sum * inv)));   // (the same roundings as where cL itself is kept)
+                for (int v = 0; v < 4; ++v) C[wt][v] = fp32_value(C[wt][v] * inv);
+            // cL, kept as the softmax bias -log2(e) * cL of the L and Z problems of position j; the four lanes of a row all hold it
+            *(ok ? c.fat(c.L.cb) + j * ROWSM + m : c.fat(c.L.trash)) = -kLog2e * row_entropy(ent, sum, den, inv);
             pack_p<T, NTB>(pb, C);
             f32x4 O[DT];
             gemm2_rows<NTB, true>(O, c, Kt, RB, ROWSB, pb);
@@ -469,9 +468,9 @@ struct HeadRes {
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const float u = fmaf(round_to<T>(acc[v]), kLog2e, cbk);
-                    const float lv = __builtin_amdgcn_exp2f(u - mx4[v]) * inv4[v];
-                    crs += lv;
-                    acc[v] = lv;
+                    const float ex = __builtin_amdgcn_exp2f(u - mx4[v]);
+                    crs = fmaf(ex, inv4[v], crs);
+                    acc[v] = fp32_value(ex * inv4[v]);
                 }
                 C[lt] = acc;
             }
@@ -553,7 +552,7 @@ struct HeadRes {
 #pragma unroll
         for (int wt = 0; wt < NTM; ++wt)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) C[wt][v] *= inv;
+            for (int v = 0; v < 4; ++v) C[wt][v] = fp32_value(C[wt][v] * inv);
         V8 pb[(NTM + 1) / 2];
         pack_p<T, NTM>(pb, C);
         f32x4 O[DT];

@@ -203,8 +203,7 @@ struct Slice {
         for (int w = 0; w < NTB; ++w)
 #pragma unroll
             for (int v = 0; v < 4; ++v) C[w][v] = fp32_value(C[w][v] * inv);
-        // cL = sum_i r log r with r = p / den (:20)
-        if (c.q == 0) c.template at<float>(c.L.cb)[c.r * ROWSM + m] = -kLog2e * fp32_value(kLn2 * (ent * inv - log2_normal(den) * (sum * inv)));
+        if (c.q == 0) c.template at<float>(c.L.cb)[c.r * ROWSM + m] = -kLog2e * row_entropy(ent, sum, den, inv);
         pack_p<T, NTB>(pb, C);
         f32x4 O[DT];
         gemm2<NTB>(c, O, pb);

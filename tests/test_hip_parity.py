@@ -407,6 +407,40 @@ def test_chained_kernel_takes_heads_in_either_order(E, H, N, D, B, T, pre, dt, l
     assert sync_status() == 0
 
 
+HEADS = [  # E, H, N, D, B, T, pre, dt, masked: strips of blocks and of block counts in the head-resident kernels, wide heads among them
+    (8, 9, 49, 48, 41, 1, False, "f16", True), (8, 9, 135, 40, 63, 2, True, "f16", False), (8, 9, 135, 64, 63, 2, False, "f16", True),
+    (8, 9, 197, 64, 14, 2, True, "f16", False), (8, 9, 100, 32, 50, 3, False, "f16", True), (8, 9, 110, 48, 35, 2, False, "f16", False),
+    (8, 9, 250, 64, 32, 3, False, "f16", True), (8, 9, 200, 72, 12, 3, True, "f16", True), (8, 9, 90, 128, 10, 2, False, "f16", False),
+    (8, 9, 197, 64, 14, 3, True, "bf16", True), (8, 9, 512, 64, 32, 2, False, "bf16", True), (8, 9, 512, 64, 32, 2, True, "f16", False),
+    (8, 9, 384, 64, 48, 2, False, "f16", True), (8, 9, 400, 64, 64, 3, False, "bf16", False), (8, 9, 120, 80, 60, 2, True, "bf16", True),
+]
+
+
+@pytest.mark.parametrize("E,H,N,D,B,T,pre,dt,masked", HEADS)
+def test_head_resident_results_are_the_chained_kernels(E, H, N, D, B, T, pre, dt, masked):
+    """AUTO runs a head in one kernel or the other by the number of heads: the two round at the same places, to the bit."""
+    q, k, v = seeded_qkv(E, H, N, D, DT[dt], seed=N + B)
+    dev = to_dev(q, k, v, block_safe_mask(E, N, B, seed=B) if masked else None)
+    assert resident_kernel_name(dev, T, B, pre) in ("resident_head_mfma", "resident_head2_mfma")
+    assert torch.equal(monarch_attention_hip(*dev, T, B, pre, variant="resident"), monarch_attention_hip(*dev, T, B, pre, variant="chained"))
+
+
+@pytest.mark.parametrize("N,D,B,T,pre,dt", [(512, 64, 32, 2, False, "bf16"), (197, 64, 14, 2, True, "f16"), (225, 72, 15, 3, False, "f16"),
+                                            (1024, 72, 32, 3, False, "f16"), (384, 64, 48, 2, False, "f16")])
+def test_a_heads_result_does_not_depend_on_the_batch(N, D, B, T, pre, dt):
+    """The first head, alone and in batches that AUTO runs in different kernels."""
+    q, k, v = seeded_qkv(8, 1, N, D, DT[dt], seed=N + D)
+    dev = [t.repeat(64, *[1] * (t.dim() - 1)) for t in to_dev(q, k, v, block_safe_mask(8, N, B, seed=B))]
+    names, first = set(), None
+    for E in (1, 64, 112, 128, 192, 256, 512):
+        part = [t[:E] for t in dev]
+        names.add(L.load().ma_fwd_kernel_name(make_params(*part, torch.empty_like(part[2]), T, B, pre, "auto")))
+        out = monarch_attention_hip(*part, T, B, pre)
+        first = out if first is None else first
+        assert torch.equal(out[:1], first), E
+    assert len(names) > 1
+
+
 @pytest.mark.parametrize("variant", ["chained", "fused"])
 @pytest.mark.parametrize("B,M,D,T,dt", [(65, 96, 64, 2, "f16"), (80, 65, 72, 1, "bf16"), (81, 80, 128, 2, "f16"), (97, 112, 32, 2, "bf16"),
                                         (112, 128, 64, 1, "f16"), (113, 72, 96, 2, "f16"), (40, 104, 64, 3, "f16")])
