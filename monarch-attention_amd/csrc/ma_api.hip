@@ -171,13 +171,13 @@ bool mfma32_supported(const ma_fwd_params* p) {
     return true;
 }
 
-int run_slice(const Problem& P, int dtype_qk, bool dry_run, hipStream_t s) {
+int run_slice(const Problem& P, int dtype_qk, SlicePlan* plan, hipStream_t s) {
     const bool h = dtype_qk == MA_F16;
     const int D = P.D;
-    if (D <= 32) return h ? launch_slice_f16_d2(P, dry_run, s) : launch_slice_bf16_d2(P, dry_run, s);
-    if (D <= 48) return h ? launch_slice_f16_d3(P, dry_run, s) : launch_slice_bf16_d3(P, dry_run, s);
-    if (D <= 64) return h ? launch_slice_f16_d4(P, dry_run, s) : launch_slice_bf16_d4(P, dry_run, s);
-    if (D <= 80) return h ? launch_slice_f16_d5(P, dry_run, s) : launch_slice_bf16_d5(P, dry_run, s);
+    if (D <= 32) return h ? launch_slice_f16_d2(P, plan, s) : launch_slice_bf16_d2(P, plan, s);
+    if (D <= 48) return h ? launch_slice_f16_d3(P, plan, s) : launch_slice_bf16_d3(P, plan, s);
+    if (D <= 64) return h ? launch_slice_f16_d4(P, plan, s) : launch_slice_bf16_d4(P, plan, s);
+    if (D <= 80) return h ? launch_slice_f16_d5(P, plan, s) : launch_slice_bf16_d5(P, plan, s);
     return MA_ERR_UNSUPPORTED;
 }
 
@@ -217,55 +217,86 @@ bool resident_head_fits(const ma_fwd_params* p, int forms = 1) {
     return p->dtype_qk != MA_F32 && run_resident(P, p->dtype_qk, true, nullptr) == MA_OK;
 }
 
-// AUTO, 16-bit: is the slice-resident kernel (ma_resident_slice.h: a workgroup per 16 positions of a head) ahead of the kernel that
-// variant v would run?  A slice has a compute unit, or half of one, to itself, so the rules are about how well heads x slices fill
-// whole passes over the 256 compute units they were measured on, and how many of a slice's 16 positions exist.  Heads that fit in
-// LDS whole stay with the head-resident kernels where those are chosen, but for blocks of 14 and 15 rows and for a single pass of
-// slices: beyond, which of the two is ahead turns on how the last pass ends (0.6 - 1.4).  In the comments: multiples of the time of the kernel
-// it replaces, at D = 32 .. 80, 64 .. 4096 tokens, 8 .. 768 heads, T = 1, 2, 3 (profiles/slice_resident_sweep.md).
-bool slice_is_ahead(const ma_fwd_params* p, int v) {
-    if (p->dtype_qk == MA_F32 || (v != MA_VARIANT_CHAINED && v != MA_VARIANT_RESIDENT)) return false;
-    const int B = p->B, M = (p->N + p->B - 1) / p->B, D = p->D;
-    if (B > 64 || M > 64) return false;
-    const long long heads = static_cast<long long>(p->E) * p->H, slices = heads * ((B + 15) / 16);
-    const bool multi = p->T >= 2, wide = D > 64;
-    if (B <= 16) {   // one slice a head: beside the head-resident kernels, which lose to padding where blocks are a little short of 16 rows
-        if (B == 16 || B < 14 || M < 12) return false;
-        if (M > 32) return multi && heads >= 192;                                             // 0.6 - 0.85
-        if (M > 16) return heads >= 112 && heads <= 288 && (multi || D <= 32);              // 0.83 - 1.0
-        if (!multi) return heads >= 96 && heads <= (wide ? 400 : 256);                       // 0.78 - 0.91
-        return wide ? heads >= (p->T == 2 ? 64 : 8) && heads <= 400                            // 0.80 - 0.94
-                    : heads <= 256 && (p->T == 2 || B == 15);                                  // 0.85 - 0.99 (others 0.96 - 1.02)
-    }
-    if (v == MA_VARIANT_RESIDENT && heads > 128 && resident_head_fits(p, 2)) return false;
-    const bool most = slices >= 192 && multi && B <= 32 && M > 16 && M <= 32 && (wide ? B >= 30 && M >= 28 : B >= 24);   // 0.79 - 0.98
-    if (slices < 224 && !most) return false;              // less than most of one pass
-    if (B <= 32) {
-        if (M <= 16) return heads <= 128 || (B >= 30 && (multi || heads >= 224));             // 0.65 - 0.94; 0.6 - 0.95
-        if (M <= 32) {
-            if (heads <= 128) return multi || B >= 24;                                        // 0.64 - 0.99
-            if (heads < 224) return multi && B >= 28 && M >= 28;                              // 0.76 - 0.98 (shorter: 0.87 - 1.03)
-            return multi || B >= (wide ? 28 : 24);                                            // 0.5 - 0.9; 0.7 - 0.97
-        }
-        if (B < 20 || (heads > 128 && heads < 224)) return false;                             // (0.89 - 1.14)
-        return multi || (B >= 28 && M <= 48);                                                 // 0.6 - 0.97; 0.8 - 1.0
-    }
-    if (B <= 48) {
-        if (D <= 32) return heads <= 85 || heads >= 224 || (multi && heads >= 112);           // 0.55 - 0.99
-        if (D <= 48) return multi && heads >= 224 && M > 20;                                  // 0.74 - 0.94
-        if (D <= 64) return multi && M > 16 && (heads >= 224 || (heads <= 85 && B >= 44));    // 0.75 - 0.97; 0.84 - 0.98
-        return multi && heads >= 512 && M > 16;                                               // 0.76 - 0.97
-    }
-    return D <= 32 && multi && B >= 56 && (heads <= 64 || (heads >= 112 && M >= 30));         // 0.63 - 0.94
-}
-// Does the slice-resident kernel take the problem: a class of its strips and columns, the state in LDS?  (16-bit operands)
-bool slice_fits(const ma_fwd_params* p) {
+// Does the slice-resident kernel (ma_resident_slice.h: a workgroup per 16 positions of a head) take the problem: a class of its
+// strips and columns, the state in LDS?  (16-bit operands)
+bool slice_fits(const ma_fwd_params* p, SlicePlan* plan) {
     Problem P = sizes_of(p);
     P.one_tile_ok = 1;
-    return run_slice(P, p->dtype_qk, true, nullptr) == MA_OK;
+    return run_slice(P, p->dtype_qk, plan, nullptr) == MA_OK;
 }
-// (the rule first: it costs a few comparisons of the host's time, 6 us calls lost 1 % otherwise)
-bool slice_pays(const ma_fwd_params* p, int v) { return slice_is_ahead(p, v) && slice_fits(p); }
+
+// AUTO, 16-bit: is the slice-resident kernel ahead of the one that variant v would run?  A slice has a compute unit, or half of one, to
+// itself and walks its problems in rounds, so its time is passes over the compute units x rounds; the chained kernel's tasks find
+// any free place, so its time is the tasks over the places beside the latency of 2 T dependent phases.  Both times are estimated in
+// us from the shape: fitted on one MI355X (256 units) to 70634 random problems (D = 32 .. 80, 1 .. 4096 tokens, 1 .. 4096 heads, T = 1 .. 6,
+// both layouts of the operands; the estimates are within 10 and 13 % of what was measured for nine in ten), the whole
+// story in profiles/slice_resident_sweep.md.
+float slice_us(const ma_fwd_params* p, const SlicePlan& plan, int M) {
+    struct Mode {
+        float call, mb, pass, round, strip, block, tile, sums;
+    };
+    static constexpr Mode kModes[4] = {                              // workgroups of
+        {1.18f, 0.51f, 3.71f, 0.066f, 0.107f, 0.091f, 0.108f, 0.019f},   // 16 waves
+        {3.59f, 0.78f, 0.88f, 0.078f, 0.067f, 0.108f, 0.067f, 0.017f},   // 12
+        {2.52f, 0.53f, 4.97f, 0.066f, 0.049f, 0.142f, 0.030f, 0.017f},   // 8, a compute unit each
+        {4.22f, 0.63f, 1.47f, 0.082f, 0.067f, 0.141f, 0.129f, 0.037f},   // 8, two on a compute unit
+    };
+    const Mode& m = kModes[plan.per_unit == 2 ? 3 : plan.waves == 16 ? 0 : plan.waves == 12 ? 1 : 2];
+    const int B = p->B, D = p->D, W = plan.waves, strips = (B + 15) / 16, tiles = (M + 15) / 16, rows = strips > tiles ? strips : tiles;
+    const long long heads = static_cast<long long>(p->E) * p->H;
+    const int xcd_units = plan.units / 8 > 0 ? plan.units / 8 : 1;
+    const long long deep = ((heads + 7) / 8 * strips + xcd_units - 1) / xcd_units;   // slices that a compute unit of the fullest XCD runs
+    const float passes = plan.per_unit == 2 ? static_cast<float>(deep / 2) + 0.65f * static_cast<float>(deep % 2) : static_cast<float>(deep);   // (a slice alone on its unit is done sooner)
+    const float cols = D % 32 == 0 ? D / 16.f : static_cast<float>((D + 15) / 16 + 1);   // (a half step of 32 columns costs a whole one)
+    const float T = static_cast<float>(p->T), r = static_cast<float>((M + W - 1) / W), l = static_cast<float>(((B < 16 ? B : 16) + W - 1) / W);
+    const float pass = m.pass + T * (r * cols * (m.round * rows + m.strip * strips) + m.block * M) +
+                       (T - 0.5f) * (l * cols * m.tile * rows + m.sums * static_cast<float>(B) / strips * tiles * tiles * static_cast<float>((D + 31) / 32));
+    const float last = strips > 2 ? 1.f + 0.08f / T : 1.f;   // (the last R phase, which takes V through the tile as well, costs long tiles more than the others)
+    return last * (m.call + m.mb * 2e-6f * heads * p->N * D + passes * pass);
+}
+float chain_us(const ma_fwd_params* p, int M, int units) {
+    const int B = p->B, D = p->D, strips = (B + 15) / 16, tiles = (M + 15) / 16;
+    const int cols = D <= 32 ? 2 : D <= 64 ? 4 : 5, pitch = D <= 32 ? 80 : D <= 64 ? 144 : 176;   // its classes of columns, bytes of a row in LDS
+    auto per_task = [](int s) { return s == 1 ? 4 : s == 2 ? 2 : 1; };
+    const int lds_r = per_task(strips) * strips * (32 * pitch + 64), lds_l = per_task(tiles) * tiles * (32 * pitch + 192);
+    const int fit = 160 * 1024 / (lds_r > lds_l ? lds_r : lds_l), places = fit < 5 ? fit : 5;   // workgroups on a compute unit
+    const int together = M > 8 ? 1 : M > 4 ? 2 : M > 2 ? 4 : M > 1 ? 8 : 16;   // positions that share an L / Z problem
+    const long long heads = static_cast<long long>(p->E) * p->H;
+    const float T = static_cast<float>(p->T), wide = static_cast<float>((heads + 7) / 8 * 8) / (static_cast<float>(units) * places);
+    const float r = T * wide * static_cast<float>((M + per_task(strips) - 1) / per_task(strips));
+    const float l = (T - 0.5f) * wide * static_cast<float>(((B + together - 1) / together + per_task(tiles) - 1) / per_task(tiles));
+    const float mb = 2e-6f * heads * D, moved = 0.68f * mb * (p->N + T * static_cast<float>(M * B));
+    const float work = moved + 2.14f * (r + l) + 0.42f * ((strips > 2 ? r : 0.f) + (tiles > 2 ? l : 0.f));
+    const float chain = 5.55f + (T - 0.5f) * (0.8f + 0.57f * static_cast<float>(strips + tiles) + 0.53f * cols);
+    return std::sqrt(chain * chain + work * work);
+}
+// Heads that the head-resident kernels run have no such estimate: their slices are ahead in a single pass over the compute units,
+// from a few blocks on (17 .. 32 rows: 0.66 - 0.9 of their time from four blocks on, 0.9 - 1.4 below) and for blocks a little
+// short of 16 rows, where the head kernels lose to padding (15 rows: 0.79 - 0.98; 14 rows, 12 - 16 blocks: 0.82 - 0.98, later
+// steps lose it).  Beyond a pass it turns on how the last one ends (0.6 - 1.6); rows of more than 64 columns, of which the head kernels
+// hold one head at a time, leave another half (0.77 - 1.0).
+int half_passes_ahead_of_heads(const ma_fwd_params* p, int M) {
+    const int B = p->B, D = p->D, T = p->T;
+    if (B < 14 || B == 16 || B > 32 || M < 3) return 0;
+    if (B > 16 && M == 3 && T > 1) return 0;
+    if (B < 16 && (M < 12 || (M > 16 && T == 1 && D > 32))) return 0;
+    if (B == 14 && D > 32 && (M > 16 || T > (D > 64 ? 3 : 2))) return 0;
+    return B == 15 && M <= 16 && D > 64 ? 3 : 2;
+}
+bool slice_pays(const ma_fwd_params* p, int v) {
+    if (p->dtype_qk == MA_F32 || (v != MA_VARIANT_CHAINED && v != MA_VARIANT_RESIDENT) || p->B > 64 || p->D > 80) return false;
+    const int M = (p->N + p->B - 1) / p->B;
+    SlicePlan plan;
+    if (M > 64) return false;
+    const int half_passes = v == MA_VARIANT_RESIDENT ? half_passes_ahead_of_heads(p, M) : 1;   // (first: a few comparisons, and most heads of this size end here)
+    if (half_passes == 0 || !slice_fits(p, &plan)) return false;
+    const long long heads = static_cast<long long>(p->E) * p->H, strips = (p->B + 15) / 16;
+    if (v == MA_VARIANT_RESIDENT) return 2 * ((heads + 7) / 8 * 8 * strips) <= static_cast<long long>(half_passes) * plan.units;
+    // (Most of a pass, or three quarters from 17 blocks on; 14 and 15 rows in up to 16 blocks any number of heads.  Below, slices are ahead
+    // too where blocks are few - 64 .. 111 heads of 17 .. 32 rows in up to 16 blocks, T >= 2: 0.66 - 0.93 -, but no call has been moved there yet.)
+    const bool one_tile = (p->B == 14 || p->B == 15) && M <= 16;
+    return (one_tile || 8 * heads * strips >= (M > 16 ? 6 : 7) * plan.units) && slice_us(p, plan, M) < chain_us(p, M, plan.units);
+}
 
 // The fused, chained and resident kernels are built for block problems of at most 128 rows.
 bool one_launch_tiles(const ma_fwd_params* p) {
@@ -510,7 +541,10 @@ int select_variant(const ma_fwd_params* p) {
         case MA_VARIANT_FUSED: return fast && one_launch_tiles(p) ? MA_VARIANT_FUSED : MA_ERR_UNSUPPORTED;
         case MA_VARIANT_CHAINED: return fast && chain_fits(p) ? MA_VARIANT_CHAINED : MA_ERR_UNSUPPORTED;
         case MA_VARIANT_RESIDENT: return (fast || fast32) && resident_fits(p, true) ? MA_VARIANT_RESIDENT : MA_ERR_UNSUPPORTED;
-        case MA_VARIANT_SLICED: return fast && slice_fits(p) ? MA_VARIANT_SLICED : MA_ERR_UNSUPPORTED;
+        case MA_VARIANT_SLICED: {
+            SlicePlan plan;
+            return fast && slice_fits(p, &plan) ? MA_VARIANT_SLICED : MA_ERR_UNSUPPORTED;
+        }
         default:
             if (fast32) return auto_fp32(p, heads, M);
             if (!fast) return MA_VARIANT_GENERIC;
@@ -1016,7 +1050,7 @@ int ma_fwd(const ma_fwd_params* p, void* stream) {
     int st = prepare(p, &pr);
     if (st != MA_OK) return st;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (pr.slice) return run_slice(pr.P, p->dtype_qk, false, s);
+    if (pr.slice) return run_slice(pr.P, p->dtype_qk, nullptr, s);
     if (pr.variant == MA_VARIANT_FUSED) return run_fused(pr, p, s);
     if (pr.variant == MA_VARIANT_CHAINED) return run_chain(pr, p, s);
     if (pr.variant == MA_VARIANT_RESIDENT) return run_resident(pr.P, p->dtype_qk, false, s);

@@ -242,16 +242,24 @@ int launch_fused_bf16_d4(const Problem& P, bool sync_ready, hipStream_t s);
 int launch_fused_bf16_d5(const Problem& P, bool sync_ready, hipStream_t s);
 int launch_fused_bf16_d8(const Problem& P, bool sync_ready, hipStream_t s);
 
+// Slice-resident forward (one launch, 16 positions of a head per workgroup).  plan: launch nothing, report whether the problem
+// fits (MA_OK / MA_ERR_UNSUPPORTED) and in which workgroups it would run.
+struct SlicePlan {
+    int waves;      // of a workgroup
+    int per_unit;   // workgroups that share a compute unit
+    int units;      // compute units of the device
+};
+int launch_slice_f16_d2(const Problem& P, SlicePlan* plan, hipStream_t s);
+int launch_slice_f16_d3(const Problem& P, SlicePlan* plan, hipStream_t s);
+int launch_slice_f16_d4(const Problem& P, SlicePlan* plan, hipStream_t s);
+int launch_slice_f16_d5(const Problem& P, SlicePlan* plan, hipStream_t s);
+int launch_slice_bf16_d2(const Problem& P, SlicePlan* plan, hipStream_t s);
+int launch_slice_bf16_d3(const Problem& P, SlicePlan* plan, hipStream_t s);
+int launch_slice_bf16_d4(const Problem& P, SlicePlan* plan, hipStream_t s);
+int launch_slice_bf16_d5(const Problem& P, SlicePlan* plan, hipStream_t s);
+
 // Resident forward (one launch, per-head state kept in LDS).  dry_run: only report
 // whether the problem fits (MA_OK / MA_ERR_UNSUPPORTED), launch nothing.
-int launch_slice_f16_d2(const Problem& P, bool dry_run, hipStream_t s);
-int launch_slice_f16_d3(const Problem& P, bool dry_run, hipStream_t s);
-int launch_slice_f16_d4(const Problem& P, bool dry_run, hipStream_t s);
-int launch_slice_f16_d5(const Problem& P, bool dry_run, hipStream_t s);
-int launch_slice_bf16_d2(const Problem& P, bool dry_run, hipStream_t s);
-int launch_slice_bf16_d3(const Problem& P, bool dry_run, hipStream_t s);
-int launch_slice_bf16_d4(const Problem& P, bool dry_run, hipStream_t s);
-int launch_slice_bf16_d5(const Problem& P, bool dry_run, hipStream_t s);
 int launch_resident_f16_d2(const Problem& P, bool dry_run, hipStream_t s);
 int launch_resident_f16_d4(const Problem& P, bool dry_run, hipStream_t s);
 int launch_resident_f16_d5(const Problem& P, bool dry_run, hipStream_t s);

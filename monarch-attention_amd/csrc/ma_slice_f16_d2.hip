@@ -2,5 +2,5 @@
 #include "ma_slice_launch.h"
 
 namespace ma {
-int launch_slice_f16_d2(const Problem& P, bool dry_run, hipStream_t s) { return mfma::launch_slice<f16, 2>(P, dry_run, s); }
+int launch_slice_f16_d2(const Problem& P, SlicePlan* plan, hipStream_t s) { return mfma::launch_slice<f16, 2>(P, plan, s); }
 }  // namespace ma

@@ -24,32 +24,33 @@ int launch_slice_w(const Problem& P, hipStream_t s) {
 // 2: 0.77 of the chained kernel's time in 12 waves, 0.85 in 8).  Eight where two slices share a compute unit and there are more
 // slices than compute units (192 heads of 512, T = 2: 24.7 us, 26.8 in 16).
 template <class T, int DT, int NTB, int NTM>
-int launch_slice_one(const Problem& P, bool dry_run, hipStream_t s) {
+int launch_slice_one(const Problem& P, SlicePlan* plan, hipStream_t s) {
+    constexpr bool kShort = NTB <= 2 && NTM <= 2;   // (their kernels of 8 waves keep to 128 registers)
+    constexpr int WIDE = kShort ? 16 : 12;
+    using Wide = Slice<T, DT, NTB, NTM, WIDE>;
     using Narrow = Slice<T, DT, NTB, NTM, 8>;
-    if (dry_run) return Narrow::takes(P.D, P.M, P.B, kSliceLds) ? MA_OK : MA_ERR_UNSUPPORTED;
-    if constexpr (NTB <= 2 && NTM <= 2) {
-        const long long slices = static_cast<long long>(P.E) * P.H * ((P.B + 15) / 16);
-        if (slices <= compute_units() || 2 * Narrow::layout(P.D, P.M).total > kSliceLds) {
-            const int err = launch_slice_w<T, DT, NTB, NTM, 16>(P, s);
-            if (err != MA_ERR_UNSUPPORTED) return err;
-        }
-    } else {
-        const int err = launch_slice_w<T, DT, NTB, NTM, 12>(P, s);
-        if (err != MA_ERR_UNSUPPORTED) return err;
+    if (!Narrow::takes(P.D, P.M, P.B, kSliceLds)) return MA_ERR_UNSUPPORTED;
+    const long long slices = static_cast<long long>(P.E) * P.H * ((P.B + 15) / 16);
+    const int units = compute_units();
+    const bool shared = kShort && slices > units && 2 * Narrow::layout(P.D, P.M).total <= kSliceLds;
+    const bool wide = !shared && Wide::takes(P.D, P.M, P.B, kSliceLds);
+    if (plan != nullptr) {
+        *plan = SlicePlan{wide ? WIDE : 8, shared ? 2 : 1, units};
+        return MA_OK;
     }
-    return launch_slice_w<T, DT, NTB, NTM, 8>(P, s);
+    return wide ? launch_slice_w<T, DT, NTB, NTM, WIDE>(P, s) : launch_slice_w<T, DT, NTB, NTM, 8>(P, s);
 }
 
 template <class T, int DT>
-int launch_slice(const Problem& P, bool dry_run, hipStream_t s) {
+int launch_slice(const Problem& P, SlicePlan* plan, hipStream_t s) {
     if (P.B > 64 || P.M > 64 || !P.one_tile_ok) return MA_ERR_UNSUPPORTED;
     auto blocks = [&](auto ntb) {
         constexpr int NTB = decltype(ntb)::value;
         switch ((P.M + 15) / 16) {
-            case 1: return launch_slice_one<T, DT, NTB, 1>(P, dry_run, s);
-            case 2: return launch_slice_one<T, DT, NTB, 2>(P, dry_run, s);
-            case 3: return launch_slice_one<T, DT, NTB, 3>(P, dry_run, s);
-            default: return launch_slice_one<T, DT, NTB, 4>(P, dry_run, s);
+            case 1: return launch_slice_one<T, DT, NTB, 1>(P, plan, s);
+            case 2: return launch_slice_one<T, DT, NTB, 2>(P, plan, s);
+            case 3: return launch_slice_one<T, DT, NTB, 3>(P, plan, s);
+            default: return launch_slice_one<T, DT, NTB, 4>(P, plan, s);
         }
     };
     switch ((P.B + 15) / 16) {

@@ -258,6 +258,27 @@ def test_sliced_by_name():
     assert lib.ma_bwd_workspace_bytes(b) == 0
 
 
+def test_auto_runs_slices_where_they_are_faster():
+    """AUTO's choice between the slice-resident kernel and the one it stands in for, at shapes where one of the two took at most
+    0.85 of the other's time (us on an MI355X: slices, the other)."""
+    lib = L.load()
+    for heads, N, D, B, T, slices, other in (
+            # few blocks, more slices than compute units
+            (768, 71, 32, 43, 2, 47.9, 22.1), (512, 36, 32, 37, 2, 32.5, 13.9), (512, 36, 32, 41, 3, 45.0, 18.7), (320, 127, 32, 33, 3, 32.3, 22.8),
+            (384, 246, 32, 43, 1, 19.8, 16.0), (128, 29, 72, 18, 3, 16.8, 12.3), (128, 4, 80, 23, 2, 12.2, 10.2),
+            # a last round of few waves or a last pass of few slices
+            (224, 1234, 40, 20, 2, 125.0, 87.2), (320, 885, 72, 25, 2, 152.7, 125.6), (320, 749, 48, 20, 2, 108.9, 87.0), (256, 712, 72, 20, 4, 192.6, 160.6),
+            (320, 548, 72, 15, 4, 187.5, 147.8), (128, 2002, 32, 34, 4, 181.1, 149.8), (192, 254, 72, 14, 6, 59.3, 52.6),
+            # the slices' own ground
+            (128, 1024, 72, 32, 3, 46.3, 77.6), (112, 260, 40, 20, 1, 8.7, 10.2), (128, 384, 40, 24, 1, 9.4, 10.9), (128, 512, 64, 32, 2, 17.1, 26.0)):
+        p = good_params()
+        p.E, p.H, p.N, p.D, p.Dv, p.B, p.T, p.variant = heads, 1, N, D, D, B, T, L.VARIANTS["auto"]
+        p.dtype_qk = p.dtype_v = L.MA_F16
+        for field in ("q_stride", "k_stride", "v_stride", "out_stride"):
+            setattr(p, field, (C.c_int64 * 3)(N * D, N * D, D))
+        assert (lib.ma_fwd_kernel_name(p) == b"resident_slice_mfma") == (slices < other), (heads, N, D, B, T)
+
+
 def test_check_maps_status_to_python_exceptions():
     with pytest.raises(ValueError):
         L.check(L.MA_ERR_SHAPE, "x")
