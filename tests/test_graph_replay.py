@@ -26,6 +26,8 @@ CASES = [  # E, H, N, D, B, T, dtype, variant
     (8, 16, 197, 64, 16, 2, "f16", "resident"),
     (1, 4, 2048, 64, 128, 2, "f16", "staged"),
     (1, 2, 300, 48, 16, 2, "f32", "auto"),
+    (2, 8, 512, 72, 32, 3, "f16", "sliced"),      # 16 positions a workgroup, Y through the workspace
+    (1, 12, 197, 64, 14, 2, "f16", "auto"),       # ... where AUTO runs it
 ]
 
 
@@ -73,7 +75,7 @@ def test_captured_forward_replays_like_eager(case, static):
         assert torch.equal(again.view(torch.uint8), want.view(torch.uint8)), f"case {case} eager call after replay {rep} differs"
 
 
-@pytest.mark.parametrize("case", [0, 1, 2, 3, 7, 8])
+@pytest.mark.parametrize("case", [0, 1, 2, 3, 7, 8, 9, 10])
 def test_captured_module_call_replays_like_eager(case):
     """The Python operator itself under capture: it allocates its output from the graph's pool, looks
     at the host-visible error word (a host read) and queues nothing but the library's kernels, so a

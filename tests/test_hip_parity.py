@@ -387,6 +387,53 @@ def test_sliced_by_name(E, H, N, D, B, T, pre, dt, masked, layout):
     assert_parity(out.cpu(), ref, dt, f"sliced {(E, H, N, D, B, T, pre, dt, masked, layout)}")
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("D", [32, 40, 48, 64, 72, 80])
+def test_every_class_of_the_slice_resident_kernel(D, dt):
+    """All classes of strips of blocks and of block counts at a head dim, at their smallest, an odd and their largest size, in every
+    kind of workgroup the launcher has: few heads (16 or 12 waves, 8 where the LDS holds no more) and, up to two strips, more
+    slices than compute units (two workgroups of 8 waves on one).  Bit-equal to the chained kernel, with masks and both pads."""
+    lib, g, ran = L.load(), torch.Generator(device=DEV).manual_seed(D), set()
+    for nb in (1, 2, 3, 4):
+        for nm in (1, 2, 3, 4):
+            for i, (B, M) in enumerate([(16 * nb, 16 * nm), (16 * nb - 15, 16 * nm - 3), (16 * nb - 2, 16 * nm - 15), (16 * nb - 7, 16 * nm - 8)]):
+                for E, H in ((1, 3), (34, 8 if nb == 1 else 4))[: 2 if nb <= 2 and nm <= 2 else 1]:
+                    N, T, pre, masked = B * M - (B // 3 if i % 2 else 0), 1 + i % 3, i % 2 == 1, i >= 2
+                    q, k, v = (torch.randn(E, H, N, D, generator=g, device=DEV).to(DT[dt]) for _ in range(3))
+                    mask = (torch.rand(E, N, generator=g, device=DEV) > 0.3) if masked else None
+                    if masked:
+                        mask[:, : N // 4 + 1] = True
+                    p = make_params(q, k, v, mask, torch.empty_like(v), T, B, pre, "sliced")
+                    if lib.ma_fwd_select_variant(p) == L.MA_ERR_UNSUPPORTED:   # (state and tiles beyond the LDS)
+                        continue
+                    ran.add((nb, nm))
+                    out = monarch_attention_hip(q, k, v, mask, T, B, pre, variant="sliced")
+                    same = torch.equal(out, monarch_attention_hip(q, k, v, mask, T, B, pre, variant="chained"))
+                    assert same and torch.isfinite(out).all(), (E, H, N, D, B, M, T, pre, masked)
+    assert len(ran) == {32: 16, 40: 16, 48: 13, 64: 11, 72: 11, 80: 8}[D], sorted(ran)
+
+
+@pytest.mark.parametrize("layout", ["heads", "tokens"])
+@pytest.mark.parametrize("M", [1, 2, 3, 5, 8, 9, 13])
+def test_slices_of_few_blocks(M, layout):
+    """Fewer blocks than waves, and (up to 8) blocks of which the chained kernel packs several positions into a problem: 112 and 128
+    heads in 17 .. 48-row blocks, both pads, masks that leave whole blocks without keys."""
+    for i, (heads, B, D, T) in enumerate([(112, 24, 64, 2), (128, 31, 72, 3), (112, 17, 40, 1), (128, 48, 32, 2)]):
+        N = B * M - (B - 3 if i == 2 else i)
+        q, k, v = seeded_qkv(heads // 8, 8, max(N, 1), D, DT["f16" if i % 2 else "bf16"], seed=M)
+        N = q.shape[2]
+        mask = torch.ones(heads // 8, N, dtype=torch.bool)
+        mask[::2, N // 2:] = False
+        mask[:, 0] = True
+        dq, dk, dv, dm = to_dev(q, k, v, mask)
+        pre = i % 2 == 0
+        want = monarch_attention_hip(dq, dk, dv, dm, T, B, pre, variant="chained")
+        out = monarch_attention_hip(*(in_layout(t, layout) for t in (dq, dk, dv)), dm, T, B, pre, variant="sliced")
+        assert torch.equal(out, want), (heads, N, D, B, T)
+        ref = monarch_attention_oracle(q[:1], k[:1], v[:1], mask[:1], T, B, pre, upcast=True)
+        assert_parity(out[:1].cpu(), ref, "f16" if i % 2 else "bf16", f"few blocks {(heads, N, D, B, T)}")
+
+
 @pytest.mark.parametrize("layouts", [("tokens", "tokens", "tokens"), ("heads", "tokens", "heads"), ("tokens", "heads", "tokens")])
 @pytest.mark.parametrize("E,H,N,D,B,T,pre,dt", [
     (2, 4, 100, 40, 16, 2, False, "f16"), (1, 8, 500, 72, 32, 2, True, "bf16"), (1, 16, 700, 80, 24, 3, False, "f16"),
