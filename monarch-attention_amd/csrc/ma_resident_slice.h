@@ -54,8 +54,8 @@ struct Slice {
     };
     // Rows an odd number of 16-byte units apart, blocks of the state 16 bytes more than their rows: neither the 16 rows of a block
     // nor the rows of 16 blocks at one position start in the same LDS banks.
-    static __host__ __device__ Layout layout(int D, int M) {
-        Layout L;
+    static constexpr __host__ __device__ Layout layout(int D, int M) {
+        Layout L{};
         L.P = 16u * ((static_cast<unsigned>(D) / 8u) | 1u);
         L.BP = 16u * L.P + 16u;
         unsigned o = 0;

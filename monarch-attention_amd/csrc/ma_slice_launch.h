@@ -12,12 +12,17 @@ constexpr size_t kSliceLds = 160 * 1024;
 template <class T, int DT, int NTB, int NTM, int W>
 int launch_slice_w(const Problem& P, hipStream_t s) {
     using SL = Slice<T, DT, NTB, NTM, W>;
-    if (!SL::takes(P.D, P.M, P.B, kSliceLds)) return MA_ERR_UNSUPPORTED;
-    const int lds_err = set_lds_limit(resident_slice_mfma<T, DT, NTB, NTM, W>, kSliceLds);
-    if (lds_err) return lds_err;
-    const long long heads = static_cast<long long>(P.E) * P.H, grid = (heads + 7) / 8 * 8 * ((P.B + 15) / 16);
-    hipLaunchKernelGGL((resident_slice_mfma<T, DT, NTB, NTM, W>), dim3(static_cast<unsigned>(grid)), dim3(64 * W), SL::layout(P.D, P.M).total, s, P);
-    return static_cast<int>(hipGetLastError());
+    // (no kernel is built for a class whose smallest problem - the fewest columns and blocks - does not fit)
+    if constexpr (SL::layout(16 * DT - (SL::kRest ? 8 : 0), SL::ROWSM - 15).total <= kSliceLds) {
+        if (!SL::takes(P.D, P.M, P.B, kSliceLds)) return MA_ERR_UNSUPPORTED;
+        const int lds_err = set_lds_limit(resident_slice_mfma<T, DT, NTB, NTM, W>, kSliceLds);
+        if (lds_err) return lds_err;
+        const long long heads = static_cast<long long>(P.E) * P.H, grid = (heads + 7) / 8 * 8 * ((P.B + 15) / 16);
+        hipLaunchKernelGGL((resident_slice_mfma<T, DT, NTB, NTM, W>), dim3(static_cast<unsigned>(grid)), dim3(64 * W), SL::layout(P.D, P.M).total, s, P);
+        return static_cast<int>(hipGetLastError());
+    } else {
+        return MA_ERR_UNSUPPORTED;
+    }
 }
 
 // As many waves as the LDS has tiles for: 16 or 8, 12 or 8 for problems of more than two strips (256 heads of 1024, 48-row blocks, T =
