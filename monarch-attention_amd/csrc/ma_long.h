@@ -2,7 +2,7 @@
 // (*_long).  The operand tiles of a problem are in LDS once, its waves walk the 16-row strips.
 //
 // What bounds them: the softmax arithmetic (48 heads of 65536 tokens, D = 64, 256 rows: vector instructions take half of the
-// cycles, at a clock that the power limit holds at 2 GHz), then the traffic (the Z step moves 1.6 GB at 4.3 TB/s, the R step with V
+// cycles, at a clock that the power limit holds at 2 GHz), then the traffic (the Z step moves 1.6 GB at 4.0 TB/s, the R step with V
 // 2.1 GB at 3.9) and, at wide head dims, how many waves fit beside the tiles.  So
 //  * problems of up to 128 rows run two strips per wave side by side, so that an operand fragment read from LDS feeds two
 //    matrix instructions (their arithmetic is that of ma_mfma.h to the bit: the chained kernel runs such problems too);
@@ -577,19 +577,19 @@ __global__ __launch_bounds__(64 * W, EU) void r_step_long(Problem P, int first) 
                 const float shift = mx - clamped, scale = __builtin_amdgcn_exp2f(shift);
                 float sum = 0.f, ent = 0.f;
 #pragma unroll
-                    for (int w = 0; w < NWT; ++w) {
-                        f32x4 p, b = {-mx, -mx, -mx, -mx};
-                        if (kMasked) b += *reinterpret_cast<const f32x4*>(kbias + 16 * w + 4 * q);
+                for (int w = 0; w < NWT; ++w) {
+                    f32x4 p, b = {-mx, -mx, -mx, -mx};
+                    if (kMasked) b += *reinterpret_cast<const f32x4*>(kbias + 16 * w + 4 * q);
 #pragma unroll
-                        for (int v = 0; v < 4; ++v) {
-                            const float d = fmaf(to_f(C[s][w][v]), cj[s], b[v]);
-                            p[v] = __builtin_amdgcn_exp2f(d);
-                            sum += p[v];
-                            ent = fmaf(p[v], d, ent);   // sum p log2 p
-                        }
-                        C[s][w] = Pack<T>::four_now(p);
-                        if (w % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                    for (int v = 0; v < 4; ++v) {
+                        const float d = fmaf(to_f(C[s][w][v]), cj[s], b[v]);
+                        p[v] = __builtin_amdgcn_exp2f(d);
+                        sum += p[v];
+                        ent = fmaf(p[v], d, ent);   // sum p log2 p
                     }
+                    C[s][w] = Pack<T>::four_now(p);
+                    if (w % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                }
                 sum = mfma::quad_rows_sum(sum);
                 ent = mfma::quad_rows_sum(ent);
                 const float den = fmaf(scale, sum, P.eps);
@@ -828,7 +828,8 @@ __global__ __launch_bounds__(64 * W, EU) void l_step_long(Problem P) {
 // longer ones lose 2 - 12 % there).  As many waves as strips, since a wave's strips would run one after the other while most of the
 // compute unit is idle.  One head of 10672 tokens, D = 72, 64-row blocks, two steps: 34.5 -> 28.6 us; of 40000, D = 64, 200-row
 // blocks: 54.3 -> 51.0; of 30000, D = 96: 59.1 -> 53.1; two heads of 22000, D = 64, 140 rows: 54.4 -> 48.3; eight of 10672, 64 rows:
-// 55.4 -> 51.1.
+// 55.4 -> 51.1.  Not for more than 192 wide rows: L and Z of 14 strips at D = 128 then spill, one head of 44100 in 210-row blocks takes 71.7
+// us in 14 waves and 67.4 in eight of two strips each, of 65536 in 256-row blocks 89.6 and 86.9, of 57600 at D = 96 (240) 69.6 and 69.4.
 // Classes of 10, 12, 14 and 16 strips; strips beyond the last row are passed over.  Measured without the classes of 10 and 14 ->
 // with them: 32 heads of 22000, D = 64, 140-row blocks, two steps 414 -> 345 us; 16 of 40000, D = 64, 200 rows 450 -> 382;
 // 16 of 48000, D = 96, 220 rows, one step 419 -> 390; 16 of 40000, D = 128, 200 rows 454 -> 429.  (Workgroups of 5 and 7 waves,
@@ -836,7 +837,7 @@ __global__ __launch_bounds__(64 * W, EU) void l_step_long(Problem P) {
 template <int STAGE, bool kV, int DT, int NWT, bool FEW>
 struct Cfg {
     static constexpr bool kWideRow = DT > 4, k16 = NWT > 12, kKeysOnly = STAGE == kStageR && !kV;
-    static constexpr bool kOne = FEW && !(STAGE == kStageR && k16 && kWideRow);   // (there the registers of 16 waves do not hold a strip)
+    static constexpr bool kOne = FEW && !(k16 && kWideRow);   // (there the registers of 14 or 16 waves do not hold a strip)
     static constexpr int W = kOne ? NWT : k16 ? 8 : DT == 8 && !kKeysOnly ? NWT : 4;
     static constexpr int SP = k16 && kWideRow && !kOne && !(kKeysOnly && DT == 6) ? 2 : 1;
     static constexpr int EU = kOne ? (NWT + 3) / 4 : !kWideRow ? 4 : SP == 2 ? 2 : k16 ? 4 : 3;
