@@ -8,23 +8,30 @@
 // are the contraction index:
 //
 //   R, pass 1, strip of query rows j (accumulator rows = keys i): S = X K^T, Gg = Ga K^T + Gy V^T -> r, g, dDot  (Ga = sm gaL);
-//      gaR[j] = sum_i dDot[j,i] K[i], gcR[j]; the row statistics (max, 1 / sum, sum_i g r).
+//      gaR[j] = sum_i dDot[j,i] K[i], gcR[j]; what pass 2 needs of the row: c0, c1 and 1 / sum (see the kernel).
 //   R, pass 2, strip of keys i (accumulator rows = query rows j): r and dDot again from the statistics;
 //      dK[i] (+)= sum_j r[j,i] Ga[j] + dDot[j,i] X[j],  dV[i] = sum_j r[j,i] Gy[j].
 //   L / Z, pass 1, strip of query blocks l (accumulator rows = key blocks k): U, g -> p, dU;
-//      dq[(l,j)] (+)= sum_k dU[l,k] aL[j,k]  (L: + round(mask_q p)[l,k] gaR[k,j]); the row statistics.
+//      dq[(l,j)] (+)= sum_k dU[l,k] aL[j,k]  (L: + round(mask_q p)[l,k] gaR[k,j]); of the row: log(mask / sum) - max, -sum g p
+//      (fp32: -max and mask / sum apart).
 //   L / Z, pass 2, strip of key blocks k: Ga[j,k] = sm sum_l dU[l,k] Q[l], gcL[j,k] = -sum_l dU[l,k],
 //      Z: gY[j,k] = sum_l round(p)[l,k] dout[l].
 //
 // The second evaluation of the logits costs matrix instructions that are otherwise idle; it saves the n x n matrices.
 //
+// Logits are rounded to the operand type where the forward that kept the states rounds them (all R stages, L and Z of up to 128
+// blocks; ma_long.h keeps those of 129 .. 256 in fp32): probabilities have to be the ones that the states were formed with.
+// Left in fp32 they are closer to the exact ones while logits are of order one, but the gradients then part from their forward with
+// the size of the logits: bf16, q and k of standard deviation 3, 2.5 .. 5 % from the reference's dq (0.6 .. 1.7 % rounded), and 2 .. 10 %
+// further from the exact one.  (The rounding costs the L and Z stages 1 - 2 us of 65 on 32 heads of 8192 tokens, training calls 0 - 2 %.)
+//
 // What bounds them: memory (each operand row once in, each gradient row once out), and with it how many waves a compute
 // unit holds while they wait.  So a pass keeps only ITS tiles in LDS: pass 1 the two operands it contracts over, pass 2
 // those of the strips - which the waves hold in registers from pass 1 and put over the first pair (LDS per workgroup: 2
-// tiles for L / Z and 3 for R, where all operands at once took 4 and 5).  A strip's accumulators of pass 2 are consumed
+// tiles for L, Z and R, 3 for R with V, where all operands at once took 4 and 5).  A strip's accumulators of pass 2 are consumed
 // two tiles at a time, and gradients that are added to are loaded at the start and seed the accumulators.
 // Behind the memory come the vector instructions, so an entry of a pass costs one exponential and about eight others: the
-// biases sit in the accumulators, the row sums are taken of unnormalised values in one sweep, pass 2 forms p from one exponent that
+// biases of what is not rounded sit in the accumulators, the row sums are taken of unnormalised values in one sweep, pass 2 forms p from one exponent that
 // holds the normaliser, and nothing branches on an entry (a select on "inside" had become a branch each).  Measured, bf16, T = 2,
 // stages Z / R with V / L / R: 32 heads of 8192 tokens in 64-row blocks 70.3 / 57.7 / 78.3 / 57.7 -> 64.3 / 62.5 / 66.2 / 49.5 us,
 // 192 heads of 512 in 32-row blocks 17.4 / 19.5 / 18.7 / 19.5 -> 18.0 / 20.5 / 18.5 / 18.2 (the two R stages averaged before).
@@ -52,12 +59,22 @@ template <class T>
 __device__ __forceinline__ f32x4 start_at(const f32x4& c) { return sizeof(T) == 2 ? c : f32x4{0.f, 0.f, 0.f, 0.f}; }
 template <class T>
 __device__ __forceinline__ f32x4 shifted(const f32x4& sum, const f32x4& c) { return sizeof(T) == 2 ? sum : sum + c; }
+// four logits as the forward holds them: rounded to the operand type
+template <class T>
+__device__ __forceinline__ f32x4 rounded(const f32x4& a) {
+    if constexpr (sizeof(T) == 4) return a;
+    else {
+        const typename mfma::Ops<T>::v4 h = {from_f<T>(a[0]), from_f<T>(a[1]), from_f<T>(a[2]), from_f<T>(a[3])};
+        return f32x4{to_f(h[0]), to_f(h[1]), to_f(h[2]), to_f(h[3])};
+    }
+}
 __device__ __forceinline__ f32x4 lds4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 
 // ---------------------------------------------------------------- R stage
 // kV: the last step's stage, the first of a backward pass (Y and dv)
+// (Two strips of up to 64 columns: five waves a SIMD as long as a wave keeps to 96 registers, which the compiler else misses by two.)
 template <class T, int DT, int NWT, int W, int PASS, bool kV>
-__global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, int first) {
+__global__ __launch_bounds__(64 * W, sizeof(T) == 2 && DT <= 4 && NWT == 2 && PASS == 0 ? 5 : 1) void r_bwd_tile(Problem P, BwdBuffers G, int first) {
     using MT = Mat<T, DT>;
     using PL = RPlan<T, DT, NWT, PASS, kV>;
     using mfma::quad_rows_max;
@@ -147,9 +164,9 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
 #pragma unroll
             for (int w = 0; w < CT1; ++w) {
                 const f32x4 kb4 = lds4(kbias + 16 * (CT1 * c + w) + 4 * q);
-                f32x4 a = start_at<T>(kb4), g = {0.f, 0.f, 0.f, 0.f};
+                f32x4 a = start_at<T>(kb4), g = {0.f, 0.f, 0.f, 0.f};   // (0 or -inf: neither changes what a is rounded to)
                 MT::gemm1(Kt, w, r, q, xb, a, ga, g);
-                a = shifted<T>(a, kb4);
+                a = rounded<T>(shifted<T>(a, kb4));
                 if (kV) MT::gemm1(Vt, w, r, q, gy, g);
                 if (NWT > 4 && w % 2 == 1) __builtin_amdgcn_sched_barrier(0);   // (keeps the tile reads from being hoisted: registers)
                 if constexpr (PL::NC1 == 1) {
@@ -343,6 +360,7 @@ __global__ __launch_bounds__(64 * W) void r_bwd_tile(Problem P, BwdBuffers G, in
                     g = shifted<T>(g, c14);
                     const f32x4 sc4 = lds4(scs + j0), c04 = lds4(c0s + j0), gl4 = lds4(gls + j0), df4 = lds4(dfs + j0);
                     const f32x4 inv4 = kF32 ? lds4(invs + j0) : f32x4{1.f, 1.f, 1.f, 1.f};
+                    a = rounded<T>(a);
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
                         const float lp = fminf(fmaf(a[v], sc4[v], c04[v]), most);
@@ -384,7 +402,7 @@ __global__ __launch_bounds__(64 * W, sizeof(T) == 2 && DT <= 4 && NWT == 8 && PA
     using mfma::quad_rows_sum;
     constexpr int NTH = 64 * W, ROWS = PL::ROWS, CT1 = PL::CT1, CT2 = PL::CT2;
     constexpr float kLog2e = mfma::kLog2e;
-    constexpr bool kF32 = sizeof(T) == 4;
+    constexpr bool kF32 = sizeof(T) == 4, kRound = !kF32 && NWT <= 8;
     static_assert(PASS != 0 || W == NWT, "one launch: every strip of the problem in the workgroup");
     extern __shared__ __attribute__((aligned(16))) char lds_raw[];
     T* tiles = reinterpret_cast<T*>(lds_raw);
@@ -461,10 +479,10 @@ __global__ __launch_bounds__(64 * W, sizeof(T) == 2 && DT <= 4 && NWT == 8 && PA
             for (int w = 0; w < CT1; ++w) {
                 const int k0 = 16 * (CT1 * c + w) + 4 * q;
                 const f32x4 ncl4 = lds4(ncl + k0), cw4 = kZ ? f32x4{0.f, 0.f, 0.f, 0.f} : lds4(cw + k0);
-                f32x4 a = start_at<T>(ncl4), g = start_at<T>(cw4);
+                f32x4 a = kRound ? f32x4{0.f, 0.f, 0.f, 0.f} : start_at<T>(ncl4), g = start_at<T>(cw4);
                 MT::gemm1(At, w, r, q, xq, a);                   // U
                 MT::gemm1(Wt, w, r, q, kZ ? xo : xq, g);         // gL = Q gaR^T + gcR (mask_q: see keep)
-                a = shifted<T>(a, ncl4);
+                a = kRound ? rounded<T>(a) + ncl4 : shifted<T>(a, ncl4);
                 if (!kZ) g = shifted<T>(g, cw4);
                 if constexpr (PL::NC1 == 1) {
                     U[w] = a;
@@ -599,13 +617,14 @@ __global__ __launch_bounds__(64 * W, sizeof(T) == 2 && DT <= 4 && NWT == 8 && PA
                     PR[u] = DU[u] = f32x4{0.f, 0.f, 0.f, 0.f};
                     if (CT2 % 2 == 1 && s + u >= CT2) continue;
                     const f32x4 c04 = lds4(c0s + l0), nd4 = lds4(nds + l0), pk4 = kF32 ? lds4(pks + l0) : f32x4{1.f, 1.f, 1.f, 1.f};
-                    f32x4 a = start_at<T>(c04), g = start_at<T>(nd4);
+                    f32x4 a = kRound ? f32x4{0.f, 0.f, 0.f, 0.f} : start_at<T>(c04), g = start_at<T>(nd4);
                     if (kZ) {
                         MT::gemm1(Qt, s + u, r, q, ak, a);
                         MT::gemm1(dOt, s + u, r, q, wk, g);
                     } else {
                         MT::gemm1(Qt, s + u, r, q, ak, a, wk, g);
                     }
+                    if (kRound) a = rounded<T>(a) + c04;
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
                         const float p = kF32 ? __builtin_amdgcn_exp2f(kLog2e * (a[v] + nck + c04[v])) * pk4[v]
