@@ -654,7 +654,7 @@ struct RProb {
             mx = fmaxf(quad_rows_max(mx), P.eps * kLog2e);
             float sum = 0.f, ent = 0.f;
 #pragma unroll
-            for (int wt = 0; wt < NWT; ++wt) {
+            for (int wt = 0; wt < NWT; ++wt)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const float d = C[wt][v] - mx;
@@ -663,7 +663,6 @@ struct RProb {
                     ent = fmaf(p, d, ent);  // sum p * log2(p)
                     C[wt][v] = p;
                 }
-            }
             sum = quad_rows_sum(sum);
             ent = quad_rows_sum(ent);
             const float den = sum + P.eps;
@@ -814,14 +813,13 @@ struct ZProb {
             mx = quad_rows_max(mx);
             float sum = 0.f;
 #pragma unroll
-            for (int wt = 0; wt < NWT; ++wt) {
+            for (int wt = 0; wt < NWT; ++wt)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const float p = __builtin_amdgcn_exp2f(C[wt][v] - mx);
                     sum += p;
                     C[wt][v] = p;
                 }
-            }
             const float inv = rcp(quad_rows_sum(sum));
 #pragma unroll
             for (int wt = 0; wt < NWT; ++wt)
@@ -971,10 +969,9 @@ struct LProb {
                 mx = quad_rows_max(mx);
                 float sum = 0.f;
 #pragma unroll
-                for (int kt = 0; kt < NWT; ++kt) {
+                for (int kt = 0; kt < NWT; ++kt)
 #pragma unroll
                     for (int v = 0; v < 4; ++v) sum += __builtin_amdgcn_exp2f(C[kt][v] - mx);
-                }
                 sum = quad_rows_sum(sum);
                 if (q == 0) {
                     mxs[l] = mx;

@@ -290,7 +290,8 @@ __device__ __forceinline__ rsrc_t state_slice(const void* base, long long eh, lo
 }
 
 // ---- launches
-// Strips of n rows in the classes 1, 2, 3, 4, 6, 8, 12, 16
+// Strips of n rows in the classes 1, 2, 3, 4, 6, 8, 12, 16 (each_launch has 5, 7 and 10 between them for 16-bit operands; the 16-bit forward
+// stages of ma_long.h have classes of their own)
 inline int strip_class(int n) {
     const int s = (n + 15) / 16;
     return s <= 4 ? s : s <= 6 ? 6 : s <= 8 ? 8 : s <= 12 ? 12 : 16;
