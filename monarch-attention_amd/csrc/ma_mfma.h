@@ -614,8 +614,8 @@ struct RProb {
         }
         problem_sync<WPP>();
         // The last strip has rows (uniform).  65 - 80 rows leave it empty in the class of 6 strips: it is passed over (16 heads of 5003,
-        // 72-row blocks, two steps: D = 64 45.2 -> 42.9 us, D = 128 75.1 -> 72.3; full classes unchanged).  Passing over its tile of
-        // keys too gives as much again, but takes 16 registers, and full strips lose 1 - 2 %; so do 8 strips with either.
+        // 72-row blocks, two steps, inputs from memory: D = 64 44.6 -> 42.3 us, D = 128 71.1 -> 70.0; full classes within 0.3 %).  Passing
+        // over its tile of keys too gives as much again, but takes 16 registers, and full strips lose 1 - 2 %; so do 8 strips with either.
         const bool full = NWT != 6 || 16 * (NWT - 1) < B;
 #pragma unroll
         for (int si = 0; si < SPW; ++si) {
