@@ -292,10 +292,15 @@ bool slice_pays(const ma_fwd_params* p, int v) {
     if (half_passes == 0 || !slice_fits(p, &plan)) return false;
     const long long heads = static_cast<long long>(p->E) * p->H, strips = (p->B + 15) / 16;
     if (v == MA_VARIANT_RESIDENT) return 2 * ((heads + 7) / 8 * 8 * strips) <= static_cast<long long>(half_passes) * plan.units;
-    // (Most of a pass, or three quarters from 17 blocks on; 14 and 15 rows in up to 16 blocks any number of heads.  Below, slices are ahead
-    // too where blocks are few - 64 .. 111 heads of 17 .. 32 rows in up to 16 blocks, T >= 2: 0.66 - 0.93 -, but no call has been moved there yet.)
-    const bool one_tile = (p->B == 14 || p->B == 15) && M <= 16;
-    return (one_tile || 8 * heads * strips >= (M > 16 ? 6 : 7) * plan.units) && slice_us(p, plan, M) < chain_us(p, M, plan.units);
+    // Most of a pass, or three quarters from 17 blocks on; 14 and 15 rows in up to 16 blocks fewer heads (64 at a single step: 8.0 us for 8.2,
+    // 12 heads 7.6 for 7.3).  Below, slices are ahead too where blocks are few - 64 .. 111 heads of 17 .. 32 rows in up to 16 blocks, T >= 2:
+    // 0.66 - 0.93 -, but no call has been moved there yet.
+    const bool one_tile = (p->B == 14 || p->B == 15) && M <= 16 && (p->T >= 2 || 4 * heads >= plan.units);
+    if (!one_tile && 8 * heads * strips < (M > 16 ? 6 : 7) * plan.units) return false;
+    // A single pass and up to 16 blocks: 0.63 - 1.04 of the chained kernel's time in 600 problems of up to 32 rows and 70 longer ones at D = 32.
+    const bool single_pass = 8 * ((heads + 7) / 8 * strips) <= plan.units;
+    if (single_pass && M <= 16 && (one_tile || strips == 2 || (strips > 2 && p->D <= 32))) return true;
+    return slice_us(p, plan, M) < chain_us(p, M, plan.units);
 }
 
 // The fused, chained and resident kernels are built for block problems of at most 128 rows.

@@ -260,7 +260,7 @@ def test_sliced_by_name():
 
 def test_auto_runs_slices_where_they_are_faster():
     """AUTO's choice between the slice-resident kernel and the one it stands in for, at shapes where one of the two took at most
-    0.85 of the other's time (us on an MI355X: slices, the other)."""
+    0.92 of the other's time (us on an MI355X: slices, the other)."""
     lib = L.load()
     for heads, N, D, B, T, slices, other in (
             # few blocks, more slices than compute units
@@ -269,6 +269,9 @@ def test_auto_runs_slices_where_they_are_faster():
             # a last round of few waves or a last pass of few slices
             (224, 1234, 40, 20, 2, 125.0, 87.2), (320, 885, 72, 25, 2, 152.7, 125.6), (320, 749, 48, 20, 2, 108.9, 87.0), (256, 712, 72, 20, 4, 192.6, 160.6),
             (320, 548, 72, 15, 4, 187.5, 147.8), (128, 2002, 32, 34, 4, 181.1, 149.8), (192, 254, 72, 14, 6, 59.3, 52.6),
+            # a single pass; few heads at a single step
+            (78, 470, 32, 48, 1, 7.6, 9.4), (80, 300, 32, 40, 1, 7.1, 8.5), (128, 214, 72, 32, 1, 10.4, 11.6), (2, 192, 48, 15, 1, 7.4, 6.5),
+            (4, 192, 48, 14, 1, 7.2, 6.6),
             # the slices' own ground
             (128, 1024, 72, 32, 3, 46.3, 77.6), (112, 260, 40, 20, 1, 8.7, 10.2), (128, 384, 40, 24, 1, 9.4, 10.9), (128, 512, 64, 32, 2, 17.1, 26.0)):
         p = good_params()
