@@ -392,10 +392,16 @@ __global__ __launch_bounds__(64 * W, sizeof(T) == 2 && DT <= 4 && NWT == 2 && PA
 }
 
 // ---------------------------------------------------------------- L and Z stages
-// (Eight strips of up to 64 columns: two workgroups of eight waves share a compute unit as long as a wave keeps to 128 registers.  The
-// L stage of 32 heads of 8192 tokens takes 66 us at 128 and 87 above.)
+// Waves a SIMD that the 16-bit kernels of one launch are held to, in the classes where a few registers would cost one.  (Eight strips of
+// up to 64 columns: two workgroups of eight waves share a compute unit as long as a wave keeps to 128 registers.  The L stage of 32 heads
+// of 8192 tokens takes 66 us at 128 and 87 above.)
+constexpr int lz_held_waves(int DT, int NWT, bool kZ) {
+    if (DT <= 4) return NWT == 8 ? 4 : kZ && NWT == 6 ? 5 : 1;
+    if (DT <= 6) return kZ && NWT == 8 ? 4 : 1;
+    return !kZ && NWT == 4 ? 4 : NWT == (kZ ? 6 : 5) ? 3 : 1;
+}
 template <class T, int DT, int NWT, int W, int PASS, bool kZ>
-__global__ __launch_bounds__(64 * W, sizeof(T) == 2 && DT <= 4 && NWT == 8 && PASS == 0 ? 4 : 1) void lz_bwd_tile(Problem P, BwdBuffers G) {
+__global__ __launch_bounds__(64 * W, sizeof(T) == 2 && PASS == 0 ? lz_held_waves(DT, NWT, kZ) : 1) void lz_bwd_tile(Problem P, BwdBuffers G) {
     using MT = Mat<T, DT>;
     using PL = LzPlan<T, DT, NWT, PASS, kZ>;
     using mfma::quad_rows_max;
