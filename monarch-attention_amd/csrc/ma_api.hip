@@ -3,6 +3,7 @@
 // the driver of the reference, monarch_attention_torch (ma/ma_torch.py:100-108):
 // (T-1) x [R step, L step], the R step that also forms Y, then the Z step.
 #include "ma_common.h"
+#include "ma_mfma_launch.h"
 
 #include <cmath>
 #include <cstdlib>
@@ -740,6 +741,7 @@ struct BwdLayout {
     uint64_t stats;
     uint64_t gaR, gcR, gaL, gcL, gY, stat, dq, dk, dv, pk, pv;
     bool tiled, rows16;                     // BwdBuffers::tiled, rows16
+    bool head;                              // the whole pass in one launch (ma_bwd_head.h)
     int parts;                              // per-tile partial buffers of dk / dv (R stage split over workgroups)
     uint64_t total;
 };
@@ -766,6 +768,33 @@ bool bwd_tiled(const ma_bwd_params* b, const ma_fwd_params* pp, bool* rows16) {
     return bits % (4 * es) == 0;
 }
 
+// Does the whole pass run as one launch, a workgroup per head (ma_bwd_head.h)?  Times are those of a training call, in multiples of
+// the stage launches' (bf16, (E, N, H, D), mask; 256 compute units).  Blocks and block counts of up to 16: always - 0.55 .. 0.75 for 512
+// heads and more of 197 - 256 tokens at T = 2, 0.82 .. 0.96 for 12 heads and more, whose calls are host time by then.  17 .. 32 rows
+// one way or both: a head has a compute unit to itself and three to five times the work, so a pass has to be mostly full.  512 tokens in
+// 32-row blocks, T = 2 | 3: 96 heads 1.00 | 1.03, 128 0.96 | 0.91, 160 0.88 | 0.83, 256 0.71 | 0.68, 264 0.95, 320 0.86, 512 0.80; 480 in
+// 24-row blocks: 128 heads 1.09 | 1.06, 160 0.96 | 0.92, 256 0.79 | 0.75, 264 1.11, 320 0.98, 528 1.02, 576 0.95; 300 tokens in
+// 16: 264 1.17, 320 1.05, 352 0.98, 528 0.94; a single step: 264 1.15 - 1.20, 320 1.05 - 1.08; D = 72, 320 tokens in 32: 192 0.92, 352 1.04,
+// 576 1.05, 768 0.93.  Few heads are calls of host time, where one launch in place of four saves 3 - 14 % (up to 48 heads, T = 2; at
+// T = 3 the one chain is longer than six launches: 1.14 - 1.22).
+bool bwd_head_pays(const ma_fwd_params* pp) {
+    const int M = (pp->N + pp->B - 1) / pp->B, strips = (pp->B + 15) / 16 + (M + 15) / 16;
+    if (strips == 2) return true;
+    const long long heads = static_cast<long long>(pp->E) * pp->H, units = mfma::compute_units(), passes = (heads + units - 1) / units;
+    if (strips == 3 && pp->D <= 64 && pp->T == 2 && heads <= units / 5) return true;
+    if (passes == 1) return 8 * heads >= (pp->D > 64 ? 6 : strips == 3 || pp->D <= 32 ? 4 : 5) * units;
+    return 8 * heads >= (pp->D > 64 ? 7 : 6) * passes * units;
+}
+bool bwd_head(const ma_bwd_params* b, const ma_fwd_params* pp, const BwdLayout& L) {
+    if (pp->B > 32 || pp->N > 32 * pp->B || !L.tiled || !L.rows16 || pp->dtype_qk == MA_F32 || pp->D % 8 != 0 || !bwd_head_pays(pp)) return false;
+    const int64_t* st[7] = {pp->q_stride, pp->k_stride, pp->v_stride, b->dout_stride, b->dq_stride, b->dk_stride, b->dv_stride};
+    for (const int64_t* t : st)   // (Head::kColOut)
+        if (((pp->N - 1) * t[2] + pp->D) * 2 >= 0x7fff0000ll) return false;
+    const Problem P = sizes_of(pp);
+    const BwdBuffers none = {};
+    return launch_bwd_head(P, none, pp->dtype_qk, 0, 0, true, nullptr) == MA_OK;
+}
+
 int bwd_prepare(const ma_bwd_params* b, bool kept, ma_fwd_params* pp, BwdLayout* L) {
     if (b == nullptr) return MA_ERR_NULL;
     *pp = b->fwd;
@@ -785,7 +814,8 @@ int bwd_prepare(const ma_bwd_params* b, bool kept, ma_fwd_params* pp, BwdLayout*
     L->tiled = bwd_tiled(b, pp, &L->rows16);
     // What a stage of the path does not use has no room of its own.  (ma_bwd's size is one for every path, so that it does
     // not depend on pointers a caller may not have yet; the T steps it runs again are the larger part of it anyway.)
-    const bool tight = kept && L->tiled, steps = pp->T > 1;
+    L->head = bwd_head(b, pp, *L);
+    const bool tight = kept && L->tiled, steps = pp->T > 1, staged = !tight || !L->head;
     const uint64_t rows = padded_rows(pp), es = tight ? elt_size(pp->dtype_qk) : 4;
     uint64_t off = kept ? 0 : state_layout(pp).total;
     auto take = [&](uint64_t* at, bool used, uint64_t bytes) {
@@ -794,11 +824,11 @@ int bwd_prepare(const ma_bwd_params* b, bool kept, ma_fwd_params* pp, BwdLayout*
     };
     const bool two_launches = pp->B > 64 || (pp->N + pp->B - 1) / pp->B > 64;   // (each_launch: longer problems may split)
     take(&L->stats, !kept, rows * 8);
-    take(&L->gaR, !tight || steps, rows * pp->D * es);
-    take(&L->gcR, !tight || steps, rows * 4);
-    take(&L->gaL, true, rows * pp->D * es);
-    take(&L->gcL, true, rows * 4);
-    take(&L->gY, true, rows * pp->Dv * es);
+    take(&L->gaR, staged && (!tight || steps), rows * pp->D * es);
+    take(&L->gcR, staged && (!tight || steps), rows * 4);
+    take(&L->gaL, staged, rows * pp->D * es);
+    take(&L->gcL, staged, rows * 4);
+    take(&L->gY, staged, rows * pp->Dv * es);
     take(&L->stat, tight && two_launches, rows * 16);
     // dq, dk, dv are contiguous: one fill kernel zeroes the three
     L->dq = off; off += rows * pp->D * 4;
@@ -916,6 +946,12 @@ int run_bwd(const ma_bwd_params* b, const void* kept, uint64_t kept_bytes, hipSt
     G.dout = static_cast<const char*>(b->dout);
     for (int i = 0; i < 3; ++i) G.dos[i] = b->dout_stride[i];
     const long long rows = static_cast<long long>(P.E) * P.H * P.M * P.B;
+    if (L.head) {
+        at_step(P, S, base, 0);
+        P.aR = base + S.aR;
+        P.cR = reinterpret_cast<float*>(base + S.cR);
+        return launch_bwd_head(P, G, pp.dtype_qk, S.slot_a, S.slot_c, false, s);
+    }
     if (!L.tiled) {
         st = launch_bwd_zero(G.dq, rows * (2LL * P.D + P.Dv), s);
         if (st) return st;

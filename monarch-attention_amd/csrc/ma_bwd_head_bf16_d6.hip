@@ -1,0 +1,8 @@
+// Backward pass of short heads in one launch, bf16, head dims of up to 96 (see ma_bwd_head.h).
+#include "ma_bwd_head.h"
+
+namespace ma {
+int launch_bwd_head_bf16_d6(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, bool dry, hipStream_t s) {
+    return bwdh::launch<bf16, 6>(P, G, slot_a, slot_c, dry, s);
+}
+}  // namespace ma
