@@ -220,9 +220,10 @@ bool resident_head_fits(const ma_fwd_params* p, int forms = 1) {
 
 // Does the slice-resident kernel (ma_resident_slice.h: a workgroup per 16 positions of a head) take the problem: a class of its
 // strips and columns, the state in LDS?  (16-bit operands)
-bool slice_fits(const ma_fwd_params* p, SlicePlan* plan) {
+bool slice_fits(const ma_fwd_params* p, SlicePlan* plan, bool keep = false) {
     Problem P = sizes_of(p);
     P.one_tile_ok = 1;
+    P.slot_rows = keep ? 1 : 0;
     return run_slice(P, p->dtype_qk, plan, nullptr) == MA_OK;
 }
 
@@ -302,6 +303,20 @@ bool slice_pays(const ma_fwd_params* p, int v) {
     const bool single_pass = 8 * ((heads + 7) / 8 * strips) <= plan.units;
     if (single_pass && M <= 16 && (one_tile || strips == 2 || (strips > 2 && p->D <= 32))) return true;
     return slice_us(p, plan, M) < chain_us(p, M, plan.units);
+}
+
+// A recorded call (ma_fwd_keep) that AUTO gives to the chained kernel: does the slice-resident one take it, writing every step's state as it
+// goes?  The same two estimates, and 0.2 us per MB of state that the chained kernel writes anyway.  Of 2076 random problems (8 .. 1024 heads,
+// D = 32 .. 80, blocks and block counts of up to 64, T = 1 .. 3) 170 are chosen, at 0.855 of the chained kernel's time; 3 % of them lose more than
+// 3 %, at most 9; of what the better kernel for each would gain this takes 84 %.  bf16, T = 2: 192 heads of 512 tokens in 32-row blocks 33.9
+// -> 30.6 us, 768 of 197 in 14 51.5 -> 40.4, 384 of 256 in 16 33.5 -> 26.5; 64 of 1024 in 32 (24.3, 28.8 in slices) and 12 of 512 (13.3, 15.3) stay.
+bool slice_keeps(const ma_fwd_params* p) {
+    if (p->variant != MA_VARIANT_AUTO || p->B > 64 || p->D > 80) return false;
+    const int M = (p->N + p->B - 1) / p->B;
+    SlicePlan plan;
+    if (M > 64 || !slice_fits(p, &plan, true)) return false;
+    const float kept = 2e-6f * static_cast<float>(p->E) * p->H * p->D * static_cast<float>(M * p->B) * static_cast<float>(2 * p->T - 1);
+    return slice_us(p, plan, M) + 0.2f * kept < 0.95f * chain_us(p, M, plan.units);
 }
 
 // The fused, chained and resident kernels are built for block problems of at most 128 rows.
@@ -1242,6 +1257,10 @@ int ma_fwd_keep(const ma_fwd_params* p, void* state, uint64_t state_bytes, void*
         pr.P.aR = base + S.aR;
         pr.P.cR = reinterpret_cast<float*>(base + S.cR);
         pr.P.slot_rows = static_cast<unsigned>(S.slot_rows);
+        if (slice_keeps(p)) {
+            pr.P.one_tile_ok = 1;
+            return run_slice(pr.P, p->dtype_qk, nullptr, s);
+        }
         pr.P.Y -= (p->T - 1) * S.slot_a;   // (Dv = D and one element type here)
         return run_chain(pr, p, s);
     }

@@ -45,8 +45,9 @@ struct Problem {
     // Query only: does a head-resident form of the resident kernel take this head?  1: the one that keeps Q, K and V
     // in LDS beside the state; 2: that one or the two-tile form (the state and one input tile at a time); 3: would a
     // launch run a head-resident form in narrow workgroups, several to a compute unit?  4: ... the four-tile form?
-    // Chained kernel, slot_rows: rows from one step's aL, cL, aR, cR to the next step's.  0: all steps share the arrays;
-    // else every step keeps its state (ma_fwd_keep; Y is given (T - 1) * slot_rows rows too low then, see chain_fwd_mfma).
+    // Chained and slice-resident kernels, slot_rows: rows from one step's aL, cL, aR, cR to the next step's.  0: all steps share the arrays;
+    // else every step keeps its state (ma_fwd_keep; the chained kernel is given Y (T - 1) * slot_rows rows too low then, see
+    // chain_fwd_mfma).
     // (They share a word: the argument block stays as long as it is.)
     union {
         int resident_head_only;

@@ -34,7 +34,8 @@
 namespace ma {
 namespace mfma {
 
-template <class T, int DT, int NTB, int NTM, int W>
+// KEEP: every step's aL, cL, aR, cR also go to memory (Problem::slot_rows, ma_fwd_keep); `cl` holds cL itself for that.
+template <class T, int DT, int NTB, int NTM, int W, bool KEEP>
 struct Slice {
     using V8 = typename Ops<T>::v8;
     using V4 = typename Ops<T>::v4;
@@ -50,7 +51,7 @@ struct Slice {
         u32x4 v[NI];
     };
     struct Layout {
-        unsigned S, St, tile, cb, cR, tokb, cs, ZR, trash, total, P, BP;
+        unsigned S, St, tile, cb, cR, tokb, cs, cl, ZR, trash, total, P, BP;
     };
     // Rows an odd number of 16-byte units apart, blocks of the state 16 bytes more than their rows: neither the 16 rows of a block
     // nor the rows of 16 blocks at one position start in the same LDS banks.  (So it is for the reads of rows; the transposed reads of
@@ -68,6 +69,7 @@ struct Slice {
         L.cR = o; o += static_cast<unsigned>(M) * 16 * 4;
         L.tokb = o; o += static_cast<unsigned>(M) * ROWSB * 4;
         L.cs = o; o += W * ROWSM * 8;
+        L.cl = o; o += KEEP ? 16 * ROWSM * 4 : 0;
         L.trash = o; o += 64 * 16;
         L.total = o;
         return L;
@@ -80,7 +82,8 @@ struct Slice {
     struct Ctx {
         char* smem;
         Layout L;
-        int wave, lane, r, q, D;
+        int wave, lane, r, q, D, j0;
+        rsrc_t aL, aR;    // KEEP: this head's rows of the step at hand
         unsigned St;      // this wave's tile
         unsigned tr, sr;  // the lane's row r of it, and of the state's position 0 at block r
         bool zin, pin;    // the lane's share of the last operand step, and its columns of the last output tile, lie inside a row
@@ -204,7 +207,11 @@ struct Slice {
         for (int w = 0; w < NTB; ++w)
 #pragma unroll
             for (int v = 0; v < 4; ++v) C[w][v] = fp32_value(C[w][v] * inv);
-        if (c.q == 0) c.template at<float>(c.L.cb)[c.r * ROWSM + m] = -kLog2e * row_entropy(ent, sum, den, inv);
+        const float cl = row_entropy(ent, sum, den, inv);
+        if (c.q == 0) {
+            c.template at<float>(c.L.cb)[c.r * ROWSM + m] = -kLog2e * cl;
+            if (KEEP) c.template at<float>(c.L.cl)[c.r * ROWSM + m] = cl;
+        }
         pack_p<T, NTB>(pb, C);
         f32x4 O[DT];
         gemm2<NTB>(c, O, pb);
@@ -213,6 +220,7 @@ struct Slice {
 #pragma unroll
             for (int v = 0; v < 4; ++v) O[dt][v] = P.sm_scale * round_to<T>(O[dt][v]);
         put_row(c, srow, O);
+        if (KEEP) store_row<T, DT, kTile>(c.aL, c.j0 + c.r < P.B ? static_cast<unsigned>((c.j0 + c.r) * P.M + m) * (2u * c.D) : kOob, c.D, O, c.q);
     }
 
     // round(x . row(t)), in log2 units, plus bias(t)
@@ -291,6 +299,7 @@ struct Slice {
             pack_p<T, NTM>(pb, U);
             f32x4 O[DT];
             gemm2<NTM>(c, O, pb);
+            if (KEEP) store_row<T, DT, kTile>(c.aR, k < P.M ? static_cast<unsigned>(k * P.B + j) * (2u * c.D) : kOob, c.D, O, c.q);
             if (k < P.M) {   // aR(k, j) over aL(j, k): this strip was its last reader
                 put_row(c, c.sr + 16 * s * c.L.BP + jj * c.L.P, O);
                 if (c.q == 0) c.template at<float>(c.L.cR)[16 * k + jj] = cr;
@@ -327,9 +336,9 @@ struct Slice {
 // heads that follow each other: rows that are no whole lines share them with the next head's where a token's heads lie side by side
 // (128 heads of 1024, D = 72, T = 3, (E, N, H, D): 312 -> 188 MB of traffic, 53.2 -> 46.4 us; D = 80, T = 1 31.7 -> 28.4; D = 64 unchanged).
 // 128 registers where two workgroups of 8 waves or one of 16 share a compute unit, else 256.
-template <class T, int DT, int NTB, int NTM, int W>
+template <class T, int DT, int NTB, int NTM, int W, bool KEEP>
 __global__ __launch_bounds__(64 * W, W == 16 || (NTB <= 2 && NTM <= 2) ? 4 : W == 12 ? 3 : 2) void resident_slice_mfma(Problem P) {
-    using SL = Slice<T, DT, NTB, NTM, W>;
+    using SL = Slice<T, DT, NTB, NTM, W, KEEP>;
     using Row = typename SL::Row;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int B = P.B, M = P.M, heads = P.E * P.H, slices = (B + 15) / 16;
@@ -347,6 +356,7 @@ __global__ __launch_bounds__(64 * W, W == 16 || (NTB <= 2 && NTM <= 2) ? 4 : W =
     c.r = c.lane & 15;
     c.q = c.lane >> 4;
     c.D = P.D;
+    c.j0 = j0;
     c.St = c.L.St + c.wave * c.L.tile;
     c.tr = c.St + c.r * c.L.P;
     c.sr = c.L.S + c.r * c.L.BP;
@@ -354,6 +364,23 @@ __global__ __launch_bounds__(64 * W, W == 16 || (NTB <= 2 && NTM <= 2) ? 4 : W =
     c.pin = 32 * SL::KS + 4 * c.q < P.D;
     const unsigned db = static_cast<unsigned>(P.D) * sizeof(T);
     const int np = M * B;
+    // KEEP: the states of step t, aL and cL out of it, aR and cR into step t + 1
+    const long long slot_a = static_cast<long long>(P.slot_rows) * db, slot_c = static_cast<long long>(P.slot_rows) * 4;
+    auto at_step = [&](int t) {
+        c.aL = make_rsrc(P.aL + t * slot_a + static_cast<long long>(head) * np * db, np * db);
+        c.aR = make_rsrc(P.aR + t * slot_a + static_cast<long long>(head) * np * db, np * db);
+    };
+    auto keep_sums = [&](int phase) {   // what phase left in LDS: rows of M floats of 16 positions, rows of 16 floats of M blocks
+        char* base = reinterpret_cast<char*>((phase & 1) ? P.cR : P.cL) + phase / 2 * slot_c;
+        const rsrc_t s = make_rsrc(base + static_cast<long long>(head) * np * 4, np * 4);
+        for (int i = threadIdx.x; i < 16 * M; i += 64 * W) {
+            const int k = (phase & 1) ? i / 16 : i % M, jj = (phase & 1) ? i % 16 : i / M;
+            const float x = (phase & 1) ? c.template at<float>(c.L.cR)[i] : c.template at<float>(c.L.cl)[jj * SL::ROWSM + k];
+            const unsigned off = static_cast<unsigned>((phase & 1) ? k * B + j0 + jj : (j0 + jj) * M + k) * 4u;
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x), s, j0 + jj < B ? off : kOob, 0, 0);
+        }
+    };
+    if (KEEP) at_step(0);
 
     // Problem n of this wave: phase ph (even: R, odd: L), round rd, and for the last step's R problems the half: K, then V
     const int last = 2 * P.T - 2, rounds_r = (M + W - 1) / W, rounds_j = (16 + W - 1) / W;
@@ -409,11 +436,18 @@ __global__ __launch_bounds__(64 * W, W == 16 || (NTB <= 2 && NTM <= 2) ? 4 : W =
             store_row<T, DT, kTile>(S.Y, j0 + c.r < B ? static_cast<unsigned>((j0 + c.r) * M + idx) * db : kOob, P.D, O, c.q);
         }
         if (!more) break;
-        if (ph != phase) __syncthreads();   // the next phase reads what this one wrote, transposed
+        if (ph != phase) {
+            __syncthreads();   // the next phase reads what this one wrote, transposed
+            if (KEEP) {
+                keep_sums(phase);
+                if (phase & 1) at_step(ph / 2);
+            }
+        }
     }
     // Y is read back by other waves of this workgroup: past the L1, behind the stores' acknowledgement
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+    if (KEEP) keep_sums(last);
     for (int jj = c.wave; jj < 16 && j0 + jj < B; jj += W) {
         const int j = j0 + jj;
         SL::issue(c, tile, S.Y, db, j * M, 1, M, np);

@@ -18,6 +18,11 @@ CASES = [  # E, H, N, D, B, T, pre, dtype, variant, masked: rows per slot that d
     (1, 2, 256, 48, 16, 2, False, "f32", None, True),
     (1, 2, 45, 20, 8, 2, True, "f16", "generic", False),
     (1, 9, 512, 64, 32, 2, False, "f16", "resident", False),  # keeps nothing: the backward runs the steps again
+    # calls that the slice-resident kernel records (its strips both ways, waves and column classes; masked, padded, one step to three)
+    (16, 12, 512, 64, 32, 2, True, "bf16", None, True), (48, 16, 197, 64, 14, 3, True, "f16", None, False), (24, 16, 256, 64, 16, 1, False, "bf16", None, True),
+    (13, 1, 60, 32, 19, 3, False, "f16", None, True), (50, 1, 21, 80, 9, 3, True, "bf16", None, False), (13, 1, 81, 48, 24, 3, True, "f16", None, True),
+    (67, 7, 53, 72, 7, 3, False, "f16", None, True), (66, 1, 1265, 32, 38, 3, True, "bf16", None, False), (79, 1, 2570, 32, 48, 2, False, "bf16", None, True),
+    (122, 1, 548, 64, 23, 3, False, "f16", None, True), (26, 1, 221, 32, 56, 3, True, "f16", None, True), (39, 13, 542, 32, 12, 3, True, "bf16", None, True),
 ]
 
 
