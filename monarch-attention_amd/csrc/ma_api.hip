@@ -182,6 +182,17 @@ int run_slice(const Problem& P, int dtype_qk, SlicePlan* plan, hipStream_t s) {
     return MA_ERR_UNSUPPORTED;
 }
 
+int run_matrix_slice(const Problem& P, int dtype_qk, float* A, hipStream_t s) {
+    const bool h = dtype_qk == MA_F16;
+    const int D = P.D;
+    if (D <= 32) return h ? launch_matrix_slice_f16_d2(P, A, s) : launch_matrix_slice_bf16_d2(P, A, s);
+    if (D <= 48) return h ? launch_matrix_slice_f16_d3(P, A, s) : launch_matrix_slice_bf16_d3(P, A, s);
+    if (D <= 64) return h ? launch_matrix_slice_f16_d4(P, A, s) : launch_matrix_slice_bf16_d4(P, A, s);
+    if (D <= 80) return h ? launch_matrix_slice_f16_d5(P, A, s) : launch_matrix_slice_bf16_d5(P, A, s);
+    if (D <= 96) return h ? launch_matrix_slice_f16_d6(P, A, s) : launch_matrix_slice_bf16_d6(P, A, s);
+    return h ? launch_matrix_slice_f16_d8(P, A, s) : launch_matrix_slice_bf16_d8(P, A, s);
+}
+
 int run_resident(const Problem& P, int dtype_qk, bool dry_run, hipStream_t s) {
     if (dtype_qk == MA_F32) return launch_head32(P, dry_run, s);
     const bool h = dtype_qk == MA_F16;
@@ -743,6 +754,21 @@ int run_steps_kept(Prepared& pr, const ma_fwd_params* p, const StateLayout& S, c
     return MA_OK;
 }
 
+// AUTO, dense matrix of 16-bit operands: is the one launch of ma_matrix_slice.h ahead of the 2 T stage launches?  1388 random problems of up to 32
+// blocks of up to 32 rows, 1 .. 200 heads, in multiples of the stage launches' time, the host's part of the call with it.  Up to 16
+// blocks: 0.74 at T = 1 (at most 1.08), 0.51 at T = 2, 0.45 at T = 3.  17 .. 32 blocks, where a wave has two blocks and an L problem four tiles:
+// D <= 80 0.77 and 0.72 at T = 2, 3 (beyond 128 heads up to 1.14); a single step 0.92 (0.75 .. 1.24) below 16 heads, 0.73 - 0.93 from there, 1.12 (up
+// to 1.57) beyond 128; D > 80, in eight waves, 0.95 (0.77 .. 1.2) below 8 heads, 0.80 above, at T = 1 1.18, 0.98 and, from 64 heads on, 0.86.  12
+// heads of 1024 tokens in 32-row blocks, T = 2: 25.1 -> 21.9 us.
+bool matrix_slice_pays(const ma_fwd_params* p) {
+    const int M = (p->N + p->B - 1) / p->B;
+    const long long heads = static_cast<long long>(p->E) * p->H;
+    if (p->B > 32 || M > 32 || !mfma_supported(p)) return false;
+    if (M <= 16) return true;
+    if (p->T == 1) return heads >= (p->D > 80 ? 64 : 16) && heads <= 128;
+    return heads >= (p->D > 80 ? 8 : 1);
+}
+
 // Workspace of the dense matrix with the probabilities of the last R step: rows of B floats, rounded up to four.
 uint64_t matrix_workspace(const ma_fwd_params* p) {
     ma_ws_layout L;
@@ -1197,6 +1223,7 @@ int ma_matrix(const ma_fwd_params* p, float* A, void* stream) {
     if (pp.H > 1 && pp.out_stride[1] == 0) pp.out_stride[1] = 1;   // output must pass the overlap check
     if (pp.variant != MA_VARIANT_AUTO && pp.variant != MA_VARIANT_GENERIC && pp.variant != MA_VARIANT_STAGED)
         return pp.variant < MA_VARIANT_AUTO || pp.variant > MA_VARIANT_SLICED ? MA_ERR_VARIANT : MA_ERR_UNSUPPORTED;
+    const bool choose = pp.variant == MA_VARIANT_AUTO;
     if (pp.variant == MA_VARIANT_AUTO) {
         const int st = check_shape(&pp);
         if (st != MA_OK) return st;
@@ -1211,6 +1238,7 @@ int ma_matrix(const ma_fwd_params* p, float* A, void* stream) {
     const bool tiled = pr.variant == MA_VARIANT_STAGED && pp.workspace_bytes >= matrix_workspace(&pp);
     if (!tiled && !generic_matrix_fits(pr.P)) return MA_ERR_UNSUPPORTED;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (choose && matrix_slice_pays(&pp) && run_matrix_slice(pr.P, pp.dtype_qk, nullptr, s) == MA_OK) return run_matrix_slice(pr.P, pp.dtype_qk, A, s);
     for (int t = 0; t < pp.T - 1; ++t) {
         st = run_r(pr, &pp, t == 0, false, s);
         if (st) return st;

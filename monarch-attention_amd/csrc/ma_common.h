@@ -242,6 +242,20 @@ int launch_matrix_f32_d5(const Problem& P, bool first, float* Rp, float* A, hipS
 int launch_matrix_f32_d6(const Problem& P, bool first, float* Rp, float* A, hipStream_t s);
 int launch_matrix_f32_d8(const Problem& P, bool first, float* Rp, float* A, hipStream_t s);
 int launch_matrix(const Problem& P, int dt, bool first, float* Rp, float* A, hipStream_t s);
+// The matrix of short sequences in one launch (ma_matrix_slice.h): D = 32, 40, 48, 64, 72, 80, 96, 128,
+// B, M <= 32.  A == nullptr: only report whether the problem fits.
+int launch_matrix_slice_bf16_d2(const Problem& P, float* A, hipStream_t s);
+int launch_matrix_slice_bf16_d3(const Problem& P, float* A, hipStream_t s);
+int launch_matrix_slice_bf16_d4(const Problem& P, float* A, hipStream_t s);
+int launch_matrix_slice_bf16_d5(const Problem& P, float* A, hipStream_t s);
+int launch_matrix_slice_bf16_d6(const Problem& P, float* A, hipStream_t s);
+int launch_matrix_slice_bf16_d8(const Problem& P, float* A, hipStream_t s);
+int launch_matrix_slice_f16_d2(const Problem& P, float* A, hipStream_t s);
+int launch_matrix_slice_f16_d3(const Problem& P, float* A, hipStream_t s);
+int launch_matrix_slice_f16_d4(const Problem& P, float* A, hipStream_t s);
+int launch_matrix_slice_f16_d5(const Problem& P, float* A, hipStream_t s);
+int launch_matrix_slice_f16_d6(const Problem& P, float* A, hipStream_t s);
+int launch_matrix_slice_f16_d8(const Problem& P, float* A, hipStream_t s);
 
 // Fused forward (one launch), by dtype and head-dim class (D <= 32/64/80/128).
 // sync_ready: the workspace's sync area is known to be zero.

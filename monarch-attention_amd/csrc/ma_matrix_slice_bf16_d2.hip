@@ -1,0 +1,6 @@
+// Dense matrix of short sequences in one launch, bf16 operands, head-dim class 2 (see ma_matrix_slice.h).
+#include "ma_matrix_slice.h"
+
+namespace ma {
+int launch_matrix_slice_bf16_d2(const Problem& P, float* A, hipStream_t s) { return mfma::launch_matrix_slice<bf16, 2>(P, A, s); }
+}  // namespace ma

@@ -34,9 +34,13 @@
 namespace ma {
 namespace mfma {
 
-// KEEP: every step's aL, cL, aR, cR also go to memory (Problem::slot_rows, ma_fwd_keep); `cl` holds cL itself for that.
-template <class T, int DT, int NTB, int NTM, int W, bool KEEP>
+// MODE kKeepSteps: every step's aL, cL, aR, cR also go to memory (Problem::slot_rows, ma_fwd_keep); `cl` holds cL itself for that.
+// kMatrix (ma_matrix_slice.h): a workgroup has `pos` <= 16 positions, the last R step leaves its probabilities in `rp`, [jj][m][i] with rows
+// of up4(B) floats, and there is no V, Y or Z.
+enum { kForward = 0, kKeepSteps = 1, kMatrix = 2 };
+template <class T, int DT, int NTB, int NTM, int W, int MODE>
 struct Slice {
+    static constexpr bool KEEP = MODE == kKeepSteps, MATRIX = MODE == kMatrix;
     using V8 = typename Ops<T>::v8;
     using V4 = typename Ops<T>::v4;
     static constexpr int KS = DT / 2, CH = 2 * DT;   // whole 32-column steps, 16-byte pieces of a full row
@@ -51,17 +55,17 @@ struct Slice {
         u32x4 v[NI];
     };
     struct Layout {
-        unsigned S, St, tile, cb, cR, tokb, cs, cl, ZR, trash, total, P, BP;
+        unsigned S, St, tile, cb, cR, tokb, cs, cl, rp, ZR, trash, total, P, BP;
     };
     // Rows an odd number of 16-byte units apart, blocks of the state 16 bytes more than their rows: neither the 16 rows of a block
     // nor the rows of 16 blocks at one position start in the same LDS banks.  (So it is for the reads of rows; the transposed reads of
     // gemm2 conflict at this pitch: 46 % of the LDS cycles of 128 heads of 1024, D = 72.)
-    static constexpr __host__ __device__ Layout layout(int D, int M) {
+    static constexpr __host__ __device__ Layout layout(int D, int M, int pos = 16, int B = 0) {
         Layout L{};
         L.P = 16u * ((static_cast<unsigned>(D) / 8u) | 1u);
-        L.BP = 16u * L.P + 16u;
+        L.BP = MATRIX ? 16u * ((static_cast<unsigned>(pos) * L.P / 16u) | 1u) : 16u * L.P + 16u;
         unsigned o = 0;
-        L.S = o; o += static_cast<unsigned>(M) * L.BP;
+        L.S = o; o += static_cast<unsigned>(M) * L.BP + (MATRIX ? 16u * L.P : 0u);   // (lanes without a position read on)
         L.tile = ROWS * L.P;
         L.St = o; o += W * L.tile;
         L.ZR = o; o += (L.P + 64u) / 16u * 16u;   // (the last operand step of a tile's or the state's last row reads on for up to 16 bytes)
@@ -70,6 +74,7 @@ struct Slice {
         L.tokb = o; o += static_cast<unsigned>(M) * ROWSB * 4;
         L.cs = o; o += W * ROWSM * 8;
         L.cl = o; o += KEEP ? 16 * ROWSM * 4 : 0;
+        L.rp = o; o += MATRIX ? static_cast<unsigned>(pos) * M * ((B + 3) / 4 * 16) : 0;
         L.trash = o; o += 64 * 16;
         L.total = o;
         return L;
@@ -82,7 +87,7 @@ struct Slice {
     struct Ctx {
         char* smem;
         Layout L;
-        int wave, lane, r, q, D, j0;
+        int wave, lane, r, q, D, j0, pos;
         rsrc_t aL, aR;    // KEEP: this head's rows of the step at hand
         unsigned St;      // this wave's tile
         unsigned tr, sr;  // the lane's row r of it, and of the state's position 0 at block r
@@ -91,7 +96,7 @@ struct Slice {
         __device__ __forceinline__ U* at(unsigned off) const { return reinterpret_cast<U*>(smem + off); }
     };
 
-    static_assert(ROWS * CH <= 640, "row_of");
+    static_assert(CH % 4 == 0 || ROWS * CH <= 640, "row_of");
     static __device__ __forceinline__ int row_of(int piece) { return CH % 4 == 0 ? piece / CH : CH == 10 ? (piece * 205) >> 11 : (piece * 171) >> 10; }
     // ---- tiles: rows of `st` bytes at tokens a + b * row (row < limit, 0 <= token < n), the rest reads as zeros
     // (The place of a piece is worked out each time: kept, the places of all pieces would take the registers of a tile.)
@@ -169,7 +174,8 @@ struct Slice {
     }
 
     // ---- R problem of block m, first half (al_cl_ref, ma/ma_torch.py:10-23): K in the wave's tile, aR rows in S
-    static __device__ __forceinline__ void r_keys(const Problem& P, const Ctx& c, int m, bool first, const Row& x0, V8 (&pb)[(NTB + 1) / 2]) {
+    static __device__ __forceinline__ void r_keys(const Problem& P, const Ctx& c, int m, bool first, const Row& x0, V8 (&pb)[(NTB + 1) / 2],
+                                                  bool probabilities = false) {
         const unsigned srow = c.L.S + m * c.L.BP + (c.tr - c.St);
         Row x;
         if (first) x = x0;
@@ -212,6 +218,13 @@ struct Slice {
             c.template at<float>(c.L.cb)[c.r * ROWSM + m] = -kLog2e * cl;
             if (KEEP) c.template at<float>(c.L.cl)[c.r * ROWSM + m] = cl;
         }
+        if (MATRIX && probabilities && c.r < c.pos) {
+            const int pitch = (P.B + 3) & ~3;
+            float* rp = c.template at<float>(c.L.rp) + (c.r * P.M + m) * pitch;
+#pragma unroll
+            for (int w = 0; w < NTB; ++w)
+                if (16 * w + 4 * c.q < pitch) *reinterpret_cast<f32x4*>(rp + 16 * w + 4 * c.q) = C[w];
+        }
         pack_p<T, NTB>(pb, C);
         f32x4 O[DT];
         gemm2<NTB>(c, O, pb);
@@ -219,7 +232,7 @@ struct Slice {
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int v = 0; v < 4; ++v) O[dt][v] = P.sm_scale * round_to<T>(O[dt][v]);
-        put_row(c, srow, O);
+        if (!MATRIX || c.r < c.pos) put_row(c, srow, O);
         if (KEEP) store_row<T, DT, kTile>(c.aL, c.j0 + c.r < P.B ? static_cast<unsigned>((c.j0 + c.r) * P.M + m) * (2u * c.D) : kOob, c.D, O, c.q);
     }
 
@@ -336,9 +349,10 @@ struct Slice {
 // heads that follow each other: rows that are no whole lines share them with the next head's where a token's heads lie side by side
 // (128 heads of 1024, D = 72, T = 3, (E, N, H, D): 312 -> 188 MB of traffic, 53.2 -> 46.4 us; D = 80, T = 1 31.7 -> 28.4; D = 64 unchanged).
 // 128 registers where two workgroups of 8 waves or one of 16 share a compute unit, else 256.
-template <class T, int DT, int NTB, int NTM, int W, bool KEEP>
+template <class T, int DT, int NTB, int NTM, int W, int MODE>
 __global__ __launch_bounds__(64 * W, W == 16 || (NTB <= 2 && NTM <= 2) ? 4 : W == 12 ? 3 : 2) void resident_slice_mfma(Problem P) {
-    using SL = Slice<T, DT, NTB, NTM, W, KEEP>;
+    using SL = Slice<T, DT, NTB, NTM, W, MODE>;
+    constexpr bool KEEP = SL::KEEP;
     using Row = typename SL::Row;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int B = P.B, M = P.M, heads = P.E * P.H, slices = (B + 15) / 16;

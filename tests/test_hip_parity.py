@@ -850,6 +850,36 @@ def test_matrix_kernel_equals_forward_on_identity(case):
     assert sync_status() == 0
 
 
+MATRIX_SHORT = [  # E, H, N, D, B, T, pre, dt, masked: one launch; strips of 1 and 2 both ways, their edges, every column class
+    (1, 1, 1, 32, 1, 2, False, "f16", False), (1, 2, 16, 64, 1, 1, False, "bf16", True), (1, 3, 45, 40, 3, 3, True, "f16", True),
+    (1, 2, 255, 64, 16, 2, True, "bf16", True), (2, 3, 272, 48, 17, 2, False, "f16", True), (1, 2, 512, 72, 32, 3, True, "f16", False),
+    (1, 1, 289, 80, 17, 2, False, "bf16", True), (1, 12, 1024, 64, 32, 2, False, "f16", False), (3, 3, 500, 96, 16, 2, True, "bf16", True),
+    (1, 2, 200, 128, 13, 3, True, "f16", True), (2, 5, 527, 128, 31, 2, False, "bf16", False),
+    # one step of 17 .. 32 blocks, heads that stay on one XCD (32 and more), several positions to a workgroup, two passes
+    (4, 4, 270, 64, 10, 1, False, "f16", True), (5, 7, 196, 32, 28, 2, True, "bf16", True), (13, 11, 120, 64, 19, 1, False, "f16", True),
+]
+
+
+@pytest.mark.parametrize("case", MATRIX_SHORT, ids=lambda c: "-".join(map(str, c)))
+def test_matrix_of_short_sequences(case):
+    """AUTO writes the matrix of short 16-bit sequences in one launch: against the oracle, on (E, N, H, D) views, twice bit for bit, every
+    entry written (the buffer that the allocator hands out held NaN before), and through the module."""
+    E, H, N, D, B, T, pre, dt, masked = case
+    q, k, _ = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in seeded_qkv(E, H, N, D, DT[dt]))
+    mask = block_safe_mask(E, N, B, seed=N) if masked else None
+    dq, dk, dm = to_dev(q, k, mask)
+    junk = torch.full((E, H, N, N), float("nan"), device=DEV)
+    del junk
+    A = monarch_matrix_hip(dq, dk, dm, T, B, pre)
+    heads = slice(0, 2)
+    assert_parity(A[:1, heads].cpu(), monarch_matrix_oracle(q[:1, heads], k[:1, heads], None if mask is None else mask[:1], T, B, pre), dt)
+    assert_parity(A[-1:, -1:].cpu(), monarch_matrix_oracle(q[-1:, -1:], k[-1:, -1:], None if mask is None else mask[-1:], T, B, pre), dt)
+    assert torch.isfinite(A).all()
+    assert torch.equal(A, MonarchAttention(B, T, "pre" if pre else "post").get_matrix(dq, dk, dm))
+    staged = monarch_matrix_hip(dq, dk, dm, T, B, pre, variant="staged")
+    assert ((A - staged).norm() / staged.norm()).item() <= 1e-5   # the same roundings; fp32 sums in another order
+
+
 @pytest.mark.parametrize("name", ["matrix_f16_eye32", "matrix_f32_eye_ragged"])
 def test_matrix_kernel_golden_vectors(name):
     g = load_golden(name)
