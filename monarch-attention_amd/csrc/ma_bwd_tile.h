@@ -72,9 +72,23 @@ __device__ __forceinline__ f32x4 lds4(const float* p) { return *reinterpret_cast
 
 // ---------------------------------------------------------------- R stage
 // kV: the last step's stage, the first of a backward pass (Y and dv)
-// (Two strips of up to 64 columns: five waves a SIMD as long as a wave keeps to 96 registers, which the compiler else misses by two.)
+// Waves a SIMD that the 16-bit kernels of one launch are held to.  A workgroup waits for its rows, computes and writes, with barriers
+// between, and what fills the gaps is another workgroup of the compute unit; one of n strips takes n of its 4 times 512 / registers
+// wave slots.  Left to itself the compiler passes the next step of that ladder by a few registers in the classes below, most of which
+// then ran one workgroup at a time.  Their spills (none to 24 words, out of the loops) cost less.  us of a stage over 14 million
+// elements of q, bf16, free -> held, with V / without:
+//   up to 64 columns: 4 strips 54.2 / 45.6 -> 52.5 / 45.8, 5 strips 92.4 / 59.3 -> 73.6 / 60.5, 6 strips 94.1 / 76.7 -> 88.4 / 67.9
+//   up to 96: 3 strips 67.9 / 61.7 -> 67.2 / 59.6, 4 strips 72.1 / 58.4 -> 68.2 / 58.2, 5 strips 123.6 / 100.7 -> 118.2 / 83.3,
+//             6 strips 89.3 / 68.3 -> 85.4 / (held: 68.9)
+//   up to 128: 3 strips 87.4 / 62.6 -> 55.9 / 48.9, 4 strips 50.9 / 40.7 -> 47.8 / 40.8, 5 strips (V held: 86.2) 77.9 / 68.4 -> - / 62.0
+// Seven and eight strips of up to 64 columns need 155 to 177 registers: held to 128 they spill 100 - 200 bytes and take 1.1 to 1.3 times as long.
+constexpr int r_held_waves(int DT, int NWT, bool kV) {
+    if (DT <= 4) return NWT == 2 ? 5 : 4 <= NWT && NWT <= 6 ? 4 : 1;
+    if (DT <= 6) return NWT == 5 ? 4 : NWT == 3 || NWT == 4 || (NWT == 6 && kV) ? 3 : 1;
+    return NWT == 5 && !kV ? 4 : NWT == 3 || NWT == 4 ? 3 : 1;
+}
 template <class T, int DT, int NWT, int W, int PASS, bool kV>
-__global__ __launch_bounds__(64 * W, sizeof(T) == 2 && DT <= 4 && NWT == 2 && PASS == 0 ? 5 : 1) void r_bwd_tile(Problem P, BwdBuffers G, int first) {
+__global__ __launch_bounds__(64 * W, sizeof(T) == 2 && PASS == 0 ? r_held_waves(DT, NWT, kV) : 1) void r_bwd_tile(Problem P, BwdBuffers G, int first) {
     using MT = Mat<T, DT>;
     using PL = RPlan<T, DT, NWT, PASS, kV>;
     using mfma::quad_rows_max;
@@ -392,13 +406,15 @@ __global__ __launch_bounds__(64 * W, sizeof(T) == 2 && DT <= 4 && NWT == 2 && PA
 }
 
 // ---------------------------------------------------------------- L and Z stages
-// Waves a SIMD that the 16-bit kernels of one launch are held to, in the classes where a few registers would cost one.  (Eight strips of
-// up to 64 columns: two workgroups of eight waves share a compute unit as long as a wave keeps to 128 registers.  The L stage of 32 heads
-// of 8192 tokens takes 66 us at 128 and 87 above.)
+// As r_held_waves.  (Eight strips of up to 64 columns: two workgroups of eight waves share a compute unit as long as a wave keeps to 128
+// registers.  The L stage of 32 heads of 8192 tokens takes 66 us at 128 and 87 above.)  us over 14 million elements, bf16, free -> held:
+// up to 64 columns Z of 5 strips 57.7 -> 48.9; up to 96 L of 4 strips 61.5 -> 59.7, 7 strips 93.2 -> 86.2, 8 strips 63.3 -> 54.4 (Z of
+// 4 strips, fp16: 48.6 -> 50.8, left free); up to 128 Z of 3 strips 53.5 -> 46.1, 4 strips 44.9 -> 39.6, L of 5 strips 65.3 -> 58.3.
 constexpr int lz_held_waves(int DT, int NWT, bool kZ) {
-    if (DT <= 4) return NWT == 8 ? 4 : kZ && NWT == 6 ? 5 : 1;
-    if (DT <= 6) return kZ && NWT == 8 ? 4 : 1;
-    return !kZ && NWT == 4 ? 4 : NWT == (kZ ? 6 : 5) ? 3 : 1;
+    if (DT <= 4) return NWT == 8 || (kZ && NWT == 5) ? 4 : kZ && NWT == 6 ? 5 : 1;
+    if (DT <= 6) return NWT == 8 || (!kZ && NWT == 7) ? 4 : !kZ && NWT == 4 ? 3 : 1;
+    if (kZ) return NWT == 3 || NWT == 4 || NWT == 6 ? 3 : 1;
+    return NWT == 4 || NWT == 5 ? 4 : 1;
 }
 template <class T, int DT, int NWT, int W, int PASS, bool kZ>
 __global__ __launch_bounds__(64 * W, sizeof(T) == 2 && PASS == 0 ? lz_held_waves(DT, NWT, kZ) : 1) void lz_bwd_tile(Problem P, BwdBuffers G) {
