@@ -81,10 +81,13 @@ __device__ __forceinline__ f32x4 lds4(const float* p) { return *reinterpret_cast
 //   up to 96: 3 strips 67.9 / 61.7 -> 67.2 / 59.6, 4 strips 72.1 / 58.4 -> 68.2 / 58.2, 5 strips 123.6 / 100.7 -> 118.2 / 83.3,
 //             6 strips 89.3 / 68.3 -> 85.4 / (held: 68.9)
 //   up to 128: 3 strips 87.4 / 62.6 -> 55.9 / 48.9, 4 strips 50.9 / 40.7 -> 47.8 / 40.8, 5 strips (V held: 86.2) 77.9 / 68.4 -> - / 62.0
-// Seven and eight strips of up to 64 columns need 155 to 177 registers: held to 128 they spill 100 - 200 bytes and take 1.1 to 1.3 times as long.
+// and, since the row sums have no branch (see there), which took up to 64 registers more,
+//   up to 32 columns: 7 strips 146 / 116 -> 111 / 92, up to 48: 142 / 115 -> 123 / 89 (8 strips 113 / 88 -> 102 / 70)
+//   up to 64: 7 strips 87.8 / 70.0 -> 80.3 / 59.8, 8 strips 57.8 / 43.1 -> 58.1 / 39.4 (7.9 million elements)
+//   up to 96: 7 strips (V held: 165) 105 / 84.0 -> - / 79.0, 8 strips held: 96.5 / 67.9 for 80.8 / 65.6
 constexpr int r_held_waves(int DT, int NWT, bool kV) {
-    if (DT <= 4) return NWT == 2 ? 5 : 4 <= NWT && NWT <= 6 ? 4 : 1;
-    if (DT <= 6) return NWT == 5 ? 4 : NWT == 3 || NWT == 4 || (NWT == 6 && kV) ? 3 : 1;
+    if (DT <= 4) return NWT == 2 ? (DT == 4 ? 5 : 1) : NWT >= 4 ? 4 : 1;
+    if (DT <= 6) return (NWT == 5 && (DT == 6 || kV)) || (NWT == 7 && !kV) ? 4 : NWT == 3 || NWT == 4 || (NWT == 6 && kV) ? 3 : 1;
     return NWT == 5 && !kV ? 4 : NWT == 3 || NWT == 4 ? 3 : 1;
 }
 template <class T, int DT, int NWT, int W, int PASS, bool kV>
@@ -204,25 +207,25 @@ __global__ __launch_bounds__(64 * W, sizeof(T) == 2 && PASS == 0 ? r_held_waves(
             for (int v = 0; v < 4; ++v) mx = __builtin_elementwise_maximum(mx, S[w][v]);
         mx = fmaxf(quad_rows_max(mx) * scale, P.eps * kLog2e);
         float sum = 0.f, hs = 0.f, es = 0.f, ehs = 0.f;   // of e, e h, e d, e h d
-        auto sums = [&](auto with_gcr) {   // (S becomes e and Gg h; fp32 keeps S and forms e again)
+        // (S becomes e and Gg h; fp32 keeps S and forms e again.  No branch on `first`, which has no use for the last two sums: across
+        // its two sides the strip's 8 NWT values were held twice)
 #pragma unroll
-            for (int w = 0; w < NWT; ++w)
+        for (int w = 0; w < NWT; ++w) {
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const float d = fmaxf(fmaf(S[w][v], scale, -mx), kFloor), e = __builtin_amdgcn_exp2f(d);
-                    const float h = fmaf(gl, d, Gg[w][v]), eh = e * h;
-                    sum += e;
-                    hs += eh;
-                    if (!kF32 && decltype(with_gcr)::value) {
-                        es = fmaf(e, d, es);
-                        ehs = fmaf(eh, d, ehs);
-                    }
-                    if (!kF32) S[w][v] = e;
-                    Gg[w][v] = h;
+            for (int v = 0; v < 4; ++v) {
+                const float d = fmaxf(fmaf(S[w][v], scale, -mx), kFloor), e = __builtin_amdgcn_exp2f(d);
+                const float h = fmaf(gl, d, Gg[w][v]), eh = e * h;
+                sum += e;
+                hs += eh;
+                if (!kF32) {
+                    es = fmaf(e, d, es);
+                    ehs = fmaf(eh, d, ehs);
+                    S[w][v] = e;
                 }
-        };
-        if (first) sums(std::false_type{});
-        else sums(std::true_type{});
+                Gg[w][v] = h;
+            }
+            if (NWT > 4 && DT != 5) __builtin_amdgcn_sched_barrier(0);   // (registers)
+        }
         sum = quad_rows_sum(sum);
         const float inv = mfma::rcp(sum + P.eps), lg = mfma::log2_normal(inv), k1 = gcl * fmaf(mfma::kLn2, lg, 1.f);
         const float dot = inv * quad_rows_sum(hs), ctr = dot - k1 * (P.eps * inv);
@@ -408,10 +411,13 @@ __global__ __launch_bounds__(64 * W, sizeof(T) == 2 && PASS == 0 ? r_held_waves(
 // ---------------------------------------------------------------- L and Z stages
 // As r_held_waves.  (Eight strips of up to 64 columns: two workgroups of eight waves share a compute unit as long as a wave keeps to 128
 // registers.  The L stage of 32 heads of 8192 tokens takes 66 us at 128 and 87 above.)  us over 14 million elements, bf16, free -> held:
-// up to 64 columns Z of 5 strips 57.7 -> 48.9; up to 96 L of 4 strips 61.5 -> 59.7, 7 strips 93.2 -> 86.2, 8 strips 63.3 -> 54.4 (Z of
-// 4 strips, fp16: 48.6 -> 50.8, left free); up to 128 Z of 3 strips 53.5 -> 46.1, 4 strips 44.9 -> 39.6, L of 5 strips 65.3 -> 58.3.
+// up to 64 columns Z of 5 strips 57.7 -> 48.9 (up to 48 columns 7 strips 83.7 -> 70.4, up to 64 59.3 -> 62); up to 80 Z of 5 strips
+// 80.7 -> 65.2, 6 strips 59.4 -> 51.3 (7: 85.8 -> 96.3, free); up to 96 L of 4 strips 61.5 -> 59.7, 7 strips 93.2 -> 86.2, 8 strips
+// 63.3 -> 54.4 (Z of 4 strips, fp16: 48.6 -> 50.8, free); up to 128 Z of 3 strips 53.5 -> 46.1, 4 strips 44.9 -> 39.6, L of 5 strips
+// 65.3 -> 58.3.
 constexpr int lz_held_waves(int DT, int NWT, bool kZ) {
-    if (DT <= 4) return NWT == 8 || (kZ && NWT == 5) ? 4 : kZ && NWT == 6 ? 5 : 1;
+    if (DT <= 4) return NWT == 8 || (kZ && (NWT == 5 || (DT == 3 && NWT == 7))) ? 4 : kZ && NWT == 6 ? 5 : 1;
+    if (DT == 5) return NWT == 8 || (kZ ? NWT == 5 || NWT == 6 : NWT == 7) ? 4 : !kZ && NWT == 4 ? 3 : 1;
     if (DT <= 6) return NWT == 8 || (!kZ && NWT == 7) ? 4 : !kZ && NWT == 4 ? 3 : 1;
     if (kZ) return NWT == 3 || NWT == 4 || NWT == 6 ? 3 : 1;
     return NWT == 4 || NWT == 5 ? 4 : 1;
