@@ -155,10 +155,16 @@ struct BwdBuffers {
     long long outs[3][3];
 };
 // one file per dtype and head-dim class (ma_bwd_tile_*.hip); B, M <= 256, D % 4 == 0, D <= 16 x the class
+int launch_bwd_tile_bf16_d2(const Problem& P, const BwdBuffers& G, int stage, bool first, bool with_v, hipStream_t s);
+int launch_bwd_tile_bf16_d3(const Problem& P, const BwdBuffers& G, int stage, bool first, bool with_v, hipStream_t s);
 int launch_bwd_tile_bf16_d4(const Problem& P, const BwdBuffers& G, int stage, bool first, bool with_v, hipStream_t s);
+int launch_bwd_tile_bf16_d5(const Problem& P, const BwdBuffers& G, int stage, bool first, bool with_v, hipStream_t s);
 int launch_bwd_tile_bf16_d6(const Problem& P, const BwdBuffers& G, int stage, bool first, bool with_v, hipStream_t s);
 int launch_bwd_tile_bf16_d8(const Problem& P, const BwdBuffers& G, int stage, bool first, bool with_v, hipStream_t s);
+int launch_bwd_tile_f16_d2(const Problem& P, const BwdBuffers& G, int stage, bool first, bool with_v, hipStream_t s);
+int launch_bwd_tile_f16_d3(const Problem& P, const BwdBuffers& G, int stage, bool first, bool with_v, hipStream_t s);
 int launch_bwd_tile_f16_d4(const Problem& P, const BwdBuffers& G, int stage, bool first, bool with_v, hipStream_t s);
+int launch_bwd_tile_f16_d5(const Problem& P, const BwdBuffers& G, int stage, bool first, bool with_v, hipStream_t s);
 int launch_bwd_tile_f16_d6(const Problem& P, const BwdBuffers& G, int stage, bool first, bool with_v, hipStream_t s);
 int launch_bwd_tile_f16_d8(const Problem& P, const BwdBuffers& G, int stage, bool first, bool with_v, hipStream_t s);
 int launch_bwd_tile_f32_d2(const Problem& P, const BwdBuffers& G, int stage, bool first, bool with_v, hipStream_t s);

@@ -11,8 +11,21 @@ int launch_bwd_tile(const Problem& P, const BwdBuffers& G, int dt, int stage, bo
                   : D <= 80 ? launch_bwd_tile_f32_d5 : D <= 96 ? launch_bwd_tile_f32_d6 : launch_bwd_tile_f32_d8;
         return f(P, G, stage, first, with_v, s);
     }
-    auto* f = dt == MA_F16 ? (D <= 64 ? launch_bwd_tile_f16_d4 : D <= 96 ? launch_bwd_tile_f16_d6 : launch_bwd_tile_f16_d8)
-                           : (D <= 64 ? launch_bwd_tile_bf16_d4 : D <= 96 ? launch_bwd_tile_bf16_d6 : launch_bwd_tile_bf16_d8);
+    // 16 bit: memory and registers bound it.  A class of their own saves operands of 17 .. 32 columns half of the tiles (backward of T = 2
+    // over 14 million elements of 92-row blocks 422 -> 304 us, 44-row blocks 267 -> 221), of 33 .. 48 and 65 .. 80 a sixth to a quarter of
+    // the accumulators (108-row blocks 375 -> 329 and 211 -> 200).  Up to 16 columns half of a 32-column tile is padding: not worth one.
+    auto* f = dt == MA_F16 ? (D <= 32   ? launch_bwd_tile_f16_d2
+                              : D <= 48 ? launch_bwd_tile_f16_d3
+                              : D <= 64 ? launch_bwd_tile_f16_d4
+                              : D <= 80 ? launch_bwd_tile_f16_d5
+                              : D <= 96 ? launch_bwd_tile_f16_d6
+                                        : launch_bwd_tile_f16_d8)
+                           : (D <= 32   ? launch_bwd_tile_bf16_d2
+                              : D <= 48 ? launch_bwd_tile_bf16_d3
+                              : D <= 64 ? launch_bwd_tile_bf16_d4
+                              : D <= 80 ? launch_bwd_tile_bf16_d5
+                              : D <= 96 ? launch_bwd_tile_bf16_d6
+                                        : launch_bwd_tile_bf16_d8);
     return f(P, G, stage, first, with_v, s);
 }
 
