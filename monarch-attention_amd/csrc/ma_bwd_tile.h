@@ -48,10 +48,17 @@ namespace bwdt {
 
 using namespace tile;
 
+// The second launch of 16 strips of 16-bit operands, eight of them per workgroup: two workgroups share a compute unit where the tiles are
+// walked in chunks of half of the LDS and a wave keeps to 128 registers (held to them from 65 columns on; narrower classes need fewer).  The stages that form two gradients of more than 80 columns do
+// not (150 to 250 registers): they take the LDS whole, see RSplit.
+template <class T>
+constexpr bool shares_lds(int DT, int NWT, int PASS, bool two_gradients) {
+    return sizeof(T) == 2 && NWT == 16 && PASS == 2 && !(two_gradients && DT >= 6);
+}
 template <class T, int DT, int NWT, int PASS, bool kV>
-using RPlan = Plan<T, DT, NWT, PASS, kV ? 2 : 1, kV ? 3 : 2, 7>;
+using RPlan = Plan<T, DT, NWT, PASS, kV ? 2 : 1, kV ? 3 : 2, 7, shares_lds<T>(DT, NWT, PASS, kV)>;
 template <class T, int DT, int NWT, int PASS, bool kZ>
-using LzPlan = Plan<T, DT, NWT, PASS, 2, kZ ? 2 : 1, 5>;
+using LzPlan = Plan<T, DT, NWT, PASS, 2, kZ ? 2 : 1, 5, shares_lds<T>(DT, NWT, PASS, kZ)>;
 
 // A term that a product's sum is shifted by: 16-bit operands start the accumulators at it; fp32 sums, which would then be rounded
 // at its magnitude in every step, take it at the end.
@@ -86,12 +93,12 @@ __device__ __forceinline__ f32x4 lds4(const float* p) { return *reinterpret_cast
 //   up to 64: 7 strips 87.8 / 70.0 -> 80.3 / 59.8, 8 strips 57.8 / 43.1 -> 58.1 / 39.4 (7.9 million elements)
 //   up to 96: 7 strips (V held: 165) 105 / 84.0 -> - / 79.0, 8 strips held: 96.5 / 67.9 for 80.8 / 65.6
 constexpr int r_held_waves(int DT, int NWT, bool kV) {
-    if (DT <= 4) return NWT == 2 ? (DT == 4 ? 5 : 1) : NWT >= 4 ? 4 : 1;
+    if (DT <= 4) return NWT == 2 ? (DT == 4 ? 5 : 1) : 4 <= NWT && NWT <= 8 ? 4 : 1;
     if (DT <= 6) return (NWT == 5 && (DT == 6 || kV)) || (NWT == 7 && !kV) ? 4 : NWT == 3 || NWT == 4 || (NWT == 6 && kV) ? 3 : 1;
     return NWT == 5 && !kV ? 4 : NWT == 3 || NWT == 4 ? 3 : 1;
 }
 template <class T, int DT, int NWT, int W, int PASS, bool kV>
-__global__ __launch_bounds__(64 * W, sizeof(T) == 2 && PASS == 0 ? r_held_waves(DT, NWT, kV) : 1) void r_bwd_tile(Problem P, BwdBuffers G, int first) {
+__global__ __launch_bounds__(64 * W, sizeof(T) == 2 && PASS == 0 ? r_held_waves(DT, NWT, kV) : DT >= 5 && W == 8 && shares_lds<T>(DT, NWT, PASS, kV) ? 4 : 1) void r_bwd_tile(Problem P, BwdBuffers G, int first) {
     using MT = Mat<T, DT>;
     using PL = RPlan<T, DT, NWT, PASS, kV>;
     using mfma::quad_rows_max;
@@ -423,7 +430,7 @@ constexpr int lz_held_waves(int DT, int NWT, bool kZ) {
     return NWT == 4 || NWT == 5 ? 4 : 1;
 }
 template <class T, int DT, int NWT, int W, int PASS, bool kZ>
-__global__ __launch_bounds__(64 * W, sizeof(T) == 2 && PASS == 0 ? lz_held_waves(DT, NWT, kZ) : 1) void lz_bwd_tile(Problem P, BwdBuffers G) {
+__global__ __launch_bounds__(64 * W, sizeof(T) == 2 && PASS == 0 ? lz_held_waves(DT, NWT, kZ) : DT >= 5 && W == 8 && shares_lds<T>(DT, NWT, PASS, kZ) ? 4 : 1) void lz_bwd_tile(Problem P, BwdBuffers G) {
     using MT = Mat<T, DT>;
     using PL = LzPlan<T, DT, NWT, PASS, kZ>;
     using mfma::quad_rows_max;
@@ -684,10 +691,29 @@ __global__ __launch_bounds__(64 * W, sizeof(T) == 2 && PASS == 0 ? lz_held_waves
 }
 
 // ---------------------------------------------------------------- launches
+// How problems of more than 128 rows that fill the device are split (16 bit).  One launch of 10 or 12 strips reads the operands once and
+// forms the statistics where they are used; its waves have 168 registers, which the R stage of 12 strips outgrows in the classes that
+// stay with two launches.  16 strips: two workgroups of four waves in pass 1, which would idle beside tiles of more than half of the LDS -
+// there one of eight.  Pass 2: see shares_lds; 96 columns and two gradients: one workgroup of 16 waves (122 registers and 76 bytes spilled).
+// us of the stages Z, R with V, L, R, bf16, before -> now, D = 64 / 96 / 128:
+//   150 rows  80, 130, 94, 101 -> 71, 100, 69, 76 (11.5 million elements) / 119, 210, 129, 139 -> 100, 164, 101, 116 / 210, 264, 192, 205 ->
+//             145, 264 (254 - 138 for 132 us in one launch), 148, 169
+//   190 rows  138, 188, 135, 148 -> 108, 188 (in one launch 203), 106, 135 / 212, 317, 225, 218 -> 150, 292, 192, 218 (221) / 310, 376, 263,
+//             308 -> 195, 376 (389), 241, 288 (R with V, 80 columns, fp16: 321 in two launches, 347 in one)
+//   250 rows  232, 400, 233, 245 -> 232, 348, 233, 245 (eight waves in pass 1: 253, 405, 243, 256) / 567, 659, 471, 444 -> 424, 576, 370, 383
+//             / 701, 737, 603, 505 -> 567, 649, 432, 447
+template <int DT, bool kV>
+struct RSplit {
+    static constexpr Split16 of{!(kV && DT == 8), kV ? DT == 6 : DT <= 4 || DT == 8, kV && DT >= 5 ? 8 : 4, kV && DT == 6 ? 16 : 8};
+};
+template <int DT, bool kZ>
+struct LzSplit {
+    static constexpr Split16 of{true, true, DT >= 5 ? 8 : 4, kZ && DT == 6 ? 16 : 8};
+};
 template <class T, int DT, bool kV>
 int launch_r(const Problem& P, const BwdBuffers& G, bool first, hipStream_t s) {
     const long long problems = static_cast<long long>(P.E) * P.H * P.M;
-    return each_launch<sizeof(T) == 4>(P.B, problems, [&](auto nwt, auto w, auto pass) {
+    return each_launch<sizeof(T) == 4, RSplit<DT, kV>>(P.B, problems, [&](auto nwt, auto w, auto pass) {
         constexpr int NWT = decltype(nwt)::value, W = decltype(w)::value, PASS = decltype(pass)::value;
         if constexpr (PASS == 0 && !RPlan<T, DT, NWT, 0, kV>::kFits) {   // three fp32 tiles of 128 rows: the passes one after the other
             static_assert(NWT > 4, "the statistics of problems of up to 64 rows have no room in the workspace");
@@ -702,7 +728,7 @@ int launch_r(const Problem& P, const BwdBuffers& G, bool first, hipStream_t s) {
 template <class T, int DT, bool kZ>
 int launch_lz(const Problem& P, const BwdBuffers& G, hipStream_t s) {
     const long long problems = static_cast<long long>(P.E) * P.H * P.B;
-    return each_launch<sizeof(T) == 4>(P.M, problems, [&](auto nwt, auto w, auto pass) {
+    return each_launch<sizeof(T) == 4, LzSplit<DT, kZ>>(P.M, problems, [&](auto nwt, auto w, auto pass) {
         constexpr int NWT = decltype(nwt)::value, W = decltype(w)::value, PASS = decltype(pass)::value;
         static_assert(LzPlan<T, DT, NWT, PASS, kZ>::kFits, "two tiles of up to 128 rows fit the LDS");
         return run(lz_bwd_tile<T, DT, NWT, W, PASS, kZ>, LzPlan<T, DT, NWT, PASS, kZ>::kLds, problems, NWT / W, W, s, P, G);

@@ -579,7 +579,7 @@ int launch_r32(const Problem& P, bool first, bool with_v, hipStream_t s) {
 template <int DT>
 int launch_l32(const Problem& P, hipStream_t s) {
     const long long problems = static_cast<long long>(P.E) * P.H * P.B;
-    return each_launch<true>(P.M, problems, [&](auto nwt, auto w, auto pass) {
+    return each_launch<true, void>(P.M, problems, [&](auto nwt, auto w, auto pass) {
         constexpr int NWT = decltype(nwt)::value, W = decltype(w)::value, PASS = decltype(pass)::value;
         return run(l_step_f32<DT, NWT, W, PASS>, LPlan<float, DT, NWT, PASS>::kLds, problems, NWT / W, W, s, P, P.stats);
     });

@@ -246,19 +246,19 @@ struct TileIn {
 };
 
 // Chunks of rows a pass with `tiles` operand tiles walks its NWT strips in, so that they fit the LDS beside `extra` bytes
-constexpr int chunks_of(int tiles, int nwt, size_t strip_bytes, size_t extra) {
+constexpr int chunks_of(int tiles, int nwt, size_t strip_bytes, size_t extra, size_t most = kLdsMax) {
     for (int nc = 1; nc < nwt; ++nc)
-        if (nwt % nc == 0 && (nc == 1 || nwt / nc % 2 == 0) && tiles * (nwt / nc) * strip_bytes + extra <= kLdsMax) return nc;
+        if (nwt % nc == 0 && (nc == 1 || nwt / nc % 2 == 0) && tiles * (nwt / nc) * strip_bytes + extra <= most) return nc;
     return nwt;
 }
 
-// LDS and chunks of a stage: TILES1 / TILES2 operand tiles in pass 1 / 2, STATS floats per row
-template <class T, int DT, int NWT, int PASS, int TILES1, int TILES2, int STATS>
+// LDS and chunks of a stage: TILES1 / TILES2 operand tiles in pass 1 / 2 (HALF2: pass 2 in half of the LDS), STATS floats per row
+template <class T, int DT, int NWT, int PASS, int TILES1, int TILES2, int STATS, bool HALF2 = false>
 struct Plan {
     using MT = Mat<T, DT>;
     static constexpr int ROWS = 16 * NWT;
     static constexpr size_t kStrip = 16 * MT::LD * sizeof(T), kStats = static_cast<size_t>(STATS) * ROWS * sizeof(float);
-    static constexpr int NC1 = chunks_of(TILES1, NWT, kStrip, kStats), NC2 = chunks_of(TILES2, NWT, kStrip, kStats);
+    static constexpr int NC1 = chunks_of(TILES1, NWT, kStrip, kStats), NC2 = chunks_of(TILES2, NWT, kStrip, kStats, HALF2 ? kLdsMax / 2 : kLdsMax);
     static constexpr int CT1 = NWT / NC1, CT2 = NWT / NC2;
     static constexpr size_t kTiles1 = TILES1 * CT1 * kStrip, kTiles2 = TILES2 * CT2 * kStrip;
     static constexpr size_t kTiles = PASS == 1 ? kTiles1 : PASS == 2 ? kTiles2 : (kTiles1 > kTiles2 ? kTiles1 : kTiles2);
@@ -300,8 +300,12 @@ inline int strip_class(int n) {
 // f(integral_constant NWT, integral_constant W, integral_constant PASS) for every launch of a stage of `problems` problems
 // of n rows.  One launch of both passes up to 128 rows, unless there are fewer problems of 6 or 8 strips than the device has
 // compute units: half of their strips per workgroup then (the graph-transformer shape has 120 problems of 128 rows).  Above 128
-// rows half of the strips per workgroup, or four where that would leave compute units without one.
-template <bool F32, class F>
+// rows, where the problems fill the device, what `Split` says, else four strips per workgroup.
+struct Split16 {   // of a 16-bit kernel: 10 and 12 strips in one launch; waves of a workgroup in pass 1 and 2 of 16
+    bool one10, one12;
+    int w1, w2;
+};
+template <bool F32, class Split, class F>
 int each_launch(int n, long long problems, F&& f) {
     auto two = [&](auto nwt, auto w1, auto w2) {
         const int st = f(nwt, w1, std::integral_constant<int, 1>{});
@@ -317,7 +321,10 @@ int each_launch(int n, long long problems, F&& f) {
         const int strips = (n + 15) / 16;
         if (fill && strips == 5) return f(integral_constant<int, 5>{}, integral_constant<int, 5>{}, one);
         if (fill && strips == 7) return f(integral_constant<int, 7>{}, integral_constant<int, 7>{}, one);
-        if (fill && (strips == 9 || strips == 10)) return two(integral_constant<int, 10>{}, integral_constant<int, 5>{}, integral_constant<int, 5>{});
+        if (fill && (strips == 9 || strips == 10)) {
+            if constexpr (Split::of.one10) return f(integral_constant<int, 10>{}, integral_constant<int, 10>{}, one);
+            else return two(integral_constant<int, 10>{}, integral_constant<int, 5>{}, integral_constant<int, 5>{});
+        }
     }
     switch (strip_class(n)) {
         case 1: return f(integral_constant<int, 1>{}, integral_constant<int, 1>{}, one);
@@ -330,11 +337,14 @@ int each_launch(int n, long long problems, F&& f) {
                              : f(integral_constant<int, 8>{}, integral_constant<int, 8>{}, one);
         case 12:
             if constexpr (!F32)
-                if (fill) return two(integral_constant<int, 12>{}, integral_constant<int, 6>{}, integral_constant<int, 6>{});
+                if (fill) {
+                    if constexpr (Split::of.one12) return f(integral_constant<int, 12>{}, integral_constant<int, 12>{}, one);
+                    else return two(integral_constant<int, 12>{}, integral_constant<int, 6>{}, integral_constant<int, 6>{});
+                }
             return two(integral_constant<int, 12>{}, integral_constant<int, 4>{}, integral_constant<int, 4>{});
         default:
             if constexpr (!F32)
-                if (fill) return two(integral_constant<int, 16>{}, integral_constant<int, 4>{}, integral_constant<int, 8>{});
+                if (fill) return two(integral_constant<int, 16>{}, integral_constant<int, Split::of.w1>{}, integral_constant<int, Split::of.w2>{});
             return two(integral_constant<int, 16>{}, integral_constant<int, 4>{}, integral_constant<int, 4>{});
     }
 }
