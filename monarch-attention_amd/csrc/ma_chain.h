@@ -98,13 +98,26 @@ __device__ __forceinline__ unsigned chain_wait(const unsigned* go, unsigned spin
     }
 }
 
+// As Split, but with a wave per strip where the workgroup has as many
+template <int NT, int W>
+struct ChainSplit {
+    static constexpr int WPP = W >= NT ? NT : kWaves, PPW = W / WPP;
+};
+template <class T, int DT, int NTB, int NTM, int W>
+struct ChainLds {
+    static constexpr size_t r = ChainSplit<NTB, W>::PPW * Lds<T, DT, NTB>::R;
+    static constexpr size_t l = ChainSplit<NTM, W>::PPW * Lds<T, DT, NTM>::L;
+    static constexpr size_t z = ChainSplit<NTM, W>::PPW * Lds<T, DT, NTM>::Z;
+    static constexpr size_t bytes = r > l ? (r > z ? r : z) : (l > z ? l : z);
+};
+
 // KEEP: every step's state stays (Problem::slot_rows).  A build of its own: the second row offset costs the others 1.5 %
 // (16 heads of 4096 tokens, one step: 17.05 -> 17.3 us).
 template <class T, int DT, int NTB, int NTM, int W, bool KEEP = false>
 __global__ __launch_bounds__(64 * W) void chain_fwd_mfma(Problem P, ChainPlan plan) {
-    using RP = RProb<T, DT, NTB>;
-    using LP = LProb<T, DT, NTM>;
-    using ZP = ZProb<T, DT, NTM>;
+    using RP = RProb<T, DT, NTB, ChainSplit<NTB, W>::WPP>;
+    using LP = LProb<T, DT, NTM, ChainSplit<NTM, W>::WPP>;
+    using ZP = ZProb<T, DT, NTM, ChainSplit<NTM, W>::WPP>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     __shared__ unsigned wg_word;   // thread 0's verdict on the wait / on being the head's last Z task
     const int wave = wave_id(), lane = threadIdx.x & 63;
@@ -155,7 +168,7 @@ __global__ __launch_bounds__(64 * W) void chain_fwd_mfma(Problem P, ChainPlan pl
     const Slices S = KEEP ? make_slices<T>(P, e, h, head, static_cast<long long>(step) * P.slot_rows, odd ? 0u : P.slot_rows)
                           : make_slices<T>(P, e, h, head);
     if (p == nph - 1) {
-        constexpr int WPP = Split<NTM, W>::WPP, PPW = Split<NTM, W>::PPW;
+        constexpr int WPP = ChainSplit<NTM, W>::WPP, PPW = ChainSplit<NTM, W>::PPW;
         const int sub = wave / WPP, wig = wave % WPP;
         const int j = (task * PPW + sub) * (NTM == 1 ? 16 >> P.pack_shift : 1);   // heads of few blocks: several positions per tile (TileIndex)
         const bool active = sub < PPW && j < P.B;
@@ -165,13 +178,13 @@ __global__ __launch_bounds__(64 * W) void chain_fwd_mfma(Problem P, ChainPlan pl
         ZP::issue(P, S, pre, active, active ? j : 0, wig, lane);
         wait_prev();
         if (failed) {
-            if (active) z_poison<T, DT, NTM>(P, S, j, wig, lane);   // the failure shows in the output
+            if (active) z_poison<T, DT, NTM, WPP>(P, S, j, wig, lane);   // the failure shows in the output
         } else {
             ZP::state(P, S, st, active, active ? j : 0, wig, lane);
             ZP::run(P, S, sm, pre, st, active, active ? j : 0, wig, lane);
         }
     } else if (odd) {
-        constexpr int WPP = Split<NTM, W>::WPP, PPW = Split<NTM, W>::PPW;
+        constexpr int WPP = ChainSplit<NTM, W>::WPP, PPW = ChainSplit<NTM, W>::PPW;
         const int sub = wave / WPP, wig = wave % WPP;
         const int j = (task * PPW + sub) * (NTM == 1 ? 16 >> P.pack_shift : 1);
         const bool active = sub < PPW && j < P.B;
@@ -185,7 +198,7 @@ __global__ __launch_bounds__(64 * W) void chain_fwd_mfma(Problem P, ChainPlan pl
             LP::run(P, S, sm, pre, st, active, active ? j : 0, wig, lane);
         }
     } else {
-        constexpr int WPP = Split<NTB, W>::WPP, PPW = Split<NTB, W>::PPW;
+        constexpr int WPP = ChainSplit<NTB, W>::WPP, PPW = ChainSplit<NTB, W>::PPW;
         const int sub = wave / WPP, wig = wave % WPP;
         const int m = task * PPW + sub;
         const bool active = sub < PPW && m < P.M;

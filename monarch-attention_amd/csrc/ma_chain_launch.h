@@ -10,13 +10,12 @@
 namespace ma {
 namespace mfma {
 
-template <class T, int DT, int NTB, int NTM, bool KEEP = false>
+template <class T, int DT, int NTB, int NTM, int W, bool KEEP = false>
 int launch_chain_one(const Problem& P, bool sync_ready, hipStream_t s) {
-    constexpr int W = kWaves;
     if constexpr (!KEEP) {
-        if (P.slot_rows != 0) return launch_chain_one<T, DT, NTB, NTM, true>(P, sync_ready, s);
+        if (P.slot_rows != 0) return launch_chain_one<T, DT, NTB, NTM, W, true>(P, sync_ready, s);
     }
-    using FL = FusedLds<T, DT, NTB, NTM, W>;   // the three kinds of block problems share one LDS allocation
+    using FL = ChainLds<T, DT, NTB, NTM, W>;   // the three kinds of block problems share one LDS allocation
     if (FL::bytes > 160 * 1024) return MA_ERR_UNSUPPORTED;
     auto kernel = chain_fwd_mfma<T, DT, NTB, NTM, W, KEEP>;
     const int lds_err = set_lds_limit(kernel, FL::bytes);
@@ -30,9 +29,9 @@ int launch_chain_one(const Problem& P, bool sync_ready, hipStream_t s) {
     const bool follow = heads % 8 == 0 && P.ks[1] < P.ks[2] && P.D * 2 % 128 != 0;
     pl.hs = follow ? pl.hx : 1;
     pl.hk = follow ? 1 : 8;
-    pl.tR = (P.M + Split<NTB, W>::PPW - 1) / Split<NTB, W>::PPW;
+    pl.tR = (P.M + ChainSplit<NTB, W>::PPW - 1) / ChainSplit<NTB, W>::PPW;
     const int per = NTM == 1 ? 16 >> P.pack_shift : 1;   // in-block positions per L / Z problem (heads of few blocks share tiles)
-    pl.tL = ((P.B + per - 1) / per + Split<NTM, W>::PPW - 1) / Split<NTM, W>::PPW;
+    pl.tL = ((P.B + per - 1) / per + ChainSplit<NTM, W>::PPW - 1) / ChainSplit<NTM, W>::PPW;
     pl.stride = chain_stride(P.T);
     pl.go_off = chain_go_offset(P.T);
     pl.spin_limit = P.test_no_spin ? 0u : 1u << 18;   // a legitimate wait lasts one phase of one head (well under a millisecond)
@@ -51,27 +50,41 @@ int launch_chain_one(const Problem& P, bool sync_ready, hipStream_t s) {
     return static_cast<int>(hipGetLastError());
 }
 
+// Waves of a workgroup.  What counts where the heads fill the device is how many workgroups a compute unit holds, so four, of which each
+// walks up to two strips - a wave per strip is 5 - 25 % behind (D = 72, two steps: 48 heads of 104 blocks of 104 rows 332 -> 388 us, 48 of 70
+// blocks of 110 rows 233 -> 289; D = 64, 48 of 128 blocks of 128 rows 348 -> 436).  One side of eight strips and one of four is where LDS and
+// registers of the eight hold the workgroups to two to four per unit, whose waves then stand idle half of the time: eight waves.  48, 16, 4 heads
+// (the last at one step) of 64 blocks of 128 rows: D = 64 171, 56, 22 -> 164, 51, 20 us; 72 276, 86, 28 -> 258, 75, 26; 128 353, 117, 33 -> 342, 110,
+// 30; of 128 blocks of 64 rows: 72 280, 86, 26 -> 249, 76, 25; 128 355, 111, 32 -> 327, 107, 31; 64 (173, 56, 20 for 170, 57, 20) and 32 stay.
+constexpr int chain_waves(int DT, int NTB, int NTM) { return (NTB == 8 && NTM == 4 && DT >= 4) || (NTB == 4 && NTM == 8 && DT >= 5) ? 8 : kWaves; }
+
+// f(integral_constant) of the strips of n rows: a class for each count.  (5 and 7 strips in the classes of 6 and 8 took their LDS, registers
+// and products with keys that are not there.  us, 48 and 16 heads at two steps: 70 blocks of 72 rows, D = 32 77, 35 -> 71, 33, 64 118, 45 ->
+// 112, 40, 72 164, 56 -> 142, 52, 128 220, 74 -> 215, 72; 104 of 104: 64 265, 82 -> 244, 75, 72 404, 127 -> 332, 104, 128 517, 160 ->
+// 494, 156; 20 of 72: 72 48, 28 -> 39, 26.)
+template <class F>
+int chain_strips(int n, F&& f) {
+    using std::integral_constant;
+    switch ((n + 15) / 16) {
+        case 1: return f(integral_constant<int, 1>{});
+        case 2: return f(integral_constant<int, 2>{});
+        case 3: return f(integral_constant<int, 3>{});
+        case 4: return f(integral_constant<int, 4>{});
+        case 5: return f(integral_constant<int, 5>{});
+        case 6: return f(integral_constant<int, 6>{});
+        case 7: return f(integral_constant<int, 7>{});
+        default: return f(integral_constant<int, 8>{});
+    }
+}
+
 template <class T, int DT>
 int launch_chain(const Problem& P, bool sync_ready, hipStream_t s) {
-    const int ntb = nt_class_chain(P.B), ntm = nt_class_chain(P.M);
-#define MA_NTM(NB)                                                              \
-    switch (ntm) {                                                              \
-        case 1: return launch_chain_one<T, DT, NB, 1>(P, sync_ready, s);        \
-        case 2: return launch_chain_one<T, DT, NB, 2>(P, sync_ready, s);        \
-        case 3: return launch_chain_one<T, DT, NB, 3>(P, sync_ready, s);        \
-        case 4: return launch_chain_one<T, DT, NB, 4>(P, sync_ready, s);        \
-        case 6: return launch_chain_one<T, DT, NB, 6>(P, sync_ready, s);        \
-        default: return launch_chain_one<T, DT, NB, 8>(P, sync_ready, s);       \
-    }
-    switch (ntb) {
-        case 1: MA_NTM(1)
-        case 2: MA_NTM(2)
-        case 3: MA_NTM(3)
-        case 4: MA_NTM(4)
-        case 6: MA_NTM(6)
-        default: MA_NTM(8)
-    }
-#undef MA_NTM
+    return chain_strips(P.B, [&](auto ntb) {
+        return chain_strips(P.M, [&](auto ntm) {
+            constexpr int NTB = decltype(ntb)::value, NTM = decltype(ntm)::value;
+            return launch_chain_one<T, DT, NTB, NTM, chain_waves(DT, NTB, NTM)>(P, sync_ready, s);
+        });
+    });
 }
 
 }  // namespace mfma

@@ -182,11 +182,11 @@ __device__ __forceinline__ float bloadf(rsrc_t r, unsigned off) {
 //          front of the stores, which is faster (2 - 4 %) for problems that read their tiles once or twice.
 //  kRun    the head-resident kernels' rows: padded, a lane's 4*DT result columns one consecutive run.
 enum { kTile = 0, kSmall = 1, kRun = 2 };
-// The layout of a problem of NWT strips here.  kTile pays where a tile is read many times - 6 and 8 strips of 128 columns (R
+// The layout of a problem of NWT strips here.  kTile pays where a tile is read many times - 5 to 8 strips of 128 columns (R
 // step of 72-row blocks at D = 128: 26.4 -> 25.2 us) - and for 2 strips of 80 columns (D = 72: 1 - 3 %); elsewhere the two are
 // within 2 %.  (The kernels of ma_tile.h use it throughout: 48 heads of 65536 tokens gained 10 %, an L step of 141 blocks at
 // D = 80 went from 70 to 45 us.)
-constexpr int layout_of_strips(int nwt, int dt) { return (nwt >= 6 && dt > 5) || (nwt == 2 && dt == 5) ? kTile : kSmall; }
+constexpr int layout_of_strips(int nwt, int dt) { return (nwt >= 5 && dt > 5) || (nwt == 2 && dt == 5) ? kTile : kSmall; }
 
 // Geometry for a head dim that needs DT 16-wide output tiles: KS 32-wide k steps, row pitch LD elements.
 template <int DT, int MODE = kTile>
@@ -213,7 +213,7 @@ struct TileCopy {
     using G = Geom<DT, layout_of_strips(ROWS / 16, DT)>;
     static constexpr int CH = G::COLS / 8;
     static constexpr int CNT = (ROWS * CH + NTH - 1) / NTH;
-    static constexpr bool EVEN = ROWS * CH % NTH == 0;   // else the last round of chunks is not for every thread
+    static constexpr int WHOLE = ROWS * CH / NTH;   // rounds of chunks for every thread
     u32x4 val[CNT];
 
     template <int SHARED, class RowOff>
@@ -222,7 +222,7 @@ struct TileCopy {
         for (int i = 0; i < CNT; ++i) {
             const int c = tix + i * NTH;
             const int row = c / CH, ch = c % CH;
-            const unsigned ro = (EVEN || c < ROWS * CH) ? rowoff(row) : kOob;
+            const unsigned ro = (i < WHOLE || c < ROWS * CH) ? rowoff(row) : kOob;
             val[i] = bload16<SHARED>(src, (ch * 8 < D) ? ro + ch * 16 : kOob);
         }
     }
@@ -230,7 +230,14 @@ struct TileCopy {
 #pragma unroll
         for (int i = 0; i < CNT; ++i) {
             const int c = tix + i * NTH;
-            if (EVEN || c < ROWS * CH) *reinterpret_cast<u32x4*>(tile + G::at(c / CH, c % CH)) = val[i];
+            if constexpr (WHOLE > 0 && WHOLE < CNT) {   // a thread without a last chunk writes the one before it again (a branch here keeps val in scratch)
+                const bool in = i < WHOLE || c < ROWS * CH;
+                const int at = in ? c : c - NTH;
+                const u32x4 x = val[i], y = val[i > 0 ? i - 1 : 0];
+                *reinterpret_cast<u32x4*>(tile + G::at(at / CH, at % CH)) = u32x4{in ? x[0] : y[0], in ? x[1] : y[1], in ? x[2] : y[2], in ? x[3] : y[3]};
+            } else {
+                if (i < WHOLE || c < ROWS * CH) *reinterpret_cast<u32x4*>(tile + G::at(c / CH, c % CH)) = val[i];
+            }
         }
     }
 };
@@ -401,16 +408,16 @@ __device__ __forceinline__ void store_row(rsrc_t dst, unsigned ro, int D, const 
 
 // How a workgroup's W waves are shared among block problems with NT strips:
 // WPP waves per problem (at most four: a wave of a 128-row problem walks two strips, one after
-// the other), PPW problems per workgroup.  Problems of 3 or 6 strips
-// (blocks and block counts of 33-48 / 81-96, e.g. the 48- and 96-token blocks of the reference's
+// the other), PPW problems per workgroup.  Problems of 3 strips
+// (blocks and block counts of 33-48, e.g. the 48-token blocks of the reference's
 // RoBERTa sweep, experiments/roberta/benchmark.py:78) run on three waves: a per-stage launch uses
 // workgroups of three waves (WG), a one-launch kernel leaves its fourth wave idle in such a phase.
 template <int NT, int W = kWaves>
 struct Split {
-    static_assert(NT == 1 || NT == 2 || NT == 3 || NT == 4 || NT == 6 || NT == 8, "strip counts are 1, 2, 3, 4, 6 or 8");
-    static constexpr int WPP = (NT == 3 || NT == 6) ? 3 : (NT < kWaves ? NT : kWaves);
+    static_assert(1 <= NT && NT <= 8, "up to 8 strips");
+    static constexpr int WPP = NT < kWaves ? NT : kWaves;
     static constexpr int PPW = W / WPP;
-    static constexpr int WG = (NT == 3 || NT == 6) ? 3 : kWaves;   // waves of a per-stage launch's workgroup
+    static constexpr int WG = NT == 3 ? 3 : kWaves;   // waves of a per-stage launch's workgroup
 };
 
 // LDS bytes of one problem slot of each stage
@@ -522,13 +529,11 @@ __device__ __forceinline__ void problem_sync() {
 // R step for one block problem (e,h,m), run by WPP waves (wig = wave in group).
 // smem: K tile, V tile, key bias.   Reference: al_cl_ref / al_y_cl_ref
 // (ma/ma_torch.py:10-23, :38-52).
-template <class T, int DT, int NWT>
+template <class T, int DT, int NWT, int WPP = Split<NWT>::WPP>
 struct RProb {
     using G = Geom<DT, Lds<T, DT, NWT>::MODE>;
     using V8 = typename Ops<T>::v8;
-    static constexpr int WPP = Split<NWT>::WPP;
-    static_assert(NWT % WPP == 0, "whole strips per wave");
-    static constexpr int SPW = NWT / WPP;   // strips per wave: 2 for blocks of more than 64 rows
+    static constexpr int SPW = (NWT + WPP - 1) / WPP;   // strips per wave: 2 for blocks of more than 64 rows in four waves or less
     static constexpr int ROWS = Lds<T, DT, NWT>::ROWS;
     static __device__ __forceinline__ int strip_of(int wig, int i) { return wig + i * WPP; }
     struct Pre {
@@ -613,13 +618,9 @@ struct RProb {
             if (tix < ROWS) kbias[tix] = (tix < P.B && token_kept(P, m * P.B - P.pad_off + tix, pre.km)) ? 0.f : kNegBig;
         }
         problem_sync<WPP>();
-        // The last strip has rows (uniform).  65 - 80 rows leave it empty in the class of 6 strips: it is passed over (16 heads of 5003,
-        // 72-row blocks, two steps, inputs from memory: D = 64 44.6 -> 42.3 us, D = 128 71.1 -> 70.0; full classes within 0.3 %).  Passing
-        // over its tile of keys too gives as much again, but takes 16 registers, and full strips lose 1 - 2 %; so do 8 strips with either.
-        const bool full = NWT != 6 || 16 * (NWT - 1) < B;
 #pragma unroll
         for (int si = 0; si < SPW; ++si) {
-          if (!full && strip_of(wig, si) == NWT - 1) continue;
+          if (NWT % WPP != 0 && strip_of(wig, si) >= NWT) continue;   // (uniform)
           f32x4 OY[DT];
           V8 pb[(NWT + 1) / 2];
           bool jv = false;
@@ -718,14 +719,12 @@ struct TileIndex {
 
 // Z step for one column problem (e,h,j).  smem: aL tile, Y tile, cL bias.
 // Reference: z_ref (ma/ma_torch.py:55-62) and the final slice (:106-108).
-template <class T, int DT, int NWT>
+template <class T, int DT, int NWT, int WPP = Split<NWT>::WPP>
 struct ZProb {
     using G = Geom<DT, Lds<T, DT, NWT>::MODE>;
     using V8 = typename Ops<T>::v8;
-    static constexpr int WPP = Split<NWT>::WPP;
     static constexpr int ROWS = Lds<T, DT, NWT>::ROWS;
-    static_assert(NWT % WPP == 0, "whole strips per wave");
-    static constexpr int SPW = NWT / WPP;   // strips per wave
+    static constexpr int SPW = (NWT + WPP - 1) / WPP;   // strips per wave
     static __device__ __forceinline__ int strip_of(int wig, int i) { return wig + i * WPP; }
     struct Pre {
         V8 xq[SPW][G::KS];   // the Q rows of this wave's strips
@@ -783,10 +782,9 @@ struct ZProb {
             if (tix < ROWS) cb[tix] = st.cbv;
         }
         problem_sync<WPP>();
-        const bool full = NWT != 6 || 16 * (NWT - 1) < P.M;   // (as in RProb)
 #pragma unroll
         for (int si = 0; si < SPW; ++si) {
-          if (!full && strip_of(wig, si) == NWT - 1) continue;
+          if (NWT % WPP != 0 && strip_of(wig, si) >= NWT) continue;   // (uniform)
           V8 pb[(NWT + 1) / 2];
           if (active) {
             const int strip = strip_of(wig, si);
@@ -839,9 +837,9 @@ struct ZProb {
 
 // NaN into the output rows of column problem (e,h,j): what a one-launch kernel writes instead of
 // results when the workgroup that owns the rows gave up waiting for the state they depend on.
-template <class T, int DT, int NWT>
+template <class T, int DT, int NWT, int WPP = Split<NWT>::WPP>
 __device__ __forceinline__ void z_poison(const Problem& P, const Slices& S, int j, int wig, int lane) {
-    constexpr int WPP = Split<NWT>::WPP, SPW = NWT / WPP;
+    constexpr int SPW = (NWT + WPP - 1) / WPP;
     const int r = lane & 15, q = lane >> 4;
     f32x4 O[DT];
 #pragma unroll
@@ -870,15 +868,14 @@ __device__ __forceinline__ void z_poison(const Problem& P, const Slices& S, int 
 // it saves the transposed copy of the probabilities in LDS (which was as large as both operand
 // tiles together and halved the workgroups per compute unit), its write, its read and the 16-lane
 // reductions of the column-wise softmax.
-template <class T, int DT, int NWT>
+template <class T, int DT, int NWT, int WPP = Split<NWT>::WPP>
 struct LProb {
     using G = Geom<DT, Lds<T, DT, NWT>::MODE>;
     using V8 = typename Ops<T>::v8;
     using LS = Lds<T, DT, NWT>;
-    static constexpr int WPP = Split<NWT>::WPP;
     static constexpr int ROWS = LS::ROWS;
     static constexpr int nth = WPP * 64;
-    static constexpr int SPW = NWT / WPP;   // strips per wave (2 for blocks counts above 64)
+    static constexpr int SPW = (NWT + WPP - 1) / WPP;   // strips per wave
     struct Pre {
         TileCopy<T, DT, ROWS, nth> qc;   // Q^T tile
         unsigned qm[SPW];                // mask word of the query token of block 16*(wig + i*WPP) + lane % 16
@@ -938,16 +935,12 @@ struct LProb {
             if (tix < ROWS) cb[tix] = st.cbv;
         }
         problem_sync<WPP>();
-        const bool full = NWT != 6 || 16 * (NWT - 1) < P.M;   // (as in RProb)
         if (active) {
             // pass 1: lane holds query block l = l0 + r, rows = key blocks 16kt + 4q + v
 #pragma unroll
             for (int si = 0; si < SPW; ++si) {
                 const int l = 16 * (wig + si * WPP) + r;
-                if (!full && wig + si * WPP == NWT - 1) {   // (pass 2 reads its statistics)
-                    if (q == 0) mxs[l] = invs[l] = 0.f;
-                    continue;
-                }
+                if (NWT % WPP != 0 && wig + si * WPP >= NWT) continue;
                 V8 xq[G::KS];
 #pragma unroll
                 for (int ks = 0; ks < G::KS; ++ks) xq[ks] = lds_row8<T>(Qt + G::at(l, 4 * ks + q));
@@ -986,7 +979,7 @@ struct LProb {
 #pragma unroll
             for (int si = 0; si < SPW; ++si) {
                 const int k = 16 * (wig + si * WPP) + r;
-                if (!full && wig + si * WPP == NWT - 1) continue;
+                if (NWT % WPP != 0 && wig + si * WPP >= NWT) continue;
                 const bool kv = ti.ok(P, k);
                 V8 xk[G::KS];
 #pragma unroll

@@ -14,15 +14,10 @@ namespace ma {
 namespace mfma {
 
 inline int dt_class(int D) { return D <= 32 ? 2 : D <= 64 ? 4 : D <= 80 ? 5 : 8; }
-// the team kernel is built for fewer classes: 96-row problems run as 128-row ones there
+// the team kernel is built for fewer classes: 65- to 112-row problems run as 128-row ones there
 inline int nt_class_one_launch(int n) {
     const int t = (n + 15) / 16;
     return t <= 4 ? (t < 1 ? 1 : t) : 8;
-}
-// the chained kernel has the 96-row class as well
-inline int nt_class_chain(int n) {
-    const int t = (n + 15) / 16;
-    return t <= 4 ? (t < 1 ? 1 : t) : t <= 6 ? 6 : 8;
 }
 // the per-stage launches have up to four strips here; longer problems run the kernels of ma_long.h
 inline int nt_class(int n) { return n <= 16 ? 1 : n <= 32 ? 2 : n <= 48 ? 3 : 4; }

@@ -23,6 +23,8 @@ CASES = [  # E, H, N, D, B, T, pre, dtype, variant, masked: rows per slot that d
     (13, 1, 60, 32, 19, 3, False, "f16", None, True), (50, 1, 21, 80, 9, 3, True, "bf16", None, False), (13, 1, 81, 48, 24, 3, True, "f16", None, True),
     (67, 7, 53, 72, 7, 3, False, "f16", None, True), (66, 1, 1265, 32, 38, 3, True, "bf16", None, False), (79, 1, 2570, 32, 48, 2, False, "bf16", None, True),
     (122, 1, 548, 64, 23, 3, False, "f16", None, True), (26, 1, 221, 32, 56, 3, True, "f16", None, True), (39, 13, 542, 32, 12, 3, True, "bf16", None, True),
+    # the chained kernel with a wave per strip: five strips one way, seven and six both ways
+    (1, 3, 5003, 128, 72, 2, True, "bf16", "chained", True), (1, 2, 60 * 70, 64, 60, 3, False, "f16", "chained", True), (1, 2, 9000, 72, 100, 2, False, "f16", "chained", False),
 ]
 
 

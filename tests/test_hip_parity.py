@@ -434,6 +434,28 @@ def test_slices_of_few_blocks(M, layout):
         assert_parity(out[:1].cpu(), ref, "f16" if i % 2 else "bf16", f"few blocks {(heads, N, D, B, T)}")
 
 
+CHAIN_STRIPS = [(sb, sm) for sb in range(1, 9) for sm in range(1, 9) if max(sb, sm) > 4]
+
+
+@pytest.mark.parametrize("sb,sm", CHAIN_STRIPS)
+def test_chained_kernel_of_more_than_64_rows(sb, sm):
+    """Every pair of strip counts of which one exceeds four, its last strips with one row and with all: the results of the stage
+    launches, the flags cleared, and one pair of heads against the oracle."""
+    i = CHAIN_STRIPS.index((sb, sm))
+    for full in (False, True):
+        B, M = (16 * sb, 16 * sm) if full else (16 * sb - 15, 16 * sm - 15)
+        D, T, pre, dt = (32, 64, 72, 128)[(i + full) % 4], 1 + (i + full) % 3, i % 2 == 1, "bf16" if (i // 2 + full) % 2 else "f16"
+        N = M * B - (0 if full else B // 2)
+        q, k, v = seeded_qkv(2, 3, N, D, DT[dt], seed=i)
+        mask = block_safe_mask(2, N, B, seed=i) if i % 3 else None
+        dev = to_dev(q, k, v, mask)
+        out = monarch_attention_hip(*dev, T, B, pre, variant="chained")
+        assert torch.equal(out, monarch_attention_hip(*dev, T, B, pre, variant="staged")), (B, M, D, T)
+        ref = monarch_attention_oracle(q[1:, 2:], k[1:, 2:], v[1:, 2:], None if mask is None else mask[1:], T, B, pre, upcast=True)
+        assert_parity(out[1:, 2:].cpu(), ref, dt, f"chained {(B, M, D, T, pre, dt)}")
+    assert sync_status() == 0
+
+
 @pytest.mark.parametrize("layouts", [("tokens", "tokens", "tokens"), ("heads", "tokens", "heads"), ("tokens", "heads", "tokens")])
 @pytest.mark.parametrize("E,H,N,D,B,T,pre,dt", [
     (2, 4, 100, 40, 16, 2, False, "f16"), (1, 8, 500, 72, 32, 2, True, "bf16"), (1, 16, 700, 80, 24, 3, False, "f16"),
@@ -1021,7 +1043,7 @@ def test_random_shapes_in_the_192_and_256_row_classes(idx, E, H, N, D, B, T, pre
 
 
 # ---------------------------------------------------------------- a wait between workgroups that runs out is loud
-@pytest.mark.parametrize("shape", [(1, 2, 1024, 64, 32, 2), (3, 8, 512, 64, 32, 3), (1, 16, 2048, 64, 64, 1)])
+@pytest.mark.parametrize("shape", [(1, 2, 1024, 64, 32, 2), (3, 8, 512, 64, 32, 3), (1, 16, 2048, 64, 64, 1), (1, 3, 70 * 80, 64, 80, 2)])
 @pytest.mark.parametrize("variant", ["fused", "chained"])
 def test_wait_that_runs_out_is_loud_and_leaves_the_workspace_usable(variant, shape):
     """MA_FLAG_TEST_NO_SPIN makes every wait of the one-launch kernels give up at once (forced from the
