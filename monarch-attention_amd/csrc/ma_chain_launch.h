@@ -50,13 +50,20 @@ int launch_chain_one(const Problem& P, bool sync_ready, hipStream_t s) {
     return static_cast<int>(hipGetLastError());
 }
 
-// Waves of a workgroup.  What counts where the heads fill the device is how many workgroups a compute unit holds, so four, of which each
-// walks up to two strips - a wave per strip is 5 - 25 % behind (D = 72, two steps: 48 heads of 104 blocks of 104 rows 332 -> 388 us, 48 of 70
-// blocks of 110 rows 233 -> 289; D = 64, 48 of 128 blocks of 128 rows 348 -> 436).  One side of eight strips and one of four is where LDS and
-// registers of the eight hold the workgroups to two to four per unit, whose waves then stand idle half of the time: eight waves.  48, 16, 4 heads
-// (the last at one step) of 64 blocks of 128 rows: D = 64 171, 56, 22 -> 164, 51, 20 us; 72 276, 86, 28 -> 258, 75, 26; 128 353, 117, 33 -> 342, 110,
-// 30; of 128 blocks of 64 rows: 72 280, 86, 26 -> 249, 76, 25; 128 355, 111, 32 -> 327, 107, 31; 64 (173, 56, 20 for 170, 57, 20) and 32 stay.
-constexpr int chain_waves(int DT, int NTB, int NTM) { return (NTB == 8 && NTM == 4 && DT >= 4) || (NTB == 4 && NTM == 8 && DT >= 5) ? 8 : kWaves; }
+// Waves of a workgroup.  What counts is how many waves with work a compute unit holds.  Four as a rule, of which each walks up to two strips: a
+// wave per strip of the larger side leaves waves idle in the other kind of phase, or fits a compute unit less often, and is up to 25 % behind (D
+// = 72, two steps: 48 heads of 104 blocks of 104 rows 332 -> 388 us, 48 of 70 blocks of 110 rows 233 -> 289; D = 64, 48 of 128 blocks of 128 rows
+// 348 -> 436).  Eight beside a side of up to five strips where the LDS of eight (of seven above 96 columns) leaves room for three workgroups
+// of four waves or less, which are half idle in the short phases: eight waves run several short problems at a time.  Two steps, 48 | 192
+// heads, four -> eight waves, us: 8 blocks of 128 rows, D = 72 37 -> 31 | 120 -> 102, 128 45 -> 40 | 161 -> 155, 20 of 120, 72 90 -> 70 | 381 -> 331,
+// 128 108 -> 94 | 474 -> 441; 116 of 20, 72 88 -> 67 | 369 -> 303; 30 of 100, 128 117 -> 112 | 540 -> 529, 72 75 -> 80 | 342 -> 383.  64 columns, eight
+// strips of a block: 8 blocks 29 -> 26 | 71 -> 68, 20 53 -> 49 | 217 -> 208, 64 (48 heads) 171 -> 164; of a position 0.98 - 1.04.
+constexpr int chain_waves(int DT, int NTB, int NTM) {
+    const int most = NTB > NTM ? NTB : NTM, least = NTB < NTM ? NTB : NTM;
+    if (most < 7 || least > 5) return kWaves;
+    if (most == 7) return DT == 8 ? 8 : kWaves;
+    return DT >= 5 || (DT == 4 && NTB == 8 && NTM <= 4) ? 8 : kWaves;
+}
 
 // f(integral_constant) of the strips of n rows: a class for each count.  (5 and 7 strips in the classes of 6 and 8 took their LDS, registers
 // and products with keys that are not there.  us, 48 and 16 heads at two steps: 70 blocks of 72 rows, D = 32 77, 35 -> 71, 33, 64 118, 45 ->
