@@ -319,8 +319,9 @@ bool slice_pays(const ma_fwd_params* p, int v) {
 // A recorded call (ma_fwd_keep) that AUTO gives to the chained kernel: does the slice-resident one take it, writing every step's state as it
 // goes?  The same two estimates, and 0.2 us per MB of state that the chained kernel writes anyway.  Of 2076 random problems (8 .. 1024 heads,
 // D = 32 .. 80, blocks and block counts of up to 64, T = 1 .. 3) 170 are chosen, at 0.855 of the chained kernel's time; 3 % of them lose more than
-// 3 %, at most 9; of what the better kernel for each would gain this takes 84 %.  bf16, T = 2: 192 heads of 512 tokens in 32-row blocks 33.9
-// -> 30.6 us, 768 of 197 in 14 51.5 -> 40.4, 384 of 256 in 16 33.5 -> 26.5; 64 of 1024 in 32 (24.3, 28.8 in slices) and 12 of 512 (13.3, 15.3) stay.
+// 3 %, at most 9; of what the better kernel for each would gain this takes 84 %.  bf16, T = 2: 768 heads of 197
+// in 14-row blocks 51.5 -> 40.4 us, 384 of 256 in 16 33.5 -> 26.5; 64 of 1024 in 32 (24.3, 28.8 in slices) and 12 of 512 (13.3, 15.3) stay.  Without
+// the margin of 5 %: of 900 random problems 21 gain 3 - 12 % (192 of 512 in 32 33.9 -> 32.3 us) and 18 lose 3 - 15 %.
 bool slice_keeps(const ma_fwd_params* p) {
     if (p->variant != MA_VARIANT_AUTO || p->B > 64 || p->D > 80) return false;
     const int M = (p->N + p->B - 1) / p->B;
