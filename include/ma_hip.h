@@ -202,7 +202,10 @@ int ma_fwd_select_variant(const ma_fwd_params* p);
 
 /* Name of the kernel that does the bulk of the work for this problem under the variant it resolves to
  * (for the per-stage variants: the R-step kernel), as it appears in a profiler's kernel list; NULL for an
- * invalid problem.  Introspection for benchmarks and profiles; no counterpart in the reference. */
+ * invalid problem.  Introspection for tests, benchmarks and profiles; no counterpart in the reference.
+ * ma_fwd_keep_kernel_name, ma_matrix_kernel_name (the kernel that writes the matrix) and ma_bwd_kernel_name say the
+ * same of the calls below.  ma_bwd_kernel_name: "head_bwd", "r_bwd_tile", or "r_bwd_kernel" for the kernels that take
+ * any strides and pointers, as for *p without pointers. */
 const char* ma_fwd_kernel_name(const ma_fwd_params* p);
 
 /* Whole forward pass: replaces monarch_attention_torch (ma/ma_torch.py:65-108).
@@ -261,6 +264,7 @@ int ma_z_step(const ma_fwd_params* p, void* stream);
  * holds (M*B + 64*M floats <= 160 KB). */
 uint64_t ma_matrix_workspace_bytes(const ma_fwd_params* p);
 int ma_matrix(const ma_fwd_params* p, float* A, void* stream);
+const char* ma_matrix_kernel_name(const ma_fwd_params* p, const float* A);
 
 /* Backward pass.  The reference has no backward code: it differentiates
  * monarch_attention_torch (ma/ma_torch.py:65-108) with PyTorch autograd, which
@@ -289,6 +293,7 @@ typedef struct ma_bwd_params {
 
 uint64_t ma_bwd_workspace_bytes(const ma_bwd_params* p);
 int ma_bwd(const ma_bwd_params* p, void* stream);
+const char* ma_bwd_kernel_name(const ma_bwd_params* p);
 
 /* Forward call of a training step: ma_fwd that leaves every step's state (aL, cL, aR, cR and the last step's Y) in
  * `state`, so that ma_bwd_kept does not run the T steps a second time.  `state`: ma_fwd_state_bytes(p) bytes of device
@@ -301,6 +306,7 @@ int ma_bwd(const ma_bwd_params* p, void* stream);
 uint64_t ma_fwd_state_bytes(const ma_fwd_params* p);
 uint64_t ma_fwd_keep_workspace_bytes(const ma_fwd_params* p);
 int ma_fwd_keep(const ma_fwd_params* p, void* state, uint64_t state_bytes, void* stream);
+const char* ma_fwd_keep_kernel_name(const ma_fwd_params* p);
 uint64_t ma_bwd_kept_workspace_bytes(const ma_bwd_params* p);
 int ma_bwd_kept(const ma_bwd_params* p, const void* state, uint64_t state_bytes, void* stream);
 

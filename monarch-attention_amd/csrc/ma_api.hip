@@ -683,6 +683,9 @@ int select_keep_variant(const ma_fwd_params* p) {
     return auto_staged(p, heads, M) ? MA_VARIANT_STAGED : MA_VARIANT_CHAINED;
 }
 
+// ma_fwd_keep's kernels for that variant: the slice-resident one in place of the chained one?
+bool keeps_slices(const ma_fwd_params* p, int v) { return v == MA_VARIANT_CHAINED && slice_keeps(p); }
+
 int prepare(const ma_fwd_params* p, Prepared* out) {
     ma_ws_layout L;
     int st = layout_of(p, &L);
@@ -738,6 +741,12 @@ void at_step(Problem& P, const StateLayout& S, char* state, int t) {
     P.cR = reinterpret_cast<float*>(state + (t > 0 ? S.cR + (t - 1) * S.slot_c : S.cL));
 }
 
+// Name of the R-step kernel of the per-stage variants (see runs_long)
+const char* r_stage_name(const ma_fwd_params* p, int v) {
+    if (v == MA_VARIANT_GENERIC) return "r_step_kernel";
+    return p->dtype_qk == MA_F32 ? "r_step_f32" : p->B > 128 ? "r_step_long" : p->B > 64 ? "r_step_pair" : "r_step_mfma";
+}
+
 // The T steps as per-stage launches, every step's state kept; no Z step.
 int run_steps_kept(Prepared& pr, const ma_fwd_params* p, const StateLayout& S, char* state, hipStream_t s) {
     Problem& P = pr.P;
@@ -775,6 +784,36 @@ uint64_t matrix_workspace(const ma_fwd_params* p) {
     ma_ws_layout L;
     if (layout_of(p, &L) != MA_OK) return 0;
     return L.total + padded_rows(p) * ((static_cast<uint64_t>(p->B) + 3) / 4 * 4) * 4;
+}
+
+// The call of ma_matrix: its arguments with the variant of the T steps, and whether one launch does it all.
+struct MatrixCall {
+    ma_fwd_params pp;
+    bool slices;
+};
+int matrix_call(const ma_fwd_params* p, const float* A, MatrixCall* c) {
+    if (p == nullptr || A == nullptr) return MA_ERR_NULL;
+    if (reinterpret_cast<uintptr_t>(A) % 4) return MA_ERR_STRIDE;
+    // the T steps on q and k alone: v and out are stand-ins that no stage of this call touches
+    ma_fwd_params& pp = c->pp;
+    pp = *p;
+    pp.v = pp.q;
+    pp.out = const_cast<float*>(A);
+    pp.Dv = pp.D;
+    pp.dtype_v = pp.dtype_qk;
+    for (int i = 0; i < 3; ++i) pp.v_stride[i] = pp.out_stride[i] = pp.q_stride[i];
+    if (pp.E > 1 && pp.out_stride[0] == 0) pp.out_stride[0] = 1;   // q may be broadcast; the stand-in
+    if (pp.H > 1 && pp.out_stride[1] == 0) pp.out_stride[1] = 1;   // output must pass the overlap check
+    c->slices = false;
+    if (pp.variant != MA_VARIANT_AUTO && pp.variant != MA_VARIANT_GENERIC && pp.variant != MA_VARIANT_STAGED)
+        return pp.variant < MA_VARIANT_AUTO || pp.variant > MA_VARIANT_SLICED ? MA_ERR_VARIANT : MA_ERR_UNSUPPORTED;
+    if (pp.variant == MA_VARIANT_AUTO) {
+        const int st = check_shape(&pp);
+        if (st != MA_OK) return st;
+        pp.variant = mfma_supported(&pp) || mfma32_supported(&pp) ? MA_VARIANT_STAGED : MA_VARIANT_GENERIC;
+        c->slices = matrix_slice_pays(&pp) && run_matrix_slice(sizes_of(&pp), pp.dtype_qk, nullptr, nullptr) == MA_OK;
+    }
+    return MA_OK;
 }
 
 // Workspace of the backward pass: (ma_bwd) the forward state and the L step's scratch, then the state gradients and
@@ -1090,8 +1129,8 @@ const char* ma_fwd_kernel_name(const ma_fwd_params* p) {
     const int v = select_variant(p);
     if (v >= 0 && runs_slices(p, v)) return "resident_slice_mfma";
     switch (v) {
-        case MA_VARIANT_GENERIC: return "r_step_kernel";
-        case MA_VARIANT_STAGED: return f32 ? "r_step_f32" : p->B > 128 ? "r_step_long" : p->B > 64 ? "r_step_pair" : "r_step_mfma";   // (see runs_long)
+        case MA_VARIANT_GENERIC:
+        case MA_VARIANT_STAGED: return r_stage_name(p, v);
         case MA_VARIANT_FUSED: return "fused_fwd_mfma";
         case MA_VARIANT_CHAINED: return "chain_fwd_mfma";
         case MA_VARIANT_RESIDENT: {
@@ -1102,6 +1141,28 @@ const char* ma_fwd_kernel_name(const ma_fwd_params* p) {
         }
         default: return nullptr;
     }
+}
+
+const char* ma_fwd_keep_kernel_name(const ma_fwd_params* p) {
+    if (check_shape(p) != MA_OK) return nullptr;
+    const int v = select_keep_variant(p);
+    if (v < 0) return nullptr;
+    return keeps_slices(p, v) ? "resident_slice_mfma" : v == MA_VARIANT_CHAINED ? "chain_fwd_mfma" : r_stage_name(p, v);
+}
+
+const char* ma_matrix_kernel_name(const ma_fwd_params* p, const float* A) {
+    if (p == nullptr) return nullptr;
+    MatrixCall c;
+    if (matrix_call(p, A, &c) != MA_OK || check_shape(&c.pp) != MA_OK) return nullptr;
+    const int v = select_variant(&c.pp);
+    return c.slices ? "matrix_slice_mfma" : v < 0 ? nullptr : v == MA_VARIANT_STAGED ? "matrix_tile" : "matrix_kernel";
+}
+
+const char* ma_bwd_kernel_name(const ma_bwd_params* b) {
+    ma_fwd_params pp;
+    BwdLayout L;
+    if (bwd_prepare(b, true, &pp, &L) != MA_OK) return nullptr;
+    return L.head ? "head_bwd" : L.tiled ? "r_bwd_tile" : "r_bwd_kernel";
 }
 
 int ma_r_step(const ma_fwd_params* p, int first, int with_v, void* stream) {
@@ -1211,27 +1272,12 @@ uint64_t ma_matrix_workspace_bytes(const ma_fwd_params* p) {
 }
 
 int ma_matrix(const ma_fwd_params* p, float* A, void* stream) {
-    if (p == nullptr || A == nullptr) return MA_ERR_NULL;
-    if (reinterpret_cast<uintptr_t>(A) % 4) return MA_ERR_STRIDE;
-    // the T steps on q and k alone: v and out are stand-ins that no stage of this call touches
-    ma_fwd_params pp = *p;
-    pp.v = pp.q;
-    pp.out = A;
-    pp.Dv = pp.D;
-    pp.dtype_v = pp.dtype_qk;
-    for (int i = 0; i < 3; ++i) pp.v_stride[i] = pp.out_stride[i] = pp.q_stride[i];
-    if (pp.E > 1 && pp.out_stride[0] == 0) pp.out_stride[0] = 1;   // q may be broadcast; the stand-in
-    if (pp.H > 1 && pp.out_stride[1] == 0) pp.out_stride[1] = 1;   // output must pass the overlap check
-    if (pp.variant != MA_VARIANT_AUTO && pp.variant != MA_VARIANT_GENERIC && pp.variant != MA_VARIANT_STAGED)
-        return pp.variant < MA_VARIANT_AUTO || pp.variant > MA_VARIANT_SLICED ? MA_ERR_VARIANT : MA_ERR_UNSUPPORTED;
-    const bool choose = pp.variant == MA_VARIANT_AUTO;
-    if (pp.variant == MA_VARIANT_AUTO) {
-        const int st = check_shape(&pp);
-        if (st != MA_OK) return st;
-        pp.variant = mfma_supported(&pp) || mfma32_supported(&pp) ? MA_VARIANT_STAGED : MA_VARIANT_GENERIC;
-    }
+    MatrixCall c;
+    int st = matrix_call(p, A, &c);
+    if (st != MA_OK) return st;
+    const ma_fwd_params& pp = c.pp;
     Prepared pr;
-    int st = prepare(&pp, &pr);
+    st = prepare(&pp, &pr);
     if (st != MA_OK) return st;
     ma_ws_layout ws;
     layout_of(&pp, &ws);
@@ -1239,7 +1285,7 @@ int ma_matrix(const ma_fwd_params* p, float* A, void* stream) {
     const bool tiled = pr.variant == MA_VARIANT_STAGED && pp.workspace_bytes >= matrix_workspace(&pp);
     if (!tiled && !generic_matrix_fits(pr.P)) return MA_ERR_UNSUPPORTED;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (choose && matrix_slice_pays(&pp) && run_matrix_slice(pr.P, pp.dtype_qk, nullptr, s) == MA_OK) return run_matrix_slice(pr.P, pp.dtype_qk, A, s);
+    if (c.slices) return run_matrix_slice(pr.P, pp.dtype_qk, A, s);
     for (int t = 0; t < pp.T - 1; ++t) {
         st = run_r(pr, &pp, t == 0, false, s);
         if (st) return st;
@@ -1286,7 +1332,7 @@ int ma_fwd_keep(const ma_fwd_params* p, void* state, uint64_t state_bytes, void*
         pr.P.aR = base + S.aR;
         pr.P.cR = reinterpret_cast<float*>(base + S.cR);
         pr.P.slot_rows = static_cast<unsigned>(S.slot_rows);
-        if (slice_keeps(p)) {
+        if (keeps_slices(p, v)) {
             pr.P.one_tile_ok = 1;
             return run_slice(pr.P, p->dtype_qk, nullptr, s);
         }

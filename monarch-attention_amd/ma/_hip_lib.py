@@ -61,7 +61,7 @@ MA_FLAG_DEVICE_EXCLUSIVE = 4
 EXPORTS = ("ma_abi_version", "ma_strerror", "ma_fwd_workspace_layout", "ma_fwd_workspace_bytes",
            "ma_workspace_init", "ma_fwd_select_variant", "ma_fwd_kernel_name", "ma_fwd", "ma_fwd_static", "ma_r_step", "ma_l_step", "ma_z_step",
            "ma_matrix_workspace_bytes", "ma_matrix", "ma_bwd_workspace_bytes", "ma_bwd", "ma_fwd_state_bytes", "ma_fwd_keep_workspace_bytes", "ma_fwd_keep",
-           "ma_bwd_kept_workspace_bytes", "ma_bwd_kept")
+           "ma_bwd_kept_workspace_bytes", "ma_bwd_kept", "ma_fwd_keep_kernel_name", "ma_matrix_kernel_name", "ma_bwd_kernel_name")
 
 _lock = threading.Lock()
 _lib = None
@@ -136,6 +136,12 @@ def load() -> C.CDLL:
         lib.ma_bwd_kept_workspace_bytes.argtypes = [C.POINTER(BwdParams)]
         lib.ma_bwd_kept.restype = C.c_int
         lib.ma_bwd_kept.argtypes = [C.POINTER(BwdParams), C.c_void_p, C.c_uint64, C.c_void_p]
+        lib.ma_fwd_keep_kernel_name.restype = C.c_char_p
+        lib.ma_fwd_keep_kernel_name.argtypes = [P]
+        lib.ma_matrix_kernel_name.restype = C.c_char_p
+        lib.ma_matrix_kernel_name.argtypes = [P, C.c_void_p]
+        lib.ma_bwd_kernel_name.restype = C.c_char_p
+        lib.ma_bwd_kernel_name.argtypes = [C.POINTER(BwdParams)]
         got = lib.ma_abi_version()
         if got != ABI_VERSION:
             raise ImportError(f"libma_hip.so has ABI version {got}, this binding needs {ABI_VERSION}")

@@ -282,6 +282,46 @@ def test_auto_runs_slices_where_they_are_faster():
         assert (lib.ma_fwd_kernel_name(p) == b"resident_slice_mfma") == (slices < other), (heads, N, D, B, T)
 
 
+def call_params(heads, N, D, B, T=2, variant="auto", dt=L.MA_BF16):
+    """A backward call on contiguous tensors (its `fwd`: the recorded forward and the matrix call), with addresses that are never read."""
+    b = L.BwdParams()
+    b.fwd = good_params()
+    p = b.fwd
+    p.E, p.H, p.N, p.D, p.Dv, p.B, p.T, p.variant = heads, 1, N, D, D, B, T, L.VARIANTS[variant]
+    p.dtype_qk = p.dtype_v = dt
+    for field in ("q_stride", "k_stride", "v_stride", "out_stride"):
+        setattr(p, field, (C.c_int64 * 3)(N * D, N * D, D))
+    b.dout_stride = b.dq_stride = b.dk_stride = b.dv_stride = (C.c_int64 * 3)(N * D, N * D, D)
+    p.q = p.k = p.v = p.out = b.dout = b.dq = b.dk = b.dv = 0x100000
+    return b
+
+
+def matrix_kernel(b):
+    return L.load().ma_matrix_kernel_name(b.fwd, 0x100000)
+
+
+def test_kernel_names_of_recorded_matrix_and_backward_calls():
+    lib = L.load()
+    assert lib.ma_fwd_keep_kernel_name(call_params(768, 197, 64, 14).fwd) == b"resident_slice_mfma"
+    assert lib.ma_fwd_keep_kernel_name(call_params(192, 512, 64, 32).fwd) == b"chain_fwd_mfma"
+    assert lib.ma_fwd_keep_kernel_name(call_params(192, 512, 64, 32, variant="staged").fwd) == b"r_step_mfma"
+    assert lib.ma_fwd_keep_kernel_name(call_params(192, 512, 64, 32, dt=L.MA_F32).fwd) == b"r_step_f32"
+    assert lib.ma_fwd_keep_kernel_name(call_params(192, 512, 60, 32, variant="generic").fwd) == b"r_step_kernel"
+    assert lib.ma_fwd_keep_kernel_name(call_params(192, 512, 64, 32, variant="resident").fwd) is None
+    assert matrix_kernel(call_params(12, 1024, 64, 32)) == b"matrix_slice_mfma"
+    assert matrix_kernel(call_params(12, 1024, 64, 32, variant="staged")) == b"matrix_tile"
+    assert matrix_kernel(call_params(12, 1024, 64, 32, dt=L.MA_F32)) == b"matrix_tile"
+    assert matrix_kernel(call_params(12, 1024, 64, 32, variant="generic")) == b"matrix_kernel"
+    assert matrix_kernel(call_params(12, 1024, 64, 32, variant="chained")) is None
+    assert lib.ma_bwd_kernel_name(call_params(192, 512, 64, 32)) == b"head_bwd"
+    assert lib.ma_bwd_kernel_name(call_params(192, 2048, 64, 64)) == b"r_bwd_tile"
+    assert lib.ma_bwd_kernel_name(call_params(192, 512, 64, 32, variant="generic")) == b"r_bwd_kernel"
+    assert lib.ma_bwd_kernel_name(call_params(192, 512, 64, 32, variant="chained")) is None
+    without = call_params(192, 512, 64, 32)
+    without.dq = None
+    assert lib.ma_bwd_kernel_name(without) == b"r_bwd_kernel"
+
+
 def test_check_maps_status_to_python_exceptions():
     with pytest.raises(ValueError):
         L.check(L.MA_ERR_SHAPE, "x")
