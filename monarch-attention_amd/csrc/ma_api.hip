@@ -895,7 +895,7 @@ int bwd_prepare(const ma_bwd_params* b, bool kept, ma_fwd_params* pp, BwdLayout*
     L->tiled = bwd_tiled(b, pp, &L->rows16);
     // What a stage of the path does not use has no room of its own.  (ma_bwd's size is one for every path, so that it does
     // not depend on pointers a caller may not have yet; the T steps it runs again are the larger part of it anyway.)
-    L->head = bwd_head(b, pp, *L);
+    L->head = pp->variant == MA_VARIANT_AUTO && bwd_head(b, pp, *L);   // (STAGED: stage launches everywhere)
     const bool tight = kept && L->tiled, steps = pp->T > 1, staged = !tight || !L->head;
     const uint64_t rows = padded_rows(pp), es = tight ? elt_size(pp->dtype_qk) : 4;
     uint64_t off = kept ? 0 : state_layout(pp).total;

@@ -108,3 +108,36 @@ def assert_parity(out, ref, dt: str, what: str = ""):
         tol = REF_ALLCLOSE[dt]
         assert torch.allclose(out.float().cpu(), ref.float().cpu(), atol=tol, rtol=tol), (what, m)
     return m
+
+
+# ---- which kernel runs: the library's own answer for these tensors
+def keep_kernel(q, k, v, mask, T, B, pre, variant=None) -> str:
+    """The kernel of a recorded forward call."""
+    from ma import _hip_lib as L
+    from ma.ma_hip import make_params
+
+    return L.load().ma_fwd_keep_kernel_name(make_params(q, k, v, mask, torch.empty_like(v), T, B, pre, variant or "auto")).decode()
+
+
+def matrix_kernel(q, k, mask, T, B, pre, variant=None) -> str:
+    """The kernel that writes the dense matrix."""
+    from ma import _hip_lib as L
+    from ma.ma_hip import make_params
+
+    E, H, N, _ = q.shape
+    A = torch.empty(E, H, N, N, device=q.device)
+    return L.load().ma_matrix_kernel_name(make_params(q, k, q, mask, q, T, B, pre, variant or "auto"), A.data_ptr()).decode()
+
+
+def bwd_kernel(q, k, v, mask, dout, T, B, pre, variant=None) -> str:
+    """The kernel of a backward call with gradients laid out like their tensors."""
+    from ma import _hip_lib as L
+    from ma.ma_hip import make_params
+
+    grads = [torch.empty_like(t) for t in (q, k, v)]
+    b = L.BwdParams()
+    b.fwd = make_params(q, k, v, mask, grads[2], T, B, pre, variant or "auto")
+    for name, t in zip(("dout", "dq", "dk", "dv"), (dout, *grads)):
+        setattr(b, name, t.data_ptr())
+        setattr(b, name + "_stride", (L.C.c_int64 * 3)(*t.stride()[:3]))
+    return L.load().ma_bwd_kernel_name(b).decode()

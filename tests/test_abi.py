@@ -322,6 +322,17 @@ def test_kernel_names_of_recorded_matrix_and_backward_calls():
     assert lib.ma_bwd_kernel_name(without) == b"r_bwd_kernel"
 
 
+def test_staged_backward_of_short_heads_runs_the_stage_launches():
+    """The one-launch backward is AUTO's; STAGED asks for the stage launches and their workspace, where AUTO would not choose them."""
+    lib = L.load()
+    for heads, N, D, B, T in ((192, 512, 64, 32, 2), (768, 197, 64, 14, 2), (12, 256, 64, 16, 3)):
+        assert lib.ma_bwd_kernel_name(call_params(heads, N, D, B, T)) == b"head_bwd"
+        assert lib.ma_bwd_kernel_name(call_params(heads, N, D, B, T, "staged")) == b"r_bwd_tile"
+        one, stages = (lib.ma_bwd_kept_workspace_bytes(call_params(heads, N, D, B, T, v)) for v in ("auto", "staged"))
+        state = heads * N * D * 2
+        assert 0 < one and stages >= one + 3 * state   # gaL, gY and gaR
+
+
 def test_check_maps_status_to_python_exceptions():
     with pytest.raises(ValueError):
         L.check(L.MA_ERR_SHAPE, "x")
