@@ -725,15 +725,16 @@ __global__ __launch_bounds__(64 * W, 2) void head_bwd(HeadArgs) {
 // Does the kernel take the problem (dry), and its launch.
 template <class T, int DT>
 int launch(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, bool dry, hipStream_t s) {
-    if (P.B > 32 || P.M > 32) return MA_ERR_UNSUPPORTED;
+    constexpr int W = 8;
+    const long long grid = (static_cast<long long>(P.E) * P.H + 7) / 8 * 8;
+    if (P.B > 32 || P.M > 32 || !launchable(grid, 64 * W)) return MA_ERR_UNSUPPORTED;
     auto go = [&](auto ntb, auto ntm) {
-        constexpr int NTB = decltype(ntb)::value, NTM = decltype(ntm)::value, W = 8;
+        constexpr int NTB = decltype(ntb)::value, NTM = decltype(ntm)::value;
         auto start = [&](auto kernel, int BP, size_t bytes) {
             if (dry) return static_cast<int>(MA_OK);
             const int attr = mfma::set_lds_limit(kernel, kLdsMax);
             if (attr) return attr;
-            const unsigned grid = 8u * static_cast<unsigned>((static_cast<long long>(P.E) * P.H + 7) / 8);
-            hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * W), bytes, s, HeadArgs{P, G, BP, slot_a, slot_c});
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(64 * W), bytes, s, HeadArgs{P, G, BP, slot_a, slot_c});
             return static_cast<int>(hipGetLastError());
         };
         for (int BP = P.B | 1; BP >= P.B; --BP) {   // (an odd BP where it fits)

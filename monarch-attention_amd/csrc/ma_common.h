@@ -312,6 +312,10 @@ inline bool head32_single_step(const Problem& P) {
            static_cast<long long>(P.E) * P.H * P.B <= kHead32T1MaxGroups;
 }
 
+// Can a launch have that many workgroups?  A dispatch counts its work items in 32 bits, and a larger launch runs some of its workgroups
+// without an error.
+constexpr bool launchable(long long groups, int threads) { return groups * threads <= 0xffffffffLL; }
+
 // Chained forward (one launch, one workgroup per block problem, flags between phases).
 int launch_chain_f16_d2(const Problem& P, bool sync_ready, hipStream_t s);
 int launch_chain_f16_d4(const Problem& P, bool sync_ready, hipStream_t s);

@@ -186,10 +186,12 @@ __global__ __launch_bounds__(64 * W, W / 4) void matrix_slice_mfma(Problem P, fl
 // A == nullptr: does the kernel take the problem?
 template <class T, int DT>
 int launch_matrix_slice(const Problem& P, float* A, hipStream_t s) {
-    const int pos = matrix_positions(static_cast<long long>(P.E) * P.H, P.B, compute_units());
+    const long long heads = static_cast<long long>(P.E) * P.H;
+    const int pos = matrix_positions(heads, P.B, compute_units());
+    const long long grid = (heads < kMatrixSpread ? heads : (heads + 7) / 8 * 8) * ((P.B + pos - 1) / pos);
     constexpr size_t kLds = 160 * 1024;
     constexpr int W = DT <= 5 ? 16 : 8;
-    if (P.B > 32 || P.M > 32) return MA_ERR_UNSUPPORTED;
+    if (P.B > 32 || P.M > 32 || !launchable(grid, 64 * W)) return MA_ERR_UNSUPPORTED;
     auto go = [&](auto ntb, auto ntm) {
         constexpr int NTB = decltype(ntb)::value, NTM = decltype(ntm)::value;
         using SL = Slice<T, DT, NTB, NTM, W, kMatrix>;
@@ -199,7 +201,6 @@ int launch_matrix_slice(const Problem& P, float* A, hipStream_t s) {
         if (A == nullptr) return static_cast<int>(MA_OK);
         const int attr = set_lds_limit(matrix_slice_mfma<T, DT, NTB, NTM, W>, kLds);
         if (attr) return attr;
-        const long long heads = static_cast<long long>(P.E) * P.H, grid = (heads < kMatrixSpread ? heads : (heads + 7) / 8 * 8) * ((P.B + pos - 1) / pos);
         hipLaunchKernelGGL((matrix_slice_mfma<T, DT, NTB, NTM, W>), dim3(static_cast<unsigned>(grid)), dim3(64 * W), lds, s, P, A, pos);
         return static_cast<int>(hipGetLastError());
     };

@@ -333,6 +333,17 @@ def test_staged_backward_of_short_heads_runs_the_stage_launches():
         assert 0 < one and stages >= one + 3 * state   # gaL, gY and gaR
 
 
+def test_head_counts_beyond_the_work_items_of_one_launch():
+    """A dispatch counts its work items in 32 bits: workgroups of 512 and 1024 threads run out of them before the stage launches' do."""
+    lib = L.load()
+    most = (2 ** 32 - 1) // 512 // 8 * 8
+    assert lib.ma_bwd_kernel_name(call_params(most, 2, 8, 1)) == b"head_bwd"
+    assert lib.ma_bwd_kernel_name(call_params(most + 1, 2, 8, 1)) == b"r_bwd_tile"
+    most = (2 ** 32 - 1) // 1024 // 8 * 8
+    assert matrix_kernel(call_params(most, 2, 32, 1)) == b"matrix_slice_mfma"
+    assert matrix_kernel(call_params(most + 1, 2, 32, 1)) == b"matrix_tile"
+
+
 def test_check_maps_status_to_python_exceptions():
     with pytest.raises(ValueError):
         L.check(L.MA_ERR_SHAPE, "x")
