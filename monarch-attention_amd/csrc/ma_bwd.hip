@@ -370,6 +370,7 @@ int launch_bwd_z(const Problem& P, const BwdBuffers& G, int dt_qk, int dt_v, hip
     }
     const int TL = tile_rows(2 * P.M, P.M);
     const size_t lds = 2ull * TL * P.M * sizeof(float);
+    if (!launchable(static_cast<long long>(P.E) * P.H * P.B, kThreads)) return MA_ERR_UNSUPPORTED;
     return dispatch_qk(dt_qk, [&](auto tq) {
         using TQ = decltype(tq);
         return dispatch_qk(dt_v, [&](auto tv) {
@@ -388,6 +389,7 @@ int launch_bwd_l(const Problem& P, const BwdBuffers& G, int dt_qk, hipStream_t s
     }
     const int TL = tile_rows(2 * P.M, P.M);
     const size_t lds = 2ull * TL * P.M * sizeof(float);
+    if (!launchable(static_cast<long long>(P.E) * P.H * P.B, kThreads)) return MA_ERR_UNSUPPORTED;
     return dispatch_qk(dt_qk, [&](auto tq) {
         using TQ = decltype(tq);
         hipLaunchKernelGGL((l_bwd_kernel<TQ>), dim3(P.E * P.H * P.B), dim3(kThreads), lds, s, P, G, TL);
@@ -403,6 +405,7 @@ int launch_bwd_r(const Problem& P, const BwdBuffers& G, int dt_qk, int dt_v, boo
     }
     const int TJ = tile_rows(3 * P.B, P.B);
     const size_t lds = 3ull * TJ * P.B * sizeof(float);
+    if (!launchable(static_cast<long long>(P.E) * P.H * P.M, kThreads)) return MA_ERR_UNSUPPORTED;
     return dispatch_qk(dt_qk, [&](auto tq) {
         using TQ = decltype(tq);
         return dispatch_qk(dt_v, [&](auto tv) {

@@ -1305,6 +1305,7 @@ int launch_lz_t(const Problem& P, const BwdBuffers& G, bool z, hipStream_t s) {
     if (TL == 0) return static_cast<int>(MA_ERR_UNSUPPORTED);
     const size_t lds = bytes(TL);
     const int nth = threads_for((TL / 16) * (up(P.M, 16) / 16));
+    if (!launchable(static_cast<long long>(P.E) * P.H * P.B, nth)) return static_cast<int>(MA_ERR_UNSUPPORTED);
     auto launch = [&](auto kernel) {
         const int attr = mfma::set_lds_limit(kernel, kLdsBudget);
         if (attr) return attr;
@@ -1351,6 +1352,7 @@ int launch_r_t(const Problem& P, const BwdBuffers& G0, bool first, bool with_v, 
     const size_t lds = bytes(TJ);
     const int nth = threads_for((TJ / 16) * (up(P.B, 16) / 16));
     const long long grid = static_cast<long long>(P.E) * P.H * P.M * (G.jt_split ? G.jt_split : 1);
+    if (!launchable(grid, nth)) return static_cast<int>(MA_ERR_UNSUPPORTED);
     auto launch = [&](auto kernel) {
         const int attr = mfma::set_lds_limit(kernel, kLdsBudget);
         if (attr) return attr;

@@ -300,6 +300,7 @@ int launch_generic_r(const Problem& P, int dt_qk, int dt_v, bool first, bool wit
     const int TJ = tile_rows(P.B, 16);
     const long long grid = static_cast<long long>(P.E) * P.H * P.M * ((P.B + TJ - 1) / TJ);
     const size_t lds = static_cast<size_t>(TJ) * P.B * sizeof(float);
+    if (!launchable(grid, kThreads)) return MA_ERR_UNSUPPORTED;
     return dispatch_qk(dt_qk, [&](auto tq) {
         using TQ = decltype(tq);
         return dispatch_qk(dt_v, [&](auto tv) {
@@ -315,6 +316,7 @@ int launch_generic_l(const Problem& P, int dt_qk, hipStream_t s) {
     const int TL = tile_rows(P.M, 16);
     const int TK = tile_rows(P.M, 16);
     const long long ehb = static_cast<long long>(P.E) * P.H * P.B;
+    if (!launchable(ehb * ((P.M + TL - 1) / TL), kThreads)) return MA_ERR_UNSUPPORTED;   // (TK = TL)
     return dispatch_qk(dt_qk, [&](auto tq) {
         using TQ = decltype(tq);
         hipLaunchKernelGGL((l_stats_kernel<TQ>), dim3(ehb * ((P.M + TL - 1) / TL)), dim3(kThreads),
@@ -331,6 +333,7 @@ int launch_generic_z(const Problem& P, int dt_qk, int dt_v, hipStream_t s) {
     const int TL = tile_rows(P.M, 16);
     const long long grid = static_cast<long long>(P.E) * P.H * P.B * ((P.M + TL - 1) / TL);
     const size_t lds = static_cast<size_t>(TL) * P.M * sizeof(float);
+    if (!launchable(grid, kThreads)) return MA_ERR_UNSUPPORTED;
     return dispatch_qk(dt_qk, [&](auto tq) {
         using TQ = decltype(tq);
         return dispatch_qk(dt_v, [&](auto tv) {
@@ -345,7 +348,7 @@ bool generic_matrix_fits(const Problem& P) {
     const int TL = tile_rows(P.M, 64);
     const size_t lds = (static_cast<size_t>(P.M) * P.B + static_cast<size_t>(TL) * P.M) * sizeof(float);
     const long long grid = static_cast<long long>(P.E) * P.H * P.B * ((P.M + TL - 1) / TL);
-    return lds <= kMatrixLdsBytes && grid <= 0x7FFFFFFFLL;
+    return lds <= kMatrixLdsBytes && launchable(grid, kThreads);
 }
 
 int launch_generic_matrix(const Problem& P, int dt_qk, float* A, bool first, hipStream_t s) {

@@ -103,9 +103,10 @@ int launch_r(const Problem& P, bool first, bool with_v, hipStream_t s) {
         constexpr int DT = decltype(dt)::value, NWT = decltype(nt)::value;
         constexpr int WG = Split<NWT>::WG, PPW = Split<NWT, WG>::PPW;
         constexpr size_t lds = PPW * Lds<T, DT, NWT>::R;
+        const long long problems = static_cast<long long>(P.E) * P.H * P.M;
+        if (!launchable((problems + PPW - 1) / PPW, 64 * WG)) return static_cast<int>(MA_ERR_UNSUPPORTED);
         const int attr = set_lds_limit(r_step_mfma<T, DT, NWT>, lds);
         if (attr) return attr;
-        const long long problems = static_cast<long long>(P.E) * P.H * P.M;
         hipLaunchKernelGGL((r_step_mfma<T, DT, NWT>), dim3((problems + PPW - 1) / PPW), dim3(64 * WG), lds, s, P,
                            first ? 1 : 0, with_v ? 1 : 0);
         return static_cast<int>(hipGetLastError());
@@ -118,10 +119,11 @@ int launch_l(const Problem& P, hipStream_t s) {
         constexpr int DT = decltype(dt)::value, NWT = decltype(nt)::value;
         constexpr int WG = Split<NWT>::WG, PPW = Split<NWT, WG>::PPW;
         constexpr size_t lds = PPW * Lds<T, DT, NWT>::L;
-        const int attr = set_lds_limit(l_step_mfma<T, DT, NWT>, lds);
-        if (attr) return attr;
         const long long per = NWT == 1 ? (16 >> P.pack_shift) : 1;   // positions per problem (see TileIndex)
         const long long problems = static_cast<long long>(P.E) * P.H * ((P.B + per - 1) / per);
+        if (!launchable((problems + PPW - 1) / PPW, 64 * WG)) return static_cast<int>(MA_ERR_UNSUPPORTED);
+        const int attr = set_lds_limit(l_step_mfma<T, DT, NWT>, lds);
+        if (attr) return attr;
         hipLaunchKernelGGL((l_step_mfma<T, DT, NWT>), dim3((problems + PPW - 1) / PPW), dim3(64 * WG), lds, s, P);
         return static_cast<int>(hipGetLastError());
     });
@@ -133,10 +135,11 @@ int launch_z(const Problem& P, hipStream_t s) {
         constexpr int DT = decltype(dt)::value, NWT = decltype(nt)::value;
         constexpr int WG = Split<NWT>::WG, PPW = Split<NWT, WG>::PPW;
         constexpr size_t lds = PPW * Lds<T, DT, NWT>::Z;
-        const int attr = set_lds_limit(z_step_mfma<T, DT, NWT>, lds);
-        if (attr) return attr;
         const long long per = NWT == 1 ? (16 >> P.pack_shift) : 1;
         const long long problems = static_cast<long long>(P.E) * P.H * ((P.B + per - 1) / per);
+        if (!launchable((problems + PPW - 1) / PPW, 64 * WG)) return static_cast<int>(MA_ERR_UNSUPPORTED);
+        const int attr = set_lds_limit(z_step_mfma<T, DT, NWT>, lds);
+        if (attr) return attr;
         hipLaunchKernelGGL((z_step_mfma<T, DT, NWT>), dim3((problems + PPW - 1) / PPW), dim3(64 * WG), lds, s, P);
         return static_cast<int>(hipGetLastError());
     });

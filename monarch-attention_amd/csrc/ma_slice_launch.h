@@ -39,6 +39,7 @@ int launch_slice_one(const Problem& P, SlicePlan* plan, hipStream_t s) {
     const int units = compute_units();
     const bool shared = kShort && slices > units && 2 * Narrow::layout(P.D, P.M).total <= kSliceLds;
     const bool wide = !shared && Wide::takes(P.D, P.M, P.B, kSliceLds);
+    if (!launchable((static_cast<long long>(P.E) * P.H + 7) / 8 * 8 * ((P.B + 15) / 16), 64 * (wide ? WIDE : 8))) return MA_ERR_UNSUPPORTED;
     if (plan != nullptr) {
         *plan = SlicePlan{wide ? WIDE : 8, shared ? 2 : 1, units};
         return MA_OK;

@@ -351,9 +351,10 @@ int each_launch(int n, long long problems, F&& f) {
 
 template <class Kernel, class... Args>
 int run(Kernel kernel, size_t lds, long long problems, int groups, int w, hipStream_t s, Args... args) {
+    const long long grid = groups == 1 ? problems : (problems + 7) / 8 * 8 * groups;
+    if (!launchable(grid, 64 * w)) return MA_ERR_UNSUPPORTED;
     const int attr = mfma::set_lds_limit(kernel, lds);
     if (attr) return attr;
-    const long long grid = groups == 1 ? problems : (problems + 7) / 8 * 8 * groups;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(64 * w), lds, s, args...);
     return static_cast<int>(hipGetLastError());
 }

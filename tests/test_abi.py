@@ -558,3 +558,22 @@ def test_workspaces_hold_what_the_path_uses():
     p.Dv = 60
     assert lib.ma_matrix_workspace_bytes(p) == lib.ma_fwd_workspace_bytes(p)
     assert lib.ma_matrix_workspace_bytes(params(2, 0, "generic").fwd) == lib.ma_fwd_workspace_bytes(params(2, 0).fwd)
+
+
+@pytest.mark.parametrize("variant,D,dt", [("staged", 8, L.MA_F16), ("staged", 8, L.MA_F32), ("generic", 3, L.MA_F16), ("sliced", 32, L.MA_F16)])
+def test_launches_of_more_than_2_to_the_32_work_items_are_refused(variant, D, dt):
+    """The runtime would run some of the workgroups and report nothing.  2^27 heads of one token."""
+    lib = L.load()
+    b = call_params(2 ** 27, 1, D, 1, 2, variant, dt)
+    p = b.fwd
+    p.eps = 1e-12
+    p.workspace = 0x100000
+    p.workspace_bytes = 1 << 50
+    assert lib.ma_fwd(p, None) == L.MA_ERR_UNSUPPORTED
+    if variant == "sliced":
+        return
+    for fn in (lambda: lib.ma_r_step(p, 1, 1, None), lambda: lib.ma_l_step(p, None), lambda: lib.ma_z_step(p, None),
+               lambda: lib.ma_fwd_keep(p, 0x100000, 1 << 50, None), lambda: lib.ma_matrix(p, 0x100000, None)):
+        assert fn() == L.MA_ERR_UNSUPPORTED
+    if variant == "staged":   # (GENERIC clears its accumulators first)
+        assert lib.ma_bwd_kept(b, 0x100000, 1 << 50, None) == L.MA_ERR_UNSUPPORTED
