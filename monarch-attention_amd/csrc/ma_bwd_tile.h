@@ -48,17 +48,18 @@ namespace bwdt {
 
 using namespace tile;
 
-// The second launch of 16 strips of 16-bit operands, eight of them per workgroup: two workgroups share a compute unit where the tiles are
-// walked in chunks of half of the LDS and a wave keeps to 128 registers (held to them from 65 columns on; narrower classes need fewer).  The stages that form two gradients of more than 80 columns do
-// not (150 to 250 registers): they take the LDS whole, see RSplit.
+// The second launch of 16 strips of 16-bit operands, four or eight of them per workgroup: two workgroups share a compute unit where the
+// tiles are walked in chunks of half of the LDS and a wave of eight keeps to 128 registers (held to them from 65 columns on; narrower
+// classes need fewer).  The stages that form two gradients of more than 80 columns do not (150 to 250 registers): they take the LDS
+// whole, see RSplit; so do launches with no second workgroup for a compute unit (WHOLE), see few_workgroups.
 template <class T>
 constexpr bool shares_lds(int DT, int NWT, int PASS, bool two_gradients) {
     return sizeof(T) == 2 && NWT == 16 && PASS == 2 && !(two_gradients && DT >= 6);
 }
-template <class T, int DT, int NWT, int PASS, bool kV>
-using RPlan = Plan<T, DT, NWT, PASS, kV ? 2 : 1, kV ? 3 : 2, 7, shares_lds<T>(DT, NWT, PASS, kV)>;
-template <class T, int DT, int NWT, int PASS, bool kZ>
-using LzPlan = Plan<T, DT, NWT, PASS, 2, kZ ? 2 : 1, 5, shares_lds<T>(DT, NWT, PASS, kZ)>;
+template <class T, int DT, int NWT, int PASS, bool kV, bool WHOLE = false>
+using RPlan = Plan<T, DT, NWT, PASS, kV ? 2 : 1, kV ? 3 : 2, 7, !WHOLE && shares_lds<T>(DT, NWT, PASS, kV)>;
+template <class T, int DT, int NWT, int PASS, bool kZ, bool WHOLE = false>
+using LzPlan = Plan<T, DT, NWT, PASS, 2, kZ ? 2 : 1, 5, !WHOLE && shares_lds<T>(DT, NWT, PASS, kZ)>;
 
 // A term that a product's sum is shifted by: 16-bit operands start the accumulators at it; fp32 sums, which would then be rounded
 // at its magnitude in every step, take it at the end.
@@ -97,10 +98,10 @@ constexpr int r_held_waves(int DT, int NWT, bool kV) {
     if (DT <= 6) return (NWT == 5 && (DT == 6 || kV)) || (NWT == 7 && !kV) ? 4 : NWT == 3 || NWT == 4 || (NWT == 6 && kV) ? 3 : 1;
     return NWT == 5 && !kV ? 4 : NWT == 3 || NWT == 4 ? 3 : 1;
 }
-template <class T, int DT, int NWT, int W, int PASS, bool kV>
+template <class T, int DT, int NWT, int W, int PASS, bool kV, bool WHOLE = false>
 __global__ __launch_bounds__(64 * W, sizeof(T) == 2 && PASS == 0 ? r_held_waves(DT, NWT, kV) : DT >= 5 && W == 8 && shares_lds<T>(DT, NWT, PASS, kV) ? 4 : 1) void r_bwd_tile(Problem P, BwdBuffers G, int first) {
     using MT = Mat<T, DT>;
-    using PL = RPlan<T, DT, NWT, PASS, kV>;
+    using PL = RPlan<T, DT, NWT, PASS, kV, WHOLE>;
     using mfma::quad_rows_max;
     using mfma::quad_rows_sum;
     constexpr int NTH = 64 * W, ROWS = PL::ROWS, CT1 = PL::CT1, CT2 = PL::CT2;
@@ -429,10 +430,10 @@ constexpr int lz_held_waves(int DT, int NWT, bool kZ) {
     if (kZ) return NWT == 3 || NWT == 4 || NWT == 6 ? 3 : 1;
     return NWT == 4 || NWT == 5 ? 4 : 1;
 }
-template <class T, int DT, int NWT, int W, int PASS, bool kZ>
+template <class T, int DT, int NWT, int W, int PASS, bool kZ, bool WHOLE = false>
 __global__ __launch_bounds__(64 * W, sizeof(T) == 2 && PASS == 0 ? lz_held_waves(DT, NWT, kZ) : DT >= 5 && W == 8 && shares_lds<T>(DT, NWT, PASS, kZ) ? 4 : 1) void lz_bwd_tile(Problem P, BwdBuffers G) {
     using MT = Mat<T, DT>;
-    using PL = LzPlan<T, DT, NWT, PASS, kZ>;
+    using PL = LzPlan<T, DT, NWT, PASS, kZ, WHOLE>;
     using mfma::quad_rows_max;
     using mfma::quad_rows_sum;
     constexpr int NTH = 64 * W, ROWS = PL::ROWS, CT1 = PL::CT1, CT2 = PL::CT2;
@@ -710,6 +711,12 @@ template <int DT, bool kZ>
 struct LzSplit {
     static constexpr Split16 of{true, true, DT >= 5 ? 8 : 4, kZ && DT == 6 ? 16 : 8};
 };
+// Does a launch of `groups` workgroups per problem leave every workgroup a compute unit to itself?  Walking its tiles in halves then only adds
+// barriers: 12 .. 64 problems of 256 rows in four workgroups each, bf16, forward and backward of one step, us, D = 48 R with V 40.2 ->
+// 38.0, 64 42.3 -> 40.0, 80 L and Z 44.6 -> 42.4 (two steps 0.97); 96 .. 240 problems, of which two share a unit, 1.03 - 1.13 of the time
+// with the LDS whole (D = 80, 240 problems 114 -> 129).
+inline bool few_workgroups(long long problems, int groups) { return (problems + 7) / 8 * 8 * groups <= mfma::compute_units(); }
+
 template <class T, int DT, bool kV>
 int launch_r(const Problem& P, const BwdBuffers& G, bool first, hipStream_t s) {
     const long long problems = static_cast<long long>(P.E) * P.H * P.M;
@@ -720,6 +727,9 @@ int launch_r(const Problem& P, const BwdBuffers& G, bool first, hipStream_t s) {
             const int st = run(r_bwd_tile<T, DT, NWT, NWT / 2, 1, kV>, RPlan<T, DT, NWT, 1, kV>::kLds, problems, 2, NWT / 2, s, P, G, first ? 1 : 0);
             return st ? st : run(r_bwd_tile<T, DT, NWT, NWT / 2, 2, kV>, RPlan<T, DT, NWT, 2, kV>::kLds, problems, 2, NWT / 2, s, P, G, first ? 1 : 0);
         } else {
+            if constexpr (W == 4 && RPlan<T, DT, NWT, PASS, kV>::NC2 != RPlan<T, DT, NWT, PASS, kV, true>::NC2)
+                if (few_workgroups(problems, NWT / W))
+                    return run(r_bwd_tile<T, DT, NWT, W, PASS, kV, true>, RPlan<T, DT, NWT, PASS, kV, true>::kLds, problems, NWT / W, W, s, P, G, first ? 1 : 0);
             return run(r_bwd_tile<T, DT, NWT, W, PASS, kV>, RPlan<T, DT, NWT, PASS, kV>::kLds, problems, NWT / W, W, s, P, G, first ? 1 : 0);
         }
     });
@@ -731,6 +741,9 @@ int launch_lz(const Problem& P, const BwdBuffers& G, hipStream_t s) {
     return each_launch<sizeof(T) == 4, LzSplit<DT, kZ>>(P.M, problems, [&](auto nwt, auto w, auto pass) {
         constexpr int NWT = decltype(nwt)::value, W = decltype(w)::value, PASS = decltype(pass)::value;
         static_assert(LzPlan<T, DT, NWT, PASS, kZ>::kFits, "two tiles of up to 128 rows fit the LDS");
+        if constexpr (W == 4 && LzPlan<T, DT, NWT, PASS, kZ>::NC2 != LzPlan<T, DT, NWT, PASS, kZ, true>::NC2)
+            if (few_workgroups(problems, NWT / W))
+                return run(lz_bwd_tile<T, DT, NWT, W, PASS, kZ, true>, LzPlan<T, DT, NWT, PASS, kZ, true>::kLds, problems, NWT / W, W, s, P, G);
         return run(lz_bwd_tile<T, DT, NWT, W, PASS, kZ>, LzPlan<T, DT, NWT, PASS, kZ>::kLds, problems, NWT / W, W, s, P, G);
     });
 }
