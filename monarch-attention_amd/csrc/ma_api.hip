@@ -849,22 +849,35 @@ bool bwd_tiled(const ma_bwd_params* b, const ma_fwd_params* pp, bool* rows16) {
     return bits % (4 * es) == 0;
 }
 
-// Does the whole pass run as one launch, a workgroup per head (ma_bwd_head.h)?  Times are those of a training call, in multiples of
-// the stage launches' (bf16, (E, N, H, D), mask; 256 compute units).  Blocks and block counts of up to 16: always - 0.55 .. 0.75 for 512
-// heads and more of 197 - 256 tokens at T = 2, 0.82 .. 0.96 for 12 heads and more, whose calls are host time by then.  17 .. 32 rows
-// one way or both: a head has a compute unit to itself and three to five times the work, so a pass has to be mostly full.  512 tokens in
-// 32-row blocks, T = 2 | 3: 96 heads 1.00 | 1.03, 128 0.96 | 0.91, 160 0.88 | 0.83, 256 0.71 | 0.68, 264 0.95, 320 0.86, 512 0.80; 480 in
-// 24-row blocks: 128 heads 1.09 | 1.06, 160 0.96 | 0.92, 256 0.79 | 0.75, 264 1.11, 320 0.98, 528 1.02, 576 0.95; 300 tokens in
-// 16: 264 1.17, 320 1.05, 352 0.98, 528 0.94; a single step: 264 1.15 - 1.20, 320 1.05 - 1.08; D = 72, 320 tokens in 32: 192 0.92, 352 1.04,
-// 576 1.05, 768 0.93.  Few heads are calls of host time, where one launch in place of four saves 3 - 14 % (up to 48 heads, T = 2; at
-// T = 3 the one chain is longer than six launches: 1.14 - 1.22).
+// Does the whole pass run as one launch, a workgroup per head (ma_bwd_head.h), or as 2 T stage launches?  A head has a compute unit to
+// itself, where eight waves walk its blocks and positions in rounds, so its time is passes over the compute units x rounds; the stage
+// launches' is the work spread over the device beside 2 T dependent launches.  Estimates in us, fitted on one MI355X (256 units) to 6488
+// random problems (D = 8 .. 96, 1 .. 4096 heads, T = 1 .. 4) by the mean of three clocks: back to back in a graph, calls from the host, and a call
+// that is waited for; within 15 and 12 % for nine in ten.  profiles/one_launch_rules_sweep.md has the table.  By the kind of problem, one
+// launch in multiples of the stages: up to 16 rows both ways 0.65 for 52 .. 256 heads, 0.77 beyond, where more than a block or two fill the rounds,
+// 0.75 for few heads but 96 columns; 17 .. 32 rows one way 0.8 - 0.87 in full passes, 1.3 - 1.6 for up to 50 heads; both ways 0.8.
+float bwd_head_us(const ma_fwd_params* p, int M, long long units) {
+    const int B = p->B, dt = p->D <= 32 ? 2 : p->D <= 64 ? 4 : 6;   // its classes of 16 columns
+    const long long heads = static_cast<long long>(p->E) * p->H, rows = static_cast<long long>(M) * B, passes = (heads + units - 1) / units;
+    const float T = static_cast<float>(p->T);
+    const float r = static_cast<float>((M + 7) / 8) * (B <= 16 ? 0.99f + 0.17f * dt : 1.63f + 0.63f * dt);
+    const float l = static_cast<float>((B + 7) / 8) * (M <= 16 ? 0.55f + 0.26f * dt : 0.62f + 0.87f * dt);
+    const bool dq_in_lds = rows * (128 * dt + 5) + 4096 * dt + 5120 <= 160 * 1024;
+    const float pass = 1.13f + T * (r + l) + (dq_in_lds ? 0.f : 0.45f / 256 * T * static_cast<float>(rows) * dt);
+    return 6.32f + 0.58f * T + static_cast<float>(passes) * pass + 2e-6f * heads * rows * p->D * (0.86f + 0.3f * T);
+}
+float bwd_stages_us(const ma_fwd_params* p, int M, long long units) {
+    const int B = p->B, dt = p->D <= 32 ? 2 : p->D <= 64 ? 4 : 6, strips = (B > 16 ? 2 : 1) + (M > 16 ? 2 : 1);
+    const float T = static_cast<float>(p->T), heads = static_cast<float>(p->E) * p->H;
+    const float chain = 8.13f + T * (0.69f * strips + 0.95f * dt - 3.06f);
+    const float problems = heads / static_cast<float>(units) * (M * (B <= 16 ? 0.028f : 0.077f) + B * (M <= 16 ? 0.018f : 0.053f));
+    const float work = 9.26f * T + problems * T * (4.05f + dt) + 2e-6f * heads * M * B * p->D * (1.13f + 1.35f * T);
+    return std::sqrt(chain * chain + work * work);
+}
+// The margin: without it 136 of the 6488 lose more than 10 %, with it 60, of 3200 chosen at 0.78 of the stages' time (at most 1.4).
 bool bwd_head_pays(const ma_fwd_params* pp) {
-    const int M = (pp->N + pp->B - 1) / pp->B, strips = (pp->B + 15) / 16 + (M + 15) / 16;
-    if (strips == 2) return true;
-    const long long heads = static_cast<long long>(pp->E) * pp->H, units = mfma::compute_units(), passes = (heads + units - 1) / units;
-    if (strips == 3 && pp->D <= 64 && pp->T == 2 && heads <= units / 5) return true;
-    if (passes == 1) return 8 * heads >= (pp->D > 64 ? 6 : strips == 3 || pp->D <= 32 ? 4 : 5) * units;
-    return 8 * heads >= (pp->D > 64 ? 7 : 6) * passes * units;
+    const int M = (pp->N + pp->B - 1) / pp->B, units = mfma::compute_units();
+    return bwd_head_us(pp, M, units) < 0.95f * bwd_stages_us(pp, M, units);
 }
 bool bwd_head(const ma_bwd_params* b, const ma_fwd_params* pp, const BwdLayout& L) {
     if (pp->B > 32 || pp->N > 32 * pp->B || !L.tiled || !L.rows16 || pp->dtype_qk == MA_F32 || pp->D % 8 != 0 || !bwd_head_pays(pp)) return false;

@@ -337,11 +337,28 @@ def test_head_counts_beyond_the_work_items_of_one_launch():
     """A dispatch counts its work items in 32 bits: workgroups of 512 and 1024 threads run out of them before the stage launches' do."""
     lib = L.load()
     most = (2 ** 32 - 1) // 512 // 8 * 8
-    assert lib.ma_bwd_kernel_name(call_params(most, 2, 8, 1)) == b"head_bwd"
-    assert lib.ma_bwd_kernel_name(call_params(most + 1, 2, 8, 1)) == b"r_bwd_tile"
+    assert lib.ma_bwd_kernel_name(call_params(most, 64, 24, 8)) == b"head_bwd"
+    assert lib.ma_bwd_kernel_name(call_params(most + 1, 64, 24, 8)) == b"r_bwd_tile"
     most = (2 ** 32 - 1) // 1024 // 8 * 8
     assert matrix_kernel(call_params(most, 2, 32, 1)) == b"matrix_slice_mfma"
     assert matrix_kernel(call_params(most + 1, 2, 32, 1)) == b"matrix_tile"
+
+
+def test_auto_runs_the_one_launch_backward_where_it_is_faster():
+    """AUTO's choice for the backward of short heads, at shapes where one side took at most 0.85 of the other's time (us of the backward
+    alone on an MI355X: one launch, stage launches)."""
+    lib = L.load()
+    for heads, N, D, B, T, one, stages in (
+            # few heads of 17 .. 32 rows one way; few blocks, of which most waves have none
+            (10, 460, 8, 30, 2, 28.0, 15.8), (14, 332, 24, 31, 2, 25.9, 16.7), (2, 249, 8, 12, 2, 22.5, 15.0), (27, 161, 64, 7, 2, 27.7, 20.2),
+            (21, 422, 8, 32, 2, 28.6, 17.5), (640, 14, 24, 19, 2, 43.0, 30.7), (1024, 37, 8, 30, 1, 39.1, 30.3), (768, 3, 96, 22, 2, 96.4, 67.4),
+            (1937, 16, 40, 7, 2, 79.4, 50.8), (2886, 3, 72, 12, 1, 88.9, 49.5), (2, 214, 96, 14, 1, 15.9, 10.8),
+            # its own ground
+            (192, 512, 64, 32, 2, 58.0, 84.0), (768, 197, 64, 14, 2, 72.0, 142.0), (23, 10, 96, 1, 3, 19.5, 27.4), (287, 178, 24, 15, 3, 39.0, 57.5),
+            (420, 281, 24, 32, 4, 96.6, 129.1), (1082, 557, 24, 20, 1, 124.7, 161.1), (224, 243, 48, 32, 2, 35.7, 49.5), (256, 53, 8, 26, 3, 27.4, 37.1),
+            (212, 567, 32, 31, 2, 51.6, 71.7), (192, 148, 24, 6, 3, 28.6, 47.9)):
+        name = lib.ma_bwd_kernel_name(call_params(heads, N, D, B, T))
+        assert name == (b"head_bwd" if one < stages else b"r_bwd_tile"), (heads, N, D, B, T)
 
 
 def test_check_maps_status_to_python_exceptions():
