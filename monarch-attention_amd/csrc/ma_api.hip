@@ -764,18 +764,23 @@ int run_steps_kept(Prepared& pr, const ma_fwd_params* p, const StateLayout& S, c
     return MA_OK;
 }
 
-// AUTO, dense matrix of 16-bit operands: is the one launch of ma_matrix_slice.h ahead of the 2 T stage launches?  1388 random problems of up to 32
-// blocks of up to 32 rows, 1 .. 200 heads, in multiples of the stage launches' time, the host's part of the call with it.  Up to 16
-// blocks: 0.74 at T = 1 (at most 1.08), 0.51 at T = 2, 0.45 at T = 3.  17 .. 32 blocks, where a wave has two blocks and an L problem four tiles:
-// D <= 80 0.77 and 0.72 at T = 2, 3 (beyond 128 heads up to 1.14); a single step 0.92 (0.75 .. 1.24) below 16 heads, 0.73 - 0.93 from there, 1.12 (up
-// to 1.57) beyond 128; D > 80, in eight waves, 0.95 (0.77 .. 1.2) below 8 heads, 0.80 above, at T = 1 1.18, 0.98 and, from 64 heads on, 0.86.  12
-// heads of 1024 tokens in 32-row blocks, T = 2: 25.1 -> 21.9 us.
+// AUTO, dense matrix of 16-bit operands: is the one launch of ma_matrix_slice.h ahead of the 2 T stage launches?  2874 random problems of up
+// to 32 blocks of up to 32 rows, 1 .. 2048 heads, in multiples of the stage launches' time, by the mean of three clocks (a replayed graph,
+// calls from the host, calls that are waited for; profiles/one_launch_rules_sweep.md).  Up to 16 blocks: 0.79 at T = 1, 0.66 at T = 2, 0.55 at
+// T = 3.  Beyond two heads per compute unit a workgroup of one to three positions, or of one or two blocks, has work for few of its waves:
+// up to 1.7, they stay away.  17 .. 32 blocks, where a wave has two blocks and an L problem four tiles: a single step 1.0 - 1.2 below 32
+// heads, 0.88 from there, 0.95 - 1.0 (up to 1.25) for more than 200 MB of matrix, which the stage launches write at the rate of the memory;
+// T = 2 0.91 from the first head up to 64 columns, 1.0 - 1.1 of 1 .. 7 heads up to 80 and of up to 31 beyond (eight waves), then 0.85; T = 3
+// 0.84, of 1 .. 7 heads above 80 columns 1.01.  12 heads of 1024 tokens in 32-row blocks, T = 2: 25.1 -> 21.9 us.
 bool matrix_slice_pays(const ma_fwd_params* p) {
     const int M = (p->N + p->B - 1) / p->B;
     const long long heads = static_cast<long long>(p->E) * p->H;
     if (p->B > 32 || M > 32 || !mfma_supported(p)) return false;
+    const bool many = heads > 2 * mfma::compute_units();
+    if (many && (p->B <= 3 || M <= 2)) return false;
     if (M <= 16) return true;
-    if (p->T == 1) return heads >= (p->D > 80 ? 64 : 16) && heads <= 128;
+    if (p->T == 1) return heads >= 32 && heads * p->N * p->N <= 50000000;   // (entries of four bytes)
+    if (p->T == 2) return heads >= (p->D > 80 ? 32 : p->D > 64 ? 8 : 1);
     return heads >= (p->D > 80 ? 8 : 1);
 }
 

@@ -10,7 +10,7 @@ must not fall back silently.
 import pytest
 import torch
 
-from helpers import (DT, assert_parity, block_safe_mask, err_metrics, golden_names, load_golden, seeded_qkv)
+from helpers import (DT, assert_parity, block_safe_mask, err_metrics, golden_names, load_golden, matrix_kernel, seeded_qkv)
 from ma import _hip_lib as L
 from ma.ma_hip import make_params, monarch_attention_hip, monarch_attention_hip_backward, monarch_matrix_hip, sync_status
 from ma.monarch_attention import MonarchAttention, PadType
@@ -875,10 +875,15 @@ def test_matrix_kernel_equals_forward_on_identity(case):
 MATRIX_SHORT = [  # E, H, N, D, B, T, pre, dt, masked: one launch; strips of 1 and 2 both ways, their edges, every column class
     (1, 1, 1, 32, 1, 2, False, "f16", False), (1, 2, 16, 64, 1, 1, False, "bf16", True), (1, 3, 45, 40, 3, 3, True, "f16", True),
     (1, 2, 255, 64, 16, 2, True, "bf16", True), (2, 3, 272, 48, 17, 2, False, "f16", True), (1, 2, 512, 72, 32, 3, True, "f16", False),
-    (1, 1, 289, 80, 17, 2, False, "bf16", True), (1, 12, 1024, 64, 32, 2, False, "f16", False), (3, 3, 500, 96, 16, 2, True, "bf16", True),
-    (1, 2, 200, 128, 13, 3, True, "f16", True), (2, 5, 527, 128, 31, 2, False, "bf16", False),
+    (1, 1, 289, 80, 17, 3, False, "bf16", True), (1, 12, 1024, 64, 32, 2, False, "f16", False), (4, 8, 500, 96, 16, 2, True, "bf16", True),
+    (1, 2, 200, 128, 13, 3, True, "f16", True), (2, 5, 527, 128, 31, 3, False, "bf16", False),
     # one step of 17 .. 32 blocks, heads that stay on one XCD (32 and more), several positions to a workgroup, two passes
-    (4, 4, 270, 64, 10, 1, False, "f16", True), (5, 7, 196, 32, 28, 2, True, "bf16", True), (13, 11, 120, 64, 19, 1, False, "f16", True),
+    (4, 8, 270, 64, 10, 1, False, "f16", True), (5, 7, 196, 32, 28, 2, True, "bf16", True), (13, 11, 120, 64, 19, 1, False, "f16", True),
+    # the builds (columns, strips of a block and of a position) that the rows above leave out
+    (1, 2, 300, 32, 10, 2, False, "bf16", True), (1, 2, 500, 32, 24, 2, True, "f16", False), (1, 3, 330, 48, 15, 3, True, "bf16", False),
+    (1, 2, 700, 40, 25, 2, False, "f16", True), (1, 2, 150, 80, 12, 2, True, "f16", True), (1, 9, 240, 72, 10, 2, False, "bf16", False),
+    (1, 2, 100, 96, 9, 2, True, "bf16", True), (1, 2, 250, 96, 20, 2, False, "f16", True), (2, 5, 420, 96, 20, 3, True, "f16", False),
+    (3, 3, 200, 128, 9, 3, False, "bf16", True), (1, 2, 300, 128, 30, 2, True, "bf16", False),
 ]
 
 
@@ -893,6 +898,7 @@ def test_matrix_of_short_sequences(case):
     junk = torch.full((E, H, N, N), float("nan"), device=DEV)
     del junk
     A = monarch_matrix_hip(dq, dk, dm, T, B, pre)
+    assert matrix_kernel(dq, dk, dm, T, B, pre) == "matrix_slice_mfma" and matrix_kernel(dq, dk, dm, T, B, pre, "staged") == "matrix_tile"
     heads = slice(0, 2)
     assert_parity(A[:1, heads].cpu(), monarch_matrix_oracle(q[:1, heads], k[:1, heads], None if mask is None else mask[:1], T, B, pre), dt)
     assert_parity(A[-1:, -1:].cpu(), monarch_matrix_oracle(q[-1:, -1:], k[-1:, -1:], None if mask is None else mask[-1:], T, B, pre), dt)
