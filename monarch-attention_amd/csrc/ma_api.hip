@@ -243,7 +243,8 @@ bool slice_fits(const ma_fwd_params* p, SlicePlan* plan, bool keep = false) {
 // any free place, so its time is the tasks over the places beside the latency of 2 T dependent phases.  Both times are estimated in
 // us from the shape: fitted on one MI355X (256 units) to 70634 random problems (D = 32 .. 80, 1 .. 4096 tokens, 1 .. 4096 heads, T = 1 .. 6,
 // both layouts of the operands; the estimates are within 10 and 13 % of what was measured for nine in ten), the whole
-// story in profiles/slice_resident_sweep.md.
+// story in profiles/slice_resident_sweep.md.  The chained kernel's workgroups of three waves, for three strips, came later: seven of them on
+// a compute unit in place of five of four (1915 problems: within 16 %).
 float slice_us(const ma_fwd_params* p, const SlicePlan& plan, int M) {
     struct Mode {
         float call, mb, pass, round, strip, block, tile, sums;
@@ -270,9 +271,10 @@ float slice_us(const ma_fwd_params* p, const SlicePlan& plan, int M) {
 float chain_us(const ma_fwd_params* p, int M, int units) {
     const int B = p->B, D = p->D, strips = (B + 15) / 16, tiles = (M + 15) / 16;
     const int cols = D <= 32 ? 2 : D <= 64 ? 4 : 5, pitch = D <= 32 ? 80 : D <= 64 ? 144 : 176;   // its classes of columns, bytes of a row in LDS
-    auto per_task = [](int s) { return s == 1 ? 4 : s == 2 ? 2 : 1; };
+    const int waves = mfma::chain_waves(cols, strips, tiles), most = waves == 3 ? 7 : 5;
+    auto per_task = [&](int s) { return waves >= s ? waves / s : 1; };
     const int lds_r = per_task(strips) * strips * (32 * pitch + 64), lds_l = per_task(tiles) * tiles * (32 * pitch + 192);
-    const int fit = 160 * 1024 / (lds_r > lds_l ? lds_r : lds_l), places = fit < 5 ? fit : 5;   // workgroups on a compute unit
+    const int fit = 160 * 1024 / (lds_r > lds_l ? lds_r : lds_l), places = fit < most ? fit : most;   // workgroups on a compute unit
     const int together = M > 8 ? 1 : M > 4 ? 2 : M > 2 ? 4 : M > 1 ? 8 : 16;   // positions that share an L / Z problem
     const long long heads = static_cast<long long>(p->E) * p->H;
     const float T = static_cast<float>(p->T), wide = static_cast<float>((heads + 7) / 8 * 8) / (static_cast<float>(units) * places);
@@ -317,11 +319,11 @@ bool slice_pays(const ma_fwd_params* p, int v) {
 }
 
 // A recorded call (ma_fwd_keep) that AUTO gives to the chained kernel: does the slice-resident one take it, writing every step's state as it
-// goes?  The same two estimates, and 0.2 us per MB of state that the chained kernel writes anyway.  Of 2076 random problems (8 .. 1024 heads,
-// D = 32 .. 80, blocks and block counts of up to 64, T = 1 .. 3) 170 are chosen, at 0.855 of the chained kernel's time; 3 % of them lose more than
-// 3 %, at most 9; of what the better kernel for each would gain this takes 84 %.  bf16, T = 2: 768 heads of 197
+// goes?  The same two estimates, and 0.2 us per MB of state that the chained kernel writes anyway.  Of 3875 random problems (8 .. 2048 heads, D = 32 .. 80,
+// blocks and block counts of up to 64, T = 1 .. 4; profiles/one_launch_rules_sweep.md) 404 are chosen, at 0.884 of the chained kernel's time;
+// 14 of them lose more than 3 %, three more than 10; of what the better kernel for each would gain this takes 77 %.  bf16, T = 2: 768 heads of 197
 // in 14-row blocks 51.5 -> 40.4 us, 384 of 256 in 16 33.5 -> 26.5; 64 of 1024 in 32 (24.3, 28.8 in slices) and 12 of 512 (13.3, 15.3) stay.  Without
-// the margin of 5 %: of 900 random problems 21 gain 3 - 12 % (192 of 512 in 32 33.9 -> 32.3 us) and 18 lose 3 - 15 %.
+// the margin of 5 % 44 lose more than 3 % for as much gained; with it 192 of 512 in 32 stays chained as well (33.9, 32.3 in slices).
 bool slice_keeps(const ma_fwd_params* p) {
     if (p->variant != MA_VARIANT_AUTO || p->B > 64 || p->D > 80) return false;
     const int M = (p->N + p->B - 1) / p->B;
@@ -337,8 +339,9 @@ bool one_launch_tiles(const ma_fwd_params* p) {
     return p->B <= 128 && M <= 128;
 }
 
-// Tasks (workgroups) of one phase of one head in the one-launch kernels: four waves per workgroup; a
-// block problem of n rows takes min(ceil(n / 16), 4) waves, rounded up to a power of two.
+// Tasks (workgroups) of one phase of one head in workgroups of four waves, a block problem of n rows on min(ceil(n / 16), 4) of them,
+// rounded up to a power of two: the team kernel's, and about the chained kernel's, whose workgroups of eight waves have fewer
+// (chain_waves) and of three up to a third more of 16-row problems - at most 16 then, beside blocks or block counts of 33 .. 48.
 long long phase_tasks(long long count, long long rows) {
     const long long strips = (rows + 15) / 16;
     const long long waves = strips <= 1 ? 1 : strips <= 2 ? 2 : 4;
@@ -346,7 +349,7 @@ long long phase_tasks(long long count, long long rows) {
     return (count + per_wg - 1) / per_wg;
 }
 
-// Can the chained kernel take the problem?  Mirrors the launcher's limits: at most 128 tasks per
+// Can the chained kernel take the problem?  Within the launcher's limits: at most 128 tasks per
 // head and phase, the heads' sync words (64-bit counters and release words of the 2T - 1 publishing
 // phases, in whole 128-byte lines) fit their part of the sync area, the grid is a 31-bit count.
 bool chain_fits(const ma_fwd_params* p) {

@@ -272,6 +272,9 @@ def test_auto_runs_slices_where_they_are_faster():
             # a single pass; few heads at a single step
             (78, 470, 32, 48, 1, 7.6, 9.4), (80, 300, 32, 40, 1, 7.1, 8.5), (128, 214, 72, 32, 1, 10.4, 11.6), (2, 192, 48, 15, 1, 7.4, 6.5),
             (4, 192, 48, 14, 1, 7.2, 6.6),
+            # 33 .. 48 rows, which the chained kernel runs in workgroups of three waves
+            (96, 1361, 32, 41, 4, 95.7, 73.3), (97, 1243, 32, 37, 3, 70.1, 57.2), (626, 423, 64, 40, 2, 104.1, 90.6), (456, 418, 48, 13, 2, 66.6, 58.7),
+            (256, 1503, 64, 45, 2, 123.2, 160.7), (512, 1523, 32, 45, 2, 153.7, 220.5),
             # the slices' own ground
             (128, 1024, 72, 32, 3, 46.3, 77.6), (112, 260, 40, 20, 1, 8.7, 10.2), (128, 384, 40, 24, 1, 9.4, 10.9), (128, 512, 64, 32, 2, 17.1, 26.0)):
         p = good_params()
@@ -280,6 +283,18 @@ def test_auto_runs_slices_where_they_are_faster():
         for field in ("q_stride", "k_stride", "v_stride", "out_stride"):
             setattr(p, field, (C.c_int64 * 3)(N * D, N * D, D))
         assert (lib.ma_fwd_kernel_name(p) == b"resident_slice_mfma") == (slices < other), (heads, N, D, B, T)
+
+
+def test_auto_records_with_slices_where_they_are_faster():
+    """The same choice for recorded calls, which write the states of all steps (us on an MI355X: slices, chained)."""
+    lib = L.load()
+    for heads, N, D, B, T, slices, chained in (
+            (38, 834, 64, 32, 3, 35.5, 28.0), (180, 1351, 64, 39, 4, 240.2, 173.3), (192, 59, 64, 43, 4, 63.2, 29.6), (88, 1572, 32, 27, 1, 30.8, 20.9),
+            (192, 1385, 64, 64, 2, 110.7, 92.2), (16, 673, 40, 16, 2, 40.4, 14.5), (12, 512, 64, 32, 2, 15.3, 13.3), (64, 1024, 64, 32, 2, 28.8, 24.3),
+            (768, 197, 64, 14, 2, 40.4, 51.5), (384, 256, 64, 16, 2, 26.5, 33.5), (1411, 144, 32, 7, 4, 113.5, 157.4), (61, 63, 32, 5, 4, 16.5, 23.2),
+            (453, 173, 80, 14, 4, 54.9, 74.7), (1244, 255, 48, 16, 1, 43.7, 66.4), (221, 42, 40, 5, 2, 12.3, 15.7), (512, 716, 32, 32, 4, 130.0, 171.5)):
+        name = lib.ma_fwd_keep_kernel_name(call_params(heads, N, D, B, T).fwd)
+        assert name == (b"resident_slice_mfma" if slices < chained else b"chain_fwd_mfma"), (heads, N, D, B, T)
 
 
 def call_params(heads, N, D, B, T=2, variant="auto", dt=L.MA_BF16):
