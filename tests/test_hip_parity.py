@@ -330,7 +330,7 @@ SLICES = [  # 14 / 15, 17 .. 32, 33 .. 48 and 49 .. 64 rows a block; every class
     (7, 16, 512, 64, 32, 2, False, "f16", True), (8, 14, 300, 40, 20, 1, True, "bf16", False), (7, 16, 1024, 72, 32, 3, False, "f16", False),
     (8, 14, 900, 80, 30, 2, True, "f16", True), (30, 12, 700, 64, 28, 2, False, "bf16", True), (8, 14, 1300, 32, 25, 2, False, "f16", True),
     (8, 14, 1300, 32, 28, 1, True, "f16", True), (5, 15, 1500, 32, 40, 2, False, "f16", True), (16, 14, 1000, 64, 44, 2, True, "f16", True),
-    (16, 14, 1600, 48, 40, 3, False, "bf16", True), (4, 14, 2500, 32, 60, 2, True, "f16", True), (4, 14, 3200, 32, 64, 3, False, "bf16", False),
+    (16, 16, 1600, 48, 40, 3, False, "bf16", True), (4, 14, 2500, 32, 60, 2, True, "f16", True), (4, 14, 3200, 32, 64, 3, False, "bf16", False),
     (16, 12, 600, 32, 15, 2, True, "f16", True), (8, 12, 800, 64, 32, 3, False, "f16", True),
 ]
 
