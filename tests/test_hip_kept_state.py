@@ -4,35 +4,42 @@ again, bit for bit, and the output equals the unrecorded call's."""
 import pytest
 import torch
 
-from helpers import DT, block_safe_mask, seeded_qkv
+from helpers import DT, block_safe_mask, keep_kernel, seeded_qkv
 from ma.ma_hip import monarch_attention_hip, monarch_attention_hip_backward
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
-CASES = [  # E, H, N, D, B, T, pre, dtype, variant, masked: rows per slot that do and do not fill a slot's 128-row grid
-    (1, 1, 64, 32, 8, 1, False, "f16", None, False),        # one step: no aR slot
-    (2, 3, 197, 64, 14, 3, True, "f16", None, True),        # ragged, three steps
-    (1, 8, 300, 72, 20, 2, False, "bf16", "chained", True),
-    (1, 2, 1000, 64, 128, 3, True, "bf16", "staged", False),
-    (1, 2, 256, 48, 16, 2, False, "f32", None, True),
-    (1, 2, 45, 20, 8, 2, True, "f16", "generic", False),
-    (1, 9, 512, 64, 32, 2, False, "f16", "resident", False),  # keeps nothing: the backward runs the steps again
+CHAIN, SLICES = "chain_fwd_mfma", "resident_slice_mfma"
+CASES = [  # E, H, N, D, B, T, pre, dtype, variant, masked, the kernel that records: rows per slot that do and do not fill a slot's 128-row grid
+    (1, 1, 64, 32, 8, 1, False, "f16", None, False, SLICES),        # one step: no aR slot
+    (2, 3, 197, 64, 14, 3, True, "f16", None, True, SLICES),        # ragged, three steps
+    (1, 8, 300, 72, 20, 2, False, "bf16", "chained", True, CHAIN),
+    (1, 2, 1000, 64, 128, 3, True, "bf16", "staged", False, "r_step_pair"),
+    (1, 2, 256, 48, 16, 2, False, "f32", None, True, "r_step_f32"),
+    (1, 2, 45, 20, 8, 2, True, "f16", "generic", False, "r_step_kernel"),
+    (1, 9, 512, 64, 32, 2, False, "f16", "resident", False, None),  # keeps nothing: the backward runs the steps again
+    (16, 12, 512, 64, 32, 2, True, "bf16", None, True, CHAIN),      # the slice-resident kernel is not far enough ahead here
     # calls that the slice-resident kernel records (its strips both ways, waves and column classes; masked, padded, one step to three)
-    (16, 12, 512, 64, 32, 2, True, "bf16", None, True), (48, 16, 197, 64, 14, 3, True, "f16", None, False), (24, 16, 256, 64, 16, 1, False, "bf16", None, True),
-    (13, 1, 60, 32, 19, 3, False, "f16", None, True), (50, 1, 21, 80, 9, 3, True, "bf16", None, False), (13, 1, 81, 48, 24, 3, True, "f16", None, True),
-    (67, 7, 53, 72, 7, 3, False, "f16", None, True), (66, 1, 1265, 32, 38, 3, True, "bf16", None, False), (79, 1, 2570, 32, 48, 2, False, "bf16", None, True),
-    (122, 1, 548, 64, 23, 3, False, "f16", None, True), (26, 1, 221, 32, 56, 3, True, "f16", None, True), (39, 13, 542, 32, 12, 3, True, "bf16", None, True),
-    # the chained kernel with a wave per strip: five strips one way, seven and six both ways
-    (1, 3, 5003, 128, 72, 2, True, "bf16", "chained", True), (1, 2, 60 * 70, 64, 60, 3, False, "f16", "chained", True), (1, 2, 9000, 72, 100, 2, False, "f16", "chained", False),
+    (48, 16, 197, 64, 14, 3, True, "f16", None, False, SLICES), (24, 16, 256, 64, 16, 1, False, "bf16", None, True, SLICES),
+    (13, 1, 60, 32, 19, 3, False, "f16", None, True, SLICES), (50, 1, 21, 80, 9, 3, True, "bf16", None, False, SLICES), (13, 1, 81, 48, 24, 3, True, "f16", None, True, SLICES),
+    (67, 7, 53, 72, 7, 3, False, "f16", None, True, SLICES), (80, 1, 2100, 32, 47, 3, True, "bf16", None, False, SLICES), (79, 1, 2570, 32, 48, 2, False, "bf16", None, True, SLICES),
+    (122, 1, 548, 64, 23, 3, False, "f16", None, True, SLICES), (26, 1, 221, 32, 56, 3, True, "f16", None, True, SLICES), (39, 13, 542, 32, 12, 3, True, "bf16", None, True, SLICES),
+    # the chained kernel in four waves of up to two strips: five strips both ways, four and five, seven and six
+    (1, 3, 5003, 128, 72, 2, True, "bf16", "chained", True, CHAIN), (1, 2, 60 * 70, 64, 60, 3, False, "f16", "chained", True, CHAIN), (1, 2, 9000, 72, 100, 2, False, "f16", "chained", False, CHAIN),
+    # ... in eight waves, where one side has seven or eight strips and the other up to five, and in three, for three strips both ways or beside one
+    (1, 3, 2393, 72, 120, 2, True, "bf16", "chained", True, CHAIN), (1, 2, 2310, 80, 20, 3, False, "f16", "chained", True, CHAIN), (1, 2, 509, 64, 128, 2, True, "f16", "chained", False, CHAIN),
+    (1, 2, 70 * 110, 128, 110, 2, False, "bf16", "chained", True, CHAIN), (1, 3, 1590, 64, 40, 3, True, "bf16", "chained", True, CHAIN),
+    (2, 4, 236, 32, 40, 2, False, "f16", "chained", True, CHAIN), (1, 5, 470, 128, 10, 2, True, "bf16", "chained", False, CHAIN),
 ]
 
 
 @pytest.mark.parametrize("case", range(len(CASES)))
 def test_kept_states_give_the_gradients_of_a_recomputation(case):
-    E, H, N, D, B, T, pre, dt, variant, masked = CASES[case]
+    E, H, N, D, B, T, pre, dt, variant, masked, kernel = CASES[case]
     q, k, v = (t.to(DEV) for t in seeded_qkv(E, H, N, D, DT[dt], seed=case))
     mask = block_safe_mask(E, N, B, seed=case).to(DEV) if masked else None
+    assert kernel is None or keep_kernel(q, k, v, mask, T, B, pre, variant) == kernel
     w = torch.randn(v.shape, generator=torch.Generator().manual_seed(case)).to(DEV).to(v.dtype)
     bwd = variant if variant in ("staged", "generic") else None
     want = monarch_attention_hip_backward(q, k, v, mask, w, T, B, pre, variant=bwd)

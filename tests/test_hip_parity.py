@@ -1049,7 +1049,9 @@ def test_random_shapes_in_the_192_and_256_row_classes(idx, E, H, N, D, B, T, pre
 
 
 # ---------------------------------------------------------------- a wait between workgroups that runs out is loud
-@pytest.mark.parametrize("shape", [(1, 2, 1024, 64, 32, 2), (3, 8, 512, 64, 32, 3), (1, 16, 2048, 64, 64, 1), (1, 3, 70 * 80, 64, 80, 2)])
+@pytest.mark.parametrize("shape", [(1, 2, 1024, 64, 32, 2), (3, 8, 512, 64, 32, 3), (1, 16, 2048, 64, 64, 1), (1, 3, 70 * 80, 64, 80, 2),
+                                   # chained workgroups of eight waves, long blocks and many blocks, and of three
+                                   (1, 3, 20 * 120, 72, 120, 2), (1, 3, 116 * 20, 72, 20, 2), (1, 3, 40 * 40, 64, 40, 2)])
 @pytest.mark.parametrize("variant", ["fused", "chained"])
 def test_wait_that_runs_out_is_loud_and_leaves_the_workspace_usable(variant, shape):
     """MA_FLAG_TEST_NO_SPIN makes every wait of the one-launch kernels give up at once (forced from the
