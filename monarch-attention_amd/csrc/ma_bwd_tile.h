@@ -93,13 +93,17 @@ __device__ __forceinline__ f32x4 lds4(const float* p) { return *reinterpret_cast
 //   up to 32 columns: 7 strips 146 / 116 -> 111 / 92, up to 48: 142 / 115 -> 123 / 89 (8 strips 113 / 88 -> 102 / 70)
 //   up to 64: 7 strips 87.8 / 70.0 -> 80.3 / 59.8, 8 strips 57.8 / 43.1 -> 58.1 / 39.4 (7.9 million elements)
 //   up to 96: 7 strips (V held: 165) 105 / 84.0 -> - / 79.0, 8 strips held: 96.5 / 67.9 for 80.8 / 65.6
+// fp16 as bf16 but for 5 strips of 81 .. 96 columns with V, where it spills 134 words for bf16's 34: us of the backward, held -> free, 66 heads of 4214,
+// D = 88, 73-row blocks, one step 392 -> 302, 51 of 2185 in 67, two steps 278 -> 221.
+template <class T>
 constexpr int r_held_waves(int DT, int NWT, bool kV) {
+    if (std::is_same<T, f16>::value && DT == 6 && NWT == 5 && kV) return 1;
     if (DT <= 4) return NWT == 2 ? (DT == 4 ? 5 : 1) : 4 <= NWT && NWT <= 8 ? 4 : 1;
     if (DT <= 6) return (NWT == 5 && (DT == 6 || kV)) || (NWT == 7 && !kV) ? 4 : NWT == 3 || NWT == 4 || (NWT == 6 && kV) ? 3 : 1;
     return NWT == 5 && !kV ? 4 : NWT == 3 || NWT == 4 ? 3 : 1;
 }
 template <class T, int DT, int NWT, int W, int PASS, bool kV, bool WHOLE = false>
-__global__ __launch_bounds__(64 * W, sizeof(T) == 2 && PASS == 0 ? r_held_waves(DT, NWT, kV) : DT >= 5 && W == 8 && shares_lds<T>(DT, NWT, PASS, kV) ? 4 : 1) void r_bwd_tile(Problem P, BwdBuffers G, int first) {
+__global__ __launch_bounds__(64 * W, sizeof(T) == 2 && PASS == 0 ? r_held_waves<T>(DT, NWT, kV) : DT >= 5 && W == 8 && shares_lds<T>(DT, NWT, PASS, kV) ? 4 : 1) void r_bwd_tile(Problem P, BwdBuffers G, int first) {
     using MT = Mat<T, DT>;
     using PL = RPlan<T, DT, NWT, PASS, kV, WHOLE>;
     using mfma::quad_rows_max;
