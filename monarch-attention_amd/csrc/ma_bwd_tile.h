@@ -698,22 +698,24 @@ __global__ __launch_bounds__(64 * W, sizeof(T) == 2 && PASS == 0 ? lz_held_waves
 // ---------------------------------------------------------------- launches
 // How problems of more than 128 rows that fill the device are split (16 bit).  One launch of 10 or 12 strips reads the operands once and
 // forms the statistics where they are used; its waves have 168 registers, which the R stage of 12 strips outgrows in the classes that
-// stay with two launches.  16 strips: two workgroups of four waves in pass 1, which would idle beside tiles of more than half of the LDS -
+// stay with two launches.  A workgroup of 12 waves has a compute unit to itself: where one launch of them gains little (R with V, 96 columns), it is
+// taken only where the last pass over the units is half full (us of the backward of one step, D = 96, two launches -> one: 302 problems 90 -> 97, 432
+// 122 -> 111, 740 183 -> 172), and R of 128 columns stays with two (of two steps 280 .. 600 problems 1.03 - 1.11 in one).  16 strips: two workgroups of four waves in pass 1, which would idle beside tiles of more than half of the LDS -
 // there one of eight.  Pass 2: see shares_lds; 96 columns and two gradients: one workgroup of 16 waves (122 registers and 76 bytes spilled).
 // us of the stages Z, R with V, L, R, bf16, before -> now, D = 64 / 96 / 128:
 //   150 rows  80, 130, 94, 101 -> 71, 100, 69, 76 (11.5 million elements) / 119, 210, 129, 139 -> 100, 164, 101, 116 / 210, 264, 192, 205 ->
 //             145, 264 (254 - 138 for 132 us in one launch), 148, 169
 //   190 rows  138, 188, 135, 148 -> 108, 188 (in one launch 203), 106, 135 / 212, 317, 225, 218 -> 150, 292, 192, 218 (221) / 310, 376, 263,
-//             308 -> 195, 376 (389), 241, 288 (R with V, 80 columns, fp16: 321 in two launches, 347 in one)
+//             308 -> 195, 376 (389), 241, 308 (288) (R with V, 80 columns, fp16: 321 in two launches, 347 in one)
 //   250 rows  232, 400, 233, 245 -> 232, 348, 233, 245 (eight waves in pass 1: 253, 405, 243, 256) / 567, 659, 471, 444 -> 424, 576, 370, 383
 //             / 701, 737, 603, 505 -> 567, 649, 432, 447
 template <int DT, bool kV>
 struct RSplit {
-    static constexpr Split16 of{!(kV && DT == 8), kV ? DT == 6 : DT <= 4 || DT == 8, kV && DT >= 5 ? 8 : 4, kV && DT == 6 ? 16 : 8};
+    static constexpr Split16 of{!(kV && DT == 8), kV ? DT == 6 : DT <= 4, kV, kV && DT >= 5 ? 8 : 4, kV && DT == 6 ? 16 : 8};
 };
 template <int DT, bool kZ>
 struct LzSplit {
-    static constexpr Split16 of{true, true, DT >= 5 ? 8 : 4, kZ && DT == 6 ? 16 : 8};
+    static constexpr Split16 of{true, true, false, DT >= 5 ? 8 : 4, kZ && DT == 6 ? 16 : 8};
 };
 // Does a launch of `groups` workgroups per problem leave every workgroup a compute unit to itself?  Walking its tiles in halves then only adds
 // barriers: 12 .. 64 problems of 256 rows in four workgroups each, bf16, forward and backward of one step, us, D = 48 R with V 40.2 ->

@@ -301,10 +301,15 @@ inline int strip_class(int n) {
 // of n rows.  One launch of both passes up to 128 rows, unless there are fewer problems of 6 or 8 strips than the device has
 // compute units: half of their strips per workgroup then (the graph-transformer shape has 120 problems of 128 rows).  Above 128
 // rows, where the problems fill the device, what `Split` says, else four strips per workgroup.
-struct Split16 {   // of a 16-bit kernel: 10 and 12 strips in one launch; waves of a workgroup in pass 1 and 2 of 16
-    bool one10, one12;
+struct Split16 {   // of a 16-bit kernel: 10 and 12 strips in one launch (12: only if the last pass is filled); waves of a workgroup in pass 1 and 2 of 16
+    bool one10, one12, filled12;
     int w1, w2;
 };
+// A workgroup to a compute unit: is the last pass over the units at least half full?
+inline bool last_pass_filled(long long problems) {
+    const int units = mfma::compute_units();
+    return (problems - 1) % units >= units / 2;
+}
 template <bool F32, class Split, class F>
 int each_launch(int n, long long problems, F&& f) {
     auto two = [&](auto nwt, auto w1, auto w2) {
@@ -338,8 +343,9 @@ int each_launch(int n, long long problems, F&& f) {
         case 12:
             if constexpr (!F32)
                 if (fill) {
-                    if constexpr (Split::of.one12) return f(integral_constant<int, 12>{}, integral_constant<int, 12>{}, one);
-                    else return two(integral_constant<int, 12>{}, integral_constant<int, 6>{}, integral_constant<int, 6>{});
+                    if constexpr (Split::of.one12)
+                        if (!Split::of.filled12 || last_pass_filled(problems)) return f(integral_constant<int, 12>{}, integral_constant<int, 12>{}, one);
+                    if constexpr (!Split::of.one12 || Split::of.filled12) return two(integral_constant<int, 12>{}, integral_constant<int, 6>{}, integral_constant<int, 6>{});
                 }
             return two(integral_constant<int, 12>{}, integral_constant<int, 4>{}, integral_constant<int, 4>{});
         default:
