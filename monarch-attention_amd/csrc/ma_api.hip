@@ -319,18 +319,20 @@ bool slice_pays(const ma_fwd_params* p, int v) {
 }
 
 // A recorded call (ma_fwd_keep) that AUTO gives to the chained kernel: does the slice-resident one take it, writing every step's state as it
-// goes?  The same two estimates, and 0.2 us per MB of state that the chained kernel writes anyway.  Of 3875 random problems (8 .. 2048 heads, D = 32 .. 80,
-// blocks and block counts of up to 64, T = 1 .. 4; profiles/one_launch_rules_sweep.md) 404 are chosen, at 0.884 of the chained kernel's time;
-// 14 of them lose more than 3 %, three more than 10; of what the better kernel for each would gain this takes 77 %.  bf16, T = 2: 768 heads of 197
-// in 14-row blocks 51.5 -> 40.4 us, 384 of 256 in 16 33.5 -> 26.5; 64 of 1024 in 32 (24.3, 28.8 in slices) and 12 of 512 (13.3, 15.3) stay.  Without
-// the margin of 5 % 44 lose more than 3 % for as much gained; with it 192 of 512 in 32 stays chained as well (33.9, 32.3 in slices).
+// goes?  The same two estimates, 0.2 us per MB of state that the chained kernel writes anyway, and a margin of 5 %, of 1.5 us for calls of less than 30.
+// Of 6138 random problems (1 .. 2048 heads, D = 32 .. 80, blocks and block counts of up to 64, T = 1 .. 4; profiles/one_launch_rules_sweep.md) 924 are
+// chosen, at 0.875 of the chained kernel's time, 16 of which lose more than 3 %; of what the better kernel for each would gain this takes 84 %.
+// With 5 % throughout 1167 at 0.899, 87 losing, 54 of these of 1 .. 7 heads (one head of 103 tokens in 7-row blocks, D = 72, T = 2 12.3 -> 14.6 us).
+// bf16, T = 2: 768 heads of 197 in 14-row blocks 51.5 -> 40.4 us, 384 of 256 in 16 33.5 -> 26.5; 64 of 1024 in 32 (24.3, 28.8 in slices), 12 of 512
+// (13.3, 15.3) and 192 of 512 (33.9, 32.3) stay.
 bool slice_keeps(const ma_fwd_params* p) {
     if (p->variant != MA_VARIANT_AUTO || p->B > 64 || p->D > 80) return false;
     const int M = (p->N + p->B - 1) / p->B;
     SlicePlan plan;
     if (M > 64 || !slice_fits(p, &plan, true)) return false;
     const float kept = 2e-6f * static_cast<float>(p->E) * p->H * p->D * static_cast<float>(M * p->B) * static_cast<float>(2 * p->T - 1);
-    return slice_us(p, plan, M) + 0.2f * kept < 0.95f * chain_us(p, M, plan.units);
+    const float chain = chain_us(p, M, plan.units);
+    return slice_us(p, plan, M) + 0.2f * kept < std::fmin(0.95f * chain, chain - 1.5f);
 }
 
 // The fused, chained and resident kernels are built for block problems of at most 128 rows.

@@ -290,7 +290,7 @@ def test_auto_records_with_slices_where_they_are_faster():
     lib = L.load()
     for heads, N, D, B, T, slices, chained in (
             (38, 834, 64, 32, 3, 35.5, 28.0), (180, 1351, 64, 39, 4, 240.2, 173.3), (192, 59, 64, 43, 4, 63.2, 29.6), (88, 1572, 32, 27, 1, 30.8, 20.9),
-            (192, 1385, 64, 64, 2, 110.7, 92.2), (16, 673, 40, 16, 2, 40.4, 14.5), (12, 512, 64, 32, 2, 15.3, 13.3), (64, 1024, 64, 32, 2, 28.8, 24.3),
+            (1, 103, 72, 7, 2, 14.6, 12.3), (12, 218, 40, 14, 2, 14.4, 12.8), (18, 143, 80, 16, 2, 15.7, 14.4), (192, 1385, 64, 64, 2, 110.7, 92.2), (16, 673, 40, 16, 2, 40.4, 14.5), (12, 512, 64, 32, 2, 15.3, 13.3), (64, 1024, 64, 32, 2, 28.8, 24.3),
             (768, 197, 64, 14, 2, 40.4, 51.5), (384, 256, 64, 16, 2, 26.5, 33.5), (1411, 144, 32, 7, 4, 113.5, 157.4), (61, 63, 32, 5, 4, 16.5, 23.2),
             (453, 173, 80, 14, 4, 54.9, 74.7), (1244, 255, 48, 16, 1, 43.7, 66.4), (221, 42, 40, 5, 2, 12.3, 15.7), (512, 716, 32, 32, 4, 130.0, 171.5)):
         name = lib.ma_fwd_keep_kernel_name(call_params(heads, N, D, B, T).fwd)

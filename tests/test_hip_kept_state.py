@@ -12,7 +12,7 @@ DEV = "cuda"
 
 CHAIN, SLICES = "chain_fwd_mfma", "resident_slice_mfma"
 CASES = [  # E, H, N, D, B, T, pre, dtype, variant, masked, the kernel that records: rows per slot that do and do not fill a slot's 128-row grid
-    (1, 1, 64, 32, 8, 1, False, "f16", None, False, SLICES),        # one step: no aR slot
+    (1, 1, 64, 32, 8, 1, False, "f16", None, False, CHAIN),        # one step: no aR slot
     (2, 3, 197, 64, 14, 3, True, "f16", None, True, SLICES),        # ragged, three steps
     (1, 8, 300, 72, 20, 2, False, "bf16", "chained", True, CHAIN),
     (1, 2, 1000, 64, 128, 3, True, "bf16", "staged", False, "r_step_pair"),
