@@ -271,7 +271,8 @@ float slice_us(const ma_fwd_params* p, const SlicePlan& plan, int M) {
 float chain_us(const ma_fwd_params* p, int M, int units) {
     const int B = p->B, D = p->D, strips = (B + 15) / 16, tiles = (M + 15) / 16;
     const int cols = D <= 32 ? 2 : D <= 64 ? 4 : 5, pitch = D <= 32 ? 80 : D <= 64 ? 144 : 176;   // its classes of columns, bytes of a row in LDS
-    const int waves = mfma::chain_waves(cols, strips, tiles), most = waves == 3 ? 7 : 5;
+    // (three strips of blocks of up to 16 rows, which run in four waves, are nearer to the terms of three as well)
+    const int waves = strips == 1 && tiles == 3 ? 3 : mfma::chain_waves(cols, strips, tiles), most = waves == 3 ? 7 : 5;
     auto per_task = [&](int s) { return waves >= s ? waves / s : 1; };
     const int lds_r = per_task(strips) * strips * (32 * pitch + 64), lds_l = per_task(tiles) * tiles * (32 * pitch + 192);
     const int fit = 160 * 1024 / (lds_r > lds_l ? lds_r : lds_l), places = fit < most ? fit : most;   // workgroups on a compute unit
@@ -343,7 +344,7 @@ bool one_launch_tiles(const ma_fwd_params* p) {
 
 // Tasks (workgroups) of one phase of one head in workgroups of four waves, a block problem of n rows on min(ceil(n / 16), 4) of them,
 // rounded up to a power of two: the team kernel's, and about the chained kernel's, whose workgroups of eight waves have fewer
-// (chain_waves) and of three up to a third more of 16-row problems - at most 16 then, beside blocks or block counts of 33 .. 48.
+// (chain_waves) and of three up to a third more of 16-row problems - at most 16 then, beside blocks of 33 .. 48 rows.
 long long phase_tasks(long long count, long long rows) {
     const long long strips = (rows + 15) / 16;
     const long long waves = strips <= 1 ? 1 : strips <= 2 ? 2 : 4;

@@ -25,17 +25,18 @@ inline int nt_class(int n) { return n <= 16 ? 1 : n <= 32 ? 2 : n <= 48 ? 3 : 4;
 // Waves of a workgroup of the chained kernel.  What counts is how many waves with work a compute unit holds.  Four as a rule, of which each walks up to two strips: a
 // wave per strip of the larger side leaves waves idle in the other kind of phase, or fits a compute unit less often, and is up to 25 % behind (D
 // = 72, two steps: 48 heads of 104 blocks of 104 rows 332 -> 388 us, 48 of 70 blocks of 110 rows 233 -> 289; D = 64, 48 of 128 blocks of 128 rows
-// 348 -> 436).  Eight beside a side of up to five strips where the LDS of eight (of seven above 96 columns) leaves room for three workgroups
+// 348 -> 436).  Eight beside a side of up to five strips where the LDS of eight (of seven above 80 columns) leaves room for three workgroups
 // of four waves or less, which are half idle in the short phases: eight waves run several short problems at a time.  Two steps, 48 | 192
 // heads, four -> eight waves, us: 8 blocks of 128 rows, D = 72 37 -> 31 | 120 -> 102, 128 45 -> 40 | 161 -> 155, 20 of 120, 72 90 -> 70 | 381 -> 331,
 // 128 108 -> 94 | 474 -> 441; 116 of 20, 72 88 -> 67 | 369 -> 303; 30 of 100, 128 117 -> 112 | 540 -> 529, 72 75 -> 80 | 342 -> 383.  64 columns, eight
 // strips of a block: 8 blocks 29 -> 26 | 71 -> 68, 20 53 -> 49 | 217 -> 208, 64 (48 heads) 171 -> 164; of a position 0.98 - 1.04.
-// Three for three strips both ways or beside one, where a fourth has nothing to do: 192 heads of 36 blocks of 40 rows, D = 32 91 -> 74, 64 116 ->
-// 107, 72 140 -> 134, 96 172 -> 162; of 48 of 48, 118 -> 105, 183 -> 172, 226 -> 221, 254 -> 246; up to 32 heads level.  (Two strips beside three
-// in six waves, whose phases are all full: 1.0 - 1.3.)
+// Three for blocks of three strips in one or three strips of blocks, where a fourth has nothing to do: 192 heads of 36 blocks of 40 rows, D = 32 91 -> 74, 64
+// 116 -> 107, 72 140 -> 134, 96 172 -> 162; of 48 of 48, 118 -> 105, 183 -> 172, 226 -> 221, 254 -> 246; up to 32 heads level.  (Three strips of blocks of up to 16
+// rows: 0.97 - 1.0 with many heads, up to 1.06 with few.  Two strips beside three in six waves, whose phases are all full: 1.0 - 1.3.)
+// 1500 random calls of these classes (1 .. 512 heads, T = 1 .. 3) in multiples of four waves' time: profiles/one_launch_rules_sweep.md.
 constexpr int chain_waves(int DT, int NTB, int NTM) {
     const int most = NTB > NTM ? NTB : NTM, least = NTB < NTM ? NTB : NTM;
-    if (most == 3 && least != 2) return 3;
+    if (NTB == 3 && (NTM == 1 || NTM == 3)) return 3;
     if (most < 7 || least > 5) return kWaves;
     if (most == 7) return DT == 8 ? 8 : kWaves;
     return DT >= 5 || (DT == 4 && NTB == 8 && NTM <= 4) ? 8 : kWaves;
