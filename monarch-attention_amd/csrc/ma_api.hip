@@ -354,7 +354,8 @@ long long phase_tasks(long long count, long long rows) {
 
 // Can the chained kernel take the problem?  Within the launcher's limits: at most 128 tasks per
 // head and phase, the heads' sync words (64-bit counters and release words of the 2T - 1 publishing
-// phases, in whole 128-byte lines) fit their part of the sync area, the grid is a 31-bit count.
+// phases, in whole 128-byte lines) fit their part of the sync area, the grid is a 31-bit count and its
+// work items a 32-bit one (blocks of 128 rows beside up to 80, in eight waves: the sync words have room for 9.1e6 tasks, 8.4e6 can be launched).
 bool chain_fits(const ma_fwd_params* p) {
     const long long M = (static_cast<long long>(p->N) + p->B - 1) / p->B;
     const long long tR = phase_tasks(M, p->B), tL = phase_tasks(p->B, M);
@@ -363,7 +364,9 @@ bool chain_fits(const ma_fwd_params* p) {
     const long long stride = (2 * nph1 + 2 + 31) / 32 * 32 + (nph1 + 31) / 32 * 32;
     if (!one_launch_tiles(p) || tR > 128 || tL > 128) return false;
     if (heads * stride > static_cast<long long>(kChainSyncBytes / 4)) return false;
-    return 8 * ((heads + 7) / 8) * p->T * (tR + tL) <= 0x7fffffffLL;
+    const long long grid = 8 * ((heads + 7) / 8) * p->T * (tR + tL);
+    const int waves = mfma::chain_waves(mfma::dt_class(p->D), (p->B + 15) / 16, static_cast<int>((M + 15) / 16));
+    return grid <= 0x7fffffffLL && launchable(grid, 64 * (waves > 4 ? waves : 4));   // (three waves: as many work items as four)
 }
 
 // Few heads whose phases fill the device: every head gets a team with one workgroup per task (64

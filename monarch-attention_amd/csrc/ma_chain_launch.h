@@ -37,11 +37,11 @@ int launch_chain_one(const Problem& P, bool sync_ready, hipStream_t s) {
     pl.spin_limit = P.test_no_spin ? 0u : 1u << 18;   // a legitimate wait lasts one phase of one head (well under a millisecond)
     // the task count of a phase is a 16-bit field of its arrival counter (and so are the sums of the
     // XCC ids: at most 15 and 225 per task); the heads' sync words must fit their part of the sync area;
-    // the grid must stay a 31-bit count
+    // the grid must stay a 31-bit count, its work items a 32-bit one
     if (pl.tR > 128 || pl.tL > 128) return MA_ERR_UNSUPPORTED;
     if (heads * pl.stride > kChainWords) return MA_ERR_UNSUPPORTED;
     const long long grid = 8ll * pl.hx * P.T * (pl.tR + pl.tL);
-    if (grid > 0x7fffffffll) return MA_ERR_UNSUPPORTED;
+    if (grid > 0x7fffffffll || !launchable(grid, 64 * W)) return MA_ERR_UNSUPPORTED;
     if (!sync_ready) {
         const int err = launch_zero_sync(P.sync, s);
         if (err) return err;

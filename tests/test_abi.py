@@ -359,6 +359,21 @@ def test_head_counts_beyond_the_work_items_of_one_launch():
     assert matrix_kernel(call_params(most + 1, 12, 32, 4)) == b"matrix_tile"
 
 
+def test_chained_launches_of_more_than_2_to_the_32_work_items_are_refused():
+    """Many steps of many heads: the sync words have room for them, a dispatch of eight-wave workgroups has not."""
+    lib = L.load()
+    for heads, N, D, B, T, fits in ((2728, 10240, 72, 128, 16, False), (2728, 10240, 128, 80, 16, False), (2400, 10240, 72, 128, 16, True),
+                                    (2728, 10240, 64, 128, 16, True), (2728, 16384, 72, 128, 16, True)):   # (the last two: workgroups of four waves)
+        p = call_params(heads, N, D, B, T, "chained").fwd
+        assert lib.ma_fwd_kernel_name(p) == (b"chain_fwd_mfma" if fits else None), (heads, N, D, B, T)
+        if not fits:
+            p.eps, p.workspace, p.workspace_bytes = 1e-12, 0x100000, 1 << 50
+            assert lib.ma_fwd(p, None) == L.MA_ERR_UNSUPPORTED
+            assert lib.ma_fwd_keep(p, 0x100000, 1 << 50, None) == L.MA_ERR_UNSUPPORTED
+            p.variant = L.VARIANTS["auto"]
+            assert lib.ma_fwd_kernel_name(p) == b"r_step_pair" and lib.ma_fwd_keep_kernel_name(p) == b"r_step_pair"
+
+
 def test_auto_runs_the_one_launch_backward_where_it_is_faster():
     """AUTO's choice for the backward of short heads, at shapes where one side took at most 0.85 of the other's time (us of the backward
     alone on an MI355X: one launch, stage launches)."""
