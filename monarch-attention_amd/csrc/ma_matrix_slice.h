@@ -144,7 +144,7 @@ __global__ __launch_bounds__(64 * W, W / 4) void matrix_slice_mfma(Problem P, fl
             const int t = (l0 + i) * B + j - P.pad_off;
             return i < rows && t >= 0 && t < N ? A + (static_cast<long long>(head) * N + t) * N : nullptr;
         };
-        if (N % 4 == 0 && B >= 4 && reinterpret_cast<uintptr_t>(A) % 16 == 0) {   // four columns per lane and store; they touch at most two blocks
+        if (N % 4 == 0 && B >= 4) {   // four columns per lane and store (A is 16-byte aligned: mfma_supported); they touch at most two blocks
             for (int n = c0 + 4 * c.lane; n < c1; n += 256) {
                 const int p = n + P.pad_off, ka = static_cast<unsigned>(p) / static_cast<unsigned>(B), ia = p - ka * B, kb = min(ka + 1, M - 1);
                 f32x4 x;
