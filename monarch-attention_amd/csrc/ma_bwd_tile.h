@@ -95,6 +95,7 @@ __device__ __forceinline__ f32x4 lds4(const float* p) { return *reinterpret_cast
 //   up to 96: 7 strips (V held: 165) 105 / 84.0 -> - / 79.0, 8 strips held: 96.5 / 67.9 for 80.8 / 65.6
 // fp16 as bf16 but for 5 strips of 81 .. 96 columns with V, where it spills 134 words for bf16's 34: us of the backward, held -> free, 66 heads of 4214,
 // D = 88, 73-row blocks, one step 392 -> 302, 51 of 2185 in 67, two steps 278 -> 221.
+// 1000 random backward calls of 17 .. 128 rows: 0.98 of the free kernels' time, at most 1.07 (profiles/one_launch_rules_sweep.md).
 template <class T>
 constexpr int r_held_waves(int DT, int NWT, bool kV) {
     if (std::is_same<T, f16>::value && DT == 6 && NWT == 5 && kV) return 1;
@@ -709,6 +710,7 @@ __global__ __launch_bounds__(64 * W, sizeof(T) == 2 && PASS == 0 ? lz_held_waves
 //             308 -> 195, 376 (389), 241, 308 (288) (R with V, 80 columns, fp16: 321 in two launches, 347 in one)
 //   250 rows  232, 400, 233, 245 -> 232, 348, 233, 245 (eight waves in pass 1: 253, 405, 243, 256) / 567, 659, 471, 444 -> 424, 576, 370, 383
 //             / 701, 737, 603, 505 -> 567, 649, 432, 447
+// 800 random backward calls of 129 .. 256 rows: 0.956, at most 1.04 (profiles/one_launch_rules_sweep.md).
 template <int DT, bool kV>
 struct RSplit {
     static constexpr Split16 of{!(kV && DT == 8), kV ? DT == 6 : DT <= 4, kV, kV && DT >= 5 ? 8 : 4, kV && DT == 6 ? 16 : 8};

@@ -33,7 +33,7 @@ inline int nt_class(int n) { return n <= 16 ? 1 : n <= 32 ? 2 : n <= 48 ? 3 : 4;
 // Three for blocks of three strips in one or three strips of blocks, where a fourth has nothing to do: 192 heads of 36 blocks of 40 rows, D = 32 91 -> 74, 64
 // 116 -> 107, 72 140 -> 134, 96 172 -> 162; of 48 of 48, 118 -> 105, 183 -> 172, 226 -> 221, 254 -> 246; up to 32 heads level.  (Three strips of blocks of up to 16
 // rows: 0.97 - 1.0 with many heads, up to 1.06 with few.  Two strips beside three in six waves, whose phases are all full: 1.0 - 1.3.)
-// 1500 random calls of these classes (1 .. 512 heads, T = 1 .. 3) in multiples of four waves' time: profiles/one_launch_rules_sweep.md.
+// 1000 random calls of these classes (1 .. 512 heads, T = 1 .. 3) in multiples of four waves' time: profiles/one_launch_rules_sweep.md.
 constexpr int chain_waves(int DT, int NTB, int NTM) {
     const int most = NTB > NTM ? NTB : NTM, least = NTB < NTM ? NTB : NTM;
     if (NTB == 3 && (NTM == 1 || NTM == 3)) return 3;
