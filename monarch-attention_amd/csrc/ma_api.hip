@@ -836,7 +836,8 @@ struct BwdLayout {
     uint64_t stats;
     uint64_t gaR, gcR, gaL, gcL, gY, stat, dq, dk, dv, pk, pv;
     bool tiled, rows16;                     // BwdBuffers::tiled, rows16
-    bool head;                              // the whole pass in one launch (ma_bwd_head.h)
+    bool head;                              // the whole pass in one launch (ma_bwd_head.h), with rows of its own in memory
+    BwdHeadUse rows;
     int parts;                              // per-tile partial buffers of dk / dv (R stage split over workgroups)
     uint64_t total;
 };
@@ -893,14 +894,14 @@ bool bwd_head_pays(const ma_fwd_params* pp) {
     const int M = (pp->N + pp->B - 1) / pp->B, units = mfma::compute_units();
     return bwd_head_us(pp, M, units) < 0.95f * bwd_stages_us(pp, M, units);
 }
-bool bwd_head(const ma_bwd_params* b, const ma_fwd_params* pp, const BwdLayout& L) {
+bool bwd_head(const ma_bwd_params* b, const ma_fwd_params* pp, BwdLayout& L) {
     if (pp->B > 32 || pp->N > 32 * pp->B || !L.tiled || !L.rows16 || pp->dtype_qk == MA_F32 || pp->D % 8 != 0 || !bwd_head_pays(pp)) return false;
     const int64_t* st[7] = {pp->q_stride, pp->k_stride, pp->v_stride, b->dout_stride, b->dq_stride, b->dk_stride, b->dv_stride};
     for (const int64_t* t : st)   // (Head::kColOut)
         if (((pp->N - 1) * t[2] + pp->D) * 2 >= 0x7fff0000ll) return false;
     const Problem P = sizes_of(pp);
     const BwdBuffers none = {};
-    return launch_bwd_head(P, none, pp->dtype_qk, 0, 0, true, nullptr) == MA_OK;
+    return launch_bwd_head(P, none, pp->dtype_qk, 0, 0, &L.rows, nullptr) == MA_OK;
 }
 
 int bwd_prepare(const ma_bwd_params* b, bool kept, ma_fwd_params* pp, BwdLayout* L) {
@@ -939,8 +940,8 @@ int bwd_prepare(const ma_bwd_params* b, bool kept, ma_fwd_params* pp, BwdLayout*
     take(&L->gY, staged, rows * pp->Dv * es);
     take(&L->stat, tight && two_launches, rows * 16);
     // dq, dk, dv are contiguous: one fill kernel zeroes the three
-    L->dq = off; off += rows * pp->D * 4;
-    L->dk = off; off += !tight || steps ? rows * pp->D * 4 : 0;   // (a single step completes dk in registers)
+    L->dq = off; off += staged || L->rows.dq ? rows * pp->D * 4 : 0;
+    L->dk = off; off += !tight || (steps && (staged || L->rows.dk)) ? rows * pp->D * 4 : 0;   // (a single step completes dk in registers)
     L->dv = off; off = align_up(off + (tight ? 0 : rows * pp->Dv * 4));
     if (L->tiled && !tight) L->stat = L->dv;   // no accumulator of dv on the tiled path (D % 4 == 0: 16 bytes a row and more)
     {
@@ -951,7 +952,7 @@ int bwd_prepare(const ma_bwd_params* b, bool kept, ma_fwd_params* pp, BwdLayout*
     }
     L->pk = off; off = align_up(off + static_cast<uint64_t>(L->parts) * rows * pp->D * 4);
     L->pv = off; off = align_up(off + static_cast<uint64_t>(L->parts) * rows * pp->Dv * 4);
-    L->total = off;
+    L->total = off != 0 ? off : kAlign;   // (ma_bwd_kept_workspace_bytes: 0 is a refusal)
     return MA_OK;
 }
 
@@ -1058,7 +1059,7 @@ int run_bwd(const ma_bwd_params* b, const void* kept, uint64_t kept_bytes, hipSt
         at_step(P, S, base, 0);
         P.aR = base + S.aR;
         P.cR = reinterpret_cast<float*>(base + S.cR);
-        return launch_bwd_head(P, G, pp.dtype_qk, S.slot_a, S.slot_c, false, s);
+        return launch_bwd_head(P, G, pp.dtype_qk, S.slot_a, S.slot_c, nullptr, s);
     }
     if (!L.tiled) {
         st = launch_bwd_zero(G.dq, rows * (2LL * P.D + P.Dv), s);

@@ -722,16 +722,19 @@ __global__ __launch_bounds__(64 * W, 2) void head_bwd(HeadArgs) {
     }
 }
 
-// Does the kernel take the problem (dry), and its launch.
+// The kernel's launch; `use`: only, does it take the problem, and what of dq and dk goes through memory?
 template <class T, int DT>
-int launch(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, bool dry, hipStream_t s) {
+int launch(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, BwdHeadUse* use, hipStream_t s) {
     constexpr int W = 8;
     const long long grid = (static_cast<long long>(P.E) * P.H + 7) / 8 * 8;
     if (P.B > 32 || P.M > 32 || !launchable(grid, 64 * W)) return MA_ERR_UNSUPPORTED;
     auto go = [&](auto ntb, auto ntm) {
         constexpr int NTB = decltype(ntb)::value, NTM = decltype(ntm)::value;
-        auto start = [&](auto kernel, int BP, size_t bytes) {
-            if (dry) return static_cast<int>(MA_OK);
+        auto start = [&](auto kernel, int BP, size_t bytes, bool dq) {
+            if (use != nullptr) {
+                *use = BwdHeadUse{dq, P.T > 1 && !Head<T, DT, NTB, NTM, W, true>::DKB};
+                return static_cast<int>(MA_OK);
+            }
             const int attr = mfma::set_lds_limit(kernel, kLdsMax);
             if (attr) return attr;
             hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(64 * W), bytes, s, HeadArgs{P, G, BP, slot_a, slot_c});
@@ -739,11 +742,11 @@ int launch(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, uns
         };
         for (int BP = P.B | 1; BP >= P.B; --BP) {   // (an odd BP where it fits)
             const size_t lds = Head<T, DT, NTB, NTM, W, true>::layout(P.M, BP).total;
-            if (lds <= kLdsMax) return start(head_bwd<T, DT, NTB, NTM, W, true>, BP, lds);
+            if (lds <= kLdsMax) return start(head_bwd<T, DT, NTB, NTM, W, true>, BP, lds, false);
         }
         for (int BP = P.B | 1; BP >= P.B; --BP) {
             const size_t lds = Head<T, DT, NTB, NTM, W, false>::layout(P.M, BP).total;
-            if (lds <= kLdsMax) return start(head_bwd<T, DT, NTB, NTM, W, false>, BP, lds);
+            if (lds <= kLdsMax) return start(head_bwd<T, DT, NTB, NTM, W, false>, BP, lds, true);
         }
         return static_cast<int>(MA_ERR_UNSUPPORTED);
     };

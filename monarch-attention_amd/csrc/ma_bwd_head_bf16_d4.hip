@@ -2,7 +2,7 @@
 #include "ma_bwd_head.h"
 
 namespace ma {
-int launch_bwd_head_bf16_d4(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, bool dry, hipStream_t s) {
-    return bwdh::launch<bf16, 4>(P, G, slot_a, slot_c, dry, s);
+int launch_bwd_head_bf16_d4(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, BwdHeadUse* use, hipStream_t s) {
+    return bwdh::launch<bf16, 4>(P, G, slot_a, slot_c, use, s);
 }
 }  // namespace ma

@@ -2,7 +2,7 @@
 #include "ma_bwd_head.h"
 
 namespace ma {
-int launch_bwd_head_f16_d2(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, bool dry, hipStream_t s) {
-    return bwdh::launch<f16, 2>(P, G, slot_a, slot_c, dry, s);
+int launch_bwd_head_f16_d2(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, BwdHeadUse* use, hipStream_t s) {
+    return bwdh::launch<f16, 2>(P, G, slot_a, slot_c, use, s);
 }
 }  // namespace ma

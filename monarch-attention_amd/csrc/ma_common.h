@@ -176,15 +176,18 @@ int launch_bwd_tile_f32_d8(const Problem& P, const BwdBuffers& G, int stage, boo
 int launch_bwd_tile(const Problem& P, const BwdBuffers& G, int dt, int stage, bool first, bool with_v, hipStream_t s);
 
 // The whole backward pass of short heads in one launch (ma_bwd_head.h): 16-bit q, k, v of one type, D % 8 == 0, rows16, D <= 96,
-// B, M <= 32, the gradients of a head's state in LDS.  slot_a, slot_c: bytes from a step's aL / aR and cL / cR to the next step's.  dry: only
-// report whether the problem fits.
-int launch_bwd_head_bf16_d2(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, bool dry, hipStream_t s);
-int launch_bwd_head_bf16_d4(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, bool dry, hipStream_t s);
-int launch_bwd_head_bf16_d6(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, bool dry, hipStream_t s);
-int launch_bwd_head_f16_d2(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, bool dry, hipStream_t s);
-int launch_bwd_head_f16_d4(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, bool dry, hipStream_t s);
-int launch_bwd_head_f16_d6(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, bool dry, hipStream_t s);
-int launch_bwd_head(const Problem& P, const BwdBuffers& G, int dt, unsigned long long slot_a, unsigned long long slot_c, bool dry, hipStream_t s);
+// B, M <= 32, the gradients of a head's state in LDS.  slot_a, slot_c: bytes from a step's aL / aR and cL / cR to the next step's.  use: only
+// report whether the problem fits, and which fp32 rows in memory it uses.
+struct BwdHeadUse {
+    bool dq, dk;
+};
+int launch_bwd_head_bf16_d2(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, BwdHeadUse* use, hipStream_t s);
+int launch_bwd_head_bf16_d4(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, BwdHeadUse* use, hipStream_t s);
+int launch_bwd_head_bf16_d6(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, BwdHeadUse* use, hipStream_t s);
+int launch_bwd_head_f16_d2(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, BwdHeadUse* use, hipStream_t s);
+int launch_bwd_head_f16_d4(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, BwdHeadUse* use, hipStream_t s);
+int launch_bwd_head_f16_d6(const Problem& P, const BwdBuffers& G, unsigned long long slot_a, unsigned long long slot_c, BwdHeadUse* use, hipStream_t s);
+int launch_bwd_head(const Problem& P, const BwdBuffers& G, int dt, unsigned long long slot_a, unsigned long long slot_c, BwdHeadUse* use, hipStream_t s);
 bool bwd_state16_ok(const Problem& P, int dt_qk, int dt_v);
 // partial buffers the R stage wants for this problem (0: it does not split blocks over workgroups)
 int bwd_r_split_tiles(const Problem& P, int dt_qk, int dt_v);

@@ -29,12 +29,12 @@ int launch_bwd_tile(const Problem& P, const BwdBuffers& G, int dt, int stage, bo
     return f(P, G, stage, first, with_v, s);
 }
 
-int launch_bwd_head(const Problem& P, const BwdBuffers& G, int dt, unsigned long long slot_a, unsigned long long slot_c, bool dry, hipStream_t s) {
+int launch_bwd_head(const Problem& P, const BwdBuffers& G, int dt, unsigned long long slot_a, unsigned long long slot_c, BwdHeadUse* use, hipStream_t s) {
     const int D = P.D;
     if (D > 96) return MA_ERR_UNSUPPORTED;   // (heads of ~ 160 tokens at D = 128: 0.98 - 1.08 of the stage launches' time)
     auto* f = dt == MA_F16 ? (D <= 32 ? launch_bwd_head_f16_d2 : D <= 64 ? launch_bwd_head_f16_d4 : launch_bwd_head_f16_d6)
                            : (D <= 32 ? launch_bwd_head_bf16_d2 : D <= 64 ? launch_bwd_head_bf16_d4 : launch_bwd_head_bf16_d6);
-    return f(P, G, slot_a, slot_c, dry, s);
+    return f(P, G, slot_a, slot_c, use, s);
 }
 
 int launch_long(const Problem& P, int dt, int stage, bool first, bool with_v, hipStream_t s) {

@@ -621,6 +621,18 @@ def test_workspaces_hold_what_the_path_uses():
     assert lib.ma_matrix_workspace_bytes(params(2, 0, "generic").fwd) == lib.ma_fwd_workspace_bytes(params(2, 0).fwd)
 
 
+def test_workspace_of_the_one_launch_backward():
+    """fp32 rows of dq and dk only where they go through memory: dq from ~ 270 tokens of 64 columns on, dk where a wave's strips of it outgrow
+    64 registers, with more than one step.  dv and the state's gradients never do."""
+    lib = L.load()
+    for heads, N, D, B, T, arrays in ((768, 197, 64, 14, 2, 0), (192, 512, 64, 32, 2, 1), (256, 512, 64, 32, 1, 1), (192, 1000, 32, 32, 2, 1),
+                                      (192, 250, 96, 16, 2, 1), (192, 480, 64, 24, 3, 2), (224, 243, 48, 32, 2, 0), (16 * 16, 323, 96, 17, 1, 1)):
+        b = call_params(heads, N, D, B, T)
+        assert lib.ma_bwd_kernel_name(b) == b"head_bwd"
+        rows = heads * -(-N // B) * B
+        assert arrays * rows * D * 4 <= lib.ma_bwd_kept_workspace_bytes(b) <= arrays * rows * D * 4 + 16 * 256, (heads, N, D, B, T)
+
+
 @pytest.mark.parametrize("variant,D,dt", [("staged", 8, L.MA_F16), ("staged", 8, L.MA_F32), ("generic", 3, L.MA_F16), ("sliced", 32, L.MA_F16)])
 def test_launches_of_more_than_2_to_the_32_work_items_are_refused(variant, D, dt):
     """The runtime would run some of the workgroups and report nothing.  2^27 heads of one token."""
